@@ -360,16 +360,14 @@ __device__ __forceinline__ void tracer_update(const GridDesc &g, const SweepArgs
 // Update of one cell by the flux difference along DIR (calcRightHandSide.hpp:288-549,
 // Cartesian, with the area correction of :156-194 applied to both faces first).  XTRA
 // compiles in the optional per-cell work (passive tracers); without it the kernels carry
-// no trace of the options.
+// no trace of the options.  p is the cell's index, A the area of its faces along DIR.
 template <class C, int DIR, bool XTRA, bool FIN = false, typename T>
-__device__ __forceinline__ double cell_update(const GridDesc &g, const SweepArgs &a, int k,
-                                              int j, int i, const T *Fm, const T *Fp,
-                                              T cmaxm, T cmaxp,
+__device__ __forceinline__ double cell_update(const GridDesc &g, const SweepArgs &a, unsigned p,
+                                              double A, int k, int j, int i, const T *Fm,
+                                              const T *Fp, T cmaxm, T cmaxp,
                                               const double *u0pre = nullptr,
                                               const double *upre = nullptr) {
-  const unsigned p = (unsigned)idx3(g, k, j, i);
   const double dtdV = a.uniform ? a.dtdV : a.dt / cell_dV<C::DIM>(g, k, j, i);
-  const double A = face_A<C::DIM, DIR>(g, k, j, i);
   double u[C::NVAR];
   if (a.flags & (SW_INIT_UC | SW_SAVE_UC0)) {
     double u0[C::NVAR];
@@ -440,16 +438,17 @@ __device__ __forceinline__ double cell_update(const GridDesc &g, const SweepArgs
   if constexpr (XTRA) {
     if (g.ntr > 0) tracer_update<C, DIR>(g, a, p, dtdV, A, (double)Fm[C::RHO], (double)Fp[C::RHO]);
   }
-  const int ig = DIR == 0 ? i : DIR == 1 ? j : k;
-  const double dl = g.dx[DIR][ig];
-  const double term = 0.5 * ((double)cmaxp + (double)cmaxm) / (dl);
   double inv = 0.0;
-  if (a.flags & SW_INVDT_SET) {
-    inv = term;
-    if (!(a.flags & SW_NO_INVDT_STORE)) st32(a.InvDt, p, inv);
-  } else if (a.flags & SW_INVDT_ADD) {
-    inv = ld32((const double *)a.InvDt, p) + term;
-    st32(a.InvDt, p, inv);
+  if (a.flags & (SW_INVDT_SET | SW_INVDT_ADD)) {
+    const int ig = DIR == 0 ? i : DIR == 1 ? j : k;
+    const double dl = g.dx[DIR][ig];
+    inv = 0.5 * ((double)cmaxp + (double)cmaxm) / (dl);
+    if (a.flags & SW_INVDT_SET) {
+      if (!(a.flags & SW_NO_INVDT_STORE)) st32(a.InvDt, p, inv);
+    } else {
+      inv = ld32((const double *)a.InvDt, p) + inv;
+      st32(a.InvDt, p, inv);
+    }
   }
   return inv;
 }
@@ -539,7 +538,8 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e,
       const bool cell_ok = lane >= 1 && lane <= 62 && c < g.end[0] && j >= g.beg[1] &&
                            j < g.end[1] && k >= g.beg[2] && k < g.end[2];
       if (cell_ok) {
-        const double inv = cell_update<C, IDIR, XTRA>(g, a, k, j, c, F, Fp, cmax, cmaxp);
+        const double inv = cell_update<C, IDIR, XTRA>(g, a, p, face_A<C::DIM, IDIR>(g, k, j, c), k,
+                                                      j, c, F, Fp, cmax, cmaxp);
         red = __double_as_longlong(inv);
       }
     }
@@ -550,14 +550,20 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e,
 }
 
 // ------------------------------------------------------------------------------------
-// y / z sweeps: marching along DIR with the stencil window in registers
+// y / z sweeps: marching along DIR with the stencil window in registers.  The columns of
+// the transverse plane are numbered with x fastest and dealt to the lanes 64 at a time
+// across row ends: blocks of 64 along x would leave a row of 130 columns (128 cells and
+// their extension) with 48 % idle lanes in its three waves, one of 514 with 11 % (whole
+// cycles: Orszag-Tang 128^3 1453 -> 1263 us, turbulence 512^3 133.4 -> 123.6 ms).
 // ------------------------------------------------------------------------------------
 struct MarchGeom {
   int ilo, ihi;   // x range (interior +- extension)
   int tlo, thi;   // range of the other transverse direction
   int ts;         // cells per segment along DIR
   int nseg;       // segments along DIR
-  int nxb;        // 64-wide x blocks
+  int nxb;        // 64-wide x blocks (k_fused2d_y)
+  int ncb;        // blocks of 64 columns (k_sweep_march)
+  int grp;        // column blocks whose segments are adjacent in launch order
 };
 
 // The stencil rows consecutive marching steps share are carried in LDS for the 3-cell
@@ -582,29 +588,35 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
   constexpr int H = NW / 2;
   const int lane = threadIdx.x & 63;
   const int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int ntr = m.thi - m.tlo;
+  const int ni = m.ihi - m.ilo;
+  const int ncol = ni * (m.thi - m.tlo);
+  // wave -> (column block, segment): groups of grp column blocks (about one x row), the
+  // segments of a group next to each other
+  const int cb = w / (m.grp * m.nseg) * m.grp + w % m.grp;
+  const int seg = w / m.grp % m.nseg;
   unsigned long long red = 0;
-  if (w < m.nxb * ntr * m.nseg) {
-    const int xb = w % m.nxb;
-    const int rest = w / m.nxb;
-    const int seg = rest % m.nseg;
-    const int tr = m.tlo + rest / m.nseg;
-    const int i = m.ilo + xb * 64 + lane;
-    const bool lane_ok = i < m.ihi;
-    const int ic = lane_ok ? i : m.ihi - 1;
+  if (cb < m.ncb) {
+    // a lane's column in the transverse plane, x fastest
+    const int t = cb * 64 + lane;
+    const bool lane_ok = t < ncol;
+    const int tc = lane_ok ? t : ncol - 1;
+    const int i = m.ilo + tc % ni;
+    const int tr = m.tlo + tc / ni;
     const int c0 = g.beg[DIR] + seg * m.ts;
     const int c1 = min(c0 + m.ts, g.end[DIR]);
     // stride along DIR and base offset of the column
     const unsigned sd = (DIR == JDIR) ? g.nt[0] : (unsigned)g.nt[0] * g.nt[1];
     const int jj = (DIR == JDIR) ? 0 : tr;  // j for the z sweep
     const int kk = (DIR == JDIR) ? tr : 0;  // k for the y sweep
-    const unsigned col = (unsigned)idx3(g, kk, jj, ic);  // index with DIR coordinate = 0
+    const unsigned col = (unsigned)idx3(g, kk, jj, i);  // index with DIR coordinate = 0
+    // area of the column's faces along DIR (constant along the column)
+    const double A = face_A<C::DIM, DIR>(g, kk, jj, i);
     const bool rhs_lane = lane_ok && i >= g.beg[0] && i < g.end[0] &&
                           ((DIR == JDIR) ? (tr >= g.beg[2] && tr < g.end[2])
                                          : (tr >= g.beg[1] && tr < g.end[1]));
     // Vs normal component: stride along DIR in the Vs array
     const unsigned vsd = (DIR == JDIR) ? g.vsn[0] : (unsigned)g.vsn[0] * g.vsn[1];
-    const unsigned vcol = (unsigned)idxs(g, 0, kk, jj, ic);
+    const unsigned vcol = (unsigned)idxs(g, 0, kk, jj, i);
     const double *VsDir = a.Vs + DIR * g.svs;  // the normal component
 
     constexpr bool CARRY = march_lds_window<C>();
@@ -724,9 +736,10 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
       } else {
         if (f > c0 && rhs_lane) {
           const int cf = f - 1;
-          const int ci = ic, cj = (DIR == JDIR) ? cf : jj, ck = (DIR == JDIR) ? kk : cf;
-          const double inv = cell_update<C, DIR, XTRA, FIN>(g, a, ck, cj, ci, Fprev, F, cprev,
-                                                            cmax, u0pre, PRE_U ? upre : nullptr);
+          const int cj = (DIR == JDIR) ? cf : jj, ck = (DIR == JDIR) ? kk : cf;
+          const double inv = cell_update<C, DIR, XTRA, FIN>(
+              g, a, col + (unsigned)cf * sd, A, ck, cj, i, Fprev, F, cprev, cmax, u0pre,
+              PRE_U ? upre : nullptr);
           const unsigned long long b = __double_as_longlong(inv);
           red = b > red ? b : red;
         }

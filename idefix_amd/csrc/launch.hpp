@@ -108,14 +108,16 @@ hipError_t launch_sweep_xtra(const GridDesc &g, const SweepArgs &a, const EmfArr
     constexpr int OT = (DIR == JDIR) ? 2 : 1;  // the other transverse direction
     m.tlo = g.beg[OT] - a.ext[OT];
     m.thi = g.end[OT] + a.ext[OT];
-    m.nxb = (m.ihi - m.ilo + 63) / 64;
+    m.nxb = 0;
+    m.ncb = (int)(((long long)(m.ihi - m.ilo) * (m.thi - m.tlo) + 63) / 64);
+    m.grp = std::min(m.ncb, (m.ihi - m.ilo + 63) / 64);
     const int nd = g.end[DIR] - g.beg[DIR];
-    const long long columns = (long long)m.nxb * (m.thi - m.tlo);
+    const long long columns = m.ncb;
     static const long long slots =
         resident_waves(k_sweep_march<C, T, DIR, FUSED, EMF, XTRA, FIN>, target_waves);
     m.ts = march_segment(columns, nd, slots);
     m.nseg = (nd + m.ts - 1) / m.ts;
-    const long long waves = columns * m.nseg;
+    const long long waves = (columns + m.grp - 1) / m.grp * m.grp * m.nseg;
     hipLaunchKernelGGL((k_sweep_march<C, T, DIR, FUSED, EMF, XTRA, FIN>), dim3(blocks_for(waves, 4)),
                        dim3(256), 0, s, g, a, e, m);
   }
