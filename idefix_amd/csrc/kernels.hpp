@@ -202,6 +202,29 @@ __device__ __forceinline__ void store_face_emf(const EmfArrays<T> &e, unsigned p
 // face) and right-face value `vr` (the left state of its right face), exactly as
 // ExtrapolatePrimVar computes them for the two faces (extrapolateToFaces.hpp:88-124,
 // :247-306).
+//
+// PPM: recon_face gives the value of the cell's right face, recon_ppm the states from the
+// window and the two face values.
+template <class C, typename T>
+__device__ __forceinline__ T recon_face(const T *w) {
+  if constexpr (C::ORDER == RECON_PPM) return ppm_face(w[1], w[2], w[3], w[4]);
+  else return T(0);
+}
+template <class C, typename T>
+__device__ __forceinline__ void recon_ppm(const T *w, int nv, T fl, T fr, T &vl, T &vr) {
+  const PpmStates<T> s = ppm_cell(w[0], w[1], w[2], w[3], w[4], fl, fr);
+  T l = s.l, r = s.r;
+  if (nv == C::RHO || nv == C::ENG) {
+    // van Leer fallback of extrapolateToFaces.hpp:260-304
+    if (r <= T(0) || l <= T(0)) {
+      const T dv = vanleer(w[3] - w[2], w[2] - w[1]);
+      r = (r <= T(0)) ? w[2] + T(0.5) * dv : r;
+      l = (l <= T(0)) ? w[2] - T(0.5) * dv : l;
+    }
+  }
+  vl = l;
+  vr = r;
+}
 template <class C, typename T>
 __device__ __forceinline__ void recon_cell(const T *w, int nv, T &vl, T &vr, T dxc = T(0),
                                            bool flat = false) {
@@ -235,16 +258,7 @@ __device__ __forceinline__ void recon_cell(const T *w, int nv, T &vl, T &vr, T d
     vr = r;
   } else {
     // w[0..4] = V(c-2) .. V(c+2)
-    T l, r;
-    ppm_states(w[0], w[1], w[2], w[3], w[4], l, r);
-    if (nv == C::RHO || nv == C::ENG) {
-      // van Leer fallback of extrapolateToFaces.hpp:260-304 (value selects, see ppm_states)
-      const T dv = vanleer(w[3] - w[2], w[2] - w[1]);
-      r = (r <= T(0)) ? w[2] + T(0.5) * dv : r;
-      l = (l <= T(0)) ? w[2] - T(0.5) * dv : l;
-    }
-    vl = l;
-    vr = r;
+    recon_ppm<C>(w, nv, ppm_face(w[0], w[1], w[2], w[3]), ppm_face(w[1], w[2], w[3], w[4]), vl, vr);
   }
 }
 template <class C>
@@ -633,8 +647,9 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
           if (s >= 1) lds[((c0 - 1 - H + s) & 1) * NV + n][tid] = win[s][n];
         }
       }
-    // right-face value of cell c0-1: the left state of the first face
-    T carry[NV], Fprev[NV], cprev = 0;
+    // right state of cell c0-1: the left state of the first face; PPM also hands on the
+    // value of its right face, the left face of the next cell
+    T carry[NV], Fprev[NV], fcar[NV], cprev = 0;
 #pragma unroll
     for (int n = 0; n < NV; n++) Fprev[n] = 0;
 #pragma unroll
@@ -643,9 +658,12 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
 #pragma unroll
       for (int s = 0; s < NW; s++) wv[s] = win[s][n];
       T dummy;
+      if (C::MHD && n == C::template BXn<DIR>()) { carry[n] = fcar[n] = wv[H]; continue; }
       if constexpr (C::ORDER == RECON_MLP) {
-        if (C::MHD && n == C::template BXn<DIR>()) { carry[n] = wv[H]; continue; }
         recon_mlp<C, DIR>(wv, n, a.mlpw, g.sv, col + (unsigned)(c0 - 1) * sd, sd, dummy, carry[n]);
+      } else if constexpr (C::ORDER == RECON_PPM) {
+        fcar[n] = recon_face<C>(wv);
+        recon_ppm<C>(wv, n, ppm_face(wv[0], wv[1], wv[2], wv[3]), fcar[n], dummy, carry[n]);
       } else {
         recon_cell<C>(wv, n, dummy, carry[n], recon_dx<C, T>(g, DIR, c0 - 1),
                       XTRA && recon_flat<C>(a, col + (unsigned)(c0 - 1) * sd));
@@ -702,16 +720,20 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
         T wv[NW];
 #pragma unroll
         for (int s = 0; s < NW; s++) wv[s] = win[s][n];
+        vL[n] = carry[n];
+        if (C::MHD && n == C::template BXn<DIR>()) {  // the normal field comes from Vs
+          vR[n] = vr_next[n] = wv[H];
+          continue;
+        }
         if constexpr (C::ORDER == RECON_MLP) {
-          if (C::MHD && n == C::template BXn<DIR>()) {
-            vR[n] = vr_next[n] = wv[H];
-          } else {
-            recon_mlp<C, DIR>(wv, n, a.mlpw, g.sv, col + (unsigned)f * sd, sd, vR[n], vr_next[n]);
-          }
+          recon_mlp<C, DIR>(wv, n, a.mlpw, g.sv, col + (unsigned)f * sd, sd, vR[n], vr_next[n]);
+        } else if constexpr (C::ORDER == RECON_PPM) {
+          const T fr = recon_face<C>(wv);
+          recon_ppm<C>(wv, n, fcar[n], fr, vR[n], vr_next[n]);
+          fcar[n] = fr;
         } else {
           recon_cell<C>(wv, n, vR[n], vr_next[n], recon_dx<C, T>(g, DIR, f), flat);
         }
-        vL[n] = carry[n];
       }
       if constexpr (C::MHD) {
         constexpr int BXn = C::template BXn<DIR>();
@@ -865,10 +887,12 @@ __device__ __forceinline__ T edge_term(const T *b, const T *v, T aL, T aR, T dL,
                                        bool plus) {
   T bL, bR, vL, vR, d;
   if constexpr (C::ORDER == RECON_PPM) {
-    ppm_states(b[1], b[2], b[3], b[4], b[5], d, bL);
-    ppm_states(b[2], b[3], b[4], b[5], b[6], bR, d);
-    ppm_states(v[1], v[2], v[3], v[4], v[5], d, vL);
-    ppm_states(v[2], v[3], v[4], v[5], v[6], vR, d);
+    // the left cell's right state and the right cell's left state share the edge's face
+    const T fb = ppm_face(b[2], b[3], b[4], b[5]), fv = ppm_face(v[2], v[3], v[4], v[5]);
+    bL = ppm_cell(b[1], b[2], b[3], b[4], b[5], ppm_face(b[1], b[2], b[3], b[4]), fb).r;
+    bR = ppm_cell(b[2], b[3], b[4], b[5], b[6], fb, ppm_face(b[3], b[4], b[5], b[6])).l;
+    vL = ppm_cell(v[1], v[2], v[3], v[4], v[5], ppm_face(v[1], v[2], v[3], v[4]), fv).r;
+    vR = ppm_cell(v[2], v[3], v[4], v[5], v[6], fv, ppm_face(v[3], v[4], v[5], v[6])).l;
   } else {
     d = mclim(b[4] - b[3], b[3] - b[2]);
     bL = b[3] + T(0.5) * d;
