@@ -227,6 +227,9 @@ SweepArgs sweep_args(idfx_ctx *c, int dir, double dt, const double *Vc, const do
     if (c->d.dim >= 2) v = v * c->dx0[1];
     if (c->d.dim >= 3) v = v * c->dx0[2];
     a.dtdV = dt / v;
+    a.areax = 1.0;  // with the association of face_A
+    if (c->d.dim >= 2) a.areax = a.areax * c->dx0[1];
+    if (c->d.dim >= 3) a.areax = a.areax * c->dx0[2];
   } else {
     a.dtdV = 0.0;
   }

@@ -74,6 +74,7 @@ struct SweepArgs {
   unsigned long long *dtmax;  // bit pattern of max(InvDt) (non-negative doubles)
   int uniform;    // all cells share one volume: dtdV below equals dt/dV(k,j,i)
   double dtdV;
+  double areax;   // likewise the area of an x face
   const float *mlpw;  // learned-limiter interface weights of this direction (RECON_MLP)
   const unsigned char *shock;  // shock flags per cell (shock flattening) or nullptr
   double *VcOut;      // SW_FINAL: output primitive state
@@ -468,54 +469,91 @@ __device__ __forceinline__ double cell_update(const GridDesc &g, const SweepArgs
 }
 
 // ------------------------------------------------------------------------------------
-// x sweep: one cell per lane.  Lane l reconstructs cell c = i0 - 1 + l once; face c
-// takes its left state from lane l-1 (a cross-lane shuffle) and its right state from the
-// lane itself, and cell c takes the flux of face c+1 from lane l+1.  A wave therefore
-// solves 63 faces and updates the 62 cells between them.
+// x sweep: one cell per lane.  Lane l reconstructs its cell c once; face c takes its left
+// state from lane l-1 (a cross-lane shuffle) and its right state from the lane itself, and
+// cell c takes the flux of face c+1 from lane l+1.  With PPM the value of a cell's left
+// face comes from lane l-1 too, which computed it as its right face.
+//
+// The sites of all rows (a row: its cells and those its first face needs) are numbered
+// through and a wave takes 64 consecutive ones across row ends, 1 + XF of them shared with
+// the next wave: it solves the faces of the lanes XF .. 62 and updates their cells.  Rows
+// cut into waves of their own would leave 31 % of the lanes idle at 128 cells a row, 8 %
+// at 512 (whole cycles: Orszag-Tang 128^3 1252 -> 1209 us, turbulence 203x150x97 3123 ->
+// 3009 us, 2-D 256^2 235 -> 226 us, 512^3 unchanged).
 // ------------------------------------------------------------------------------------
-// occupancy target of the x sweep: 4 waves per SIMD (<= 128 VGPRs).  The 8-variable MHD
-// states spill a little at 128 (2-D; 3-D PPM in FP64: 36 B per lane) but still run faster
-// than at 3 waves (3-D PPM HLLD at 512^3: 11.7 against 12.4 ms); the other 3-D
-// reconstructions in FP64 spill more (up to 64 B) and stay at 3.
+// Lanes before the first face a wave solves: the cell on its left, and with PPM the cell
+// whose right face is that cell's left one.
+template <class C>
+constexpr int x_first() {
+  return C::ORDER == RECON_PPM ? 2 : 1;
+}
+// n / d for n < 2^31 by one high product: m = ceil(2^(31 + l) / d), s = l - 1, l = ceil(log2 d)
+// (Granlund and Montgomery 1994); d = 1 has m = 0.
+struct FastDiv {
+  unsigned d, m, s;
+};
+__device__ __forceinline__ unsigned fast_div(unsigned n, const FastDiv &f) {
+  return f.m == 0 ? n : __umulhi(n, f.m) >> f.s;
+}
+struct XGeom {
+  FastDiv ns;  // sites per row: cells beg - XF .. end
+  FastDiv nj;  // rows per plane
+  int nsites;  // sites of all rows
+};
+// occupancy target of the x sweep: 4 waves per SIMD (<= 128 VGPRs) where the state fits
+// with few spills; the 8-variable MHD state with PPM spills at 128 and runs faster at 3
+// (turbulence 512^3: 10.1 against 11.1 ms a launch; 2-D 256^2: 16.1 against 18.0 us), as do
+// the other 3-D reconstructions.
 template <class C>
 constexpr int x_waves_per_eu() {
-  return (C::DIM == 3 && C::ORDER != RECON_PPM) ? 3 : 4;
+  return (C::DIM == 3 && C::ORDER != RECON_PPM) || (C::MHD && C::NVAR >= 8 && C::ORDER == RECON_PPM) ? 3 : 4;
 }
 template <class C, typename T, bool FUSED, int EMF, bool XTRA>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(x_waves_per_eu<C>())))
-void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e,
-                                                 int nseg) {
+void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
   constexpr int NV = C::NVAR;
   constexpr int NW = window<C>();
   constexpr int H = NW / 2;
+  constexpr int XF = x_first<C>();
   const int lane = threadIdx.x & 63;
   const int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int nj = g.end[1] - g.beg[1] + 2 * a.ext[1];
-  const int nk = g.end[2] - g.beg[2] + 2 * a.ext[2];
-  const bool wave_ok = w < nseg * nj * nk;
   unsigned long long red = 0;
-  if (wave_ok) {
-    const int seg = w % nseg;
-    const int r = w / nseg;
-    const int j = g.beg[1] - a.ext[1] + r % nj;
-    const int k = g.beg[2] - a.ext[2] + r / nj;
-    const int c = g.beg[0] - 1 + seg * 62 + lane;  // this lane's cell; its left face is c-1/2
-    const int cc = c <= g.end[0] ? c : g.end[0];     // clamped for the loads
+  const int first = w * (63 - XF);  // the wave's first site
+  if (first + XF < m.nsites) {
+    // lanes past the last site repeat it; none of their faces or cells is theirs
+    const bool lane_ok = first + lane < m.nsites;
+    const unsigned site = (unsigned)min(first + lane, m.nsites - 1);
+    const unsigned r = C::DIM >= 2 ? fast_div(site, m.ns) : 0;
+    const unsigned rk = C::DIM >= 3 ? fast_div(r, m.nj) : 0;
+    const int c = g.beg[0] - XF + (int)(site - r * m.ns.d);  // this lane's cell; its left face is c-1/2
+    const int j = g.beg[1] - a.ext[1] + (int)(r - rk * m.nj.d);
+    const int k = g.beg[2] - a.ext[2] + (int)rk;
     const unsigned row = (unsigned)idx3(g, k, j, 0);
+    const unsigned p = row + (unsigned)c;
 
     // reconstruct the lane's cell: vl = right state of face c, vr = left state of face c+1
     T vl[NV], vr[NV];
-    const bool flat = XTRA && recon_flat<C>(a, row + (unsigned)cc);
+    const bool flat = XTRA && recon_flat<C>(a, p);
 #pragma unroll
     for (int n = 0; n < NV; n++) {
+      if (C::MHD && n == C::BX1) {  // the normal field comes from Vs
+        vl[n] = vr[n] = T(0);
+        continue;
+      }
       T wv[NW];
 #pragma unroll
-      for (int s = 0; s < NW; s++) wv[s] = (T)ld32(a.Vc + n * g.sv, row + (unsigned)(cc - H + s));
+      for (int s = 0; s < NW; s++) {
+        // a row's first PPM site only gives its right face: V(c-2) may lie outside
+        const unsigned q = (XF == 2 && s == 0) ? row + (unsigned)max(c - H, 0) : p + (unsigned)(s - H);
+        wv[s] = (T)ld32(a.Vc + n * g.sv, q);
+      }
       if constexpr (C::ORDER == RECON_MLP) {
-        if (C::MHD && n == C::BX1) { vl[n] = vr[n] = wv[H]; continue; }  // normal field: Vs
-        recon_mlp<C, IDIR>(wv, n, a.mlpw, g.sv, row + (unsigned)cc, 1u, vl[n], vr[n]);
+        recon_mlp<C, IDIR>(wv, n, a.mlpw, g.sv, p, 1u, vl[n], vr[n]);
+      } else if constexpr (C::ORDER == RECON_PPM) {
+        const T fr = recon_face<C>(wv);
+        recon_ppm<C>(wv, n, __shfl_up(fr, 1), fr, vl[n], vr[n]);
       } else {
-        recon_cell<C>(wv, n, vl[n], vr[n], recon_dx<C, T>(g, 0, cc), flat);
+        recon_cell<C>(wv, n, vl[n], vr[n], recon_dx<C, T>(g, 0, c), flat);
       }
     }
     T vL[NV], vR[NV];
@@ -525,16 +563,13 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e,
       vR[n] = vl[n];
     }
     if constexpr (C::MHD) {
-      vL[C::BX1] = (T)ld32(a.Vs, (unsigned)idxs(g, 0, k, j, cc));
+      vL[C::BX1] = (T)ld32(a.Vs, (unsigned)idxs(g, 0, k, j, c));
       vR[C::BX1] = vL[C::BX1];
     }
     T F[NV], cmax;
     FaceEmf<T> E;
-    const bool wrote = riemann<C, IDIR>(vL, vR, F, cmax, E, EMF,
-                                        eos_face<C, T>(g, row + (unsigned)(cc - 1), row + (unsigned)cc));
-    const bool face_ok = lane >= 1 && c <= g.end[0];
-    const bool own_face = face_ok && (lane <= 62 || c == g.end[0]);
-    const unsigned p = row + (unsigned)c;
+    const bool wrote = riemann<C, IDIR>(vL, vR, F, cmax, E, EMF, eos_face<C, T>(g, p - 1u, p));
+    const bool own_face = lane_ok && lane >= XF && lane <= 62 && c >= g.beg[0];
     if (own_face) store_face_emf<C, IDIR>(e, p, EMF, E);
     if constexpr (!FUSED) {
       if (own_face) {
@@ -549,11 +584,11 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e,
 #pragma unroll
       for (int n = 0; n < NV; n++) Fp[n] = __shfl_down(F[n], 1);
       const T cmaxp = __shfl_down(cmax, 1);
-      const bool cell_ok = lane >= 1 && lane <= 62 && c < g.end[0] && j >= g.beg[1] &&
-                           j < g.end[1] && k >= g.beg[2] && k < g.end[2];
+      const bool cell_ok = own_face && c < g.end[0] && j >= g.beg[1] && j < g.end[1] &&
+                           k >= g.beg[2] && k < g.end[2];
       if (cell_ok) {
-        const double inv = cell_update<C, IDIR, XTRA>(g, a, p, face_A<C::DIM, IDIR>(g, k, j, c), k,
-                                                      j, c, F, Fp, cmax, cmaxp);
+        const double A = a.uniform ? a.areax : face_A<C::DIM, IDIR>(g, k, j, c);
+        const double inv = cell_update<C, IDIR, XTRA>(g, a, p, A, k, j, c, F, Fp, cmax, cmaxp);
         red = __double_as_longlong(inv);
       }
     }

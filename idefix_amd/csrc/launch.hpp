@@ -90,17 +90,31 @@ inline int march_segment(long long columns, int nd, long long slots) {
   return bt;
 }
 
+inline FastDiv fast_div_of(unsigned d) {
+  FastDiv f{d, 0, 0};
+  if (d > 1) {
+    unsigned l = 0;  // ceil(log2 d)
+    while ((1ULL << l) < d) l++;
+    f.m = (unsigned)(((1ULL << (31 + l)) + d - 1) / d);
+    f.s = l - 1;
+  }
+  return f;
+}
+
 template <class C, typename T, int DIR, bool FUSED, int EMF, bool XTRA, bool FIN = false>
 hipError_t launch_sweep_xtra(const GridDesc &g, const SweepArgs &a, const EmfArrays<T> &e,
                             int target_waves, hipStream_t s) {
   if constexpr (DIR == IDIR) {
-    const int nint = g.end[0] - g.beg[0];
-    const int nseg = (nint + 61) / 62;
-    const long long nj = g.end[1] - g.beg[1] + 2 * a.ext[1];
-    const long long nk = g.end[2] - g.beg[2] + 2 * a.ext[2];
-    const long long waves = (long long)nseg * nj * nk;
+    constexpr int XF = x_first<C>();
+    const unsigned nj = (unsigned)(g.end[1] - g.beg[1] + 2 * a.ext[1]);
+    const unsigned nk = (unsigned)(g.end[2] - g.beg[2] + 2 * a.ext[2]);
+    XGeom m;
+    m.ns = fast_div_of((unsigned)(g.end[0] - g.beg[0] + XF + 1));
+    m.nj = fast_div_of(nj);
+    m.nsites = (int)(m.ns.d * nj * nk);  // below 2^31: a block has fewer than 2^29 cells
+    const long long waves = (m.nsites - XF + 62 - XF) / (63 - XF);
     hipLaunchKernelGGL((k_sweep_x<C, T, FUSED, EMF, XTRA>), dim3(blocks_for(waves, 4)), dim3(256), 0, s, g,
-                       a, e, nseg);
+                       a, e, m);
   } else {
     MarchGeom m;
     m.ilo = g.beg[0] - a.ext[0];

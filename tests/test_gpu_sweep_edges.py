@@ -1,0 +1,58 @@
+"""Sweeps at the sizes where their lane mapping can go wrong: the sites of an x sweep and the
+columns of a y or z sweep are dealt to waves of 64 lanes across row ends, so rows shorter
+than a wave, rows that end at or next to a wave's last lanes, and last waves with one site
+are compared with the oracle cell by cell (FP64 bar of tests/pairs.py)."""
+import pytest
+
+from idefix_amd import problems
+from tests.pairs import cfg_kwargs, compare_state, make_pair
+
+pytestmark = pytest.mark.gpu
+
+# a wave of the x sweep solves 62 sites (PLM) or 61 (PPM); a row holds nx + 2 or nx + 3
+SIZES_3D = [(4, 5, 3), (7, 4, 6), (58, 3, 4), (59, 4, 3), (61, 3, 3), (64, 3, 4), (121, 3, 3),
+            (125, 4, 3), (130, 3, 3), (3, 33, 18)]
+
+
+@pytest.mark.parametrize("recon,nstages", [("plm", 2), ("ppm", 3)])
+@pytest.mark.parametrize("n", SIZES_3D)
+def test_mhd_3d(n, recon, nstages):
+    kw = cfg_kwargs(3, n, emf="uct_contact", recon=recon, nstages=nstages, cfl=0.3)
+    o, g = make_pair(kw, problems.random_mhd)
+    o.set_boundaries()
+    assert o.cycle() == 0
+    g.cycle()
+    compare_state(o, g, what="%s %s" % (recon, n))
+    assert g.dt == pytest.approx(o.dt, rel=1e-12)
+
+
+@pytest.mark.parametrize("recon", ["plm", "ppm"])
+@pytest.mark.parametrize("n", [(5, 40), (58, 9), (60, 7), (122, 6), (128, 5)])
+def test_mhd_2d_three_components(n, recon):
+    kw = cfg_kwargs(2, n, comps=3, emf="uct_contact", recon=recon, nstages=3, cfl=0.3)
+    o, g = make_pair(kw, problems.random_mhd)
+    o.set_boundaries()
+    assert o.cycle() == 0
+    g.cycle()
+    compare_state(o, g, what="%s %s" % (recon, n))
+
+
+@pytest.mark.parametrize("recon", ["plm", "ppm"])
+@pytest.mark.parametrize("n", [(3,), (59,), (61,), (62,), (123,), (124,), (125,), (1000,)])
+def test_hd_1d(n, recon):
+    kw = cfg_kwargs(1, n, mhd=False, solver="hllc", recon=recon, bc="outflow", gamma=1.4, cfl=0.3)
+    o, g = make_pair(kw, problems.random_hd)
+    o.set_boundaries()
+    assert o.cycle() == 0
+    g.cycle()
+    compare_state(o, g, what="%s %s" % (recon, n))
+
+
+@pytest.mark.parametrize("n", [(3, 4, 5), (60, 5, 4), (62, 3, 3), (64, 4, 4)])
+def test_hd_3d_outflow(n):
+    kw = cfg_kwargs(3, n, mhd=False, solver="hllc", recon="plm", bc="outflow", gamma=1.4, cfl=0.3)
+    o, g = make_pair(kw, problems.random_hd)
+    o.set_boundaries()
+    assert o.cycle() == 0
+    g.cycle()
+    compare_state(o, g, what="%s" % (n,))
