@@ -62,15 +62,64 @@ template <typename T> __device__ __forceinline__ T fab(T a) { return fabs(a); }
 __device__ __forceinline__ float fmn(float a, float b) { return fminf(a, b); }
 __device__ __forceinline__ float fmx(float a, float b) { return fmaxf(a, b); }
 __device__ __forceinline__ float fab(float a) { return fabsf(a); }
-template <typename T> __device__ __forceinline__ T sqrt_(T a) { return sqrt(a); }
 __device__ __forceinline__ float sqrt_(float a) { return sqrtf(a); }
+
+// Division and square root, correctly rounded, without the scaling steps of the compiler's
+// own expansion (two div_scale, a div_fmas that waits for VCC, two ldexp) and with the
+// reciprocal of a denominator refined once for all its quotients: v_rcp, two Newton steps,
+// then per quotient a product, its exact remainder and one correction (Markstein 1990).
+// div_fixup gives zero, infinite and NaN operands their IEEE results.  Equal to a / b bit
+// for bit while the denominator and the quotient are normal and the numerator is zero or
+// at least 2^-969 (its remainder is then exact; below, the last bit of a quotient may
+// differ), to sqrt(x) for x = 0 or x >= 2^-767.  An HLLD face has 20 quotients with 12
+// denominators and 6 square roots; whole cycles: Orszag-Tang 512^2 147 -> 139 us, 128^3 1209
+// -> 1164 us, turbulence 203x150x97 3009 -> 2950 us.
+template <typename T>
+struct Recip {
+  T b, r;  // denominator, refined reciprocal
+};
+__device__ __forceinline__ Recip<double> recip(double b) {
+  double r = __builtin_amdgcn_rcp(b);
+  r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+  r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+  return {b, r};
+}
+__device__ __forceinline__ double quot(double a, const Recip<double> &d) {
+  double q = a * d.r;
+  q = __builtin_fma(__builtin_fma(-d.b, q, a), d.r, q);
+  return __builtin_amdgcn_div_fixup(q, d.b, a);
+}
+__device__ __forceinline__ Recip<float> recip(float b) {
+  float r = __builtin_amdgcn_rcpf(b);
+  r = __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
+  return {b, r};
+}
+__device__ __forceinline__ float quot(float a, const Recip<float> &d) {
+  float q = a * d.r;
+  q = __builtin_fmaf(__builtin_fmaf(-d.b, q, a), d.r, q);
+  q = __builtin_fmaf(__builtin_fmaf(-d.b, q, a), d.r, q);
+  return __builtin_amdgcn_div_fixupf(q, d.b, a);
+}
+__device__ __forceinline__ double div_(double a, double b) { return quot(a, recip(b)); }
+// a single quotient in FP32: the compiler's, whose scaling FP32's range may need
+__device__ __forceinline__ float div_(float a, float b) { return a / b; }
+__device__ __forceinline__ double sqrt_(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = __builtin_fma(-h, g, 0.5);
+  h = __builtin_fma(h, e, h);
+  g = __builtin_fma(g, e, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return (x == 0.0 || x == __builtin_inf()) ? x : g;
+}
 
 // ------------------------------------------------------------------------------------
 // Slope limiters: src/fluid/RiemannSolver/slopeLimiter.hpp
 // ------------------------------------------------------------------------------------
 template <typename T>
 __device__ __forceinline__ T vanleer(T dvp, T dvm) {  // slopeLimiter.hpp:54-57
-  return (dvp * dvm > T(0) ? T(2) * dvp * dvm / (dvp + dvm) : T(0));
+  return (dvp * dvm > T(0) ? div_(T(2) * dvp * dvm, dvp + dvm) : T(0));
 }
 template <typename T>
 __device__ __forceinline__ T mclim(T dvp, T dvm) {  // slopeLimiter.hpp:67-75
@@ -133,7 +182,7 @@ __device__ __forceinline__ float flip(float x, float s) {
 template <typename T, bool FAST>
 __device__ __forceinline__ T ppm_div(T a, T b) {
   if constexpr (FAST) return a * __builtin_amdgcn_rcpf(b);
-  else return a / b;
+  else return div_(a, b);
 }
 template <typename T, bool FAST = false>
 __device__ __forceinline__ T ppm_face(T vm1, T v0, T vp1, T vp2) {
@@ -195,8 +244,9 @@ __device__ __forceinline__ void ppm_states(T vm2, T vm1, T v0, T vp1, T vp2, T &
 // ------------------------------------------------------------------------------------
 // Pointwise conversions: src/fluid/convertConsToPrim.hpp, eos_adiabatic.hpp:39-45
 // ------------------------------------------------------------------------------------
+// gm1: gamma - 1
 template <class C, typename T>
-__device__ __forceinline__ void prim2cons(const T *v, T *u, T gamma) {
+__device__ __forceinline__ void prim2cons(const T *v, T *u, const Recip<T> &gm1) {
   // K_PrimToCons, convertConsToPrim.hpp:69-100
   u[C::RHO] = v[C::RHO];
   u[C::MX1] = v[C::MX1] * v[C::RHO];
@@ -212,7 +262,7 @@ __device__ __forceinline__ void prim2cons(const T *v, T *u, T gamma) {
     T v2 = v[C::MX1] * v[C::MX1];
     if constexpr (C::COMP >= 2) v2 = v2 + v[C::MX2] * v[C::MX2];
     if constexpr (C::COMP >= 3) v2 = v2 + v[C::MX3] * v[C::MX3];
-    const T eint = v[C::ENG] / (gamma - T(1.0));
+    const T eint = quot(v[C::ENG], gm1);
     if constexpr (C::MHD) {
       u[C::BX1] = v[C::BX1];
       if constexpr (C::COMP >= 2) u[C::BX2] = v[C::BX2];
@@ -227,15 +277,21 @@ __device__ __forceinline__ void prim2cons(const T *v, T *u, T gamma) {
   }
 }
 
+template <class C, typename T>
+__device__ __forceinline__ void prim2cons(const T *v, T *u, T gamma) {
+  prim2cons<C>(v, u, recip(gamma - T(1.0)));
+}
+
 // K_ConsToPrim, convertConsToPrim.hpp:15-67: always evaluated in FP64 (the
 // energy-to-pressure recovery suffers cancellation at low plasma beta).
 // SMALL_PRESSURE_FIX = 1e-5 (fluid_defs.hpp:23); the re-synced energy is local.
 template <class C>
 __device__ __forceinline__ void cons2prim(const double *u, double *v, double gamma) {
   v[C::RHO] = u[C::RHO];
-  v[C::MX1] = u[C::MX1] / u[C::RHO];
-  if constexpr (C::COMP >= 2) v[C::MX2] = u[C::MX2] / u[C::RHO];
-  if constexpr (C::COMP >= 3) v[C::MX3] = u[C::MX3] / u[C::RHO];
+  const Recip<double> rho = recip(u[C::RHO]);
+  v[C::MX1] = quot(u[C::MX1], rho);
+  if constexpr (C::COMP >= 2) v[C::MX2] = quot(u[C::MX2], rho);
+  if constexpr (C::COMP >= 3) v[C::MX3] = quot(u[C::MX3], rho);
   if constexpr (C::ISO) {
     if constexpr (C::MHD) {
       v[C::BX1] = u[C::BX1];
@@ -246,7 +302,7 @@ __device__ __forceinline__ void cons2prim(const double *u, double *v, double gam
     double m2 = u[C::MX1] * u[C::MX1];
     if constexpr (C::COMP >= 2) m2 = m2 + u[C::MX2] * u[C::MX2];
     if constexpr (C::COMP >= 3) m2 = m2 + u[C::MX3] * u[C::MX3];
-    const double kin = 0.5 / u[C::RHO] * m2;
+    const double kin = quot(0.5, rho) * m2;
     if constexpr (C::MHD) {
       v[C::BX1] = u[C::BX1];
       if constexpr (C::COMP >= 2) v[C::BX2] = u[C::BX2];
@@ -271,13 +327,14 @@ template <class C>
 __device__ __forceinline__ void cons2prim_part(const double *u, double *v) {
   static_assert(C::MHD && !C::ISO, "the split conversion is for adiabatic MHD");
   v[C::RHO] = u[C::RHO];
-  v[C::MX1] = u[C::MX1] / u[C::RHO];
-  if constexpr (C::COMP >= 2) v[C::MX2] = u[C::MX2] / u[C::RHO];
-  if constexpr (C::COMP >= 3) v[C::MX3] = u[C::MX3] / u[C::RHO];
+  const Recip<double> rho = recip(u[C::RHO]);
+  v[C::MX1] = quot(u[C::MX1], rho);
+  if constexpr (C::COMP >= 2) v[C::MX2] = quot(u[C::MX2], rho);
+  if constexpr (C::COMP >= 3) v[C::MX3] = quot(u[C::MX3], rho);
   double m2 = u[C::MX1] * u[C::MX1];
   if constexpr (C::COMP >= 2) m2 = m2 + u[C::MX2] * u[C::MX2];
   if constexpr (C::COMP >= 3) m2 = m2 + u[C::MX3] * u[C::MX3];
-  const double kin = 0.5 / u[C::RHO] * m2;
+  const double kin = quot(0.5, rho) * m2;
   v[C::ENG] = u[C::ENG] - kin;
 }
 template <class C>
@@ -354,15 +411,17 @@ __device__ __forceinline__ void hllc_hd(const T *vL, const T *vR, T *flux, T &cm
   constexpr int Xt = C::template Xt<DIR>();
   constexpr int Xb = C::template Xb<DIR>();
   T uL[NV], uR[NV], fL[NV], fR[NV];
-  const T cL = sqrt_(gamma * (vL[C::ENG] / vL[C::RHO]));
-  const T cR = sqrt_(gamma * (vR[C::ENG] / vR[C::RHO]));
+  const Recip<T> rhoL = recip(vL[C::RHO]), rhoR = recip(vR[C::RHO]);
+  const T cL = sqrt_(gamma * quot(vL[C::ENG], rhoL));
+  const T cR = sqrt_(gamma * quot(vR[C::ENG], rhoR));
   const T cminL = vL[Xn] - cL, cmaxL = vL[Xn] + cL;
   const T cminR = vR[Xn] - cR, cmaxR = vR[Xn] + cR;
   const T SL = fmn(cminL, cminR);
   const T SR = fmx(cmaxL, cmaxR);
   cmax = fmx(fab(SL), fab(SR));
-  prim2cons<C>(vL, uL, gamma);
-  prim2cons<C>(vR, uR, gamma);
+  const Recip<T> gm1 = recip(gamma - T(1));
+  prim2cons<C>(vL, uL, gm1);
+  prim2cons<C>(vR, uR, gm1);
   kflux<C, DIR>(fL, vL, uL);
   kflux<C, DIR>(fR, vR, uR);
   if (SL > T(0)) {
@@ -377,9 +436,9 @@ __device__ __forceinline__ void hllc_hd(const T *vL, const T *vR, T *flux, T &cm
     const T qR = vR[C::ENG] + uR[Xn] * (vR[Xn] - SR);
     const T wL = vL[C::RHO] * (vL[Xn] - SL);
     const T wR = vR[C::RHO] * (vR[Xn] - SR);
-    const T vs = (qR - qL) / (wR - wL);
-    usL[C::RHO] = uL[C::RHO] * (SL - vL[Xn]) / (SL - vs);
-    usR[C::RHO] = uR[C::RHO] * (SR - vR[Xn]) / (SR - vs);
+    const T vs = div_(qR - qL, wR - wL);
+    usL[C::RHO] = div_(uL[C::RHO] * (SL - vL[Xn]), SL - vs);
+    usR[C::RHO] = div_(uR[C::RHO] * (SR - vR[Xn]), SR - vs);
     usL[Xn] = usL[C::RHO] * vs;
     usR[Xn] = usR[C::RHO] * vs;
     if constexpr (C::COMP >= 2) {
@@ -390,10 +449,10 @@ __device__ __forceinline__ void hllc_hd(const T *vL, const T *vR, T *flux, T &cm
       usL[Xb] = usL[C::RHO] * vL[Xb];
       usR[Xb] = usR[C::RHO] * vR[Xb];
     }
-    usL[C::ENG] = uL[C::ENG] / vL[C::RHO] +
-                  (vs - vL[Xn]) * (vs + vL[C::ENG] / (vL[C::RHO] * (SL - vL[Xn])));
-    usR[C::ENG] = uR[C::ENG] / vR[C::RHO] +
-                  (vs - vR[Xn]) * (vs + vR[C::ENG] / (vR[C::RHO] * (SR - vR[Xn])));
+    usL[C::ENG] = quot(uL[C::ENG], rhoL) +
+                  (vs - vL[Xn]) * (vs + div_(vL[C::ENG], vL[C::RHO] * (SL - vL[Xn])));
+    usR[C::ENG] = quot(uR[C::ENG], rhoR) +
+                  (vs - vR[Xn]) * (vs + div_(vR[C::ENG], vR[C::RHO] * (SR - vR[Xn])));
     usL[C::ENG] *= usL[C::RHO];
     usR[C::ENG] *= usR[C::RHO];
     if (vs >= T(0)) {
@@ -570,7 +629,9 @@ __device__ __forceinline__ bool roe_hd(const T *vL, const T *vR, T *flux, T &cma
 template <typename T>
 struct StarPre {
   bool valid;
-  T duL, duR, scrh, Sc, usLRHO, usRRHO, sqrL, sqrR;
+  T duL, duR, scrh, Sc, usLRHO, usRRHO;
+  Recip<T> slS, srS;    // sl - Sc, sr - Sc
+  Recip<T> sqrL, sqrR;  // square roots of the star densities
 };
 
 template <class C, int DIR, typename T>
@@ -580,12 +641,14 @@ __device__ __forceinline__ void star_pre(const T *vL, const T *vR, const T *uL, 
   P.valid = true;
   P.duL = sl - vL[Xn];
   P.duR = sr - vR[Xn];
-  P.scrh = T(1) / (P.duR * uR[C::RHO] - P.duL * uL[C::RHO]);
+  P.scrh = div_(T(1), P.duR * uR[C::RHO] - P.duL * uL[C::RHO]);
   P.Sc = (P.duR * uR[Xn] - P.duL * uL[Xn] - ptR + ptL) * P.scrh;
-  P.usLRHO = uL[C::RHO] * P.duL / (sl - P.Sc);
-  P.usRRHO = uR[C::RHO] * P.duR / (sr - P.Sc);
-  P.sqrL = sqrt_(P.usLRHO);
-  P.sqrR = sqrt_(P.usRRHO);
+  P.slS = recip(sl - P.Sc);
+  P.srS = recip(sr - P.Sc);
+  P.usLRHO = quot(uL[C::RHO] * P.duL, P.slS);
+  P.usRRHO = quot(uR[C::RHO] * P.duR, P.srS);
+  P.sqrL = recip(sqrt_(P.usLRHO));
+  P.sqrR = recip(sqrt_(P.usRRHO));
 }
 
 // Face data for constrained transport (storeFlux.hpp:14-208) with the signs of
@@ -621,7 +684,7 @@ __device__ __forceinline__ void store_face_emf(const T *vL, const T *vR, const T
   } else if (emf == EMF_UCT_HLL) {
     const T ar = fmx(T(0), sr);
     const T al = fmn(T(0), sl);
-    const T scrh = T(1) / (ar - al);
+    const T scrh = div_(T(1), ar - al);
     if constexpr (CO > 1) {
       E.Et = -st * (ar * vL[Xt] - al * vR[Xt]) * scrh;
       if constexpr (CO >= 3) E.Eb = -sb * (ar * vL[Xb] - al * vR[Xb]) * scrh;
@@ -633,7 +696,7 @@ __device__ __forceinline__ void store_face_emf(const T *vL, const T *vR, const T
   } else {
     // K_StoreHLLD, storeFlux.hpp:77-208 (HAVE_ENERGY branch)
     bool revert_to_hll = false;
-    const T Bn = (sr * vR[BXn] - sl * vL[BXn]) / (sr - sl);
+    const T Bn = div_(sr * vR[BXn] - sl * vL[BXn], sr - sl);
     T scrh, Sc, SaL, SaR;
     if constexpr (C::ISO) {
       // storeFlux.hpp:139-147: one averaged density across the fan
@@ -648,16 +711,16 @@ __device__ __forceinline__ void store_face_emf(const T *vL, const T *vR, const T
       StarPre<T> P = pre;
       if (!P.valid) star_pre<C, DIR>(vL, vR, uL, uR, sl, sr, ptL, ptR, P);
       Sc = P.Sc;
-      SaL = Sc - fab(Bn) / P.sqrL;
-      SaR = Sc + fab(Bn) / P.sqrR;
+      SaL = Sc - quot(fab(Bn), P.sqrL);
+      SaR = Sc + quot(fab(Bn), P.sqrR);
     }
     if ((SaL - sl) < T(1e-4) * (Sc - sl)) revert_to_hll = true;
     if ((SaR - sr) > -T(1e-4) * (sr - Sc)) revert_to_hll = true;
-    const T chiL = (vL[Xn] - Sc) * (sl - Sc) / (SaL + sl - T(2) * Sc);
-    const T chiR = (vR[Xn] - Sc) * (sr - Sc) / (SaR + sr - T(2) * Sc);
-    const T nuL = (SaL + sl) / (fab(SaL) + fab(sl));
-    const T nuR = (SaR + sr) / (fab(SaR) + fab(sr));
-    const T nuLR = (SaL + SaR) / (fab(SaL) + fab(SaR));
+    const T chiL = div_((vL[Xn] - Sc) * (sl - Sc), SaL + sl - T(2) * Sc);
+    const T chiR = div_((vR[Xn] - Sc) * (sr - Sc), SaR + sr - T(2) * Sc);
+    const T nuL = div_(SaL + sl, fab(SaL) + fab(sl));
+    const T nuR = div_(SaR + sr, fab(SaR) + fab(sr));
+    const T nuLR = div_(SaL + SaR, fab(SaL) + fab(SaR));
     if (fab(SaR - SaL) > T(1.e-9) * fab(sr - sl)) {
       E.dL = T(0.5) * (chiL * nuL - chiL * nuLR) + T(0.5) * (fab(SaL) - nuLR * SaL);
       E.dR = T(0.5) * (chiR * nuR - chiR * nuLR) + T(0.5) * (fab(SaR) - nuLR * SaR);
@@ -671,7 +734,7 @@ __device__ __forceinline__ void store_face_emf(const T *vL, const T *vR, const T
     }
     const T ar = fmx(T(0), sr);
     const T al = fmn(T(0), sl);
-    scrh = T(1) / (ar - al);
+    scrh = div_(T(1), ar - al);
     if (revert_to_hll) {
       E.aL = ar * scrh;
       E.aR = -al * scrh;
@@ -713,7 +776,7 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
     T Bmag2 = b1 * b1 + Btmag2;
     cL = gpr - Bmag2;
     cL = gpr + Bmag2 + sqrt_(cL * cL + T(4) * gpr * Btmag2);
-    cL = sqrt_(T(0.5) * cL / vL[C::RHO]);
+    cL = sqrt_(div_(T(0.5) * cL, vL[C::RHO]));
   }
   {
     T gpr = gamma * vR[C::ENG];
@@ -724,7 +787,7 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
     T Bmag2 = b1 * b1 + Btmag2;
     cR = gpr - Bmag2;
     cR = gpr + Bmag2 + sqrt_(cR * cR + T(4) * gpr * Btmag2);
-    cR = sqrt_(T(0.5) * cR / vR[C::RHO]);
+    cR = sqrt_(div_(T(0.5) * cR, vR[C::RHO]));
   }
   const T cminL = vL[Xn] - cL, cmaxL = vL[Xn] + cL;
   const T cminR = vR[Xn] - cR, cmaxR = vR[Xn] + cR;
@@ -732,8 +795,9 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
   const T sr = fmx(cmaxL, cmaxR);
   cmax = fmx(fab(sl), fab(sr));
 
-  prim2cons<C>(vL, uL, gamma);
-  prim2cons<C>(vR, uR, gamma);
+  const Recip<T> gm1 = recip(gamma - T(1));
+  prim2cons<C>(vL, uL, gm1);
+  prim2cons<C>(vR, uR, gm1);
   kflux<C, DIR>(fluxL, vL, uL);
   kflux<C, DIR>(fluxR, vR, uR);
 
@@ -760,7 +824,7 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
     T scrh, scrhL, scrhR, duL, duR, sBx, Bx, SM, S1L, S1R, pts, sqrL, sqrR;
     T vsL = 0, vsR = 0, wsL = 0, wsR = 0;
     bool revert_to_hllc = false;
-    scrh = T(1) / (sr - sl);
+    scrh = div_(T(1), sr - sl);
     Bx = (sr * vR[BXn] - sl * vL[BXn]) * scrh;
     sBx = (Bx > T(0) ? T(1) : T(-1));
     StarPre<T> P = pre;
@@ -774,14 +838,14 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
     pts *= scrh;
     usL[C::RHO] = P.usLRHO;
     usR[C::RHO] = P.usRRHO;
-    sqrL = P.sqrL;
-    sqrR = P.sqrR;
-    S1L = SM - fab(Bx) / sqrL;
-    S1R = SM + fab(Bx) / sqrR;
+    sqrL = P.sqrL.b;
+    sqrR = P.sqrR.b;
+    S1L = SM - quot(fab(Bx), P.sqrL);
+    S1R = SM + quot(fab(Bx), P.sqrR);
     if ((S1L - sl) < T(1.e-4) * (SM - sl)) revert_to_hllc = true;
     if ((S1R - sr) > -T(1.e-4) * (sr - SM)) revert_to_hllc = true;
     if (revert_to_hllc) {
-      scrh = T(1) / (sr - sl);
+      scrh = div_(T(1), sr - sl);
       T Uhll_n, Uhll_t = 0, Uhll_b = 0;
       Uhll_n = (sr * uR[BXn] - sl * uL[BXn] + fluxL[BXn] - fluxR[BXn]) * scrh;
       if constexpr (CO >= 2) Uhll_t = (sr * uR[BXt] - sl * uL[BXt] + fluxL[BXt] - fluxR[BXt]) * scrh;
@@ -791,8 +855,8 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
       if constexpr (CO >= 3) usL[BXb] = usR[BXb] = Uhll_b;
       S1L = S1R = SM;
     } else {
-      scrhL = (uL[C::RHO] * duL * duL - Bx * Bx) / (uL[C::RHO] * duL * (sl - SM) - Bx * Bx);
-      scrhR = (uR[C::RHO] * duR * duR - Bx * Bx) / (uR[C::RHO] * duR * (sr - SM) - Bx * Bx);
+      scrhL = div_(uL[C::RHO] * duL * duL - Bx * Bx, uL[C::RHO] * duL * (sl - SM) - Bx * Bx);
+      scrhR = div_(uR[C::RHO] * duR * duR - Bx * Bx, uR[C::RHO] * duR * (sr - SM) - Bx * Bx);
       usL[BXn] = Bx;
       if constexpr (CO >= 2) usL[BXt] = uL[BXt] * scrhL;
       if constexpr (CO >= 3) usL[BXb] = uL[BXb] * scrhL;
@@ -800,8 +864,8 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
       if constexpr (CO >= 2) usR[BXt] = uR[BXt] * scrhR;
       if constexpr (CO >= 3) usR[BXb] = uR[BXb] * scrhR;
     }
-    scrhL = Bx / (uL[C::RHO] * duL);
-    scrhR = Bx / (uR[C::RHO] * duR);
+    scrhL = div_(Bx, uL[C::RHO] * duL);
+    scrhR = div_(Bx, uR[C::RHO] * duR);
     if constexpr (CO >= 2) {
       vsL = vL[Xt] - scrhL * (usL[BXt] - uL[BXt]);
       vsR = vR[Xt] - scrhR * (usR[BXt] - uR[BXt]);
@@ -829,8 +893,7 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
       if constexpr (CO >= 3) s = s + wsL * usL[BXb];
       scrhL -= s;
     }
-    usL[C::ENG] = duL * uL[C::ENG] - ptL * vL[Xn] + pts * SM + Bx * scrhL;
-    usL[C::ENG] /= sl - SM;
+    usL[C::ENG] = quot(duL * uL[C::ENG] - ptL * vL[Xn] + pts * SM + Bx * scrhL, P.slS);
     scrhR = vR[Xn] * Bx;
     if constexpr (CO >= 2) scrhR = scrhR + vR[Xt] * uR[BXt];
     if constexpr (CO >= 3) scrhR = scrhR + vR[Xb] * uR[BXb];
@@ -840,8 +903,7 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
       if constexpr (CO >= 3) s = s + wsR * usR[BXb];
       scrhR -= s;
     }
-    usR[C::ENG] = duR * uR[C::ENG] - ptR * vR[Xn] + pts * SM + Bx * scrhR;
-    usR[C::ENG] /= sr - SM;
+    usR[C::ENG] = quot(duR * uR[C::ENG] - ptR * vR[Xn] + pts * SM + Bx * scrhR, P.srS);
 
     if (S1L >= T(0)) {
 #pragma unroll
@@ -853,13 +915,14 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
       T vss = 0, wss = 0, ussl[NV], ussr[NV];
       ussl[C::RHO] = usL[C::RHO];
       ussr[C::RHO] = usR[C::RHO];
+      const Recip<T> sq = recip(sqrL + sqrR);
       if constexpr (CO >= 2) {
         vss = sqrL * vsL + sqrR * vsR + (usR[BXt] - usL[BXt]) * sBx;
-        vss /= sqrL + sqrR;
+        vss = quot(vss, sq);
       }
       if constexpr (CO >= 3) {
         wss = sqrL * wsL + sqrR * wsR + (usR[BXb] - usL[BXb]) * sBx;
-        wss /= sqrL + sqrR;
+        wss = quot(wss, sq);
       }
       ussl[Xn] = ussl[C::RHO] * SM;
       ussr[Xn] = ussr[C::RHO] * SM;
@@ -874,12 +937,12 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
       ussl[BXn] = ussr[BXn] = Bx;
       if constexpr (CO >= 2) {
         ussl[BXt] = sqrL * usR[BXt] + sqrR * usL[BXt] + sqrL * sqrR * (vsR - vsL) * sBx;
-        ussl[BXt] /= sqrL + sqrR;
+        ussl[BXt] = quot(ussl[BXt], sq);
         ussr[BXt] = ussl[BXt];
       }
       if constexpr (CO >= 3) {
         ussl[BXb] = sqrL * usR[BXb] + sqrR * usL[BXb] + sqrL * sqrR * (wsR - wsL) * sBx;
-        ussl[BXb] /= sqrL + sqrR;
+        ussl[BXb] = quot(ussl[BXb], sq);
         ussr[BXb] = ussl[BXb];
       }
       scrhL = SM * Bx;
