@@ -1,6 +1,7 @@
-// Training of the learned limiter: hand-written FP32 kernels for the forward pass, the
-// loss, the backward pass, the weight-gradient reductions and Adam, behind the C ABI of
-// include/idefix_amd.h (idfx_mlp_*).  No counterpart in the reference.
+// Training of the learned limiter: hand-written FP32 kernels behind the C ABI of
+// include/idefix_amd.h (idfx_mlp_*).  No counterpart in the reference.  A step is two
+// kernels: k_train (forward, loss, backward and the weight gradients of a block's rows,
+// FP32 matrix cores) and k_reduce (sums the blocks' gradients and applies Adam).
 //
 // Parameters are packed as in oracle/mlp.py: W1 [48][64], b1 [64], W2 [64][64], b2 [64],
 // W3 [64][16], b3 [16] (row-major [in][out]), 8336 floats.  A batch row of X holds
@@ -24,147 +25,275 @@ constexpr int P_W1 = 0, P_B1 = P_W1 + NF * NH, P_W2 = P_B1 + NH, P_B2 = P_W2 + N
               P_W3 = P_B2 + NH, P_B3 = P_W3 + NH * NO, P_N = P_B3 + NO;
 constexpr float GELU_K = 1.702f;
 constexpr int ROW = 72, ROW_WP = 48, ROW_OM = 64;  // batch row: features | wp | om
-constexpr int WG_ROWS = 512;  // rows per block of the weight-gradient reduction
+constexpr int TR = 32;            // rows of a tile: two waves of 16
+constexpr int MAX_BLOCKS = 512;   // blocks of k_train: two per CU
 
 __device__ __forceinline__ float sig(float z) { return 1.0f / (1.0f + expf(-z)); }
-__device__ __forceinline__ float gelu(float z) { return z * sig(GELU_K * z); }
-__device__ __forceinline__ float gelu_d(float z) {
-  const float s = sig(GELU_K * z);
+// derivative of z s with s = sig(GELU_K z)
+__device__ __forceinline__ float gelu_d(float z, float s) {
   return s + GELU_K * z * s * (1.0f - s);
 }
 
-// Z = A W + b, H = gelu(Z) (or Z when act == 0); A has K columns in rows of lda floats;
-// one thread per (row, output unit).
-__global__ __launch_bounds__(256) void k_dense_fwd(const float *A, int K, int lda, const float *W,
-                                                   const float *b, int N, float *Z, float *H,
-                                                   int act, int B) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)B * N) return;
-  const int r = (int)(t / N), j = (int)(t % N);
-  float z = b[j];
-  for (int k = 0; k < K; k++) z += A[(long long)r * lda + k] * W[k * N + j];
-  Z[t] = z;
-  if (H) H[t] = act ? gelu(z) : z;
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // batch rows: any float address
+
+// D += A B on 16x16x4 FP32 matrix instructions: lane 16 g + q gives A[q][g] and B[g][q]
+// and holds D[4 g + r][q], r = 0 .. 3.
+__device__ __forceinline__ f4 mfma(float a, float b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Output layer: wL = wpL + z3[2v], wR = wpR - z3[2v], the row's loss, and dZ3 = dloss/dz3 (1/B included).
-__global__ __launch_bounds__(256) void k_out_loss(const float *Z3, const float *X,
-                                                  const float *TAU, int B, float *dZ3,
-                                                  float *rowloss) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= B) return;
-  float l = 0.0f;
-  const float inv = 1.0f / (float)B;
-  const float *xr = X + (long long)r * ROW;
-  for (int v = 0; v < 8; v++) {
-    const float x2 = xr[6 * v + 2], x3 = xr[6 * v + 3];
-    const float d = x3 - x2;
-    const float tau = TAU[(long long)r * 8 + v];
-    const float om2 = xr[ROW_OM + v] * xr[ROW_OM + v];
-    const float z = Z3[(long long)r * NO + 2 * v];
-    const float wl = xr[ROW_WP + 2 * v] + z;
-    const float wr = xr[ROW_WP + 2 * v + 1] - z;
-    const float el = x2 + wl * d - tau;
-    const float er = x3 - wr * d - tau;
-    l += om2 * (el * el + er * er);
-    dZ3[(long long)r * NO + 2 * v] = om2 * 2.0f * (el + er) * d * inv;
-    dZ3[(long long)r * NO + 2 * v + 1] = 0.0f;
+// LDS, in floats.  Weights, rows padded so that a lane's four consecutive inputs come in
+// one 16-byte read without bank conflicts (row strides of an odd number of 16-byte units):
+// transposed [out][in] for the forward pass, [in][out] for the backward pass.  The tile's
+// activations and deltas [row][unit] take their place for the weight gradients (strides of
+// 16 mod 32 floats).
+constexpr int L_WT1 = 0, S_WT1 = 52, L_WT2 = L_WT1 + NH * S_WT1, S_W2 = 68,
+              L_W2 = L_WT2 + NH * S_W2, L_WT3 = L_W2 + NH * S_W2, L_W3 = L_WT3 + NO * S_W2,
+              S_W3 = 20, L_B = L_W3 + NH * S_W3, L_END = L_B + 2 * NH + NO;
+constexpr int S_X = 48, S_H = 80, S_O = 16, L_X = 0, L_H1 = L_X + TR * S_X,
+              L_H2 = L_H1 + TR * S_H, L_D1 = L_H2 + TR * S_H, L_D2 = L_D1 + TR * S_H,
+              L_D3 = L_D2 + TR * S_H;
+static_assert(L_D3 + TR * S_O <= L_END, "the gradient buffers reuse the weights' space");
+
+// acc[t] += W[16 t + .][16 NI units] in over the inputs in[NI] (units 16 i + 4 g + r of the
+// lane's row in in[i][r]); w is the lane's row of the weights, rows 16 apart by 16 stride.
+template <int NT, int NI>
+__device__ __forceinline__ void layer(const float *w, int stride, const f4 *in, f4 *acc) {
+#pragma unroll
+  for (int i = 0; i < NI; i++) {
+    f4 a[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) a[t] = *reinterpret_cast<const f4 *>(w + 16 * t * stride + 16 * i);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int t = 0; t < NT; t++) acc[t] = mfma(a[t][r], in[i][r], acc[t]);
   }
-  rowloss[r] = l;
 }
 
-// dZp = (dZ W^T) * gelu'(Zp); one thread per (row, input unit).
-__global__ __launch_bounds__(256) void k_dense_bwd(const float *dZ, int N, const float *W,
-                                                   int K, const float *Zp, float *dZp, int B) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)B * K) return;
-  const int r = (int)(t / K), k = (int)(t % K);
-  float s = 0.0f;
-  for (int j = 0; j < N; j++) s += dZ[(long long)r * N + j] * W[k * N + j];
-  dZp[t] = s * gelu_d(Zp[t]);
-}
-
-// Partial weight and bias gradients of one layer over WG_ROWS rows per block (A has K
-// columns in rows of lda floats):
-// out[blk][off + k N + n] = sum_r A[r][k] dZ[r][n] (k < K), out[blk][off + K N + n] =
-// sum_r dZ[r][n].
-__global__ __launch_bounds__(256) void k_wgrad(const float *A, int K, int lda, const float *dZ,
-                                               int N, int B, float *partial, int off) {
-  __shared__ float sa[16][NH + 1];
-  __shared__ float sz[16][NH];
-  const int total = (K + 1) * N;
-  float acc[17];
+// Forward pass, loss, backward pass and weight gradients of tiles of 32 rows.  A wave takes
+// 16 rows through all layers with the weights as the A operand and the activations as the
+// B operand: a layer's accumulator (unit 4 g + r of row q in lane 16 g + q) is the next
+// layer's B operand as it stands, so activations stay in registers.  For the gradients
+// (sums over rows) the activations and deltas pass through LDS, each wave computing half
+// of every layer's output tiles over all 32 rows; they accumulate in registers over the
+// block's tiles and go out once per block.  Everything is FP32 (products, accumulators,
+// activations).  208 + 128 matrix instructions per 16 rows: 2.2 us of the matrix cores'
+// time at 8192 rows; the kernel is bound by its serial chain of layers.  A step of 8192
+// rows takes 51 us; the eleven kernels this replaces (one thread per activation, scalar
+// products) took 716, 555 of them in the weight gradients.
+__global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU, int B,
+                                               const float *P, float *partial,
+                                               double *lossp) {
+  __shared__ __attribute__((aligned(16))) float lds[L_END];
+  __shared__ double lred[2];
+  const int tid = threadIdx.x, wave = tid >> 6, q = tid & 15, g = (tid >> 4) & 3;
+  f4 g1[3][2], g2[4][2], g3[2];
 #pragma unroll
-  for (int m = 0; m < 17; m++) acc[m] = 0.0f;
-  const int r0 = blockIdx.x * WG_ROWS;
-  const int r1 = min(r0 + WG_ROWS, B);
-  for (int rt = r0; rt < r1; rt += 16) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < 16 * NH; e += 256) {
-      const int rr = e / NH, c = e % NH;
-      const int r = rt + rr;
-      sa[rr][c] = (r < r1 && c < K) ? A[(long long)r * lda + c] : 0.0f;
-      sz[rr][c] = (r < r1 && c < N) ? dZ[(long long)r * N + c] : 0.0f;
+  for (int n = 0; n < 2; n++) {
+#pragma unroll
+    for (int m = 0; m < 3; m++) g1[m][n] = f4{0, 0, 0, 0};
+#pragma unroll
+    for (int m = 0; m < 4; m++) g2[m][n] = f4{0, 0, 0, 0};
+    g3[n] = f4{0, 0, 0, 0};
+  }
+  float gb = 0.0f, gb3 = 0.0f;  // bias gradients: unit tid of layers 1 | 2, unit tid of 3
+  double loss = 0.0;
+  const float inv = 1.0f / (float)B;
+  for (int tile = blockIdx.x; tile * TR < B; tile += gridDim.x) {
+    __syncthreads();  // the previous tile's gradient buffers have been read
+    for (int e = tid; e < NF * NH; e += 128) lds[L_WT1 + (e % NH) * S_WT1 + e / NH] = P[P_W1 + e];
+    for (int e = tid; e < NH * NH; e += 128) {
+      const float v = P[P_W2 + e];
+      lds[L_WT2 + (e % NH) * S_W2 + e / NH] = v;
+      lds[L_W2 + e / NH * S_W2 + e % NH] = v;
     }
-    if (threadIdx.x < 16) sa[threadIdx.x][NH] = (rt + threadIdx.x < r1) ? 1.0f : 0.0f;
+    for (int e = tid; e < NH * NO; e += 128) {
+      const float v = P[P_W3 + e];
+      lds[L_WT3 + (e % NO) * S_W2 + e / NO] = v;
+      lds[L_W3 + e / NO * S_W3 + e % NO] = v;
+    }
+    for (int e = tid; e < 2 * NH + NO; e += 128)
+      lds[L_B + e] = P[e < NH ? P_B1 + e : e < 2 * NH ? P_B2 + e - NH : P_B3 + e - 2 * NH];
     __syncthreads();
+
+    const int row = tile * TR + 16 * wave + q;
+    const bool ok = row < B;
+    const float *xr = X + (long long)(ok ? row : B - 1) * ROW;
+    f4 x[3], z1[4], z2[4], z3;
 #pragma unroll
-    for (int m = 0; m < 17; m++) {
-      const int e = threadIdx.x + 256 * m;
-      if (e < total) {
-        const int k = e / N, n = e % N;
-        const int kk = k < K ? k : NH;  // the bias row reads the ones column
-        float s = acc[m];
-        for (int rr = 0; rr < 16; rr++) s += sa[rr][kk] * sz[rr][n];
-        acc[m] = s;
+    for (int i = 0; i < 3; i++) x[i] = *reinterpret_cast<const f4u *>(xr + 16 * i + 4 * g);
+    // the lane's output variables 2 g and 2 g + 1
+    float x2[2], x3[2], d[2], om2[2], tau[2], wpl[2], wpr[2];
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+      const int v = 2 * g + n;
+      x2[n] = xr[6 * v + 2];
+      x3[n] = xr[6 * v + 3];
+      d[n] = x3[n] - x2[n];
+      const float om = xr[ROW_OM + v];
+      om2[n] = ok ? om * om : 0.0f;
+      wpl[n] = xr[ROW_WP + 2 * v];
+      wpr[n] = xr[ROW_WP + 2 * v + 1];
+      tau[n] = TAU[(long long)(ok ? row : B - 1) * 8 + v];
+    }
+    f4 s1[4], s2[4], h[4], h1[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) z1[t] = *reinterpret_cast<const f4 *>(lds + L_B + 16 * t + 4 * g);
+    layer<4, 3>(lds + L_WT1 + q * S_WT1 + 4 * g, S_WT1, x, z1);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        s1[t][r] = sig(GELU_K * z1[t][r]);
+        h1[t][r] = z1[t][r] * s1[t][r];
+      }
+#pragma unroll
+    for (int t = 0; t < 4; t++) z2[t] = *reinterpret_cast<const f4 *>(lds + L_B + NH + 16 * t + 4 * g);
+    layer<4, 4>(lds + L_WT2 + q * S_W2 + 4 * g, S_W2, h1, z2);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        s2[t][r] = sig(GELU_K * z2[t][r]);
+        h[t][r] = z2[t][r] * s2[t][r];
+      }
+    z3 = *reinterpret_cast<const f4 *>(lds + L_B + 2 * NH + 4 * g);
+    layer<1, 4>(lds + L_WT3 + q * S_W2 + 4 * g, S_W2, h, &z3);
+    // loss and dloss/dz3 (1/B included): wL = wpL + z3[2v], wR = wpR - z3[2v]
+    f4 d3 = f4{0, 0, 0, 0};
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+      const float z = z3[2 * n];
+      const float el = x2[n] + (wpl[n] + z) * d[n] - tau[n];
+      const float er = x3[n] - (wpr[n] - z) * d[n] - tau[n];
+      loss += (double)(om2[n] * (el * el + er * er));
+      d3[2 * n] = om2[n] * 2.0f * (el + er) * d[n] * inv;
+    }
+    f4 d2[4], d1[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const float *w3 = lds + L_W3 + (16 * t + q) * S_W3 + 4 * g;
+      d2[t] = mfma(w3[0], d3[0], f4{0, 0, 0, 0});
+      d2[t] = mfma(w3[2], d3[2], d2[t]);
+      d1[t] = f4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) d2[t][r] *= gelu_d(z2[t][r], s2[t][r]);
+    layer<4, 4>(lds + L_W2 + q * S_W2 + 4 * g, S_W2, d2, d1);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) d1[t][r] *= gelu_d(z1[t][r], s1[t][r]);
+    __syncthreads();  // both waves are done with the weights
+    {
+      const int rr = 16 * wave + q;
+#pragma unroll
+      for (int i = 0; i < 3; i++)
+        *reinterpret_cast<f4 *>(lds + L_X + rr * S_X + 16 * i + 4 * g) = x[i];
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const int o = rr * S_H + 16 * t + 4 * g;
+        *reinterpret_cast<f4 *>(lds + L_H1 + o) = h1[t];
+        *reinterpret_cast<f4 *>(lds + L_H2 + o) = h[t];
+        *reinterpret_cast<f4 *>(lds + L_D1 + o) = d1[t];
+        *reinterpret_cast<f4 *>(lds + L_D2 + o) = d2[t];
+      }
+      *reinterpret_cast<f4 *>(lds + L_D3 + rr * S_O + 4 * g) = d3;
+    }
+    __syncthreads();
+    // gradients: this wave's output units are the tiles 2 wave, 2 wave + 1 of layers 1 and
+    // 2; of layer 3 its input units are.  Rows past the batch have zero deltas.
+#pragma unroll
+    for (int k = 0; k < TR; k += 4) {
+      const float *b1 = lds + L_D1 + (k + g) * S_H + 32 * wave + q, *b2 = b1 + (L_D2 - L_D1);
+      const float *ax = lds + L_X + (k + g) * S_X + q, *ah = lds + L_H1 + (k + g) * S_H + q;
+      const float *a2 = lds + L_H2 + (k + g) * S_H + 32 * wave + q;
+      const float dz3 = lds[L_D3 + (k + g) * S_O + q];
+#pragma unroll
+      for (int n = 0; n < 2; n++) {
+#pragma unroll
+        for (int m = 0; m < 3; m++) g1[m][n] = mfma(ax[16 * m], b1[16 * n], g1[m][n]);
+#pragma unroll
+        for (int m = 0; m < 4; m++) g2[m][n] = mfma(ah[16 * m], b2[16 * n], g2[m][n]);
+        g3[n] = mfma(a2[16 * n], dz3, g3[n]);
       }
     }
+    for (int r = 0; r < TR; r++) {
+      gb += lds[(wave ? L_D2 : L_D1) + r * S_H + (tid & 63)];
+      if (tid < NO) gb3 += lds[L_D3 + r * S_O + tid];
+    }
   }
+  float *out = partial + (long long)blockIdx.x * P_N;
 #pragma unroll
-  for (int m = 0; m < 17; m++) {
-    const int e = threadIdx.x + 256 * m;
-    if (e < total) partial[(long long)blockIdx.x * P_N + off + e] = acc[m];
-  }
-}
-
-__global__ __launch_bounds__(256) void k_reduce_partials(const float *partial, int nblk,
-                                                         float *G) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= P_N) return;
-  float s = 0.0f;
-  for (int b = 0; b < nblk; b++) s += partial[(long long)b * P_N + e];
-  G[e] = s;
-}
-
-// Adam (Kingma & Ba 2015) with bias correction; step t is 1-based.
-__global__ __launch_bounds__(256) void k_adam(float *P, const float *G, float *M, float *V, int n,
-                                              float lr, float b1, float b2, float eps, float c1,
-                                              float c2) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const float g = G[e];
-  const float m = b1 * M[e] + (1.0f - b1) * g;
-  const float v = b2 * V[e] + (1.0f - b2) * g * g;
-  M[e] = m;
-  V[e] = v;
-  P[e] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
-}
-
-// Sum of the row losses into a device double (one block).
-__global__ __launch_bounds__(256) void k_sum_loss(const float *rowloss, int B, double *out) {
-  __shared__ double red[256];
-  double s = 0.0;
-  for (int r = threadIdx.x; r < B; r += 256) s += rowloss[r];
-  red[threadIdx.x] = s;
+  for (int n = 0; n < 2; n++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int col = 32 * wave + 16 * n + q, m0 = 4 * g + r;
+#pragma unroll
+      for (int m = 0; m < 3; m++) out[P_W1 + (16 * m + m0) * NH + col] = g1[m][n][r];
+#pragma unroll
+      for (int m = 0; m < 4; m++) out[P_W2 + (16 * m + m0) * NH + col] = g2[m][n][r];
+      out[P_W3 + (32 * wave + 16 * n + m0) * NO + q] = g3[n][r];
+    }
+  out[(wave ? P_B2 : P_B1) + (tid & 63)] = gb;
+  if (tid < NO) out[P_B3 + tid] = gb3;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
+  if ((tid & 63) == 0) lred[wave] = loss;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = red[0] / B;
+  if (tid == 0) lossp[blockIdx.x] = lred[0] + lred[1];
 }
 
-unsigned nblocks(long long n) { return (unsigned)((n + 255) / 256); }
+// G = sum of the blocks' gradients, 32 parameters per block of 256 threads (8 slices of the
+// blocks, then the slices, in a fixed order), and with ADAM the step (Kingma & Ba 2015,
+// bias correction c1, c2).  Block 0 also sums the loss.
+struct AdamArgs {
+  float lr, b1, b2, eps, c1, c2;
+};
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_reduce(const float *partial, const double *lossp,
+                                                int nblk, int B, float *G, double *loss,
+                                                float *P, float *M, float *V, AdamArgs a) {
+  __shared__ float red[8][32];
+  __shared__ double lred[256];
+  const int c = threadIdx.x & 31, sl = threadIdx.x >> 5;
+  const int e = blockIdx.x * 32 + c;
+  float s = 0.0f;
+  if (e < P_N)
+    for (int b = sl; b < nblk; b += 8) s += partial[(long long)b * P_N + e];
+  red[sl][c] = s;
+  __syncthreads();
+  if (sl == 0 && e < P_N) {
+    float gr = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; k++) gr += red[k][c];
+    G[e] = gr;
+    if constexpr (ADAM) {
+      const float m = a.b1 * M[e] + (1.0f - a.b1) * gr;
+      const float v = a.b2 * V[e] + (1.0f - a.b2) * gr * gr;
+      M[e] = m;
+      V[e] = v;
+      P[e] -= a.lr * (m / a.c1) / (sqrtf(v / a.c2) + a.eps);
+    }
+  }
+  if (blockIdx.x == 0) {
+    double l = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += 256) l += lossp[b];
+    lred[threadIdx.x] = l;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if ((int)threadIdx.x < w) lred[threadIdx.x] += lred[threadIdx.x + w];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) *loss = lred[0] / B;
+  }
+}
+
+int train_blocks(int B) { return std::min(MAX_BLOCKS, (B + TR - 1) / TR); }
 
 }  // namespace
 
@@ -173,8 +302,8 @@ struct idfx_mlp {
   long step = 0;
   std::vector<void *> allocs;
   float *P = nullptr, *G = nullptr, *M = nullptr, *V = nullptr;
-  float *Z1, *H1, *Z2, *H2, *Z3, *dZ3, *dZ2, *dZ1, *partial, *rowloss;
-  double *loss = nullptr;
+  float *partial = nullptr;                  // gradients per block of k_train
+  double *loss = nullptr, *lossp = nullptr;  // mean loss; loss sums per block
 };
 
 namespace {
@@ -188,30 +317,18 @@ int mlp_alloc(idfx_mlp *h, float **p, long long n) {
   return IDFX_OK;
 }
 
-// forward + loss + backward + gradient into h->G (asynchronous on s)
-int grad_enqueue(idfx_mlp *h, const float *X, const float *TAU, int B, hipStream_t s) {
-  const float *P = h->P;
-  hipLaunchKernelGGL(k_dense_fwd, dim3(nblocks((long long)B * NH)), dim3(256), 0, s, X, NF, ROW,
-                     P + P_W1, P + P_B1, NH, h->Z1, h->H1, 1, B);
-  hipLaunchKernelGGL(k_dense_fwd, dim3(nblocks((long long)B * NH)), dim3(256), 0, s, h->H1, NH,
-                     NH, P + P_W2, P + P_B2, NH, h->Z2, h->H2, 1, B);
-  hipLaunchKernelGGL(k_dense_fwd, dim3(nblocks((long long)B * NO)), dim3(256), 0, s, h->H2, NH,
-                     NH, P + P_W3, P + P_B3, NO, h->Z3, (float *)nullptr, 0, B);
-  hipLaunchKernelGGL(k_out_loss, dim3(nblocks(B)), dim3(256), 0, s, h->Z3, X, TAU, B, h->dZ3,
-                     h->rowloss);
-  hipLaunchKernelGGL(k_dense_bwd, dim3(nblocks((long long)B * NH)), dim3(256), 0, s, h->dZ3, NO,
-                     P + P_W3, NH, h->Z2, h->dZ2, B);
-  hipLaunchKernelGGL(k_dense_bwd, dim3(nblocks((long long)B * NH)), dim3(256), 0, s, h->dZ2, NH,
-                     P + P_W2, NH, h->Z1, h->dZ1, B);
-  const int nblk = (B + WG_ROWS - 1) / WG_ROWS;
-  hipLaunchKernelGGL(k_wgrad, dim3(nblk), dim3(256), 0, s, X, NF, ROW, h->dZ1, NH, B, h->partial,
-                     P_W1);
-  hipLaunchKernelGGL(k_wgrad, dim3(nblk), dim3(256), 0, s, h->H1, NH, NH, h->dZ2, NH, B,
-                     h->partial, P_W2);
-  hipLaunchKernelGGL(k_wgrad, dim3(nblk), dim3(256), 0, s, h->H2, NH, NH, h->dZ3, NO, B,
-                     h->partial, P_W3);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(nblocks(P_N)), dim3(256), 0, s, h->partial, nblk, h->G);
-  hipLaunchKernelGGL(k_sum_loss, dim3(1), dim3(256), 0, s, h->rowloss, B, h->loss);
+// forward + loss + backward + gradient into h->G, with adam its step (asynchronous on s)
+int grad_enqueue(idfx_mlp *h, const float *X, const float *TAU, int B, const AdamArgs *adam,
+                 hipStream_t s) {
+  const int nblk = train_blocks(B);
+  const dim3 rgrid((P_N + 31) / 32);
+  hipLaunchKernelGGL(k_train, dim3(nblk), dim3(128), 0, s, X, TAU, B, h->P, h->partial, h->lossp);
+  if (adam)
+    hipLaunchKernelGGL(k_reduce<true>, rgrid, dim3(256), 0, s, h->partial, h->lossp, nblk, B, h->G,
+                       h->loss, h->P, h->M, h->V, *adam);
+  else
+    hipLaunchKernelGGL(k_reduce<false>, rgrid, dim3(256), 0, s, h->partial, h->lossp, nblk, B,
+                       h->G, h->loss, h->P, h->M, h->V, AdamArgs{});
   return hipGetLastError() == hipSuccess ? IDFX_OK : IDFX_E_LAUNCH;
 }
 
@@ -226,26 +343,17 @@ int idfx_mlp_create(int max_batch, idfx_mlp **out) {
   *out = nullptr;
   idfx_mlp *h = new idfx_mlp();
   h->cap = max_batch;
-  const long long B = max_batch;
-  const int nblk = (max_batch + WG_ROWS - 1) / WG_ROWS;
+  const int nblk = train_blocks(max_batch);
   int st = IDFX_OK;
   float **bufs[] = {&h->P, &h->G, &h->M, &h->V};
   for (float **b : bufs)
     if (st == IDFX_OK) st = mlp_alloc(h, b, P_N);
-  if (st == IDFX_OK) st = mlp_alloc(h, &h->Z1, B * NH);
-  if (st == IDFX_OK) st = mlp_alloc(h, &h->H1, B * NH);
-  if (st == IDFX_OK) st = mlp_alloc(h, &h->Z2, B * NH);
-  if (st == IDFX_OK) st = mlp_alloc(h, &h->H2, B * NH);
-  if (st == IDFX_OK) st = mlp_alloc(h, &h->Z3, B * NO);
-  if (st == IDFX_OK) st = mlp_alloc(h, &h->dZ3, B * NO);
-  if (st == IDFX_OK) st = mlp_alloc(h, &h->dZ2, B * NH);
-  if (st == IDFX_OK) st = mlp_alloc(h, &h->dZ1, B * NH);
   if (st == IDFX_OK) st = mlp_alloc(h, &h->partial, (long long)nblk * P_N);
-  if (st == IDFX_OK) st = mlp_alloc(h, &h->rowloss, B);
   if (st == IDFX_OK) {
     float *l = nullptr;
-    st = mlp_alloc(h, &l, 2);
+    st = mlp_alloc(h, &l, 2 * (1 + nblk));
     h->loss = reinterpret_cast<double *>(l);
+    h->lossp = h->loss ? h->loss + 1 : nullptr;
   }
   if (st != IDFX_OK) {
     idfx_mlp_destroy(h);
@@ -283,7 +391,7 @@ int idfx_mlp_loss_grad(idfx_mlp *h, const float *X, const float *TAU, int B, dou
                        float *grad, void *stream) {
   if (!h || !X || !TAU || B < 1 || B > h->cap) return IDFX_E_ARGS;
   hipStream_t s = (hipStream_t)stream;
-  int st = grad_enqueue(h, X, TAU, B, s);
+  int st = grad_enqueue(h, X, TAU, B, nullptr, s);
   if (st != IDFX_OK) return st;
   if (hipStreamSynchronize(s) != hipSuccess) return IDFX_E_LAUNCH;
   if (loss && hipMemcpy(loss, h->loss, sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
@@ -297,15 +405,12 @@ int idfx_mlp_train_step(idfx_mlp *h, const float *X, const float *TAU, int B, fl
                         void *stream) {
   if (!h || !X || !TAU || B < 1 || B > h->cap || !(lr > 0.0f)) return IDFX_E_ARGS;
   hipStream_t s = (hipStream_t)stream;
-  int st = grad_enqueue(h, X, TAU, B, s);
-  if (st != IDFX_OK) return st;
-  h->step++;
-  const float b1 = 0.9f, b2 = 0.999f;
-  const float c1 = 1.0f - (float)std::pow(0.9, (double)h->step);
-  const float c2 = 1.0f - (float)std::pow(0.999, (double)h->step);
-  hipLaunchKernelGGL(k_adam, dim3(nblocks(P_N)), dim3(256), 0, s, h->P, h->G, h->M, h->V, P_N, lr,
-                     b1, b2, 1e-8f, c1, c2);
-  return hipGetLastError() == hipSuccess ? IDFX_OK : IDFX_E_LAUNCH;
+  const double t = (double)(h->step + 1);
+  const AdamArgs adam{lr, 0.9f, 0.999f, 1e-8f, 1.0f - (float)std::pow(0.9, t),
+                      1.0f - (float)std::pow(0.999, t)};
+  const int st = grad_enqueue(h, X, TAU, B, &adam, s);
+  if (st == IDFX_OK) h->step++;
+  return st;
 }
 
 int idfx_mlp_loss(idfx_mlp *h, double *loss, void *stream) {
