@@ -464,9 +464,27 @@ hipError_t launch_mlp_dir(const GridDesc &g, const double *Vc, const MlpNet &net
       n[d] = g.nt[d];
     }
   }
-  const long long waves = (long long)((n[0] + 63) / 64) * n[1] * n[2];
+  MlpGeom m{};
+  m.lo0 = lo[0];
+  m.lo1 = lo[1];
+  m.lo2 = lo[2];
+  m.nx = fast_div_of((unsigned)n[0]);
+  m.nj = fast_div_of((unsigned)n[1]);
+  long long waves;
+  if constexpr (DIR == IDIR) {
+    m.n = n[0] * n[1] * n[2];  // fewer than 2^29
+    waves = (m.n + 63) / 64;
+  } else {
+    m.n = n[0] * n[DIR == JDIR ? 2 : 1];
+    m.nf = n[DIR];
+    const long long ncb = (m.n + 15) / 16;
+    static const long long slots = resident_waves(k_mlp_infer<C, DIR>, 256 * 32);
+    m.ts = march_segment(ncb, m.nf, slots);
+    m.nseg = (m.nf + m.ts - 1) / m.ts;
+    waves = ncb * m.nseg;
+  }
   hipLaunchKernelGGL((k_mlp_infer<C, DIR>), dim3(blocks_for(waves, 4)), dim3(256), 0, s, g, Vc,
-                     net, W, lo[0], lo[1], lo[2], n[0], n[1], n[2]);
+                     net, W, m);
   return hipGetLastError();
 }
 
