@@ -4,12 +4,11 @@
 // [dir][k][j][i] with one extra face along each active direction for Vs
 // (src/fluid/fluid.hpp:529-560).  Kernels index with the ghost-inclusive np_tot extents.
 //
-// Sweeps.  The x sweep gives one face per lane: a wave covers 64 faces and updates the
-// 63 cells between them, taking the right-hand flux from the neighbouring lane with a
-// cross-lane shuffle.  The y and z sweeps march: a lane owns one x column and walks a
-// segment of cells along the sweep direction, carrying the stencil window, the
-// reconstructed state of the previous cell and the previous face flux in registers, so
-// every cell is reconstructed once and every face solved once (plus one face per
+// Sweeps.  The x sweep gives one face per lane and takes the right-hand flux from the
+// neighbouring lane with a cross-lane shuffle.  The y and z sweeps march: a lane owns one x
+// column and walks a segment of cells along the sweep direction, carrying the stencil
+// window and the reconstructed state of the previous cell (in LDS) and the previous face
+// flux, so every cell is reconstructed once and every face solved once (plus one face per
 // segment).  In FUSED mode the flux divergence goes straight into Uc in FP64 and the
 // intercell flux never reaches HBM; in flux-only mode the kernel writes FluxRiemann
 // like the reference (needed when a user flux hook is enrolled).
@@ -531,29 +530,36 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
     const unsigned row = (unsigned)idx3(g, k, j, 0);
     const unsigned p = row + (unsigned)c;
 
+    // every load first: the limiters below branch, and loads between them would each wait
+    // for memory on their own (512^3 PPM: 9.9 -> 8.1 ms a launch)
+    T wv[NV][NW], bn = T(0);
+#pragma unroll
+    for (int n = 0; n < NV; n++) {
+      if (C::MHD && n == C::BX1) continue;  // the normal field comes from Vs
+#pragma unroll
+      for (int s = 0; s < NW; s++) {
+        // a row's first PPM site only gives its right face: V(c-2) may lie outside
+        const unsigned q = (XF == 2 && s == 0) ? row + (unsigned)max(c - H, 0) : p + (unsigned)(s - H);
+        wv[n][s] = (T)ld32(a.Vc + n * g.sv, q);
+      }
+    }
+    if constexpr (C::MHD) bn = (T)ld32(a.Vs, (unsigned)idxs(g, 0, k, j, c));
     // reconstruct the lane's cell: vl = right state of face c, vr = left state of face c+1
     T vl[NV], vr[NV];
     const bool flat = XTRA && recon_flat<C>(a, p);
 #pragma unroll
     for (int n = 0; n < NV; n++) {
-      if (C::MHD && n == C::BX1) {  // the normal field comes from Vs
+      if (C::MHD && n == C::BX1) {
         vl[n] = vr[n] = T(0);
         continue;
       }
-      T wv[NW];
-#pragma unroll
-      for (int s = 0; s < NW; s++) {
-        // a row's first PPM site only gives its right face: V(c-2) may lie outside
-        const unsigned q = (XF == 2 && s == 0) ? row + (unsigned)max(c - H, 0) : p + (unsigned)(s - H);
-        wv[s] = (T)ld32(a.Vc + n * g.sv, q);
-      }
       if constexpr (C::ORDER == RECON_MLP) {
-        recon_mlp<C, IDIR>(wv, n, a.mlpw, g.sv, p, 1u, vl[n], vr[n]);
+        recon_mlp<C, IDIR>(wv[n], n, a.mlpw, g.sv, p, 1u, vl[n], vr[n]);
       } else if constexpr (C::ORDER == RECON_PPM) {
-        const T fr = recon_face<C>(wv);
-        recon_ppm<C>(wv, n, __shfl_up(fr, 1), fr, vl[n], vr[n]);
+        const T fr = recon_face<C>(wv[n]);
+        recon_ppm<C>(wv[n], n, __shfl_up(fr, 1), fr, vl[n], vr[n]);
       } else {
-        recon_cell<C>(wv, n, vl[n], vr[n], recon_dx<C, T>(g, 0, c), flat);
+        recon_cell<C>(wv[n], n, vl[n], vr[n], recon_dx<C, T>(g, 0, c), flat);
       }
     }
     T vL[NV], vR[NV];
@@ -563,8 +569,8 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
       vR[n] = vl[n];
     }
     if constexpr (C::MHD) {
-      vL[C::BX1] = (T)ld32(a.Vs, (unsigned)idxs(g, 0, k, j, c));
-      vR[C::BX1] = vL[C::BX1];
+      vL[C::BX1] = bn;
+      vR[C::BX1] = bn;
     }
     T F[NV], cmax;
     FaceEmf<T> E;
@@ -604,6 +610,11 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
 // across row ends: blocks of 64 along x would leave a row of 130 columns (128 cells and
 // their extension) with 48 % idle lanes in its three waves, one of 514 with 11 % (whole
 // cycles: Orszag-Tang 128^3 1453 -> 1263 us, turbulence 512^3 133.4 -> 123.6 ms).
+//
+// With the window in LDS, the next row loaded a step ahead and every other load of a step
+// before its reconstruction, the 512^3 PPM sweeps take 7.2 (y) and 8.4 ms (z) a launch at
+// 228-238 VGPRs; with the window in registers and its leading row loaded when needed they
+// took 7.8 and 9.5 ms (256 VGPRs and 44 B of spills).
 // ------------------------------------------------------------------------------------
 struct MarchGeom {
   int ilo, ihi;   // x range (interior +- extension)
@@ -615,17 +626,11 @@ struct MarchGeom {
   int grp;        // column blocks whose segments are adjacent in launch order
 };
 
-// The stencil rows consecutive marching steps share are carried in LDS for the 3-cell
-// window (PLM, learned limiter); PPM keeps its 5-row window in registers.
-template <class C>
-constexpr bool march_lds_window() {
-  return window<C>() == 3;
-}
 // 3 waves per SIMD fit the 2-D march of the 6-variable MHD state without spills; the 3-D
 // one and the 8-variable 2-D one would spill, so they stay at 2
 template <class C>
 constexpr int march_waves_per_eu() {
-  return (march_lds_window<C>() && C::DIM == 2 && C::NVAR < 8) ? 3 : 2;
+  return (window<C>() == 3 && C::DIM == 2 && C::NVAR < 8) ? 3 : 2;
 }
 template <class C, typename T, int DIR, bool FUSED, int EMF, bool XTRA, bool FIN = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(march_waves_per_eu<C>())))
@@ -668,61 +673,49 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
     const unsigned vcol = (unsigned)idxs(g, 0, kk, jj, i);
     const double *VsDir = a.Vs + DIR * g.svs;  // the normal component
 
-    constexpr bool CARRY = march_lds_window<C>();
-    // window rows f-1, f of thread t at lds[(row & 1) * NV + n][t]
-    __shared__ T lds[CARRY ? 2 * NV : 1][256];
+    // What a step hands to the next one passes through LDS, out of the registers the Riemann
+    // solve needs: the window's last NW - 1 rows (a ring, row r at slot r mod NW - 1), the
+    // right state of cell f - 1 (the left state of face f) and, with PPM, the value of face
+    // f.  The normal field has no slot: it comes from Vs.
+    constexpr bool PPM = C::ORDER == RECON_PPM;
+    constexpr int NS = C::MHD ? NV - 1 : NV;
+    constexpr int RW = NW > 1 ? NW - 1 : 1;  // 1, 2 or 4
+    __shared__ T ring[RW * NS][256], hand[NS][256];
     const int tid = threadIdx.x;
-    T win[NW][NV];
-#pragma unroll
-    for (int s = 0; s < NW; s++)
-#pragma unroll
-      for (int n = 0; n < NV; n++) {
-        win[s][n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 - 1 - H + s) * sd);
-        if constexpr (CARRY) {
-          if (s >= 1) lds[((c0 - 1 - H + s) & 1) * NV + n][tid] = win[s][n];
-        }
-      }
-    // right state of cell c0-1: the left state of the first face; PPM also hands on the
-    // value of its right face, the left face of the next cell
-    T carry[NV], Fprev[NV], fcar[NV], cprev = 0;
-#pragma unroll
-    for (int n = 0; n < NV; n++) Fprev[n] = 0;
+    auto is_bn = [](int n) { return C::MHD && n == C::template BXn<DIR>(); };
+    auto slot = [](int n) { return C::MHD && n > C::template BXn<DIR>() ? n - 1 : n; };
+    auto row = [&](int r, int n) -> T & { return ring[(r & (RW - 1)) * NS + slot(n)][tid]; };
+    T Fprev[NV], fcar[NV], cprev = 0;
+    // the leading row of a step's window is loaded a step ahead, before the Riemann solve, so
+    // that it arrives under it
+    T nxt[NV];
 #pragma unroll
     for (int n = 0; n < NV; n++) {
+      Fprev[n] = 0;
+      if (is_bn(n)) continue;
       T wv[NW];
 #pragma unroll
-      for (int s = 0; s < NW; s++) wv[s] = win[s][n];
-      T dummy;
-      if (C::MHD && n == C::template BXn<DIR>()) { carry[n] = fcar[n] = wv[H]; continue; }
+      for (int s = 0; s < NW; s++) {
+        wv[s] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 - 1 - H + s) * sd);
+        if (NW > 1 && s >= 1) row(c0 - 1 - H + s, n) = wv[s];
+      }
+      nxt[n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 + H) * sd);
+      T dummy, right;
       if constexpr (C::ORDER == RECON_MLP) {
-        recon_mlp<C, DIR>(wv, n, a.mlpw, g.sv, col + (unsigned)(c0 - 1) * sd, sd, dummy, carry[n]);
-      } else if constexpr (C::ORDER == RECON_PPM) {
+        recon_mlp<C, DIR>(wv, n, a.mlpw, g.sv, col + (unsigned)(c0 - 1) * sd, sd, dummy, right);
+      } else if constexpr (PPM) {
         fcar[n] = recon_face<C>(wv);
-        recon_ppm<C>(wv, n, ppm_face(wv[0], wv[1], wv[2], wv[3]), fcar[n], dummy, carry[n]);
+        recon_ppm<C>(wv, n, ppm_face(wv[0], wv[1], wv[2], wv[3]), fcar[n], dummy, right);
       } else {
-        recon_cell<C>(wv, n, dummy, carry[n], recon_dx<C, T>(g, DIR, c0 - 1),
+        recon_cell<C>(wv, n, dummy, right, recon_dx<C, T>(g, DIR, c0 - 1),
                       XTRA && recon_flat<C>(a, col + (unsigned)(c0 - 1) * sd));
       }
+      hand[slot(n)][tid] = right;
     }
     for (int f = c0; f <= c1; f++) {
-      // shift the window to cell f and load its leading row
-      if constexpr (CARRY) {
-#pragma unroll
-        for (int n = 0; n < NV; n++) {
-          win[0][n] = lds[((f - 1) & 1) * NV + n][tid];
-          win[1][n] = lds[(f & 1) * NV + n][tid];
-          win[2][n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(f + 1) * sd);
-          lds[((f + 1) & 1) * NV + n][tid] = win[2][n];  // replaces row f-1, read above
-        }
-      } else {
-#pragma unroll
-        for (int s = 0; s < NW - 1; s++)
-#pragma unroll
-          for (int n = 0; n < NV; n++) win[s][n] = win[s + 1][n];
-#pragma unroll
-        for (int n = 0; n < NV; n++)
-          win[NW - 1][n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(f + H) * sd);
-      }
+      // the normal field of face f, ahead of the reconstruction
+      T bn = T(0);
+      if constexpr (C::MHD) bn = (T)ld32(VsDir, vcol + (unsigned)f * vsd);
       // FIN: the begin state of cell f - 1 (updated at the end of this step), loaded now
       // so that its latency overlaps the reconstruction and the Riemann solve
       double u0pre[NV];
@@ -734,12 +727,10 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
               u0pre[n] = ld32((const double *)a.Uc0 + n * g.sv, col + (unsigned)(f - 1) * sd);
         }
       }
-      // the 3-D sweeps without per-cell options, except Roe's and the final FP64 one: the
-      // accumulated state of cell f - 1 (the register room this needs is there only in
-      // those; the FP32 sweeps have it at their 3 waves per SIMD)
+      // the 3-D sweeps without per-cell options, except Roe's: the accumulated state of cell
+      // f - 1 (the register room this needs is there only in those)
       double upre[NV];
-      constexpr bool PRE_U = FUSED && !XTRA && C::DIM == 3 && C::SOLVER != SOLVER_ROE &&
-                             (!FIN || std::is_same<T, float>::value);
+      constexpr bool PRE_U = FUSED && !XTRA && C::DIM == 3 && C::SOLVER != SOLVER_ROE;
       if constexpr (PRE_U) {
         if (f > c0 && rhs_lane) {
 #pragma unroll
@@ -748,32 +739,36 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
               upre[n] = ld32((const double *)a.Uc + n * g.sv, col + (unsigned)(f - 1) * sd);
         }
       }
-      T vL[NV], vR[NV], vr_next[NV];
+      T vL[NV], vR[NV];
       const bool flat = XTRA && recon_flat<C>(a, col + (unsigned)f * sd);
 #pragma unroll
       for (int n = 0; n < NV; n++) {
-        T wv[NW];
-#pragma unroll
-        for (int s = 0; s < NW; s++) wv[s] = win[s][n];
-        vL[n] = carry[n];
-        if (C::MHD && n == C::template BXn<DIR>()) {  // the normal field comes from Vs
-          vR[n] = vr_next[n] = wv[H];
+        if (is_bn(n)) {
+          vL[n] = vR[n] = bn;
           continue;
         }
+        T wv[NW];  // the window of cell f
+#pragma unroll
+        for (int s = 0; s < NW - 1; s++) wv[s] = row(f - H + s, n);
+        wv[NW - 1] = nxt[n];
+        if (NW > 1) row(f + H, n) = nxt[n];  // replaces row f - H, read above
+        vL[n] = hand[slot(n)][tid];
+        T right;
         if constexpr (C::ORDER == RECON_MLP) {
-          recon_mlp<C, DIR>(wv, n, a.mlpw, g.sv, col + (unsigned)f * sd, sd, vR[n], vr_next[n]);
-        } else if constexpr (C::ORDER == RECON_PPM) {
+          recon_mlp<C, DIR>(wv, n, a.mlpw, g.sv, col + (unsigned)f * sd, sd, vR[n], right);
+        } else if constexpr (PPM) {
           const T fr = recon_face<C>(wv);
-          recon_ppm<C>(wv, n, fcar[n], fr, vR[n], vr_next[n]);
+          recon_ppm<C>(wv, n, fcar[n], fr, vR[n], right);
           fcar[n] = fr;
         } else {
-          recon_cell<C>(wv, n, vR[n], vr_next[n], recon_dx<C, T>(g, DIR, f), flat);
+          recon_cell<C>(wv, n, vR[n], right, recon_dx<C, T>(g, DIR, f), flat);
         }
+        hand[slot(n)][tid] = right;
       }
-      if constexpr (C::MHD) {
-        constexpr int BXn = C::template BXn<DIR>();
-        vL[BXn] = (T)ld32(VsDir, vcol + (unsigned)f * vsd);
-        vR[BXn] = vL[BXn];
+      if (f < c1) {
+#pragma unroll
+        for (int n = 0; n < NV; n++)
+          nxt[n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(f + 1 + H) * sd);
       }
       T F[NV], cmax;
       FaceEmf<T> E;
@@ -802,10 +797,7 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
         }
       }
 #pragma unroll
-      for (int n = 0; n < NV; n++) {
-        carry[n] = vr_next[n];
-        Fprev[n] = F[n];
-      }
+      for (int n = 0; n < NV; n++) Fprev[n] = F[n];
       cprev = cmax;
     }
   }
