@@ -1147,20 +1147,25 @@ __global__ __launch_bounds__(256) void k_evolve_b(GridDesc g, double *Vs, double
 
 // CalcCornerEMF (uct_contact) and EvolveMagField of a 3-D block in one kernel, for the
 // stage path (the reference-granularity entry points keep k_corner_emf + k_evolve_b).
-// A block of 8 waves owns a tile of 63 face columns (i) x 7 face rows (j) and marches
-// along k over a segment of face planes.  Lane l of wave w computes the three edge EMFs at
-// edge (k, j0 + w, i0 + l) of each plane k with the arithmetic of k_corner_emf
-// (contact_edges3), so the tile's 64 x 8 edges cover its faces and the one halo column
-// and row they need; the edges of plane k stay in registers (own column), reach the
-// neighbouring column by a shuffle and the neighbouring row through LDS (three plane
-// buffers, one barrier per plane), and the face data and cell EMFs of plane k - 1 are
-// the previous step's plane k.  After plane k, the faces of plane k - 1 are updated with
-// the arithmetic of k_evolve_b (mode / wc / w0 as there), in place: every face has one
-// owner and no other block reads Vs.  A lane loads the old values (and RK begin values)
-// of the faces it updates in a step at the top of that step, so their latency overlaps
-// the edge work and the barrier.  Only faces the next stage reads are updated: each
-// face field over [beg, end] along its own direction and [beg, end) across; the edge
-// arrays ex, ey, ez are not written.
+// A block of 12 waves covers 64 columns (i) x 12 rows (j), owns the 62 x 10 faces inside, and
+// marches along k over a segment of face planes.  A lane loads only what sits at its own
+// (k, j, i): the cell's v and B, six face EMFs, three upwind weights.  The edge EMFs at
+// (k, j, i) (contact_edges3, the arithmetic of k_corner_emf) also need the column before
+// (shuffles and LDS), the row before (LDS, from the neighbouring wave) and the plane before
+// (registers).  The lanes of the first column and row only feed their neighbours, those of
+// the last only give theirs the edges at i + 1 and j + 1.  One barrier per plane: two
+// buffers each for what a lane loaded and for its edges.  After plane k, the faces of plane
+// k - 1 are updated with the arithmetic of k_evolve_b (mode / wc / w0 as there), in place:
+// every face has one owner and no other block reads Vs.  The next plane's loads and the old
+// values (and RK begin values) of the faces updated in a step are issued before the step's
+// barrier.  Only faces the next stage reads are updated: each face field over [beg, end]
+// along its own direction and [beg, end) across; the edge arrays ex, ey, ez are not written.
+//
+// The kernel is bound by HBM: 139 B a cell it cannot do without (3.9 ms at 512^3 at the
+// copy rate).  Tiles follow each other along x, then y, so that the tiles an XCD works on at
+// a time share their edge columns' cache lines and halo rows in its L2.  5.2 ms at 512^3 and
+// 147 us at 203x150x97; with every lane loading all four cells and the face data around its
+// edge, and tiles following each other along y, 7.6 ms and 208 us.
 // Cell EMFs of one cell from 32-bit offsets (the arithmetic of cell_emf).
 template <class C, typename T>
 __device__ __forceinline__ void cell_emf32(const double *Vc, long long sv, unsigned p, T &E1,
@@ -1192,54 +1197,86 @@ __device__ __forceinline__ void evolve_face_pre(double *Vs, double *Vs0, unsigne
   st32(Vs, q, (mode == 2) ? wc * upd + w0 * old0 : upd);
 }
 
+// tile of k_ct3d: faces per block in i and j (512^3 FP64, 8 waves of 62 x 6: 5.5 ms, 12
+// waves: 5.2 ms, 16 waves, which must fit 128 VGPRs: 5.9 ms)
+constexpr int CT_TI = 62, CT_TJ = 10;
 template <class C, typename T>
-__global__ __launch_bounds__(512) void k_ct3d(GridDesc g, const double *Vc, double *Vs,
+__global__ __launch_bounds__((CT_TJ + 2) * 64, 3) void k_ct3d(GridDesc g, const double *Vc, double *Vs,
                                               double *Vs0, EmfArrays<T> e, double dt, int mode,
-                                              double wc, double w0, int ntj, int nseg,
-                                              int kseg) {
+                                              double wc, double w0, int nti, int ntj, int kseg) {
   static_assert(C::MHD && C::DIM == 3 && C::COMP == 3, "k_ct3d is the 3-D MHD CT");
-  constexpr int TI = 63, TJ = 7;
-  __shared__ T lez[3][8][64], lex[3][8][64];
+  constexpr int TI = CT_TI, TJ = CT_TJ, NW = TJ + 2;
+  __shared__ T sE1[2][NW][64], sE3[2][NW][64], sezi[2][NW][64], sexk[2][NW][64];
+  __shared__ T lez[2][NW][64], lex[2][NW][64];
+  __shared__ unsigned char ssvx[2][NW][64], ssvz[2][NW][64];
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // each XCD takes a contiguous run of (tile, segment) indices, so that neighbouring
-  // tiles, which read each other's halo rows and columns, share an L2
+  // each XCD takes a contiguous run of tiles, x fastest, then y, then the k segments
   const int blk = xcd_contiguous_block();
-  const int seg = blk % nseg;
-  const int tile = blk / nseg;
-  const int ti = tile / ntj, tj = tile % ntj;
-  const int i = g.beg[0] + TI * ti + l, j = g.beg[1] + TJ * tj + w;
+  const int ti = blk % nti, tj = blk / nti % ntj, seg = blk / (nti * ntj);
+  const int i = g.beg[0] - 1 + TI * ti + l, j = g.beg[1] - 1 + TJ * tj + w;
   const int ks = g.beg[2] + kseg * seg;
   const int ke = min(ks + kseg, g.end[2] + 1);  // face planes [ks, ke)
   const int klast = min(ke, g.end[2]);          // last edge plane
-  const bool edge_ok = i <= g.end[0] && j <= g.end[1];
-  const unsigned sy = (unsigned)g.nt[0], sz = (unsigned)g.nt[0] * (unsigned)g.nt[1];
+  const bool in = i <= g.end[0] && j <= g.end[1];
+  const unsigned sz = (unsigned)g.nt[0] * (unsigned)g.nt[1];
   const unsigned vy = (unsigned)g.vsn[0], vz = (unsigned)g.vsn[0] * (unsigned)g.vsn[1];
   double *Vs1 = Vs + g.svs, *Vs2 = Vs + 2 * g.svs;
   double *Vs01 = Vs0 + g.svs, *Vs02 = Vs0 + 2 * g.svs;
-  // plane k - 1 data carried from the previous step
-  T E1m0 = 0, E1m1 = 0, E2m0 = 0, E2m1 = 0;  // E1 of cells (k-1, j-1+dj, i), E2 of (k-1, j, i-1+di)
-  T svx_m = 0, svy_m = 0, exj_m = 0, eyi_m = 0;
-  if (edge_ok) {
-    const unsigned p = (unsigned)idx3(g, ks - 1, j, i);
-    T a1, a2, a3;
-    cell_emf32<C, T>(Vc, g.sv, p - sy, E1m0, a2, a3);
-    cell_emf32<C, T>(Vc, g.sv, p, E1m1, E2m1, a3);
-    cell_emf32<C, T>(Vc, g.sv, p - 1, a1, E2m0, a3);
-    svx_m = sv_val<T>(ld32(e.svx, p));
-    svy_m = sv_val<T>(ld32(e.svy, p));
-    exj_m = ld32(e.exj, p);
-    eyi_m = ld32(e.eyi, p);
-  }
-  T pex = 0, pey = 0, pez = 0;  // edges of the previous plane, own column
+  const int lm = l > 0 ? l - 1 : 0, wm = w > 0 ? w - 1 : 0, wp = w < NW - 1 ? w + 1 : w;
+  // what the lane loads of a plane
+  double v1 = 0, v2 = 0, v3 = 0, b1 = 0, b2 = 0, b3 = 0;
+  T ezi = 0, ezj = 0, exj = 0, exk = 0, eyi = 0, eyk = 0;
+  unsigned cx = 0, cy = 0, cz = 0;
+  unsigned p = in ? (unsigned)idx3(g, ks - 1, j, i) : 0u;
+  auto load = [&]() {
+    v1 = ld32(Vc + C::MX1 * g.sv, p);
+    v2 = ld32(Vc + C::MX2 * g.sv, p);
+    v3 = ld32(Vc + C::MX3 * g.sv, p);
+    b1 = ld32(Vc + C::BX1 * g.sv, p);
+    b2 = ld32(Vc + C::BX2 * g.sv, p);
+    b3 = ld32(Vc + C::BX3 * g.sv, p);
+    ezi = ld32(e.ezi, p);
+    ezj = ld32(e.ezj, p);
+    exj = ld32(e.exj, p);
+    exk = ld32(e.exk, p);
+    eyi = ld32(e.eyi, p);
+    eyk = ld32(e.eyk, p);
+    cx = ld32(e.svx, p);
+    cy = ld32(e.svy, p);
+    cz = ld32(e.svz, p);
+  };
+  if (in) load();
+  // plane k - 1: cell EMFs of (j-1, i), (j, i), (j, i-1), weights and face EMFs; edges
+  T E1m0 = 0, E1m1 = 0, E2m0 = 0, E2m1 = 0, svx_m = 0, svy_m = 0, exj_m = 0, eyi_m = 0;
+  T pex = 0, pey = 0, pez = 0;
   // dt / dx of the lane's column and row (clamped indices: lanes past the block's end
   // compute no face)
   const double rdx = dt / g.dx[0][min(i, g.nt[0] - 1)], rdy = dt / g.dx[1][min(j, g.nt[1] - 1)];
-  const double mrdx = -dt / g.dx[0][min(i, g.nt[0] - 1)];
-  const bool own = l < TI && w < TJ;
-  for (int k = ks; k <= klast; k++) {
-    // the faces of plane k - 1 this lane updates in this step: their old values (and RK
-    // begin values) are loaded before the edge work and the barrier; only this lane
-    // writes them, later in this step
+  const bool own = l >= 1 && l <= TI && w >= 1 && w <= TJ;
+  for (int k = ks - 1; k <= klast; k++) {  // plane ks - 1 only primes
+    const int bf = k & 1;
+    // cell EMFs (the arithmetic of cell_emf) of the loaded plane
+    const T E1 = ((T)v3 * (T)b2 - (T)v2 * (T)b3);
+    const T E2 = ((T)v1 * (T)b3 - (T)v3 * (T)b1);
+    const T E3 = ((T)v2 * (T)b1 - (T)v1 * (T)b2);
+    ContactFaces<T> f;
+    f.ezi = ezi;
+    f.ezj = ezj;
+    f.exj = exj;
+    f.exk = exk;
+    f.eyi = eyi;
+    f.eyk = eyk;
+    const unsigned cyc = cy, czc = cz;
+    f.svx = sv_val<T>((unsigned char)cx);
+    f.svy = sv_val<T>((unsigned char)cy);
+    f.svz = sv_val<T>((unsigned char)cz);
+    sE1[bf][w][l] = E1;
+    sE3[bf][w][l] = E3;
+    sezi[bf][w][l] = ezi;
+    sexk[bf][w][l] = exk;
+    ssvx[bf][w][l] = (unsigned char)cx;
+    ssvz[bf][w][l] = (unsigned char)cz;
+    // the faces of plane k - 1 this lane updates in this step
     const int kk = k - 1;
     const unsigned q = (unsigned)kk * vz + (unsigned)j * vy + (unsigned)i;
     const bool u1 = k > ks && own && i <= g.end[0] && j < g.end[1] && kk < g.end[2];
@@ -1258,60 +1295,61 @@ __global__ __launch_bounds__(512) void k_ct3d(GridDesc g, const double *Vc, doub
       o3 = ld32(Vs2, q);
       if (mode == 2) z3 = ld32(Vs02, q);
     }
-    const double rdz = (k > ks && kk < g.end[2]) ? dt / g.dx[2][kk] : 0.0;
-    T cex = 0, cey = 0, cez = 0;
-    if (edge_ok) {
-      const unsigned p = (unsigned)idx3(g, k, j, i);
-      T E1[2][2][2], E2[2][2][2], E3[2][2][2];
-      cell_emf32<C, T>(Vc, g.sv, p - sy - 1, E1[1][0][0], E2[1][0][0], E3[1][0][0]);
-      cell_emf32<C, T>(Vc, g.sv, p - sy, E1[1][0][1], E2[1][0][1], E3[1][0][1]);
-      cell_emf32<C, T>(Vc, g.sv, p - 1, E1[1][1][0], E2[1][1][0], E3[1][1][0]);
-      cell_emf32<C, T>(Vc, g.sv, p, E1[1][1][1], E2[1][1][1], E3[1][1][1]);
-      E1[0][0][1] = E1m0;
-      E1[0][1][1] = E1m1;
-      E2[0][1][0] = E2m0;
-      E2[0][1][1] = E2m1;
-      ContactFaces<T> f;
-      f.svx = sv_val<T>(ld32(e.svx, p));
-      f.svx_jm = sv_val<T>(ld32(e.svx, p - sy));
-      f.svx_km = svx_m;
-      f.svy = sv_val<T>(ld32(e.svy, p));
-      f.svy_im = sv_val<T>(ld32(e.svy, p - 1));
-      f.svy_km = svy_m;
-      f.svz = sv_val<T>(ld32(e.svz, p));
-      f.svz_jm = sv_val<T>(ld32(e.svz, p - sy));
-      f.svz_im = sv_val<T>(ld32(e.svz, p - 1));
-      f.ezi = ld32(e.ezi, p);
-      f.ezi_jm = ld32(e.ezi, p - sy);
-      f.ezj = ld32(e.ezj, p);
-      f.ezj_im = ld32(e.ezj, p - 1);
-      f.exj = ld32(e.exj, p);
-      f.exj_km = exj_m;
-      f.exk = ld32(e.exk, p);
-      f.exk_jm = ld32(e.exk, p - sy);
-      f.eyi = ld32(e.eyi, p);
-      f.eyi_km = eyi_m;
-      f.eyk = ld32(e.eyk, p);
-      f.eyk_im = ld32(e.eyk, p - 1);
-      contact_edges3(f, E1, E2, E3, cex, cey, cez);
-      E1m0 = E1[1][0][1];
-      E1m1 = E1[1][1][1];
-      E2m0 = E2[1][1][0];
-      E2m1 = E2[1][1][1];
-      svx_m = f.svx;
-      svy_m = f.svy;
-      exj_m = f.exj;
-      eyi_m = f.eyi;
+    if (in && k < klast) {
+      p += sz;
+      load();
     }
-    lez[k % 3][w][l] = cez;
-    lex[k % 3][w][l] = cex;
     __syncthreads();
+    // the column, row and corner before
+    const T E3_im = sE3[bf][w][lm], E3_jm = sE3[bf][wm][l], E3_ijm = sE3[bf][wm][lm];
+    const T E1_jm = sE1[bf][wm][l];
+    f.ezi_jm = sezi[bf][wm][l];
+    f.exk_jm = sexk[bf][wm][l];
+    f.svx_jm = sv_val<T>(ssvx[bf][wm][l]);
+    f.svz_jm = sv_val<T>(ssvz[bf][wm][l]);
+    const T E2_im = __shfl_up(E2, 1);
+    f.ezj_im = __shfl_up(f.ezj, 1);
+    f.eyk_im = __shfl_up(f.eyk, 1);
+    f.svy_im = sv_val<T>((unsigned char)__shfl_up(cyc, 1));
+    f.svz_im = sv_val<T>((unsigned char)__shfl_up(czc, 1));
+    T cex = 0, cey = 0, cez = 0;
+    if (k >= ks) {
+      f.svx_km = svx_m;
+      f.svy_km = svy_m;
+      f.exj_km = exj_m;
+      f.eyi_km = eyi_m;
+      T A1[2][2][2], A2[2][2][2], A3[2][2][2];  // [dk][dj][di], the ones the edges use
+      A1[0][0][1] = E1m0;
+      A1[0][1][1] = E1m1;
+      A1[1][0][1] = E1_jm;
+      A1[1][1][1] = E1;
+      A2[0][1][0] = E2m0;
+      A2[0][1][1] = E2m1;
+      A2[1][1][0] = E2_im;
+      A2[1][1][1] = E2;
+      A3[1][0][0] = E3_ijm;
+      A3[1][0][1] = E3_jm;
+      A3[1][1][0] = E3_im;
+      A3[1][1][1] = E3;
+      contact_edges3(f, A1, A2, A3, cex, cey, cez);
+      lez[bf][w][l] = cez;
+      lex[bf][w][l] = cex;
+    }
+    E1m0 = E1_jm;
+    E1m1 = E1;
+    E2m0 = E2_im;
+    E2m1 = E2;
+    svx_m = f.svx;
+    svy_m = f.svy;
+    exj_m = f.exj;
+    eyi_m = f.eyi;
     if (k > ks) {
       // faces of plane kk = k - 1 from the edges of planes kk (p*) and k (c*)
+      const double rdz = kk < g.end[2] ? dt / g.dx[2][kk] : 0.0;
       const T ez_ip = __shfl_down(pez, 1);
       const T ey_ip = __shfl_down(pey, 1);
-      const T ez_jp = lez[kk % 3][w < 7 ? w + 1 : w][l];
-      const T ex_jp = lex[kk % 3][w < 7 ? w + 1 : w][l];
+      const T ez_jp = lez[bf ^ 1][wp][l];
+      const T ex_jp = lex[bf ^ 1][wp][l];
       if (u1) {  // BX1s
         double r = 0.0 - rdy * ((double)ez_jp - (double)pez);
         r = r + rdz * ((double)cey - (double)pey);
@@ -1323,7 +1361,7 @@ __global__ __launch_bounds__(512) void k_ct3d(GridDesc g, const double *Vc, doub
         evolve_face_pre(Vs1, Vs01, q, o2, z2, r, mode, wc, w0);
       }
       if (u3) {  // BX3s at face plane kk
-        const double r = mrdx * ((double)ey_ip - (double)pey) + rdy * ((double)ex_jp - (double)pex);
+        const double r = -rdx * ((double)ey_ip - (double)pey) + rdy * ((double)ex_jp - (double)pex);
         evolve_face_pre(Vs2, Vs02, q, o3, z3, r, mode, wc, w0);
       }
     }
@@ -1334,11 +1372,11 @@ __global__ __launch_bounds__(512) void k_ct3d(GridDesc g, const double *Vc, doub
   if (ke == g.end[2] + 1) {
     // the top face plane of the block (BX3s at end) from the last edge plane
     const int kk = g.end[2];
+    __syncthreads();
     const T ey_ip = __shfl_down(pey, 1);
-    const T ex_jp = lex[kk % 3][w < 7 ? w + 1 : w][l];
-    if (l < TI && w < TJ && i < g.end[0] && j < g.end[1]) {
-      const double r = -dt / g.dx[0][i] * ((double)ey_ip - (double)pey) +
-                       dt / g.dx[1][j] * ((double)ex_jp - (double)pex);
+    const T ex_jp = lex[kk & 1][wp][l];
+    if (own && i < g.end[0] && j < g.end[1]) {
+      const double r = -rdx * ((double)ey_ip - (double)pey) + rdy * ((double)ex_jp - (double)pex);
       const unsigned q = (unsigned)kk * vz + (unsigned)j * vy + (unsigned)i;
       evolve_face(Vs2, Vs02, q, r, mode, wc, w0);
     }

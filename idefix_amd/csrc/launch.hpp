@@ -239,18 +239,19 @@ hipError_t launch_ct3d(const GridDesc &g, const double *Vc, double *Vs, double *
                        const void *emf, double dt, int mode, double wc, double w0,
                        hipStream_t s) {
   if constexpr (C::MHD && C::DIM == 3) {
-    // tiles of 63 x 7 faces in (i, j); k segments so that the grid holds about 2048
-    // blocks of 8 waves (several rounds of the chip's resident blocks)
+    // k segments: march_segment's rule with blocks for columns and the chip's 256 CUs (one
+    // block each) for slots.  From 256 tiles on, 512 slots, which leads to fewer, longer
+    // segments: the XCDs then work near one plane (512^3, 468 tiles: 5.2 against 5.6 ms;
+    // 203x150x97, 64 tiles, with 512: 161 against 147 us).
     const int nfi = g.end[0] - g.beg[0] + 1, nfj = g.end[1] - g.beg[1] + 1;
     const int nfk = g.end[2] - g.beg[2] + 1;
-    const int nti = (nfi + 62) / 63, ntj = (nfj + 6) / 7;
+    const int nti = (nfi + CT_TI - 1) / CT_TI, ntj = (nfj + CT_TJ - 1) / CT_TJ;
     const long long tiles = (long long)nti * ntj;
-    int nseg = (int)std::max<long long>(1, std::min<long long>(nfk, (2048 + tiles - 1) / tiles));
-    const int kseg = (nfk + nseg - 1) / nseg;
-    nseg = (nfk + kseg - 1) / kseg;
-    hipLaunchKernelGGL((k_ct3d<C, T>), dim3((unsigned)(tiles * nseg)), dim3(512), 0, s, g, Vc,
-                       Vs, Vs0, *static_cast<const EmfArrays<T> *>(emf), dt, mode, wc, w0, ntj,
-                       nseg, kseg);
+    const int kseg = march_segment(tiles, nfk, tiles >= 256 ? 512 : 256);
+    const int nseg = (nfk + kseg - 1) / kseg;
+    hipLaunchKernelGGL((k_ct3d<C, T>), dim3((unsigned)(tiles * nseg)), dim3((CT_TJ + 2) * 64), 0, s,
+                       g, Vc, Vs, Vs0, *static_cast<const EmfArrays<T> *>(emf), dt, mode, wc, w0,
+                       nti, ntj, kseg);
     return hipGetLastError();
   }
   return hipErrorInvalidValue;

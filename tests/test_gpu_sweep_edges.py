@@ -56,3 +56,20 @@ def test_hd_3d_outflow(n):
     assert o.cycle() == 0
     g.cycle()
     compare_state(o, g, what="%s" % (n,))
+
+
+@pytest.mark.parametrize("nstages", [2, 3])
+@pytest.mark.parametrize("n", [(3, 5, 4), (61, 6, 3), (62, 7, 3), (63, 5, 4), (124, 12, 3), (125, 13, 3),
+                               (5, 3, 40)])
+def test_ct3d_tiles(n, nstages):
+    """The fused constrained transport (fusion level 2: at every size) at the edges of its
+    tiles of 62 x 6 faces and of its k segments."""
+    kw = cfg_kwargs(3, n, emf="uct_contact", recon="ppm" if min(n) >= 3 else "plm", nstages=nstages,
+                    cfl=0.3)
+    o, g = make_pair(kw, problems.random_mhd)
+    g.set_fusion(2)
+    o.set_boundaries()
+    for _ in range(2):
+        assert o.cycle() == 0
+        g.cycle()
+    compare_state(o, g, what="ct3d %s" % (n,))
