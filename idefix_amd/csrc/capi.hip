@@ -724,10 +724,11 @@ int idfx_check_divb(idfx_ctx *c, const double *Vs, double *divb, void *stream) {
 
 // One RK stage on the fused path.  When newdt_host is given in stage 0, the InvDt
 // maximum is copied to pinned memory asynchronously and ctx->ev_dt records it.
-// Boundary step of a stage.  In a box periodic along every active direction whose
-// interior cell field equals the face average (every stage after the first of a cycle:
-// the previous stage's ConsToPrim wrote it), one kernel fills every ghost zone with the
-// same values as the per-direction fill followed by ReconstructVcField.
+// Boundary step of a stage.  In a box periodic along every active direction one kernel
+// fills every ghost zone with the same values as the per-direction fill followed by
+// ReconstructVcField; the interior cell field is taken from the faces too unless it
+// already equals their average (every stage after the first of a cycle: the previous
+// stage's ConsToPrim wrote it).
 static bool all_periodic(const idfx_ctx *c) {
   for (int d = 0; d < c->d.dim; d++)
     if (c->d.lbound[d] != IDFX_BC_PERIODIC || c->d.rbound[d] != IDFX_BC_PERIODIC) return false;
@@ -735,8 +736,8 @@ static bool all_periodic(const idfx_ctx *c) {
 }
 static int stage_boundaries(idfx_ctx *c, double *Vc, double *Vs, bool cell_field_consistent,
                             hipStream_t s) {
-  if (all_periodic(c) && (cell_field_consistent || !c->d.mhd))
-    return check(c->ops->boundary_periodic(c->g, Vc, Vs, s));
+  if (all_periodic(c))
+    return check(c->ops->boundary_periodic(c->g, Vc, Vs, !cell_field_consistent, s));
   return idfx_set_boundaries(c, Vc, Vs, s);
 }
 

@@ -29,8 +29,9 @@ struct Ops {
                              double wc, double w0, hipStream_t s) = nullptr;
   hipError_t (*vc_field)(const GridDesc &g, const double *Vs, double *X,
                          hipStream_t s) = nullptr;
-  // all-periodic box: every ghost zone in one pass (see k_boundary_periodic)
-  hipError_t (*boundary_periodic)(const GridDesc &g, double *Vc, double *Vs,
+  // all-periodic box: every ghost zone in one pass, with field the interior cell field too
+  // (see k_boundary_periodic)
+  hipError_t (*boundary_periodic)(const GridDesc &g, double *Vc, double *Vs, bool field,
                                   hipStream_t s) = nullptr;
   hipError_t (*boundary)(const GridDesc &g, double *Vc, double *Vs, int dir, int lbc, int rbc,
                          hipStream_t s) = nullptr;
@@ -312,7 +313,8 @@ hipError_t launch_boundary(const GridDesc &g, double *Vc, double *Vs, int dir, i
 }
 
 template <class C>
-hipError_t launch_boundary_periodic(const GridDesc &g, double *Vc, double *Vs, hipStream_t s) {
+hipError_t launch_boundary_periodic(const GridDesc &g, double *Vc, double *Vs, bool field,
+                                    hipStream_t s) {
   constexpr int NF = C::MHD ? C::DIM : 0;
   long long total = 0;
   for (int f = -1; f < NF; f++)
@@ -325,7 +327,12 @@ hipError_t launch_boundary_periodic(const GridDesc &g, double *Vc, double *Vs, h
       }
       total += sz;
     }
-  hipLaunchKernelGGL((k_boundary_periodic<C>), dim3(blocks_for(total)), dim3(256), 0, s, g, Vc, Vs);
+  if (field && C::MHD) {
+    total += (long long)(g.end[0] - g.beg[0]) * (g.end[1] - g.beg[1]) * (g.end[2] - g.beg[2]);
+    hipLaunchKernelGGL((k_boundary_periodic<C, true>), dim3(blocks_for(total)), dim3(256), 0, s, g, Vc, Vs);
+  } else {
+    hipLaunchKernelGGL((k_boundary_periodic<C, false>), dim3(blocks_for(total)), dim3(256), 0, s, g, Vc, Vs);
+  }
   return hipGetLastError();
 }
 
