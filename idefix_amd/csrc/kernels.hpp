@@ -50,9 +50,9 @@ enum : int {
   SW_INVDT_ADD = 8,    // InvDt += term
   SW_DT_REDUCE = 16,   // fold max(InvDt) of the updated cells into *dtmax
   SW_NO_INVDT_STORE = 32,  // keep InvDt in registers only (requires SW_INVDT_SET)
-  // last sweep of a 3-D stage on the ping-pong schedule (the FIN kernels): the updated
-  // cell state goes through AddAndStore and the field-independent part of ConsToPrim
-  // into VcOut instead of back into Uc
+  // last sweep of a stage on the ping-pong schedule (the FIN kernels; hydro, 3-D MHD): the
+  // updated cell state goes through AddAndStore and ConsToPrim (with MHD its
+  // field-independent part) into VcOut instead of back into Uc
   SW_FINAL = 64,
   SW_RK = 128,         // with SW_FINAL: U = wc U + w0 U0 (stages after the first)
   SW_WRITE_UC = 256,   // with SW_FINAL: also store the combined U into Uc
@@ -418,8 +418,9 @@ __device__ __forceinline__ double cell_update(const GridDesc &g, const SweepArgs
   }
   if constexpr (FIN) {
     // the stage's last sweep (ping-pong schedule): the new state, its RK combination as
-    // in AddAndStore, and rho, v and E - kinetic energy of ConsToPrim into VcOut; the
-    // pressure and the cell field follow once the faces are updated (k_prs_from_faces)
+    // in AddAndStore, and ConsToPrim into VcOut: all of it for hydro; for MHD rho, v and E -
+    // kinetic energy, the pressure and the cell field following once the faces are updated
+    // (k_prs_from_faces)
     double un[C::NVAR], vo[C::NVAR];
 #pragma unroll
     for (int n = 0; n < C::NVAR; n++) {
@@ -435,7 +436,8 @@ __device__ __forceinline__ double cell_update(const GridDesc &g, const SweepArgs
       for (int n = 0; n < C::NVAR; n++)
         if (!C::is_ct_field(n)) st32(a.Uc + n * g.sv, p, un[n]);
     }
-    cons2prim_part<C>(un, vo);
+    if constexpr (C::MHD) cons2prim_part<C>(un, vo);
+    else cons2prim<C>(un, vo, g.gamma);
 #pragma unroll
     for (int n = 0; n < C::NVAR; n++)
       if (!C::is_ct_field(n)) st32(a.VcOut + n * g.sv, p, vo[n]);
@@ -507,7 +509,7 @@ template <class C>
 constexpr int x_waves_per_eu() {
   return (C::DIM == 3 && C::ORDER != RECON_PPM) || (C::MHD && C::NVAR >= 8 && C::ORDER == RECON_PPM) ? 3 : 4;
 }
-template <class C, typename T, bool FUSED, int EMF, bool XTRA>
+template <class C, typename T, bool FUSED, int EMF, bool XTRA, bool FIN = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(x_waves_per_eu<C>())))
 void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
   constexpr int NV = C::NVAR;
@@ -594,7 +596,7 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
                            k >= g.beg[2] && k < g.end[2];
       if (cell_ok) {
         const double A = a.uniform ? a.areax : face_A<C::DIM, IDIR>(g, k, j, c);
-        const double inv = cell_update<C, IDIR, XTRA>(g, a, p, A, k, j, c, F, Fp, cmax, cmaxp);
+        const double inv = cell_update<C, IDIR, XTRA, FIN>(g, a, p, A, k, j, c, F, Fp, cmax, cmaxp);
         red = __double_as_longlong(inv);
       }
     }

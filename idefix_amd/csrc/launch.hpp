@@ -114,7 +114,7 @@ hipError_t launch_sweep_xtra(const GridDesc &g, const SweepArgs &a, const EmfArr
     m.nj = fast_div_of(nj);
     m.nsites = (int)(m.ns.d * nj * nk);  // below 2^31: a block has fewer than 2^29 cells
     const long long waves = (m.nsites - XF + 62 - XF) / (63 - XF);
-    hipLaunchKernelGGL((k_sweep_x<C, T, FUSED, EMF, XTRA>), dim3(blocks_for(waves, 4)), dim3(256), 0, s, g,
+    hipLaunchKernelGGL((k_sweep_x<C, T, FUSED, EMF, XTRA, FIN>), dim3(blocks_for(waves, 4)), dim3(256), 0, s, g,
                        a, e, m);
   } else {
     MarchGeom m;
@@ -145,10 +145,10 @@ template <class C, typename T, int DIR, bool FUSED, int EMF>
 hipError_t launch_sweep_dir(const GridDesc &g, const SweepArgs &a, const EmfArrays<T> &e,
                             int target_waves, hipStream_t s) {
   if (a.flags & SW_FINAL) {
-    // the z sweep of the 3-D ping-pong schedule (adiabatic MHD, uct_contact, no per-cell
-    // options)
-    if constexpr (DIR == KDIR && C::DIM == 3 && C::MHD && !C::ISO && FUSED &&
-                  EMF == EMF_UCT_CONTACT) {
+    // the last sweep of the ping-pong schedule (hydro; 3-D adiabatic MHD with uct_contact;
+    // no per-cell options)
+    if constexpr (DIR == C::DIM - 1 && FUSED &&
+                  (!C::MHD || (C::DIM == 3 && !C::ISO && EMF == EMF_UCT_CONTACT))) {
       if (a.shock != nullptr || g.ntr > 0) return hipErrorInvalidValue;
       return launch_sweep_xtra<C, T, DIR, FUSED, EMF, false, true>(g, a, e, target_waves, s);
     } else {

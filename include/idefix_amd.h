@@ -219,11 +219,12 @@ int idfx_stage(idfx_ctx *ctx, int stage, int nstages, double dt, double cfl, dou
  * the dt update (CFL_max_var, first-cycle check, dt < 1e-15).  *t and *dt are updated;
  * ncycles is the index of this cycle.  On return the interior cells and interior faces of
  * Vc/Vs (and Uc) hold the new state; with the fused schedules (idfx_ctx_set_fusion: 2-D
- * MHD, and 3-D adiabatic MHD with uct_contact, no tracers, no shock flattening, no
+ * MHD, and 3-D adiabatic MHD with uct_contact and hydro, no tracers, no shock flattening, no
  * user-defined sides, whose stages alternate between Vc and context-owned state arrays)
  * the ghost zones hold the boundary values of an earlier stage, which the next stage's
  * boundary fill rewrites before any use, and the corner (2-D also y-face) EMF scratch
- * arrays are not written.  The first 3-D RK3 cycle allocates one more state array. */
+ * arrays are not written.  The first RK3 cycle of 3-D MHD or hydro allocates one more state
+ * array. */
 int idfx_cycle(idfx_ctx *ctx, int nstages, double cfl, double cfl_max_var, long ncycles,
                double *t, double *dt, double *Vc, double *Vs, double *Uc, double *InvDt,
                void *stream);
@@ -237,7 +238,9 @@ int idfx_cycle(idfx_ctx *ctx, int nstages, double cfl, double cfl_max_var, long 
  * leaves the edge EMF arrays unwritten and the face fields of ghost columns as they were;
  * for adiabatic 3-D MHD (no tracers, no shock flattening, no user-defined sides) the last
  * sweep also applies AddAndStore and the field-independent part of ConvertConsToPrim into
- * the next state array, and a pointwise kernel adds pressure and cell field.
+ * the next state array, and a pointwise kernel adds pressure and cell field.  Hydro (same
+ * conditions) starts with the last sweep doing both in full; level 0 makes ConvertConsToPrim
+ * its own kernel there too.
  * In 3-D, level 1 takes the fused CT kernel on blocks of at least 5 * 2^19 interior cells
  * and k_corner_emf + k_evolve_b below (the faster choice on MI355X); level 2 takes the
  * fused CT kernel at every size.  All levels give identical interior cells, faces and Uc.

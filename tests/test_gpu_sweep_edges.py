@@ -73,3 +73,28 @@ def test_ct3d_tiles(n, nstages):
         assert o.cycle() == 0
         g.cycle()
     compare_state(o, g, what="ct3d %s" % (n,))
+
+
+@pytest.mark.parametrize("nstages", [2, 3])
+@pytest.mark.parametrize("n,csiso", [((61,), None), ((61,), 0.9), ((130,), None), ((60, 7), None),
+                                     ((60, 7), 0.9), ((9, 66), None), ((5, 4, 6), None),
+                                     ((61, 4, 3), None)])
+def test_hydro_ping_pong_equals_in_place(n, nstages, csiso):
+    """Hydro stages whose last sweep converts the state (the default) against the schedule
+    with ConsToPrim as a kernel of its own: every bit of Vc and Uc, and dt, over three
+    cycles; and the oracle."""
+    import torch
+    kw = cfg_kwargs(len(n), n, mhd=False, solver="hllc", recon="plm", bc="outflow" if len(n) < 3 else
+                    "periodic", gamma=1.4, cfl=0.3, nstages=nstages, csiso=csiso)
+    o, g = make_pair(kw, problems.random_hd)
+    _, h = make_pair(kw, problems.random_hd)
+    h.set_fusion(0)
+    o.set_boundaries()
+    for _ in range(3):
+        assert o.cycle() == 0
+        g.cycle()
+        h.cycle()
+    assert g.dt == h.dt
+    assert torch.equal(g.interior(g.Vc), h.interior(h.Vc))
+    assert torch.equal(g.interior(g.Uc), h.interior(h.Uc))
+    compare_state(o, g, what="hydro %s" % (n,))
