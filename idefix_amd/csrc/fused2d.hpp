@@ -39,14 +39,11 @@ __device__ __forceinline__ T lane_at(T v, int lane, int off) {
   return __shfl(v, lane + off);
 }
 
-// 3 waves per SIMD for the 6-variable state; the 8-variable one (three vector components)
-// needs about 220 VGPRs and runs at 2
-template <class C>
-constexpr int fused2d_waves_per_eu() {
-  return C::NVAR >= 8 ? 2 : 3;
-}
+// Loads ahead and the window in LDS take 230-256 VGPRs and, with PPM, half a CU's LDS: 2
+// waves per SIMD.  (2048^2 PLM, 6 variables: 295 us a launch; at 3 waves, each load where it
+// is used, 351.)
 template <class C, typename T, int EMF, bool XTRA>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused2d_waves_per_eu<C>())))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGeom m) {
   static_assert(C::DIM == 2 && C::MHD, "2-D MHD only");
   constexpr int NV = C::NVAR;
@@ -77,106 +74,163 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
     const double dtdx1 = a.dt / g.dx[0][cc];  // evolveMagField.hpp:67 (dt/dx1(i))
     constexpr int emf = EMF;  // the corner-EMF scheme is a compile-time choice here
 
-    // PLM: the stencil rows a marching step shares with the next ones are carried in LDS
-    // (slot q of thread t at lds[q][t]) instead of being fetched again: each step then
-    // reads every input row once.  PPM reloads them (its wider window does not fit).
-    constexpr bool CARRY = C::ORDER != RECON_PPM;
+    // What a marching step shares with the next ones is carried in LDS (slot q of thread t
+    // at lds[q][t]): the window's last NW - 1 rows, the right state of the previous cell
+    // and, but for PPM's wider edge stencils, the rows the corner EMF reads.
+    constexpr bool PPM = C::ORDER == RECON_PPM;
+    constexpr bool CARRY = !PPM;
     constexpr bool HLLE = emf == EMF_UCT_HLL || emf == EMF_UCT_HLLD;
     constexpr bool NEED_E3 = emf == EMF_UCT0 || emf == EMF_UCT_CONTACT;
-    constexpr int RW = NW - 1;                  // window rows carried (PLM: f-1, f)
-    constexpr int S_BX = RW * NV;               // uct_hll(d): BX1s rows f-2 .. f (ring of 4)
+    constexpr int RW = NW - 1;                  // window rows carried (PLM 2, PPM 4)
+    constexpr int NS = NV - 1;                  // the normal field BX2 comes from Vs
+    constexpr int S_HD = RW * NS;               // right state of cell f-1
+    constexpr int S_BX = S_HD + NS;             // uct_hll(d): BX1s rows f-2 .. f (ring of 4)
     constexpr int S_EZ = S_BX + 4;              //             ezi rows f-2 .. f (ring of 4)
-    constexpr int S_AD = S_EZ + 4;              //             axL axR dxL dxR of row f-1
-    constexpr int S_E1 = RW * NV;               // others: ezi of row f-1
+    constexpr int S_AD = CARRY ? S_EZ + 4 : S_BX;  //          axL axR dxL dxR of row f-1
+    constexpr int S_E1 = S_BX;                  // others: ezi of row f-1
     constexpr int S_S1 = S_E1 + 1;              //         svx of row f-1
-    constexpr int NSLOT = CARRY ? (HLLE ? S_AD + 4 : S_S1 + 1) : 1;
+    constexpr int NSLOT = HLLE ? S_AD + 4 : S_S1 + 1;
     __shared__ T lds[NSLOT][256];
     const int tid = threadIdx.x;
-    auto wslot = [&](int row, int n) -> T & { return lds[(row & (RW - 1)) * NV + n][tid]; };
+    auto sl = [](int n) { return n > BX2 ? n - 1 : n; };
+    auto wslot = [&](int row, int n) -> T & { return lds[(row & (RW - 1)) * NS + sl(n)][tid]; };
     auto ld_row = [&](const T *arr, int row) { return ld32(arr, (unsigned)row * sd + col); };
 
-    T carry[NV], Fprev[NV];
+    T Fprev[NV], fcar[NV];
     T cprev = 0, ezprev = 0;
     double b2prev = 0.0;
-    // right-face value of cell c0-1: the left state of the first face
+    // right state of cell c0-1: the left state of the first face (PPM: and the value of that
+    // face)
 #pragma unroll
     for (int n = 0; n < NV; n++) {
       Fprev[n] = 0;
-      carry[n] = 0;
-      const bool keep = n != BX2 || NEED_E3;
-      if (n == BX2 && !(CARRY && keep)) continue;  // the normal field comes from Vs
+      fcar[n] = 0;
+      if (n == BX2) continue;
       T wv[NW];
 #pragma unroll
       for (int q = 0; q < NW; q++)
         wv[q] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 - 1 - H + q) * sd);
-      if constexpr (CARRY) {
-        if (keep) {
 #pragma unroll
-          for (int q = 1; q < NW; q++) wslot(c0 - 1 - H + q, n) = wv[q];
-        }
-      }
-      if (n == BX2) continue;
-      T dummy;
-      if constexpr (C::ORDER == RECON_MLP)
-        recon_mlp<C, JDIR>(wv, n, a.mlpw, g.sv, col + (unsigned)(c0 - 1) * sd, sd, dummy, carry[n]);
-      else
-        recon_cell<C>(wv, n, dummy, carry[n], recon_dx<C, T>(g, 1, c0 - 1),
+      for (int q = 1; q < NW; q++) wslot(c0 - 1 - H + q, n) = wv[q];
+      T dummy, right;
+      if constexpr (C::ORDER == RECON_MLP) {
+        recon_mlp<C, JDIR>(wv, n, a.mlpw, g.sv, col + (unsigned)(c0 - 1) * sd, sd, dummy, right);
+      } else if constexpr (PPM) {
+        fcar[n] = recon_face<C>(wv);
+        recon_ppm<C>(wv, n, ppm_face(wv[0], wv[1], wv[2], wv[3]), fcar[n], dummy, right);
+      } else {
+        recon_cell<C>(wv, n, dummy, right, recon_dx<C, T>(g, 1, c0 - 1),
                       XTRA && recon_flat<C>(a, col + (unsigned)(c0 - 1) * sd));
+      }
+      lds[S_HD + sl(n)][tid] = right;
     }
-    if constexpr (CARRY) {
-      if constexpr (HLLE) {
+    if constexpr (HLLE) {
+      if constexpr (CARRY) {
 #pragma unroll
         for (int r = c0 - 2; r <= c0; r++) {
           lds[S_BX + (r & 3)][tid] = (T)ld32(s.Vs_in, (unsigned)r * vsd + col);
           lds[S_EZ + (r & 3)][tid] = ld_row(e.ezi, r);
         }
-        lds[S_AD + 0][tid] = ld_row(e.axL, c0 - 1);
-        lds[S_AD + 1][tid] = ld_row(e.axR, c0 - 1);
-        lds[S_AD + 2][tid] = ld_row(e.dxL, c0 - 1);
-        lds[S_AD + 3][tid] = ld_row(e.dxR, c0 - 1);
-      } else {
-        lds[S_E1][tid] = ld_row(e.ezi, c0 - 1);
-        if constexpr (emf == EMF_UCT_CONTACT) lds[S_S1][tid] = sv_val<T>(ld32(e.svx, (unsigned)(c0 - 1) * sd + col));
       }
+      lds[S_AD + 0][tid] = ld_row(e.axL, c0 - 1);
+      lds[S_AD + 1][tid] = ld_row(e.axR, c0 - 1);
+      lds[S_AD + 2][tid] = ld_row(e.dxL, c0 - 1);
+      lds[S_AD + 3][tid] = ld_row(e.dxR, c0 - 1);
+    } else {
+      lds[S_E1][tid] = ld_row(e.ezi, c0 - 1);
+      if constexpr (emf == EMF_UCT_CONTACT) lds[S_S1][tid] = sv_val<T>(ld32(e.svx, (unsigned)(c0 - 1) * sd + col));
+    }
+    // the leading row of a step's window and its face field are loaded a step ahead, before
+    // the Riemann solve, so that they arrive under it
+    T nxt[NV];
+    double b2nxt = ld32(Vs1_in, (unsigned)c0 * vsd + col);
+#pragma unroll
+    for (int n = 0; n < NV; n++)
+      nxt[n] = n == BX2 ? T(0) : (T)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 + H) * sd);
+    // cell-centred E3 = vx2 Bx1 - vx1 Bx2 of cell f - 1, and the cell field BX2 of cell f
+    T E3_cm = T(0), bc2 = T(0);
+    if constexpr (NEED_E3) {
+      auto lc = [&](int n) { return (T)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 - 1) * sd); };
+      E3_cm = lc(C::MX2) * lc(C::BX1) - lc(C::MX1) * lc(BX2);
+      bc2 = (T)ld32(a.Vc + BX2 * g.sv, col + (unsigned)c0 * sd);
     }
     for (int f = c0; f <= c1; f++) {
       // ---- 1. y face f -------------------------------------------------------------
-      T win[NW][NV];
-#pragma unroll
-      for (int n = 0; n < NV; n++) {
-        const bool keep = n != BX2 || NEED_E3;
-        if (!keep) continue;
-        if constexpr (CARRY) {
-#pragma unroll
-          for (int q = 0; q < NW - 1; q++) win[q][n] = wslot(f - H + q, n);
-          win[NW - 1][n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(f + H) * sd);
-          wslot(f + H, n) = win[NW - 1][n];  // replaces row f-H, read above
-        } else {
-#pragma unroll
-          for (int q = 0; q < NW; q++)
-            win[q][n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(f - H + q) * sd);
-        }
+      const double b2old = b2nxt;
+      // what else the step reads, ahead of the reconstruction: the branches below would make
+      // each load wait for memory on its own (the begin state only where registers allow)
+      constexpr bool PRE_U0 = C::NVAR < 8;
+      const unsigned pf = (unsigned)f * sd + col, qf = (unsigned)f * vsd + col;
+      const unsigned p = pf - sd, q1 = qf - vsd;  // cell and x face of row f - 1
+      auto xf = [&](const T *arr, int r) { return ld32(arr, (unsigned)r * sd + col); };
+      T axL, axR, dxL, dxR, bhi, vhi, ezi_f;
+      unsigned char svx_f = 0;
+      double b1old = 0.0, z2 = 0.0, z1 = 0.0, upre[NV], u0pre[NV], invpre = 0.0;
+      if constexpr (HLLE) {
+        constexpr int SHI = C::ORDER == RECON_PPM ? 6 : 5;
+        axL = xf(e.axL, f);
+        axR = xf(e.axR, f);
+        dxL = xf(e.dxL, f);
+        dxR = xf(e.dxR, f);
+        bhi = (T)ld32(s.Vs_in, (unsigned)(f - 4 + SHI) * vsd + col);
+        vhi = xf(e.ezi, f - 4 + SHI);
+        if constexpr (!(CARRY && std::is_same<T, double>::value)) b1old = ld32(s.Vs_in, q1);
+      } else {
+        b1old = ld32(s.Vs_in, q1);
+        ezi_f = xf(e.ezi, f);
+        if constexpr (emf == EMF_UCT_CONTACT) svx_f = ld32(e.svx, pf);
       }
-      T vL[NV], vR[NV], vr_next[NV];
-      const bool flat = XTRA && recon_flat<C>(a, col + (unsigned)f * sd);
+      if (s.rk == 2) {
+        z2 = ld32((const double *)Vs1_0, qf);
+        if (f > c0) z1 = ld32((const double *)s.Vs0, q1);
+      }
+      if (f > c0 && cell_col) {
+#pragma unroll
+        for (int n = 0; n < NV; n++)
+          if (!C::is_ct_field(n)) upre[n] = ld32((const double *)a.Uc + n * g.sv, p);
+        if (PRE_U0 && s.rk == 2) {
+#pragma unroll
+          for (int n = 0; n < NV; n++)
+            if (!C::is_ct_field(n)) u0pre[n] = ld32((const double *)a.Uc0 + n * g.sv, p);
+        }
+        if (a.flags & SW_INVDT_ADD) invpre = ld32((const double *)a.InvDt, p);
+      }
+      T vL[NV], vR[NV];
+      T wc[NV];  // cell f
+      const bool flat = XTRA && recon_flat<C>(a, pf);
 #pragma unroll
       for (int n = 0; n < NV; n++) {
-        vL[n] = carry[n];
-        if (n == BX2) {
-          vR[n] = vr_next[n] = 0;
-          continue;
-        }
+        if (n == BX2) continue;
         T wv[NW];
 #pragma unroll
-        for (int q = 0; q < NW; q++) wv[q] = win[q][n];
-        if constexpr (C::ORDER == RECON_MLP)
-          recon_mlp<C, JDIR>(wv, n, a.mlpw, g.sv, col + (unsigned)f * sd, sd, vR[n], vr_next[n]);
-        else
-          recon_cell<C>(wv, n, vR[n], vr_next[n], recon_dx<C, T>(g, 1, f), flat);
+        for (int q = 0; q < NW - 1; q++) wv[q] = wslot(f - H + q, n);
+        wv[NW - 1] = nxt[n];
+        wslot(f + H, n) = nxt[n];  // replaces row f - H, read above
+        wc[n] = wv[H];
+        vL[n] = lds[S_HD + sl(n)][tid];
+        T right;
+        if constexpr (C::ORDER == RECON_MLP) {
+          recon_mlp<C, JDIR>(wv, n, a.mlpw, g.sv, pf, sd, vR[n], right);
+        } else if constexpr (PPM) {
+          const T fr = recon_face<C>(wv);
+          recon_ppm<C>(wv, n, fcar[n], fr, vR[n], right);
+          fcar[n] = fr;
+        } else {
+          recon_cell<C>(wv, n, vR[n], right, recon_dx<C, T>(g, 1, f), flat);
+        }
+        lds[S_HD + sl(n)][tid] = right;
       }
-      const double b2old = ld32(Vs1_in, (unsigned)f * vsd + col);
+      T E3_c = T(0);
+      if constexpr (NEED_E3) E3_c = wc[C::MX2] * wc[C::BX1] - wc[C::MX1] * bc2;
       vL[BX2] = (T)b2old;
       vR[BX2] = vL[BX2];
+      if (f < c1) {
+        b2nxt = ld32(Vs1_in, qf + vsd);
+#pragma unroll
+        for (int n = 0; n < NV; n++)
+          if (n != BX2) nxt[n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(f + 1 + H) * sd);
+        if constexpr (NEED_E3) bc2 = (T)ld32(a.Vc + BX2 * g.sv, pf + sd);
+      }
       T F[NV], cmax;
       FaceEmf<T> E;
       riemann<C, JDIR>(vL, vR, F, cmax, E, emf,
@@ -189,8 +243,6 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
 
       // ---- 2. corner EMF ez(c, f) ----------------------------------------------------
       T ez;
-      auto xf = [&](const T *arr, int row) { return ld32(arr, (unsigned)row * sd + col); };
-      double b1old;  // BX1s of row f-1
       if constexpr (HLLE) {
         constexpr int SLO = C::ORDER == RECON_PPM ? 1 : 2;
         constexpr int SHI = C::ORDER == RECON_PPM ? 6 : 5;
@@ -204,22 +256,14 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
         }
         T aL, aR, dL, dR;
         {
-          const T axL = xf(e.axL, f), axR = xf(e.axR, f), dxL = xf(e.dxL, f), dxR = xf(e.dxR, f);
-          if constexpr (CARRY) {
-            aL = T(0.5) * (lds[S_AD + 0][tid] + axL);
-            aR = T(0.5) * (lds[S_AD + 1][tid] + axR);
-            dL = T(0.5) * (lds[S_AD + 2][tid] + dxL);
-            dR = T(0.5) * (lds[S_AD + 3][tid] + dxR);
-            lds[S_AD + 0][tid] = axL;
-            lds[S_AD + 1][tid] = axR;
-            lds[S_AD + 2][tid] = dxL;
-            lds[S_AD + 3][tid] = dxR;
-          } else {
-            aL = T(0.5) * (xf(e.axL, f - 1) + axL);
-            aR = T(0.5) * (xf(e.axR, f - 1) + axR);
-            dL = T(0.5) * (xf(e.dxL, f - 1) + dxL);
-            dR = T(0.5) * (xf(e.dxR, f - 1) + dxR);
-          }
+          aL = T(0.5) * (lds[S_AD + 0][tid] + axL);
+          aR = T(0.5) * (lds[S_AD + 1][tid] + axR);
+          dL = T(0.5) * (lds[S_AD + 2][tid] + dxL);
+          dR = T(0.5) * (lds[S_AD + 3][tid] + dxR);
+          lds[S_AD + 0][tid] = axL;
+          lds[S_AD + 1][tid] = axR;
+          lds[S_AD + 2][tid] = dxL;
+          lds[S_AD + 3][tid] = dxR;
         }
         ez = edge_term<C>(b, v, aL, aR, dL, dR, true);
         // y faces: B = BX1s of x face c and v = ezi along y (rows f-4+s)
@@ -229,16 +273,18 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
             b[q] = lds[S_BX + ((f - 4 + q) & 3)][tid];
             v[q] = lds[S_EZ + ((f - 4 + q) & 3)][tid];
           }
-          b[SHI] = (T)ld32(s.Vs_in, (unsigned)(f - 4 + SHI) * vsd + col);
-          v[SHI] = xf(e.ezi, f - 4 + SHI);
+          b[SHI] = bhi;
+          v[SHI] = vhi;
           lds[S_BX + ((f - 4 + SHI) & 3)][tid] = b[SHI];
           lds[S_EZ + ((f - 4 + SHI) & 3)][tid] = v[SHI];
         } else {
 #pragma unroll
-          for (int q = SLO; q <= SHI; q++) {
+          for (int q = SLO; q < SHI; q++) {
             b[q] = (T)ld32(s.Vs_in, (unsigned)(f - 4 + q) * vsd + col);
             v[q] = xf(e.ezi, f - 4 + q);
           }
+          b[SHI] = bhi;
+          v[SHI] = vhi;
         }
         aL = T(0.5) * (lane_at(E.aL, lane, -1) + E.aL);
         aR = T(0.5) * (lane_at(E.aR, lane, -1) + E.aR);
@@ -247,28 +293,15 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
         ez += edge_term<C>(b, v, aL, aR, dL, dR, false);
         // BX1s of row f-1 is slot 3 of the stencil (exact when T is double)
         if constexpr (CARRY && std::is_same<T, double>::value) b1old = b[3];
-        else b1old = ld32(s.Vs_in, (unsigned)(f - 1) * vsd + col);
       } else {
-        b1old = ld32(s.Vs_in, (unsigned)(f - 1) * vsd + col);
         const T ezj_c = E.Et;
         const T ezj_m = lane_at(E.Et, lane, -1);
-        const T ezi_f = xf(e.ezi, f);
-        T ezi_m;
-        if constexpr (CARRY) {
-          ezi_m = lds[S_E1][tid];
-          lds[S_E1][tid] = ezi_f;
-        } else {
-          ezi_m = xf(e.ezi, f - 1);
-        }
+        const T ezi_m = lds[S_E1][tid];
+        lds[S_E1][tid] = ezi_f;
         if constexpr (emf == EMF_ARITHMETIC) {
           ez = T(0.25) * (ezi_f + ezi_m + ezj_c + ezj_m);
         } else {
-          // cell-centred E3 = vx2 Bx1 - vx1 Bx2 of cells (c, f-1), (c, f) and column c-1
-          auto e3 = [&](int q) {
-            return win[q][C::MX2] * win[q][C::BX1] - win[q][C::MX1] * win[q][C::BX2];
-          };
-          const T E3_cm = e3(H - 1);  // cell (c, f-1)
-          const T E3_c = e3(H);       // cell (c, f)
+          // cells (c, f-1), (c, f) and column c-1
           const T E3_mm = lane_at(E3_cm, lane, -1);
           const T E3_m = lane_at(E3_c, lane, -1);
           if constexpr (emf == EMF_UCT0) {
@@ -278,14 +311,9 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
             const T a4 = T(2) * ezj_m - T(0.5) * (E3_mm + E3_m);
             ez = T(0.25) * (a1 + a2 + a3 + a4);
           } else {
-            const T svx_c = sv_val<T>(ld32(e.svx, (unsigned)f * sd + col));
-            T svx_m;
-            if constexpr (CARRY) {
-              svx_m = lds[S_S1][tid];
-              lds[S_S1][tid] = svx_c;
-            } else {
-              svx_m = sv_val<T>(ld32(e.svx, (unsigned)(f - 1) * sd + col));
-            }
+            const T svx_c = sv_val<T>(svx_f);
+            const T svx_m = lds[S_S1][tid];
+            lds[S_S1][tid] = svx_c;
             const T svy_c = E.sv, svy_m = lane_at(E.sv, lane, -1);
             const T ez_l2 = (1 - svx_m) * (ezj_c - E3_cm) + (svx_m) * (ezj_m - E3_mm);
             const T ez_r2 = (1 - svx_c) * (ezj_c - E3_c) + (svx_c) * (ezj_m - E3_m);
@@ -299,17 +327,15 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
       // ---- 3. face fields ------------------------------------------------------------
       const T ezp = lane_at(ez, lane, 1);
       double b2new = b2old + dtdx1 * ((double)ezp - (double)ez);
-      if (s.rk == 2) b2new = s.wc * b2new + s.w0 * ld32((const double *)Vs1_0, (unsigned)f * vsd + col);
+      if (s.rk == 2) b2new = s.wc * b2new + s.w0 * z2;
       if (cell_col && (f < c1 || c1 == g.end[1])) {
-        const unsigned q = (unsigned)f * vsd + col;
-        if (s.rk == 1) st32(Vs1_0, q, b2old);
-        st32(Vs1_out, q, b2new);
+        if (s.rk == 1) st32(Vs1_0, qf, b2old);
+        st32(Vs1_out, qf, b2new);
       }
       if (f > c0) {
         const int fr = f - 1;
-        const unsigned q1 = (unsigned)fr * vsd + col;
         double b1new = b1old + (0.0 - a.dt / g.dx[1][fr] * ((double)ez - (double)ezprev));
-        if (s.rk == 2) b1new = s.wc * b1new + s.w0 * ld32((const double *)s.Vs0, q1);
+        if (s.rk == 2) b1new = s.wc * b1new + s.w0 * z1;
         const double b1next = __shfl(b1new, lane + 1);
         if (out_col) {
           if (s.rk == 1) st32(s.Vs0, q1, b1old);
@@ -317,7 +343,6 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
         }
         // ---- 4. cell (c, f-1) ---------------------------------------------------------
         if (cell_col) {
-          const unsigned p = (unsigned)fr * sd + col;
           const double dtdV = a.uniform ? a.dtdV : a.dt / cell_dV<2>(g, 0, fr, c);
           const double A = face_A<2, JDIR>(g, 0, fr, c);
           double u[NV], v[NV];
@@ -325,11 +350,10 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
           for (int n = 0; n < NV; n++) {
             if (C::is_ct_field(n)) continue;
             const double rhs = -dtdV * ((double)F[n] * A - (double)Fprev[n] * A);
-            u[n] = ld32((const double *)a.Uc + n * g.sv, p) + rhs;
+            u[n] = upre[n] + rhs;
           }
-          const double term = 0.5 * ((double)cmax + (double)cprev) / (g.dx[1][fr]);
           if (a.flags & SW_INVDT_ADD) {
-            const double inv = ld32((const double *)a.InvDt, p) + term;
+            const double inv = invpre + 0.5 * ((double)cmax + (double)cprev) / (g.dx[1][fr]);
             st32(a.InvDt, p, inv);
             const unsigned long long bb = __double_as_longlong(inv);
             red = bb > red ? bb : red;
@@ -338,7 +362,7 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
 #pragma unroll
             for (int n = 0; n < NV; n++)
               if (!C::is_ct_field(n))
-                u[n] = s.wc * u[n] + s.w0 * ld32((const double *)a.Uc0 + n * g.sv, p);
+                u[n] = s.wc * u[n] + s.w0 * (PRE_U0 ? u0pre[n] : ld32((const double *)a.Uc0 + n * g.sv, p));
           }
           u[C::BX1] = 0.5 * (b1new + b1next);
           u[C::BX2] = 0.5 * (b2prev + b2new);
@@ -352,10 +376,8 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
         }
       }
 #pragma unroll
-      for (int n = 0; n < NV; n++) {
-        carry[n] = vr_next[n];
-        Fprev[n] = F[n];
-      }
+      for (int n = 0; n < NV; n++) Fprev[n] = F[n];
+      E3_cm = E3_c;
       cprev = cmax;
       ezprev = ez;
       b2prev = b2new;

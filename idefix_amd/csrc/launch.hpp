@@ -74,21 +74,34 @@ long long resident_waves(K kernel, int target_waves) {
   return (long long)nb * 4 * std::max(1, target_waves / 32);
 }
 
-// Segment length of a marching kernel: minimises the modelled duration
-// ceil(waves / slots) x (ts + 2), waves = columns x ceil(nd / ts), where ts + 2 counts the
-// ts cells, the extra face and the window priming of one segment.
-inline int march_segment(long long columns, int nd, long long slots) {
+// Segment length of a marching kernel: minimises the modelled duration (ts + 2) x s over
+// the segment's cells ts, waves = columns x ceil(nd / ts); ts + 2 counts the extra face and
+// the window priming of one segment, and s, a step's duration, is the waves that share a
+// SIMD, but at least `fill`, the number that run side by side without slowing each other;
+// past the resident waves (slots), whole rounds of them.  The FP64 MHD kernels, bound by
+// instruction latency when alone on a SIMD and by issue beyond, have a fill of 2: their small
+// grids take short segments (2-D turbulence 256^2 marches 1 cell instead of 4, 1280 waves
+// instead of 320: 211 -> 166 us a cycle; Orszag-Tang 512^2 122 -> 115).  The others wait for
+// memory and gain up to the last resident wave (fill 0): with a fill of 2 the inference took
+// 261 instead of 193 us at 128^3, the hydro z sweep of 181x133x120 121 instead of 104.
+inline int march_segment(long long columns, int nd, long long slots, double fill) {
+  const double simds = 1024.0, full = (double)slots / simds;
+  if (fill <= 0.0 || fill > full) fill = full;
   double best = 1e300;
   int bt = nd;
-  for (int ts = std::min(nd, 4); ts <= nd; ts++) {
+  for (int ts = 1; ts <= nd; ts++) {
     const long long waves = columns * ((nd + ts - 1) / ts);
-    const double cost = (double)((waves + slots - 1) / slots) * (ts + 2);
-    if (cost < best) {
-      best = cost;
+    const double s = waves <= slots ? std::max(fill, waves / simds) : (double)((waves + slots - 1) / slots) * full;
+    if (s * (ts + 2) < best) {
+      best = s * (ts + 2);
       bt = ts;
     }
   }
   return bt;
+}
+template <class C, typename T>
+constexpr double march_fill() {
+  return C::MHD && std::is_same<T, double>::value ? 2.0 : 0.0;
 }
 
 inline FastDiv fast_div_of(unsigned d) {
@@ -130,7 +143,7 @@ hipError_t launch_sweep_xtra(const GridDesc &g, const SweepArgs &a, const EmfArr
     const long long columns = m.ncb;
     static const long long slots =
         resident_waves(k_sweep_march<C, T, DIR, FUSED, EMF, XTRA, FIN>, target_waves);
-    m.ts = march_segment(columns, nd, slots);
+    m.ts = march_segment(columns, nd, slots, march_fill<C, T>());
     m.nseg = (nd + m.ts - 1) / m.ts;
     const long long waves = (columns + m.grp - 1) / m.grp * m.grp * m.nseg;
     hipLaunchKernelGGL((k_sweep_march<C, T, DIR, FUSED, EMF, XTRA, FIN>), dim3(blocks_for(waves, 4)),
@@ -240,15 +253,24 @@ hipError_t launch_ct3d(const GridDesc &g, const double *Vc, double *Vs, double *
                        const void *emf, double dt, int mode, double wc, double w0,
                        hipStream_t s) {
   if constexpr (C::MHD && C::DIM == 3) {
-    // k segments: march_segment's rule with blocks for columns and the chip's 256 CUs (one
-    // block each) for slots.  From 256 tiles on, 512 slots, which leads to fewer, longer
+    // k segments of kseg planes: the least rounds of the chip's 256 CUs (one block each) x
+    // (kseg + 2).  From 256 tiles on, 512 slots, which leads to fewer, longer
     // segments: the XCDs then work near one plane (512^3, 468 tiles: 5.2 against 5.6 ms;
     // 203x150x97, 64 tiles, with 512: 161 against 147 us).
     const int nfi = g.end[0] - g.beg[0] + 1, nfj = g.end[1] - g.beg[1] + 1;
     const int nfk = g.end[2] - g.beg[2] + 1;
     const int nti = (nfi + CT_TI - 1) / CT_TI, ntj = (nfj + CT_TJ - 1) / CT_TJ;
     const long long tiles = (long long)nti * ntj;
-    const int kseg = march_segment(tiles, nfk, tiles >= 256 ? 512 : 256);
+    const long long slots = tiles >= 256 ? 512 : 256;
+    int kseg = nfk;
+    double best = 1e300;
+    for (int q = std::min(nfk, 4); q <= nfk; q++) {
+      const double cost = (double)((tiles * ((nfk + q - 1) / q) + slots - 1) / slots) * (q + 2);
+      if (cost < best) {
+        best = cost;
+        kseg = q;
+      }
+    }
     const int nseg = (nfk + kseg - 1) / kseg;
     hipLaunchKernelGGL((k_ct3d<C, T>), dim3((unsigned)(tiles * nseg)), dim3((CT_TJ + 2) * 64), 0, s,
                        g, Vc, Vs, Vs0, *static_cast<const EmfArrays<T> *>(emf), dt, mode, wc, w0,
@@ -425,14 +447,14 @@ hipError_t launch_fused2d_y_emf(const GridDesc &g, const SweepArgs &a, const voi
   const int nd = g.end[1] - g.beg[1];
   if (a.shock != nullptr) {
     static const long long slots = resident_waves(k_fused2d_y<C, T, EMF, true>, target_waves);
-    m.ts = march_segment(m.nxb, nd, slots);
+    m.ts = march_segment(m.nxb, nd, slots, march_fill<C, T>());
     m.nseg = (nd + m.ts - 1) / m.ts;
     const long long waves = (long long)m.nxb * m.nseg;
     hipLaunchKernelGGL((k_fused2d_y<C, T, EMF, true>), dim3(blocks_for(waves, 4)), dim3(256), 0,
                        s, g, a, *static_cast<const EmfArrays<T> *>(emf), f, m);
   } else {
     static const long long slots = resident_waves(k_fused2d_y<C, T, EMF, false>, target_waves);
-    m.ts = march_segment(m.nxb, nd, slots);
+    m.ts = march_segment(m.nxb, nd, slots, march_fill<C, T>());
     m.nseg = (nd + m.ts - 1) / m.ts;
     const long long waves = (long long)m.nxb * m.nseg;
     hipLaunchKernelGGL((k_fused2d_y<C, T, EMF, false>), dim3(blocks_for(waves, 4)), dim3(256), 0,
@@ -487,7 +509,7 @@ hipError_t launch_mlp_dir(const GridDesc &g, const double *Vc, const MlpNet &net
     m.nf = n[DIR];
     const long long ncb = (m.n + 15) / 16;
     static const long long slots = resident_waves(k_mlp_infer<C, DIR>, 256 * 32);
-    m.ts = march_segment(ncb, m.nf, slots);
+    m.ts = march_segment(ncb, m.nf, slots, 0.0);
     m.nseg = (m.nf + m.ts - 1) / m.ts;
     waves = ncb * m.nseg;
   }

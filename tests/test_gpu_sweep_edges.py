@@ -98,3 +98,18 @@ def test_hydro_ping_pong_equals_in_place(n, nstages, csiso):
     assert torch.equal(g.interior(g.Vc), h.interior(h.Vc))
     assert torch.equal(g.interior(g.Uc), h.interior(h.Uc))
     compare_state(o, g, what="hydro %s" % (n,))
+
+
+@pytest.mark.parametrize("emf,recon", [("uct_hlld", "plm"), ("uct_hlld", "ppm"), ("uct_contact", "plm"),
+                                       ("uct_contact", "ppm"), ("uct0", "plm"), ("arithmetic", "ppm")])
+@pytest.mark.parametrize("n", [(4, 3), (57, 4), (60, 5), (62, 3), (63, 9), (124, 4), (20, 70)])
+def test_mhd_2d_fused(n, emf, recon):
+    """The fused second half of a 2-D stage at the edges of its waves' columns (57 to 62 of 64
+    lanes own one) and at the one-cell segments small grids take."""
+    kw = cfg_kwargs(2, n, emf=emf, recon=recon, nstages=2, cfl=0.3)
+    o, g = make_pair(kw, problems.random_mhd)
+    o.set_boundaries()
+    for _ in range(2):
+        assert o.cycle() == 0
+        g.cycle()
+    compare_state(o, g, what="%s %s %s" % (emf, recon, n))
