@@ -43,23 +43,32 @@ __device__ __forceinline__ f4 mfma(float a, float b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// LDS, in floats.  Weights, rows padded so that a lane's four consecutive inputs come in
-// one 16-byte read without bank conflicts (row strides of an odd number of 16-byte units):
-// transposed [out][in] for the forward pass, [in][out] for the backward pass.  The tile's
-// activations and deltas [row][unit] take their place for the weight gradients (strides of
-// 16 mod 32 floats).
-constexpr int L_WT1 = 0, S_WT1 = 52, L_WT2 = L_WT1 + NH * S_WT1, S_W2 = 68,
-              L_W2 = L_WT2 + NH * S_W2, L_WT3 = L_W2 + NH * S_W2, L_W3 = L_WT3 + NO * S_W2,
-              S_W3 = 20, L_B = L_W3 + NH * S_W3, L_END = L_B + 2 * NH + NO;
+// LDS, in floats.  Weights [in][out], rows padded to strides (68, 20) that keep the reads of
+// both passes free of bank conflicts: forward a lane reads one output of four inputs 4 g + r,
+// backward four consecutive outputs of one input.  The tile's activations and deltas
+// [row][unit] take their place for the weight gradients (strides of 16 mod 32 floats).
+constexpr int S_W = 68, S_W3 = 20, L_W1 = 0, L_W2 = L_W1 + NF * S_W, L_W3 = L_W2 + NH * S_W,
+              L_B = L_W3 + NH * S_W3, L_WEND = L_B + 2 * NH + NO;
 constexpr int S_X = 48, S_H = 80, S_O = 16, L_X = 0, L_H1 = L_X + TR * S_X,
               L_H2 = L_H1 + TR * S_H, L_D1 = L_H2 + TR * S_H, L_D2 = L_D1 + TR * S_H,
               L_D3 = L_D2 + TR * S_H;
-static_assert(L_D3 + TR * S_O <= L_END, "the gradient buffers reuse the weights' space");
+constexpr int L_GEND = L_D3 + TR * S_O, L_END = L_GEND > L_WEND ? L_GEND : L_WEND;
 
-// acc[t] += W[16 t + .][16 NI units] in over the inputs in[NI] (units 16 i + 4 g + r of the
-// lane's row in in[i][r]); w is the lane's row of the weights, rows 16 apart by 16 stride.
+// Forward: acc[t] += W^T in over the inputs in[NI] (inputs 16 i + 4 g + r of the lane's row
+// in in[i][r]); w points at the lane's input 4 g and output q of tile 0.
 template <int NT, int NI>
-__device__ __forceinline__ void layer(const float *w, int stride, const f4 *in, f4 *acc) {
+__device__ __forceinline__ void forward(const float *w, int stride, const f4 *in, f4 *acc) {
+#pragma unroll
+  for (int i = 0; i < NI; i++)
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+        acc[t] = mfma(w[(16 * i + r) * stride + 16 * t], in[i][r], acc[t]);
+}
+// Backward: acc[t] += W in over the outputs; w points at the lane's input q and output 4 g.
+template <int NT, int NI>
+__device__ __forceinline__ void backward(const float *w, int stride, const f4 *in, f4 *acc) {
 #pragma unroll
   for (int i = 0; i < NI; i++) {
     f4 a[NT];
@@ -81,8 +90,9 @@ __device__ __forceinline__ void layer(const float *w, int stride, const f4 *in, 
 // block's tiles and go out once per block.  Everything is FP32 (products, accumulators,
 // activations).  208 + 128 matrix instructions per 16 rows: 2.2 us of the matrix cores'
 // time at 8192 rows; the kernel is bound by its serial chain of layers.  A step of 8192
-// rows takes 51 us; the eleven kernels this replaces (one thread per activation, scalar
-// products) took 716, 555 of them in the weight gradients.
+// rows takes 31 us, 18 of them here (33 with the weights loaded and transposed one float at a
+// time); the eleven kernels this replaces (one thread per activation, scalar products) took
+// 716, 555 of them in the weight gradients.
 __global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU, int B,
                                                const float *P, float *partial,
                                                double *lossp) {
@@ -103,19 +113,38 @@ __global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU,
   const float inv = 1.0f / (float)B;
   for (int tile = blockIdx.x; tile * TR < B; tile += gridDim.x) {
     __syncthreads();  // the previous tile's gradient buffers have been read
-    for (int e = tid; e < NF * NH; e += 128) lds[L_WT1 + (e % NH) * S_WT1 + e / NH] = P[P_W1 + e];
-    for (int e = tid; e < NH * NH; e += 128) {
-      const float v = P[P_W2 + e];
-      lds[L_WT2 + (e % NH) * S_W2 + e / NH] = v;
-      lds[L_W2 + e / NH * S_W2 + e % NH] = v;
+    {
+      // 16 consecutive floats of a thread's loads in flight at a time; every block of P
+      // starts at a multiple of four floats
+      const f4 *p1 = reinterpret_cast<const f4 *>(P + P_W1), *p2 = reinterpret_cast<const f4 *>(P + P_W2);
+      const f4 *p3 = reinterpret_cast<const f4 *>(P + P_W3);
+      f4 v1[NF * NH / 512], v2[NH * NH / 512], v3[NH * NO / 512];
+#pragma unroll
+      for (int n = 0; n < NF * NH / 512; n++) v1[n] = p1[tid + 128 * n];
+#pragma unroll
+      for (int n = 0; n < NH * NH / 512; n++) v2[n] = p2[tid + 128 * n];
+#pragma unroll
+      for (int n = 0; n < NH * NO / 512; n++) v3[n] = p3[tid + 128 * n];
+      const float bias = P[tid < NH ? P_B1 + tid : P_B2 + tid - NH];
+      const float bias3 = tid < NO ? P[P_B3 + tid] : 0.0f;
+#pragma unroll
+      for (int n = 0; n < NF * NH / 512; n++) {
+        const int e = tid + 128 * n;  // 16 groups of four per row
+        *reinterpret_cast<f4 *>(lds + L_W1 + e / 16 * S_W + e % 16 * 4) = v1[n];
+      }
+#pragma unroll
+      for (int n = 0; n < NH * NH / 512; n++) {
+        const int e = tid + 128 * n;
+        *reinterpret_cast<f4 *>(lds + L_W2 + e / 16 * S_W + e % 16 * 4) = v2[n];
+      }
+#pragma unroll
+      for (int n = 0; n < NH * NO / 512; n++) {
+        const int e = tid + 128 * n;  // four groups per row
+        *reinterpret_cast<f4 *>(lds + L_W3 + e / 4 * S_W3 + e % 4 * 4) = v3[n];
+      }
+      lds[L_B + tid] = bias;
+      if (tid < NO) lds[L_B + 2 * NH + tid] = bias3;
     }
-    for (int e = tid; e < NH * NO; e += 128) {
-      const float v = P[P_W3 + e];
-      lds[L_WT3 + (e % NO) * S_W2 + e / NO] = v;
-      lds[L_W3 + e / NO * S_W3 + e % NO] = v;
-    }
-    for (int e = tid; e < 2 * NH + NO; e += 128)
-      lds[L_B + e] = P[e < NH ? P_B1 + e : e < 2 * NH ? P_B2 + e - NH : P_B3 + e - 2 * NH];
     __syncthreads();
 
     const int row = tile * TR + 16 * wave + q;
@@ -141,7 +170,7 @@ __global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU,
     f4 s1[4], s2[4], h[4], h1[4];
 #pragma unroll
     for (int t = 0; t < 4; t++) z1[t] = *reinterpret_cast<const f4 *>(lds + L_B + 16 * t + 4 * g);
-    layer<4, 3>(lds + L_WT1 + q * S_WT1 + 4 * g, S_WT1, x, z1);
+    forward<4, 3>(lds + L_W1 + 4 * g * S_W + q, S_W, x, z1);
 #pragma unroll
     for (int t = 0; t < 4; t++)
 #pragma unroll
@@ -151,7 +180,7 @@ __global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU,
       }
 #pragma unroll
     for (int t = 0; t < 4; t++) z2[t] = *reinterpret_cast<const f4 *>(lds + L_B + NH + 16 * t + 4 * g);
-    layer<4, 4>(lds + L_WT2 + q * S_W2 + 4 * g, S_W2, h1, z2);
+    forward<4, 4>(lds + L_W2 + 4 * g * S_W + q, S_W, h1, z2);
 #pragma unroll
     for (int t = 0; t < 4; t++)
 #pragma unroll
@@ -160,7 +189,7 @@ __global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU,
         h[t][r] = z2[t][r] * s2[t][r];
       }
     z3 = *reinterpret_cast<const f4 *>(lds + L_B + 2 * NH + 4 * g);
-    layer<1, 4>(lds + L_WT3 + q * S_W2 + 4 * g, S_W2, h, &z3);
+    forward<1, 4>(lds + L_W3 + 4 * g * S_W3 + q, S_W3, h, &z3);
     // loss and dloss/dz3 (1/B included): wL = wpL + z3[2v], wR = wpR - z3[2v]
     f4 d3 = f4{0, 0, 0, 0};
 #pragma unroll
@@ -183,7 +212,7 @@ __global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU,
     for (int t = 0; t < 4; t++)
 #pragma unroll
       for (int r = 0; r < 4; r++) d2[t][r] *= gelu_d(z2[t][r], s2[t][r]);
-    layer<4, 4>(lds + L_W2 + q * S_W2 + 4 * g, S_W2, d2, d1);
+    backward<4, 4>(lds + L_W2 + q * S_W + 4 * g, S_W, d2, d1);
 #pragma unroll
     for (int t = 0; t < 4; t++)
 #pragma unroll
@@ -222,6 +251,7 @@ __global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU,
         g3[n] = mfma(a2[16 * n], dz3, g3[n]);
       }
     }
+#pragma unroll
     for (int r = 0; r < TR; r++) {
       gb += lds[(wave ? L_D2 : L_D1) + r * S_H + (tid & 63)];
       if (tid < NO) gb3 += lds[L_D3 + r * S_O + tid];
@@ -250,7 +280,8 @@ __global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU,
 
 // G = sum of the blocks' gradients, 32 parameters per block of 256 threads (8 slices of the
 // blocks, then the slices, in a fixed order), and with ADAM the step (Kingma & Ba 2015,
-// bias correction c1, c2).  Block 0 also sums the loss.
+// bias correction c1, c2).  Block 0 also sums the loss.  Eight loads in flight per thread: 6
+// instead of 11 us for 256 blocks.
 struct AdamArgs {
   float lr, b1, b2, eps, c1, c2;
 };
@@ -263,8 +294,17 @@ __global__ __launch_bounds__(256) void k_reduce(const float *partial, const doub
   const int c = threadIdx.x & 31, sl = threadIdx.x >> 5;
   const int e = blockIdx.x * 32 + c;
   float s = 0.0f;
-  if (e < P_N)
-    for (int b = sl; b < nblk; b += 8) s += partial[(long long)b * P_N + e];
+  if (e < P_N) {
+    int b = sl;
+    for (; b + 56 < nblk; b += 64) {  // eight loads in flight
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) v[k] = partial[(long long)(b + 8 * k) * P_N + e];
+#pragma unroll
+      for (int k = 0; k < 8; k++) s += v[k];
+    }
+    for (; b < nblk; b += 8) s += partial[(long long)b * P_N + e];
+  }
   red[sl][c] = s;
   __syncthreads();
   if (sl == 0 && e < P_N) {
