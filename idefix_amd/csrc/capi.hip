@@ -91,6 +91,7 @@ struct idfx_ctx {
   unsigned long long *dtmax = nullptr, *divb = nullptr;  // device scalars
   unsigned char *shock = nullptr;  // shock flags (shock flattening on)
   unsigned long long *host = nullptr;                    // pinned readback
+  bool dt_clean = true;  // dtmax is zero (once the work enqueued so far has run)
   hipEvent_t ev_dt = nullptr;
   int target_waves = 8192;
   bool fp32 = false;
@@ -565,11 +566,10 @@ int idfx_ctx_array(idfx_ctx *c, int which, double **ptr) {
   return *ptr ? IDFX_OK : IDFX_E_ARGS;
 }
 
-int idfx_enforce_boundary_dir(idfx_ctx *c, int dir, double *Vc, double *Vs, void *stream) {
-  if (!c || !Vc || (c->d.mhd && !Vs) || dir < 0 || dir >= c->d.dim) return IDFX_E_ARGS;
+static int enforce_dir(idfx_ctx *c, int dir, double *Vc, double *Vs, DtTake tk, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   // built-in side types (user-defined sides are left alone by the kernel)
-  IDFX_TRY(check(c->ops->boundary(c->g, Vc, Vs, dir, c->d.lbound[dir], c->d.rbound[dir], s)));
+  IDFX_TRY(check(c->ops->boundary(c->g, Vc, Vs, dir, c->d.lbound[dir], c->d.rbound[dir], tk, s)));
   for (int side = 0; side < 2; side++) {
     const int bc = side == 0 ? c->d.lbound[dir] : c->d.rbound[dir];
     if (bc != IDFX_BC_USERDEF) continue;
@@ -578,6 +578,11 @@ int idfx_enforce_boundary_dir(idfx_ctx *c, int dir, double *Vc, double *Vs, void
     c->user_fn(c->user_arg, dir, side, c->t_bound, Vc, Vs, stream);
   }
   return IDFX_OK;
+}
+
+int idfx_enforce_boundary_dir(idfx_ctx *c, int dir, double *Vc, double *Vs, void *stream) {
+  if (!c || !Vc || (c->d.mhd && !Vs) || dir < 0 || dir >= c->d.dim) return IDFX_E_ARGS;
+  return enforce_dir(c, dir, Vc, Vs, DtTake{}, stream);
 }
 
 int idfx_reconstruct_normal_field(idfx_ctx *c, int dir, double *Vs, void *stream) {
@@ -589,15 +594,19 @@ int idfx_reconstruct_normal_field(idfx_ctx *c, int dir, double *Vs, void *stream
   return check(c->ops->normal_field(c->g, Vs, dir, recL, recR, (hipStream_t)stream));
 }
 
-int idfx_set_boundaries(idfx_ctx *c, double *Vc, double *Vs, void *stream) {
-  if (!c || !Vc || (c->d.mhd && !Vs)) return IDFX_E_ARGS;
+static int set_boundaries(idfx_ctx *c, double *Vc, double *Vs, DtTake tk, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   for (int dir = 0; dir < c->d.dim; dir++) {
-    IDFX_TRY(idfx_enforce_boundary_dir(c, dir, Vc, Vs, stream));
+    IDFX_TRY(enforce_dir(c, dir, Vc, Vs, dir == 0 ? tk : DtTake{}, stream));
     if (c->d.mhd) IDFX_TRY(idfx_reconstruct_normal_field(c, dir, Vs, stream));
   }
   if (c->d.mhd) IDFX_TRY(check(c->ops->vc_field(c->g, Vs, Vc, s)));
   return IDFX_OK;
+}
+
+int idfx_set_boundaries(idfx_ctx *c, double *Vc, double *Vs, void *stream) {
+  if (!c || !Vc || (c->d.mhd && !Vs)) return IDFX_E_ARGS;
+  return set_boundaries(c, Vc, Vs, DtTake{}, stream);
 }
 
 int idfx_ctx_set_userdef_boundary(idfx_ctx *c, idfx_userdef_boundary_fn fn, void *arg) {
@@ -703,6 +712,7 @@ int idfx_evolve_stage(idfx_ctx *c, double t, double dt, const double *Vc, double
 int idfx_compute_timestep(idfx_ctx *c, const double *InvDt, double *dtmin, void *stream) {
   if (!c || !dtmin) return IDFX_E_ARGS;
   hipStream_t s = (hipStream_t)stream;
+  c->dt_clean = false;
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, c->dtmax);
   hipLaunchKernelGGL(k_invdt_max, dim3(1024), dim3(256), 0, s, c->g, InvDt ? InvDt : c->InvDt,
                      c->dtmax);
@@ -732,8 +742,6 @@ int idfx_check_divb(idfx_ctx *c, const double *Vs, double *divb, void *stream) {
   return IDFX_OK;
 }
 
-// One RK stage on the fused path.  When newdt_host is given in stage 0, the InvDt
-// maximum is copied to pinned memory asynchronously and ctx->ev_dt records it.
 // Boundary step of a stage.  In a box periodic along every active direction one kernel
 // fills every ghost zone with the same values as the per-direction fill followed by
 // ReconstructVcField; the interior cell field is taken from the faces too unless it
@@ -745,10 +753,39 @@ static bool all_periodic(const idfx_ctx *c) {
   return true;
 }
 static int stage_boundaries(idfx_ctx *c, double *Vc, double *Vs, bool cell_field_consistent,
-                            hipStream_t s) {
+                            DtTake tk, hipStream_t s) {
   if (all_periodic(c))
-    return check(c->ops->boundary_periodic(c->g, Vc, Vs, !cell_field_consistent, s));
-  return idfx_set_boundaries(c, Vc, Vs, s);
+    return check(c->ops->boundary_periodic(c->g, Vc, Vs, !cell_field_consistent, tk, s));
+  return set_boundaries(c, Vc, Vs, tk, s);
+}
+
+// What a stage does for the next time step.  A cycle of several stages reduces InvDt in the
+// first (DT_REDUCE) and takes the maximum to the host, with ctx->ev_dt behind it, in the
+// second's boundary kernel (DT_TAKE); DT_ALL does everything in one stage.
+enum { DT_NONE, DT_REDUCE, DT_TAKE, DT_ALL };
+// dtmax is cleared by its last reader, or here after any other use.
+static int dt_begin(idfx_ctx *c, int dt, hipStream_t s) {
+  if (dt != DT_REDUCE && dt != DT_ALL) return IDFX_OK;
+  if (!c->dt_clean) {
+    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, c->dtmax);
+    IDFX_TRY(check(hipGetLastError()));
+  }
+  c->dt_clean = false;
+  return IDFX_OK;
+}
+static DtTake dt_take(idfx_ctx *c, int dt) {
+  return dt == DT_TAKE ? DtTake{c->dtmax, c->host} : DtTake{};
+}
+static int dt_taken(idfx_ctx *c, int dt, hipStream_t s) {
+  if (dt != DT_TAKE) return IDFX_OK;
+  c->dt_clean = true;
+  return check(hipEventRecord(c->ev_dt, s));
+}
+static int dt_copy(idfx_ctx *c, int dt, hipStream_t s) {
+  if (dt != DT_ALL) return IDFX_OK;
+  IDFX_TRY(check(hipMemcpyAsync(c->host, c->dtmax, sizeof(unsigned long long),
+                                hipMemcpyDeviceToHost, s)));
+  return check(hipEventRecord(c->ev_dt, s));
 }
 
 // VcOut (ping-pong schedule, pp_ok): the last sweep writes the stage's new state into VcOut,
@@ -757,21 +794,23 @@ static int stage_boundaries(idfx_ctx *c, double *Vc, double *Vs, bool cell_field
 // sweep's conversion saves writing and reading Uc and Uc0 once more, 61 us a stage.)
 static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double *Vc, double *Vs,
                          double *Uc, double *InvDt, int skip_boundaries, int write_uc,
-                         bool want_dt, hipStream_t s, bool consistent = false,
+                         int dt_mode, hipStream_t s, bool consistent = false,
                          double *VcOut = nullptr) {
   static const double WC[2][2] = {{0.5, 0.0}, {0.25, 2.0 / 3.0}};
   static const double W0[2][2] = {{0.5, 0.0}, {0.75, 1.0 / 3.0}};
   if (!skip_boundaries) {
     Region r(c, IDFX_REGION_BOUNDARIES, s);
-    IDFX_TRY(stage_boundaries(c, Vc, Vs, consistent, s));
+    IDFX_TRY(stage_boundaries(c, Vc, Vs, consistent, dt_take(c, dt_mode), s));
   }
+  IDFX_TRY(dt_taken(c, dt_mode, s));
+  const bool want_dt = dt_mode == DT_REDUCE || dt_mode == DT_ALL;
   double wc = 0.0, w0 = 0.0;
   if (stage > 0) {
     wc = WC[nstages - 2][stage - 1];
     w0 = W0[nstages - 2][stage - 1];
   }
   const int dim = c->d.dim;
-  if (want_dt) hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, c->dtmax);
+  IDFX_TRY(dt_begin(c, dt_mode, s));
   for (int dir = 0; dir < dim; dir++) {
     int flags = 0;
     if (dir == 0) {
@@ -828,11 +867,7 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
   } else if (c->d.mhd && stage > 0) {
     // 1-D MHD keeps Vs constant; AddAndStore still applies (a no-op on equal values)
   }
-  if (want_dt) {
-    IDFX_TRY(check(hipMemcpyAsync(c->host, c->dtmax, sizeof(unsigned long long),
-                                  hipMemcpyDeviceToHost, s)));
-    IDFX_TRY(check(hipEventRecord(c->ev_dt, s)));
-  }
+  IDFX_TRY(dt_copy(c, dt_mode, s));
   const int lo[3] = {c->g.beg[0], c->g.beg[1], c->g.beg[2]};
   const int hi[3] = {c->g.end[0], c->g.end[1], c->g.end[2]};
   const int flags = (stage > 0 ? 1 : 0) | (write_uc ? 2 : 0);
@@ -850,15 +885,17 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
 // which writes the interior of the output pair.  Same arithmetic as stage_enqueue.
 static int stage_fused2d(idfx_ctx *c, int stage, int nstages, double dt, double *Vc_in,
                          double *Vs_in, double *Vc_out, double *Vs_out, double *Uc,
-                         double *InvDt, int write_uc, bool want_dt, hipStream_t s,
+                         double *InvDt, int write_uc, int dt_mode, hipStream_t s,
                          bool consistent) {
   static const double WC[2][2] = {{0.5, 0.0}, {0.25, 2.0 / 3.0}};
   static const double W0[2][2] = {{0.5, 0.0}, {0.75, 1.0 / 3.0}};
   {
     Region r(c, IDFX_REGION_BOUNDARIES, s);
-    IDFX_TRY(stage_boundaries(c, Vc_in, Vs_in, consistent, s));
+    IDFX_TRY(stage_boundaries(c, Vc_in, Vs_in, consistent, dt_take(c, dt_mode), s));
   }
-  if (want_dt) hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, c->dtmax);
+  IDFX_TRY(dt_taken(c, dt_mode, s));
+  IDFX_TRY(dt_begin(c, dt_mode, s));
+  const bool want_dt = dt_mode == DT_REDUCE || dt_mode == DT_ALL;
   int flags = SW_INIT_UC;
   if (stage == 0 && nstages > 1) flags |= SW_SAVE_UC0;
   if (stage == 0) flags |= SW_INVDT_SET;
@@ -889,11 +926,7 @@ static int stage_fused2d(idfx_ctx *c, int stage, int nstages, double dt, double 
     Region r(c, IDFX_REGION_FUSED2D_Y, s);
     IDFX_TRY(check(c->ops->fused2d_y(c->g, ay, c->emf(), f, c->target_waves, s)));
   }
-  if (want_dt) {
-    IDFX_TRY(check(hipMemcpyAsync(c->host, c->dtmax, sizeof(unsigned long long),
-                                  hipMemcpyDeviceToHost, s)));
-    IDFX_TRY(check(hipEventRecord(c->ev_dt, s)));
-  }
+  IDFX_TRY(dt_copy(c, dt_mode, s));
   return IDFX_OK;
 }
 
@@ -983,7 +1016,7 @@ int idfx_stage(idfx_ctx *c, int stage, int nstages, double dt, double cfl, doubl
   hipStream_t s = (hipStream_t)stream;
   const bool want_dt = stage == 0 && newdt_host != nullptr;
   IDFX_TRY(stage_enqueue(c, stage, nstages, dt, Vc, Vs, Uc, InvDt, skip_boundaries, write_uc,
-                         want_dt, s));
+                         want_dt ? DT_ALL : DT_NONE, s));
   if (want_dt) {
     IDFX_TRY(check(hipEventSynchronize(c->ev_dt)));
     *newdt_host = cfl * (1.0 / bits_to_double(*c->host));
@@ -1030,20 +1063,21 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
   const double tstage[3] = {t0, t0 + *dt, 0.25 * (t0 + *dt + *dt) + 0.75 * t0};
   for (int stage = 0; stage < nstages; stage++) {
     c->t_bound = tstage[stage];
+    const int dt_mode = nstages == 1 ? DT_ALL : stage == 0 ? DT_REDUCE : stage == 1 ? DT_TAKE : DT_NONE;
     if (pp3 && stage >= pp_first) {
       IDFX_TRY(stage_enqueue(c, stage, nstages, *dt, pin[stage], Vs, Uc, InvDt, 0,
-                             stage == nstages - 1, stage == 0, s, stage > 0, pout[stage]));
+                             stage == nstages - 1, dt_mode, s, stage > 0, pout[stage]));
     } else if (!fused || stage < first_fused) {
       IDFX_TRY(stage_enqueue(c, stage, nstages, *dt, Vc, Vs, Uc, InvDt, 0,
-                             stage == nstages - 1, stage == 0, s, stage > 0));
+                             stage == nstages - 1, dt_mode, s, stage > 0));
     } else {
       const bool fwd = (stage - first_fused) % 2 == 0;
       IDFX_TRY(stage_fused2d(c, stage, nstages, *dt, fwd ? Vc : c->Vc2, fwd ? Vs : c->Vs2,
                              fwd ? c->Vc2 : Vc, fwd ? c->Vs2 : Vs, Uc, InvDt,
-                             stage == nstages - 1, stage == 0, s, stage > 0));
+                             stage == nstages - 1, dt_mode, s, stage > 0));
     }
   }
-  // the dt readback of stage 0 completes while the later stages still run
+  // stage 0's InvDt maximum reaches the host while the later stages still run
   IDFX_TRY(check(hipEventSynchronize(c->ev_dt)));
   const double newdt = cfl * (1.0 / bits_to_double(*c->host));
   *t = t0 + *dt;

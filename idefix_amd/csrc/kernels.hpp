@@ -1554,6 +1554,19 @@ __global__ __launch_bounds__(256) void k_vc_field(GridDesc g, const double *Vs, 
     X[C::BX3 * g.sv + p] = 0.5 * (Vs[idxs(g, 2, k, j, i)] + Vs[idxs(g, 2, k + 1, j, i)]);
 }
 
+// The InvDt maximum of a cycle's first stage on its way to the host: the next stage's
+// boundary kernel stores it to pinned memory and clears it for the next cycle, in place of a
+// clearing kernel and a copy.  dtmax == nullptr: nothing to take.
+struct DtTake {
+  unsigned long long *dtmax, *host;
+};
+__device__ __forceinline__ void take_dt(const DtTake &tk) {
+  if (tk.dtmax != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
+    __hip_atomic_store(tk.host, *tk.dtmax, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    *tk.dtmax = 0ULL;
+  }
+}
+
 // Ghost zones of a box periodic in every active direction, all directions at once: every
 // ghost cell of Vc and ghost face of each Vs component takes the value at the periodic
 // image of its ghost coordinates (faces along their own direction wrap with period
@@ -1569,7 +1582,9 @@ __global__ __launch_bounds__(256) void k_vc_field(GridDesc g, const double *Vs, 
 // direction and k_vc_field, and 32-bit index arithmetic, whole cycles: Orszag-Tang 512^2 139
 // -> 128 us, 128^3 1063 -> 1016 us.)
 template <class C, bool FIELD>
-__global__ __launch_bounds__(256) void k_boundary_periodic(GridDesc g, double *Vc, double *Vs) {
+__global__ __launch_bounds__(256) void k_boundary_periodic(GridDesc g, double *Vc, double *Vs,
+                                                           DtTake tk) {
+  take_dt(tk);
   constexpr int NF = C::MHD ? C::DIM : 0;
   // all site counts stay below 2^31: a block has fewer than 2^29 cells
   unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1739,7 +1754,8 @@ enum BcType { BC_PERIODIC = 0, BC_OUTFLOW = 1, BC_REFLECTIVE = 2, BC_USERDEF = 3
 // periodic), for the sides whose type is not user-defined.
 template <class C>
 __global__ __launch_bounds__(256) void k_boundary(GridDesc g, double *Vc, double *Vs, int dir,
-                                                  int lbc, int rbc) {
+                                                  int lbc, int rbc, DtTake tk) {
+  take_dt(tk);
   // enumerate ghost sites of the cell array and of the three face arrays in one grid
   const int ng = g.beg[dir];
   const int nint = g.end[dir] - g.beg[dir];

@@ -32,9 +32,9 @@ struct Ops {
   // all-periodic box: every ghost zone in one pass, with field the interior cell field too
   // (see k_boundary_periodic)
   hipError_t (*boundary_periodic)(const GridDesc &g, double *Vc, double *Vs, bool field,
-                                  hipStream_t s) = nullptr;
+                                  DtTake tk, hipStream_t s) = nullptr;
   hipError_t (*boundary)(const GridDesc &g, double *Vc, double *Vs, int dir, int lbc, int rbc,
-                         hipStream_t s) = nullptr;
+                         DtTake tk, hipStream_t s) = nullptr;
   hipError_t (*normal_field)(const GridDesc &g, double *Vs, int dir, int recL, int recR,
                              hipStream_t s) = nullptr;
   hipError_t (*correct_flux)(int dir, const GridDesc &g, double *Flux, hipStream_t s) = nullptr;
@@ -321,7 +321,7 @@ hipError_t launch_vc_field(const GridDesc &g, const double *Vs, double *X, hipSt
 
 template <class C>
 hipError_t launch_boundary(const GridDesc &g, double *Vc, double *Vs, int dir, int lbc, int rbc,
-                           hipStream_t s) {
+                           DtTake tk, hipStream_t s) {
   constexpr int NF = C::MHD ? C::DIM : 0;
   long long total = 0;
   for (int f = -1; f < NF; f++) {
@@ -330,13 +330,13 @@ hipError_t launch_boundary(const GridDesc &g, double *Vc, double *Vs, int dir, i
     total += sz;
   }
   hipLaunchKernelGGL((k_boundary<C>), dim3(blocks_for(total)), dim3(256), 0, s, g, Vc, Vs, dir,
-                     lbc, rbc);
+                     lbc, rbc, tk);
   return hipGetLastError();
 }
 
 template <class C>
 hipError_t launch_boundary_periodic(const GridDesc &g, double *Vc, double *Vs, bool field,
-                                    hipStream_t s) {
+                                    DtTake tk, hipStream_t s) {
   constexpr int NF = C::MHD ? C::DIM : 0;
   long long total = 0;
   for (int f = -1; f < NF; f++)
@@ -351,9 +351,11 @@ hipError_t launch_boundary_periodic(const GridDesc &g, double *Vc, double *Vs, b
     }
   if (field && C::MHD) {
     total += (long long)(g.end[0] - g.beg[0]) * (g.end[1] - g.beg[1]) * (g.end[2] - g.beg[2]);
-    hipLaunchKernelGGL((k_boundary_periodic<C, true>), dim3(blocks_for(total)), dim3(256), 0, s, g, Vc, Vs);
+    hipLaunchKernelGGL((k_boundary_periodic<C, true>), dim3(blocks_for(total)), dim3(256), 0, s, g, Vc, Vs,
+                       tk);
   } else {
-    hipLaunchKernelGGL((k_boundary_periodic<C, false>), dim3(blocks_for(total)), dim3(256), 0, s, g, Vc, Vs);
+    hipLaunchKernelGGL((k_boundary_periodic<C, false>), dim3(blocks_for(total)), dim3(256), 0, s, g, Vc, Vs,
+                       tk);
   }
   return hipGetLastError();
 }
