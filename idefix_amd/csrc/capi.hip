@@ -566,6 +566,11 @@ int idfx_ctx_array(idfx_ctx *c, int which, double **ptr) {
   return *ptr ? IDFX_OK : IDFX_E_ARGS;
 }
 
+static bool all_periodic(const idfx_ctx *c) {
+  for (int d = 0; d < c->d.dim; d++)
+    if (c->d.lbound[d] != IDFX_BC_PERIODIC || c->d.rbound[d] != IDFX_BC_PERIODIC) return false;
+  return true;
+}
 static int enforce_dir(idfx_ctx *c, int dir, double *Vc, double *Vs, DtTake tk, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   // built-in side types (user-defined sides are left alone by the kernel)
@@ -606,6 +611,9 @@ static int set_boundaries(idfx_ctx *c, double *Vc, double *Vs, DtTake tk, void *
 
 int idfx_set_boundaries(idfx_ctx *c, double *Vc, double *Vs, void *stream) {
   if (!c || !Vc || (c->d.mhd && !Vs)) return IDFX_E_ARGS;
+  // one kernel for the same values in a box periodic in every direction
+  if (all_periodic(c))
+    return check(c->ops->boundary_periodic(c->g, Vc, Vs, true, DtTake{}, (hipStream_t)stream));
   return set_boundaries(c, Vc, Vs, DtTake{}, stream);
 }
 
@@ -714,8 +722,7 @@ int idfx_compute_timestep(idfx_ctx *c, const double *InvDt, double *dtmin, void 
   hipStream_t s = (hipStream_t)stream;
   c->dt_clean = false;
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, c->dtmax);
-  hipLaunchKernelGGL(k_invdt_max, dim3(1024), dim3(256), 0, s, c->g, InvDt ? InvDt : c->InvDt,
-                     c->dtmax);
+  launch_invdt_max(c->g, InvDt ? InvDt : c->InvDt, c->dtmax, s);
   IDFX_TRY(check(hipGetLastError()));
   unsigned long long b;
   IDFX_TRY(read_u64(c, c->dtmax, &b, s));
@@ -747,11 +754,6 @@ int idfx_check_divb(idfx_ctx *c, const double *Vs, double *divb, void *stream) {
 // ReconstructVcField; the interior cell field is taken from the faces too unless it
 // already equals their average (every stage after the first of a cycle: the previous
 // stage's ConsToPrim wrote it).
-static bool all_periodic(const idfx_ctx *c) {
-  for (int d = 0; d < c->d.dim; d++)
-    if (c->d.lbound[d] != IDFX_BC_PERIODIC || c->d.rbound[d] != IDFX_BC_PERIODIC) return false;
-  return true;
-}
 static int stage_boundaries(idfx_ctx *c, double *Vc, double *Vs, bool cell_field_consistent,
                             DtTake tk, hipStream_t s) {
   if (all_periodic(c))
@@ -837,8 +839,7 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
       }
       IDFX_TRY(do_sweep_unfused(c, dir, dt, Vc, Vs, Uc, InvDt, c->Flux, s));
       if (dir == dim - 1 && want_dt)
-        hipLaunchKernelGGL(k_invdt_max, dim3(1024), dim3(256), 0, s, c->g,
-                           InvDt ? InvDt : c->InvDt, c->dtmax);
+        launch_invdt_max(c->g, InvDt ? InvDt : c->InvDt, c->dtmax, s);
     } else {
       IDFX_TRY(shock_step(c, dir, Vc, s));
       if (VcOut && dir == dim - 1)

@@ -1685,18 +1685,20 @@ static __global__ __launch_bounds__(256) void k_add_and_store(double *U, const d
   if (p < n) U[p] = wl * U[p] + wr * U0[p];
 }
 
-// max over the interior of InvDt (bit pattern), for ComputeTimestep (dataBlock.cpp:333-364)
-static __global__ __launch_bounds__(256) void k_invdt_max(GridDesc g, const double *InvDt,
+// max over the interior of InvDt (bit pattern), for ComputeTimestep (dataBlock.cpp:333-364).
+// About eight cells a thread, so that the blocks' atomics on the one result stay few (1024
+// blocks whatever the size, and 64-bit index divisions: 14.8 us at 96x80x72; the array reads
+// in 1 us).
+static __global__ __launch_bounds__(256) void k_invdt_max(GridDesc g, const double *InvDt, FastDiv ni,
+                                                   FastDiv nj, unsigned n,
                                                    unsigned long long *out) {
-  const int ni = g.end[0] - g.beg[0], nj = g.end[1] - g.beg[1], nk = g.end[2] - g.beg[2];
-  const long long n = (long long)ni * nj * nk;
   unsigned long long m = 0;
-  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n;
-       t += (long long)gridDim.x * blockDim.x) {
-    const int i = g.beg[0] + t % ni;
-    const int j = g.beg[1] + (t / ni) % nj;
-    const int k = g.beg[2] + t / ((long long)ni * nj);
-    const unsigned long long b = __double_as_longlong(InvDt[idx3(g, k, j, i)]);
+#pragma unroll 4
+  for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
+    const unsigned r = fast_div(t, ni), rk = fast_div(r, nj);
+    const unsigned p = (unsigned)idx3(g, g.beg[2] + (int)rk, g.beg[1] + (int)(r - rk * nj.d),
+                                      g.beg[0] + (int)(t - r * ni.d));
+    const unsigned long long b = __double_as_longlong(ld32(InvDt, p));
     m = b > m ? b : m;
   }
   block_max_atomic(m, out);

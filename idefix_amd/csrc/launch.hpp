@@ -115,6 +115,14 @@ inline FastDiv fast_div_of(unsigned d) {
   return f;
 }
 
+inline void launch_invdt_max(const GridDesc &g, const double *InvDt, unsigned long long *out,
+                             hipStream_t s) {
+  const unsigned ni = g.end[0] - g.beg[0], nj = g.end[1] - g.beg[1], nk = g.end[2] - g.beg[2];
+  const unsigned n = ni * nj * nk;
+  hipLaunchKernelGGL(k_invdt_max, dim3(std::min(1024u, blocks_for(n, 2048))), dim3(256), 0, s, g, InvDt,
+                     fast_div_of(ni), fast_div_of(nj), n, out);
+}
+
 template <class C, typename T, int DIR, bool FUSED, int EMF, bool XTRA, bool FIN = false>
 hipError_t launch_sweep_xtra(const GridDesc &g, const SweepArgs &a, const EmfArrays<T> &e,
                             int target_waves, hipStream_t s) {
