@@ -763,7 +763,7 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
   constexpr int BXn = C::template BXn<DIR>();
   constexpr int BXt = C::template BXt<DIR>();
   constexpr int BXb = C::template BXb<DIR>();
-  T uL[NV], uR[NV], fluxL[NV], fluxR[NV];
+  T uL[NV], uR[NV];
 
   // fast magnetosonic speeds, hlldMHD.hpp:183-226
   T cL, cR;
@@ -795,11 +795,14 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
   const T sr = fmx(cmaxL, cmaxR);
   cmax = fmx(fab(sl), fab(sr));
 
-  const Recip<T> gm1 = recip(gamma - T(1));
-  prim2cons<C>(vL, uL, gm1);
-  prim2cons<C>(vR, uR, gm1);
-  kflux<C, DIR>(fluxL, vL, uL);
-  kflux<C, DIR>(fluxR, vR, uR);
+  // conserved density, normal momentum and field here; the rest of PrimToCons, the physical
+  // flux and the star energies belong to the side of the contact the face lies on and are
+  // computed for that side alone: 110 of the 750 operations that a wave whose faces all lie
+  // on one side skips for the other
+  uL[C::RHO] = vL[C::RHO];
+  uR[C::RHO] = vR[C::RHO];
+  uL[Xn] = vL[Xn] * vL[C::RHO];
+  uR[Xn] = vR[Xn] * vR[C::RHO];
 
   T b2L = vL[C::BX1] * vL[C::BX1];
   if constexpr (CO >= 2) b2L = b2L + vL[C::BX2] * vL[C::BX2];
@@ -813,169 +816,143 @@ __device__ __forceinline__ void hlld_mhd(const T *vL, const T *vR, T *flux, T &c
   pre.valid = false;
   if (emf == EMF_UCT_HLLD) star_pre<C, DIR>(vL, vR, uL, uR, sl, sr, ptL, ptR, pre);
 
-  if (sl > T(0)) {
-#pragma unroll
-    for (int n = 0; n < NV; n++) flux[n] = fluxL[n];
-  } else if (sr < T(0)) {
-#pragma unroll
-    for (int n = 0; n < NV; n++) flux[n] = fluxR[n];
-  } else {
-    T usL[NV], usR[NV];
-    T scrh, scrhL, scrhR, duL, duR, sBx, Bx, SM, S1L, S1R, pts, sqrL, sqrR;
-    T vsL = 0, vsR = 0, wsL = 0, wsR = 0;
+  // the face's side, and how far into the fan it lies: OUTER (beyond the fast wave), FIRST
+  // (between fast and Alfven wave), SECOND (between Alfven wave and contact)
+  enum { OUTER, FIRST, SECOND };
+  int region = OUTER;
+  bool left = sl > T(0);
+  StarPre<T> P = pre;
+  T sBx = 0, Bx = 0, SM = 0, S1L = 0, S1R = 0, pts = 0;
+  T vsL = 0, vsR = 0, wsL = 0, wsR = 0;           // transverse star velocities
+  T BnL = 0, BnR = 0, BtL = 0, BtR = 0, BbL = 0, BbR = 0;  // star fields
+  T vss = 0, wss = 0, Btss = 0, Bbss = 0;         // between the Alfven waves
+  if (!(sl > T(0)) && !(sr < T(0))) {
     bool revert_to_hllc = false;
-    scrh = div_(T(1), sr - sl);
+    T scrh = div_(T(1), sr - sl);
     Bx = (sr * vR[BXn] - sl * vL[BXn]) * scrh;
     sBx = (Bx > T(0) ? T(1) : T(-1));
-    StarPre<T> P = pre;
     if (!P.valid) star_pre<C, DIR>(vL, vR, uL, uR, sl, sr, ptL, ptR, P);
-    duL = P.duL;
-    duR = P.duR;
-    scrh = P.scrh;
+    const T duL = P.duL, duR = P.duR;
     SM = P.Sc;
     pts = duR * uR[C::RHO] * ptL - duL * uL[C::RHO] * ptR +
           vL[C::RHO] * vR[C::RHO] * duR * duL * (vR[Xn] - vL[Xn]);
-    pts *= scrh;
-    usL[C::RHO] = P.usLRHO;
-    usR[C::RHO] = P.usRRHO;
-    sqrL = P.sqrL.b;
-    sqrR = P.sqrR.b;
+    pts *= P.scrh;
     S1L = SM - quot(fab(Bx), P.sqrL);
     S1R = SM + quot(fab(Bx), P.sqrR);
     if ((S1L - sl) < T(1.e-4) * (SM - sl)) revert_to_hllc = true;
     if ((S1R - sr) > -T(1.e-4) * (sr - SM)) revert_to_hllc = true;
     if (revert_to_hllc) {
-      scrh = div_(T(1), sr - sl);
-      T Uhll_n, Uhll_t = 0, Uhll_b = 0;
-      Uhll_n = (sr * uR[BXn] - sl * uL[BXn] + fluxL[BXn] - fluxR[BXn]) * scrh;
-      if constexpr (CO >= 2) Uhll_t = (sr * uR[BXt] - sl * uL[BXt] + fluxL[BXt] - fluxR[BXt]) * scrh;
-      if constexpr (CO >= 3) Uhll_b = (sr * uR[BXb] - sl * uL[BXb] + fluxL[BXb] - fluxR[BXb]) * scrh;
-      usL[BXn] = usR[BXn] = Uhll_n;
-      if constexpr (CO >= 2) usL[BXt] = usR[BXt] = Uhll_t;
-      if constexpr (CO >= 3) usL[BXb] = usR[BXb] = Uhll_b;
+      // the field of the HLL state; F(B) = v_n B - B_n v, zero along the normal
+      BnL = BnR = (sr * vR[BXn] - sl * vL[BXn] + T(0) - T(0)) * scrh;
+      if constexpr (CO >= 2)
+        BtL = BtR = (sr * vR[BXt] - sl * vL[BXt] + (vL[Xn] * vL[BXt] - vL[BXn] * vL[Xt]) -
+                     (vR[Xn] * vR[BXt] - vR[BXn] * vR[Xt])) * scrh;
+      if constexpr (CO >= 3)
+        BbL = BbR = (sr * vR[BXb] - sl * vL[BXb] + (vL[Xn] * vL[BXb] - vL[BXn] * vL[Xb]) -
+                     (vR[Xn] * vR[BXb] - vR[BXn] * vR[Xb])) * scrh;
       S1L = S1R = SM;
     } else {
-      scrhL = div_(uL[C::RHO] * duL * duL - Bx * Bx, uL[C::RHO] * duL * (sl - SM) - Bx * Bx);
-      scrhR = div_(uR[C::RHO] * duR * duR - Bx * Bx, uR[C::RHO] * duR * (sr - SM) - Bx * Bx);
-      usL[BXn] = Bx;
-      if constexpr (CO >= 2) usL[BXt] = uL[BXt] * scrhL;
-      if constexpr (CO >= 3) usL[BXb] = uL[BXb] * scrhL;
-      usR[BXn] = Bx;
-      if constexpr (CO >= 2) usR[BXt] = uR[BXt] * scrhR;
-      if constexpr (CO >= 3) usR[BXb] = uR[BXb] * scrhR;
+      BnL = BnR = Bx;
+      if constexpr (CO >= 2) {
+        const T kL = div_(uL[C::RHO] * duL * duL - Bx * Bx, uL[C::RHO] * duL * (sl - SM) - Bx * Bx);
+        const T kR = div_(uR[C::RHO] * duR * duR - Bx * Bx, uR[C::RHO] * duR * (sr - SM) - Bx * Bx);
+        BtL = vL[BXt] * kL;
+        BtR = vR[BXt] * kR;
+        if constexpr (CO >= 3) {
+          BbL = vL[BXb] * kL;
+          BbR = vR[BXb] * kR;
+        }
+      }
     }
-    scrhL = div_(Bx, uL[C::RHO] * duL);
-    scrhR = div_(Bx, uR[C::RHO] * duR);
     if constexpr (CO >= 2) {
-      vsL = vL[Xt] - scrhL * (usL[BXt] - uL[BXt]);
-      vsR = vR[Xt] - scrhR * (usR[BXt] - uR[BXt]);
+      const T kL = div_(Bx, uL[C::RHO] * duL), kR = div_(Bx, uR[C::RHO] * duR);
+      vsL = vL[Xt] - kL * (BtL - vL[BXt]);
+      vsR = vR[Xt] - kR * (BtR - vR[BXt]);
+      if constexpr (CO >= 3) {
+        wsL = vL[Xb] - kL * (BbL - vL[BXb]);
+        wsR = vR[Xb] - kR * (BbR - vR[BXb]);
+      }
     }
-    if constexpr (CO >= 3) {
-      wsL = vL[Xb] - scrhL * (usL[BXb] - uL[BXb]);
-      wsR = vR[Xb] - scrhR * (usR[BXb] - uR[BXb]);
-    }
-    usL[Xn] = usL[C::RHO] * SM;
-    usR[Xn] = usR[C::RHO] * SM;
-    if constexpr (CO >= 2) {
-      usL[Xt] = usL[C::RHO] * vsL;
-      usR[Xt] = usR[C::RHO] * vsR;
-    }
-    if constexpr (CO >= 3) {
-      usL[Xb] = usL[C::RHO] * wsL;
-      usR[Xb] = usR[C::RHO] * wsR;
-    }
-    scrhL = vL[Xn] * Bx;
-    if constexpr (CO >= 2) scrhL = scrhL + vL[Xt] * uL[BXt];
-    if constexpr (CO >= 3) scrhL = scrhL + vL[Xb] * uL[BXb];
-    {
-      T s = SM * Bx;
-      if constexpr (CO >= 2) s = s + vsL * usL[BXt];
-      if constexpr (CO >= 3) s = s + wsL * usL[BXb];
-      scrhL -= s;
-    }
-    usL[C::ENG] = quot(duL * uL[C::ENG] - ptL * vL[Xn] + pts * SM + Bx * scrhL, P.slS);
-    scrhR = vR[Xn] * Bx;
-    if constexpr (CO >= 2) scrhR = scrhR + vR[Xt] * uR[BXt];
-    if constexpr (CO >= 3) scrhR = scrhR + vR[Xb] * uR[BXb];
-    {
-      T s = SM * Bx;
-      if constexpr (CO >= 2) s = s + vsR * usR[BXt];
-      if constexpr (CO >= 3) s = s + wsR * usR[BXb];
-      scrhR -= s;
-    }
-    usR[C::ENG] = quot(duR * uR[C::ENG] - ptR * vR[Xn] + pts * SM + Bx * scrhR, P.srS);
-
+    region = FIRST;
     if (S1L >= T(0)) {
-#pragma unroll
-      for (int n = 0; n < NV; n++) flux[n] = fluxL[n] + sl * (usL[n] - uL[n]);
+      left = true;
     } else if (S1R <= T(0)) {
-#pragma unroll
-      for (int n = 0; n < NV; n++) flux[n] = fluxR[n] + sr * (usR[n] - uR[n]);
+      left = false;
     } else {
-      T vss = 0, wss = 0, ussl[NV], ussr[NV];
-      ussl[C::RHO] = usL[C::RHO];
-      ussr[C::RHO] = usR[C::RHO];
+      region = SECOND;
+      left = SM >= T(0);
+      const T sqrL = P.sqrL.b, sqrR = P.sqrR.b;
       const Recip<T> sq = recip(sqrL + sqrR);
       if constexpr (CO >= 2) {
-        vss = sqrL * vsL + sqrR * vsR + (usR[BXt] - usL[BXt]) * sBx;
-        vss = quot(vss, sq);
+        vss = quot(sqrL * vsL + sqrR * vsR + (BtR - BtL) * sBx, sq);
+        Btss = quot(sqrL * BtR + sqrR * BtL + sqrL * sqrR * (vsR - vsL) * sBx, sq);
       }
       if constexpr (CO >= 3) {
-        wss = sqrL * wsL + sqrR * wsR + (usR[BXb] - usL[BXb]) * sBx;
-        wss = quot(wss, sq);
-      }
-      ussl[Xn] = ussl[C::RHO] * SM;
-      ussr[Xn] = ussr[C::RHO] * SM;
-      if constexpr (CO >= 2) {
-        ussl[Xt] = ussl[C::RHO] * vss;
-        ussr[Xt] = ussr[C::RHO] * vss;
-      }
-      if constexpr (CO >= 3) {
-        ussl[Xb] = ussl[C::RHO] * wss;
-        ussr[Xb] = ussr[C::RHO] * wss;
-      }
-      ussl[BXn] = ussr[BXn] = Bx;
-      if constexpr (CO >= 2) {
-        ussl[BXt] = sqrL * usR[BXt] + sqrR * usL[BXt] + sqrL * sqrR * (vsR - vsL) * sBx;
-        ussl[BXt] = quot(ussl[BXt], sq);
-        ussr[BXt] = ussl[BXt];
-      }
-      if constexpr (CO >= 3) {
-        ussl[BXb] = sqrL * usR[BXb] + sqrR * usL[BXb] + sqrL * sqrR * (wsR - wsL) * sBx;
-        ussl[BXb] = quot(ussl[BXb], sq);
-        ussr[BXb] = ussl[BXb];
-      }
-      scrhL = SM * Bx;
-      if constexpr (CO >= 2) scrhL = scrhL + vsL * usL[BXt];
-      if constexpr (CO >= 3) scrhL = scrhL + wsL * usL[BXb];
-      {
-        T s = SM * Bx;
-        if constexpr (CO >= 2) s = s + vss * ussl[BXt];
-        if constexpr (CO >= 3) s = s + wss * ussl[BXb];
-        scrhL -= s;
-      }
-      scrhR = SM * Bx;
-      if constexpr (CO >= 2) scrhR = scrhR + vsR * usR[BXt];
-      if constexpr (CO >= 3) scrhR = scrhR + wsR * usR[BXb];
-      {
-        T s = SM * Bx;
-        if constexpr (CO >= 2) s = s + vss * ussr[BXt];
-        if constexpr (CO >= 3) s = s + wss * ussr[BXb];
-        scrhR -= s;
-      }
-      ussl[C::ENG] = usL[C::ENG] - sqrL * scrhL * sBx;
-      ussr[C::ENG] = usR[C::ENG] + sqrR * scrhR * sBx;
-      if (SM >= T(0)) {
-#pragma unroll
-        for (int n = 0; n < NV; n++)
-          flux[n] = fluxL[n] + S1L * (ussl[n] - usL[n]) + sl * (usL[n] - uL[n]);
-      } else {
-#pragma unroll
-        for (int n = 0; n < NV; n++)
-          flux[n] = fluxR[n] + S1R * (ussr[n] - usR[n]) + sr * (usR[n] - uR[n]);
+        wss = quot(sqrL * wsL + sqrR * wsR + (BbR - BbL) * sBx, sq);
+        Bbss = quot(sqrL * BbR + sqrR * BbL + sqrL * sqrR * (wsR - wsL) * sBx, sq);
       }
     }
   }
+
+  // flux of one side
+  const Recip<T> gm1 = recip(gamma - T(1));
+  auto side = [&](const T *v, T *u, T pt, T du, T sx, T s1, T rhos, const Recip<T> &sS, T sqr, T vs,
+                  T ws, T Bn, T Bt, T Bb, bool right) {
+    T f[NV];
+    prim2cons<C>(v, u, gm1);
+    kflux<C, DIR>(f, v, u);
+    if (region == OUTER) {
+#pragma unroll
+      for (int n = 0; n < NV; n++) flux[n] = f[n];
+      return;
+    }
+    T us[NV];
+    us[C::RHO] = rhos;
+    us[Xn] = rhos * SM;
+    us[BXn] = Bn;
+    T vb = v[Xn] * Bx, vbs = SM * Bx;
+    if constexpr (CO >= 2) {
+      us[Xt] = rhos * vs;
+      us[BXt] = Bt;
+      vb = vb + v[Xt] * u[BXt];
+      vbs = vbs + vs * Bt;
+    }
+    if constexpr (CO >= 3) {
+      us[Xb] = rhos * ws;
+      us[BXb] = Bb;
+      vb = vb + v[Xb] * u[BXb];
+      vbs = vbs + ws * Bb;
+    }
+    us[C::ENG] = quot(du * u[C::ENG] - pt * v[Xn] + pts * SM + Bx * (vb - vbs), sS);
+    if (region == FIRST) {
+#pragma unroll
+      for (int n = 0; n < NV; n++) flux[n] = f[n] + sx * (us[n] - u[n]);
+      return;
+    }
+    T uss[NV];
+    uss[C::RHO] = rhos;
+    uss[Xn] = rhos * SM;
+    uss[BXn] = Bx;
+    T vbss = SM * Bx;
+    if constexpr (CO >= 2) {
+      uss[Xt] = rhos * vss;
+      uss[BXt] = Btss;
+      vbss = vbss + vss * Btss;
+    }
+    if constexpr (CO >= 3) {
+      uss[Xb] = rhos * wss;
+      uss[BXb] = Bbss;
+      vbss = vbss + wss * Bbss;
+    }
+    const T de = sqr * (vbs - vbss) * sBx;
+    uss[C::ENG] = right ? us[C::ENG] + de : us[C::ENG] - de;
+#pragma unroll
+    for (int n = 0; n < NV; n++) flux[n] = f[n] + s1 * (uss[n] - us[n]) + sx * (us[n] - u[n]);
+  };
+  if (left)
+    side(vL, uL, ptL, P.duL, sl, S1L, P.usLRHO, P.slS, P.sqrL.b, vsL, wsL, BnL, BtL, BbL, false);
+  else
+    side(vR, uR, ptR, P.duR, sr, S1R, P.usRRHO, P.srS, P.sqrR.b, vsR, wsR, BnR, BtR, BbR, true);
 
   store_face_emf<C, DIR>(vL, vR, uL, uR, flux, sl, sr, ptL, ptR, E, emf, pre);
 }
