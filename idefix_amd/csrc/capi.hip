@@ -126,7 +126,8 @@ struct idfx_ctx {
   bool pp_ok = false;
   bool pp_hd_on = false;  // hydro: off at fusion level 0 (MHD follows fused3d_on)
   double *Vc2 = nullptr, *Vs2 = nullptr;
-  double *Vc3 = nullptr;  // 3-D ping-pong with three stages: the first stage's output
+  // ping-pong with three stages: the first stage's output (2-D MHD: and its faces)
+  double *Vc3 = nullptr, *Vs3 = nullptr;
   bool vc3_failed = false;  // its allocation failed once: RK3 keeps the in-place first stage
   // enrolled user boundary (IDFX_BC_USERDEF sides) and the time it is called with
   idfx_userdef_boundary_fn user_fn = nullptr;
@@ -1030,34 +1031,33 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
   if (!c || !t || !dt || nstages < 1 || nstages > 3) return IDFX_E_ARGS;
   hipStream_t s = (hipStream_t)stream;
   const double t0 = *t;
-  // fused 2-D stages ping-pong between (Vc, Vs) and the context's pair; an odd stage count
-  // runs its first stage in place so that the last stage writes the caller's arrays
+  // fused 2-D MHD stages write cells and faces into another pair of arrays, 3-D MHD and
+  // hydro stages their cells (Vs updated in place).  RK2 Vc -> Vc2 -> Vc; RK3 Vc -> Vc3 ->
+  // Vc2 -> Vc (the third array allocated at the first such cycle; without it the first RK3
+  // stage runs in place on the per-kernel schedule and the others alternate Vc -> Vc2 -> Vc;
+  // 2-D turbulence 256^2: 154 us a cycle without it, 140 with it)
   const bool fused = c->fused2d_on && nstages >= 2 && Vs;
-  // 3-D MHD and hydro: the same alternation between (Vc, Vs) and (Vc2, Vs), Vs updated in
-  // place
   const bool pp3 = c->pp_ok && nstages >= 2 && (c->d.mhd ? c->fused3d_on && Vs : c->pp_hd_on);
-  const int first_fused = (nstages % 2 == 1) ? 1 : 0;
-  // 3-D ping-pong inputs and outputs per stage: RK2 Vc -> Vc2 -> Vc; RK3 Vc -> Vc3 -> Vc2
-  // -> Vc (Vc3 allocated at the first such cycle; without it the first RK3 stage runs in
-  // place on the per-kernel ConsToPrim and the others alternate Vc -> Vc2 -> Vc)
-  if (pp3 && nstages == 3 && !c->Vc3 && !c->vc3_failed &&
-      alloc_n(c, &c->Vc3, c->n3 * c->nvar) != IDFX_OK) {
-    c->Vc3 = nullptr;
-    c->vc3_failed = true;
-    (void)hipGetLastError();  // the failed allocation must not surface as a launch error
+  if ((pp3 || fused) && nstages == 3 && !c->Vc3 && !c->vc3_failed) {
+    double *v = nullptr, *b = nullptr;
+    if (alloc_n(c, &v, c->n3 * c->nvar) == IDFX_OK && (!fused || alloc_n(c, &b, c->nvs) == IDFX_OK)) {
+      c->Vc3 = v;
+      c->Vs3 = b;
+    } else {
+      c->vc3_failed = true;
+      (void)hipGetLastError();  // the failed allocation must not surface as a launch error
+    }
   }
   double *pin[3] = {Vc, c->Vc2, Vc}, *pout[3] = {c->Vc2, Vc, nullptr};
+  double *bin[3] = {Vs, c->Vs2, Vs}, *bout[3] = {c->Vs2, Vs, nullptr};
   int pp_first = 0;
   if (nstages == 3) {
-    if (c->Vc3) {
-      pin[0] = Vc, pout[0] = c->Vc3;
-      pin[1] = c->Vc3, pout[1] = c->Vc2;
-      pin[2] = c->Vc2, pout[2] = Vc;
-    } else {
-      pp_first = 1;
-      pin[1] = Vc, pout[1] = c->Vc2;
-      pin[2] = c->Vc2, pout[2] = Vc;
-    }
+    pp_first = c->Vc3 ? 0 : 1;
+    pout[0] = c->Vc3, bout[0] = c->Vs3;
+    pin[1] = c->Vc3 ? c->Vc3 : Vc, bin[1] = c->Vc3 ? c->Vs3 : Vs;
+    pout[1] = c->Vc2, bout[1] = c->Vs2;
+    pin[2] = c->Vc2, bin[2] = c->Vs2;
+    pout[2] = Vc, bout[2] = Vs;
   }
   // stage times of the boundary calls (TimeIntegrator::Cycle advances t by dt after each
   // stage, then t = wc t + w0 t0): t0, t0 + dt, and t0 + dt/2 for the third RK3 stage
@@ -1065,18 +1065,15 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
   for (int stage = 0; stage < nstages; stage++) {
     c->t_bound = tstage[stage];
     const int dt_mode = nstages == 1 ? DT_ALL : stage == 0 ? DT_REDUCE : stage == 1 ? DT_TAKE : DT_NONE;
-    if (pp3 && stage >= pp_first) {
-      IDFX_TRY(stage_enqueue(c, stage, nstages, *dt, pin[stage], Vs, Uc, InvDt, 0,
-                             stage == nstages - 1, dt_mode, s, stage > 0, pout[stage]));
-    } else if (!fused || stage < first_fused) {
-      IDFX_TRY(stage_enqueue(c, stage, nstages, *dt, Vc, Vs, Uc, InvDt, 0,
-                             stage == nstages - 1, dt_mode, s, stage > 0));
-    } else {
-      const bool fwd = (stage - first_fused) % 2 == 0;
-      IDFX_TRY(stage_fused2d(c, stage, nstages, *dt, fwd ? Vc : c->Vc2, fwd ? Vs : c->Vs2,
-                             fwd ? c->Vc2 : Vc, fwd ? c->Vs2 : Vs, Uc, InvDt,
-                             stage == nstages - 1, dt_mode, s, stage > 0));
-    }
+    const bool last = stage == nstages - 1;
+    if (stage < pp_first || !(pp3 || fused))
+      IDFX_TRY(stage_enqueue(c, stage, nstages, *dt, Vc, Vs, Uc, InvDt, 0, last, dt_mode, s, stage > 0));
+    else if (pp3)
+      IDFX_TRY(stage_enqueue(c, stage, nstages, *dt, pin[stage], Vs, Uc, InvDt, 0, last, dt_mode, s,
+                             stage > 0, pout[stage]));
+    else
+      IDFX_TRY(stage_fused2d(c, stage, nstages, *dt, pin[stage], bin[stage], pout[stage], bout[stage],
+                             Uc, InvDt, last, dt_mode, s, stage > 0));
   }
   // stage 0's InvDt maximum reaches the host while the later stages still run
   IDFX_TRY(check(hipEventSynchronize(c->ev_dt)));

@@ -223,8 +223,8 @@ int idfx_stage(idfx_ctx *ctx, int stage, int nstages, double dt, double cfl, dou
  * user-defined sides, whose stages alternate between Vc and context-owned state arrays)
  * the ghost zones hold the boundary values of an earlier stage, which the next stage's
  * boundary fill rewrites before any use, and the corner (2-D also y-face) EMF scratch
- * arrays are not written.  The first RK3 cycle of 3-D MHD or hydro allocates one more state
- * array. */
+ * arrays are not written.  The first RK3 cycle on these schedules allocates one more state array
+ * (2-D MHD: and face array). */
 int idfx_cycle(idfx_ctx *ctx, int nstages, double cfl, double cfl_max_var, long ncycles,
                double *t, double *dt, double *Vc, double *Vs, double *Uc, double *InvDt,
                void *stream);
