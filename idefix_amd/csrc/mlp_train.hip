@@ -25,8 +25,8 @@ constexpr int P_W1 = 0, P_B1 = P_W1 + NF * NH, P_W2 = P_B1 + NH, P_B2 = P_W2 + N
               P_W3 = P_B2 + NH, P_B3 = P_W3 + NH * NO, P_N = P_B3 + NO;
 constexpr float GELU_K = 1.702f;
 constexpr int ROW = 72, ROW_WP = 48, ROW_OM = 64;  // batch row: features | wp | om
-constexpr int TR = 32;            // rows of a tile: two waves of 16
-constexpr int MAX_BLOCKS = 512;   // blocks of k_train: two per CU
+constexpr int TR = 32;            // rows of a tile: two groups of 16
+constexpr int MAX_BLOCKS = 256;   // blocks of k_train: one per CU
 
 __device__ __forceinline__ float sig(float z) { return 1.0f / (1.0f + expf(-z)); }
 // derivative of z s with s = sig(GELU_K z)
@@ -45,112 +45,80 @@ __device__ __forceinline__ f4 mfma(float a, float b, f4 c) {
 
 // LDS, in floats.  Weights [in][out], rows padded to strides (68, 20) that keep the reads of
 // both passes free of bank conflicts: forward a lane reads one output of four inputs 4 g + r,
-// backward four consecutive outputs of one input.  The tile's activations and deltas
-// [row][unit] take their place for the weight gradients (strides of 16 mod 32 floats).
+// backward four consecutive outputs of one input.  Then the tile's features, activations and
+// deltas [row][unit] (strides of 16 mod 32 floats).
 constexpr int S_W = 68, S_W3 = 20, L_W1 = 0, L_W2 = L_W1 + NF * S_W, L_W3 = L_W2 + NH * S_W,
               L_B = L_W3 + NH * S_W3, L_WEND = L_B + 2 * NH + NO;
-constexpr int S_X = 48, S_H = 80, S_O = 16, L_X = 0, L_H1 = L_X + TR * S_X,
+constexpr int S_X = 48, S_H = 80, S_O = 16, L_X = L_WEND, L_H1 = L_X + TR * S_X,
               L_H2 = L_H1 + TR * S_H, L_D1 = L_H2 + TR * S_H, L_D2 = L_D1 + TR * S_H,
-              L_D3 = L_D2 + TR * S_H;
-constexpr int L_GEND = L_D3 + TR * S_O, L_END = L_GEND > L_WEND ? L_GEND : L_WEND;
+              L_D3 = L_D2 + TR * S_H, L_END = L_D3 + TR * S_O;
+static_assert(L_X % 4 == 0 && L_B % 4 == 0, "16-byte reads");
 
-// Forward: acc[t] += W^T in over the inputs in[NI] (inputs 16 i + 4 g + r of the lane's row
-// in in[i][r]); w points at the lane's input 4 g and output q of tile 0.
-template <int NT, int NI>
-__device__ __forceinline__ void forward(const float *w, int stride, const f4 *in, f4 *acc) {
-#pragma unroll
-  for (int i = 0; i < NI; i++)
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-#pragma unroll
-      for (int t = 0; t < NT; t++)
-        acc[t] = mfma(w[(16 * i + r) * stride + 16 * t], in[i][r], acc[t]);
-}
-// Backward: acc[t] += W in over the outputs; w points at the lane's input q and output 4 g.
-template <int NT, int NI>
-__device__ __forceinline__ void backward(const float *w, int stride, const f4 *in, f4 *acc) {
-#pragma unroll
-  for (int i = 0; i < NI; i++) {
-    f4 a[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) a[t] = *reinterpret_cast<const f4 *>(w + 16 * t * stride + 16 * i);
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-#pragma unroll
-      for (int t = 0; t < NT; t++) acc[t] = mfma(a[t][r], in[i][r], acc[t]);
-  }
-}
-
-// Forward pass, loss, backward pass and weight gradients of tiles of 32 rows.  A wave takes
-// 16 rows through all layers with the weights as the A operand and the activations as the
-// B operand: a layer's accumulator (unit 4 g + r of row q in lane 16 g + q) is the next
-// layer's B operand as it stands, so activations stay in registers.  For the gradients
-// (sums over rows) the activations and deltas pass through LDS, each wave computing half
-// of every layer's output tiles over all 32 rows; they accumulate in registers over the
-// block's tiles and go out once per block.  Everything is FP32 (products, accumulators,
-// activations).  208 + 128 matrix instructions per 16 rows: 2.2 us of the matrix cores'
-// time at 8192 rows; the kernel is bound by its serial chain of layers.  A step of 8192
-// rows takes 31 us, 18 of them here (33 with the weights loaded and transposed one float at a
-// time); the eleven kernels this replaces (one thread per activation, scalar products) took
-// 716, 555 of them in the weight gradients.
-__global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU, int B,
+// Forward pass, loss, backward pass and weight gradients of tiles of 32 rows.  A group of
+// four waves takes 16 rows through the layers, each wave one tile of 16 units of the hidden
+// layers (all four compute the 16 outputs), with the weights as the A operand and the
+// activations as the B operand: a lane holds units 4 g + r of row q, r = 0 .. 3.  Between
+// layers the activations and deltas pass through LDS, where the gradients (sums over rows)
+// need them too; each of the block's eight waves computes four of their 32 tiles of 16 x 16
+// over all 32 rows.  They accumulate in registers over the block's tiles and go out once per
+// block.  Everything is FP32 (products, accumulators, activations).
+//
+// 208 + 128 matrix instructions per 16 rows: 2.2 us of the matrix cores' time at 8192 rows;
+// the kernel is bound by its serial chain of layers, which four waves a row group shorten:
+// 14 us at 8192 rows (a step 27), against 18 (31) with one wave per 16 rows and the activations
+// in registers; 131,072 rows: a step 109 against 117.
+// The eleven kernels this replaces (one thread per activation, scalar products) took 716 us a
+// step, 555 of them in the weight gradients.
+__global__ __launch_bounds__(512) void k_train(const float *X, const float *TAU, int B,
                                                const float *P, float *partial,
                                                double *lossp) {
   __shared__ __attribute__((aligned(16))) float lds[L_END];
   __shared__ double lred[2];
   const int tid = threadIdx.x, wave = tid >> 6, q = tid & 15, g = (tid >> 4) & 3;
-  f4 g1[3][2], g2[4][2], g3[2];
-#pragma unroll
-  for (int n = 0; n < 2; n++) {
-#pragma unroll
-    for (int m = 0; m < 3; m++) g1[m][n] = f4{0, 0, 0, 0};
-#pragma unroll
-    for (int m = 0; m < 4; m++) g2[m][n] = f4{0, 0, 0, 0};
-    g3[n] = f4{0, 0, 0, 0};
+  const int grp = wave >> 2, u = wave & 3;  // row group, tile of 16 hidden units
+  {
+    // the weights: 16-byte loads, all in flight together; every block of P starts at a
+    // multiple of four floats
+    const f4 *p1 = reinterpret_cast<const f4 *>(P + P_W1), *p2 = reinterpret_cast<const f4 *>(P + P_W2);
+    const f4 *p3 = reinterpret_cast<const f4 *>(P + P_W3);
+    constexpr int Q1 = NF * NH / 4, Q2 = NH * NH / 4, Q3 = NH * NO / 4;  // 768, 1024, 256
+    const f4 a0 = p1[tid], a1 = p1[min(tid + 512, Q1 - 1)], b0 = p2[tid], b1 = p2[tid + 512];
+    const f4 c0 = p3[min(tid, Q3 - 1)];
+    const float bias = tid < NH       ? P[P_B1 + tid]
+                       : tid < 2 * NH ? P[P_B2 + tid - NH]
+                       : tid < 2 * NH + NO ? P[P_B3 + tid - 2 * NH] : 0.0f;
+    auto put = [&](int base, int e, f4 v) {  // 16 groups of four per row
+      *reinterpret_cast<f4 *>(lds + base + e / 16 * S_W + e % 16 * 4) = v;
+    };
+    put(L_W1, tid, a0);
+    if (tid + 512 < Q1) put(L_W1, tid + 512, a1);
+    put(L_W2, tid, b0);
+    put(L_W2, tid + 512, b1);
+    static_assert(Q2 == 1024, "two 16-byte groups of W2 per thread");
+    if (tid < Q3) *reinterpret_cast<f4 *>(lds + L_W3 + tid / 4 * S_W3 + tid % 4 * 4) = c0;
+    if (tid < 2 * NH + NO) lds[L_B + tid] = bias;
   }
-  float gb = 0.0f, gb3 = 0.0f;  // bias gradients: unit tid of layers 1 | 2, unit tid of 3
+  // this wave's gradient tiles: waves 0-2 input block `wave` of layer 1, 3-6 input block
+  // wave - 3 of layer 2, each with all four output blocks; wave 7 the four input blocks of
+  // layer 3
+  const int am = wave < 3 ? L_X + 16 * wave : wave < 7 ? L_H1 + 16 * (wave - 3) : L_H2;
+  const int as = wave < 3 ? S_X : S_H, an = wave < 7 ? 0 : 16;
+  const int bm = wave < 3 ? L_D1 : wave < 7 ? L_D2 : L_D3;
+  const int bs = wave < 7 ? S_H : S_O, bnn = wave < 7 ? 16 : 0;
+  f4 gr[4];
+#pragma unroll
+  for (int n = 0; n < 4; n++) gr[n] = f4{0, 0, 0, 0};
+  // bias gradients: thread tid sums unit tid of layer 1, tid - 64 of 2, tid - 128 of 3
+  const int gcol = tid < NH ? L_D1 + tid : tid < 2 * NH ? L_D2 + tid - NH : L_D3 + tid - 2 * NH;
+  const int gstr = tid < 2 * NH ? S_H : S_O;
+  float gb = 0.0f;
   double loss = 0.0;
   const float inv = 1.0f / (float)B;
   for (int tile = blockIdx.x; tile * TR < B; tile += gridDim.x) {
-    __syncthreads();  // the previous tile's gradient buffers have been read
-    {
-      // 16 consecutive floats of a thread's loads in flight at a time; every block of P
-      // starts at a multiple of four floats
-      const f4 *p1 = reinterpret_cast<const f4 *>(P + P_W1), *p2 = reinterpret_cast<const f4 *>(P + P_W2);
-      const f4 *p3 = reinterpret_cast<const f4 *>(P + P_W3);
-      f4 v1[NF * NH / 512], v2[NH * NH / 512], v3[NH * NO / 512];
-#pragma unroll
-      for (int n = 0; n < NF * NH / 512; n++) v1[n] = p1[tid + 128 * n];
-#pragma unroll
-      for (int n = 0; n < NH * NH / 512; n++) v2[n] = p2[tid + 128 * n];
-#pragma unroll
-      for (int n = 0; n < NH * NO / 512; n++) v3[n] = p3[tid + 128 * n];
-      const float bias = P[tid < NH ? P_B1 + tid : P_B2 + tid - NH];
-      const float bias3 = tid < NO ? P[P_B3 + tid] : 0.0f;
-#pragma unroll
-      for (int n = 0; n < NF * NH / 512; n++) {
-        const int e = tid + 128 * n;  // 16 groups of four per row
-        *reinterpret_cast<f4 *>(lds + L_W1 + e / 16 * S_W + e % 16 * 4) = v1[n];
-      }
-#pragma unroll
-      for (int n = 0; n < NH * NH / 512; n++) {
-        const int e = tid + 128 * n;
-        *reinterpret_cast<f4 *>(lds + L_W2 + e / 16 * S_W + e % 16 * 4) = v2[n];
-      }
-#pragma unroll
-      for (int n = 0; n < NH * NO / 512; n++) {
-        const int e = tid + 128 * n;  // four groups per row
-        *reinterpret_cast<f4 *>(lds + L_W3 + e / 4 * S_W3 + e % 4 * 4) = v3[n];
-      }
-      lds[L_B + tid] = bias;
-      if (tid < NO) lds[L_B + 2 * NH + tid] = bias3;
-    }
-    __syncthreads();
-
-    const int row = tile * TR + 16 * wave + q;
+    const int lr = 16 * grp + q, row = tile * TR + lr;
     const bool ok = row < B;
     const float *xr = X + (long long)(ok ? row : B - 1) * ROW;
-    f4 x[3], z1[4], z2[4], z3;
+    f4 x[3];
 #pragma unroll
     for (int i = 0; i < 3; i++) x[i] = *reinterpret_cast<const f4u *>(xr + 16 * i + 4 * g);
     // the lane's output variables 2 g and 2 g + 1
@@ -167,29 +135,46 @@ __global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU,
       wpr[n] = xr[ROW_WP + 2 * v + 1];
       tau[n] = TAU[(long long)(ok ? row : B - 1) * 8 + v];
     }
-    f4 s1[4], s2[4], h[4], h1[4];
+    __syncthreads();  // weights stored; the previous tile's gradients have been summed
+    if (u < 3) *reinterpret_cast<f4 *>(lds + L_X + lr * S_X + 16 * u + 4 * g) = x[u];
+    // hidden layers: this wave's units 16 u + 4 g + r
+    const int ho = lr * S_H + 16 * u + 4 * g, hrow = lr * S_H + 4 * g;
+    f4 z1 = *reinterpret_cast<const f4 *>(lds + L_B + 16 * u + 4 * g), s1, s2;
 #pragma unroll
-    for (int t = 0; t < 4; t++) z1[t] = *reinterpret_cast<const f4 *>(lds + L_B + 16 * t + 4 * g);
-    forward<4, 3>(lds + L_W1 + 4 * g * S_W + q, S_W, x, z1);
+    for (int i = 0; i < 3; i++)
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+      for (int r = 0; r < 4; r++)
+        z1 = mfma(lds[L_W1 + (16 * i + 4 * g + r) * S_W + 16 * u + q], x[i][r], z1);
+    f4 h;
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        s1[t][r] = sig(GELU_K * z1[t][r]);
-        h1[t][r] = z1[t][r] * s1[t][r];
-      }
+    for (int r = 0; r < 4; r++) {
+      s1[r] = sig(GELU_K * z1[r]);
+      h[r] = z1[r] * s1[r];
+    }
+    *reinterpret_cast<f4 *>(lds + L_H1 + ho) = h;
+    __syncthreads();
+    f4 z2 = *reinterpret_cast<const f4 *>(lds + L_B + NH + 16 * u + 4 * g);
 #pragma unroll
-    for (int t = 0; t < 4; t++) z2[t] = *reinterpret_cast<const f4 *>(lds + L_B + NH + 16 * t + 4 * g);
-    forward<4, 4>(lds + L_W2 + 4 * g * S_W + q, S_W, h1, z2);
+    for (int i = 0; i < 4; i++) {
+      const f4 in = *reinterpret_cast<const f4 *>(lds + L_H1 + hrow + 16 * i);
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+      for (int r = 0; r < 4; r++)
+        z2 = mfma(lds[L_W2 + (16 * i + 4 * g + r) * S_W + 16 * u + q], in[r], z2);
+    }
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        s2[t][r] = sig(GELU_K * z2[t][r]);
-        h[t][r] = z2[t][r] * s2[t][r];
-      }
-    z3 = *reinterpret_cast<const f4 *>(lds + L_B + 2 * NH + 4 * g);
-    forward<1, 4>(lds + L_W3 + 4 * g * S_W3 + q, S_W3, h, &z3);
+    for (int r = 0; r < 4; r++) {
+      s2[r] = sig(GELU_K * z2[r]);
+      h[r] = z2[r] * s2[r];
+    }
+    *reinterpret_cast<f4 *>(lds + L_H2 + ho) = h;
+    __syncthreads();
+    f4 z3 = *reinterpret_cast<const f4 *>(lds + L_B + 2 * NH + 4 * g);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const f4 in = *reinterpret_cast<const f4 *>(lds + L_H2 + hrow + 16 * i);
+#pragma unroll
+      for (int r = 0; r < 4; r++) z3 = mfma(lds[L_W3 + (16 * i + 4 * g + r) * S_W3 + q], in[r], z3);
+    }
     // loss and dloss/dz3 (1/B included): wL = wpL + z3[2v], wR = wpR - z3[2v]
     f4 d3 = f4{0, 0, 0, 0};
 #pragma unroll
@@ -197,83 +182,53 @@ __global__ __launch_bounds__(128) void k_train(const float *X, const float *TAU,
       const float z = z3[2 * n];
       const float el = x2[n] + (wpl[n] + z) * d[n] - tau[n];
       const float er = x3[n] - (wpr[n] - z) * d[n] - tau[n];
-      loss += (double)(om2[n] * (el * el + er * er));
+      if (u == 0) loss += (double)(om2[n] * (el * el + er * er));
       d3[2 * n] = om2[n] * 2.0f * (el + er) * d[n] * inv;
     }
-    f4 d2[4], d1[4];
+    if (u == 0) *reinterpret_cast<f4 *>(lds + L_D3 + lr * S_O + 4 * g) = d3;
+    // deltas; outputs 2 v + 1 have none
+    const float *w3 = lds + L_W3 + (16 * u + q) * S_W3 + 4 * g;
+    f4 d2 = mfma(w3[0], d3[0], f4{0, 0, 0, 0});
+    d2 = mfma(w3[2], d3[2], d2);
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-      const float *w3 = lds + L_W3 + (16 * t + q) * S_W3 + 4 * g;
-      d2[t] = mfma(w3[0], d3[0], f4{0, 0, 0, 0});
-      d2[t] = mfma(w3[2], d3[2], d2[t]);
-      d1[t] = f4{0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) d2[t][r] *= gelu_d(z2[t][r], s2[t][r]);
-    backward<4, 4>(lds + L_W2 + q * S_W + 4 * g, S_W, d2, d1);
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) d1[t][r] *= gelu_d(z1[t][r], s1[t][r]);
-    __syncthreads();  // both waves are done with the weights
-    {
-      const int rr = 16 * wave + q;
-#pragma unroll
-      for (int i = 0; i < 3; i++)
-        *reinterpret_cast<f4 *>(lds + L_X + rr * S_X + 16 * i + 4 * g) = x[i];
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int o = rr * S_H + 16 * t + 4 * g;
-        *reinterpret_cast<f4 *>(lds + L_H1 + o) = h1[t];
-        *reinterpret_cast<f4 *>(lds + L_H2 + o) = h[t];
-        *reinterpret_cast<f4 *>(lds + L_D1 + o) = d1[t];
-        *reinterpret_cast<f4 *>(lds + L_D2 + o) = d2[t];
-      }
-      *reinterpret_cast<f4 *>(lds + L_D3 + rr * S_O + 4 * g) = d3;
-    }
+    for (int r = 0; r < 4; r++) d2[r] *= gelu_d(z2[r], s2[r]);
+    *reinterpret_cast<f4 *>(lds + L_D2 + ho) = d2;
     __syncthreads();
-    // gradients: this wave's output units are the tiles 2 wave, 2 wave + 1 of layers 1 and
-    // 2; of layer 3 its input units are.  Rows past the batch have zero deltas.
+    f4 d1 = f4{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const f4 in = *reinterpret_cast<const f4 *>(lds + L_D2 + hrow + 16 * i);
+      const f4 w = *reinterpret_cast<const f4 *>(lds + L_W2 + (16 * u + q) * S_W + 16 * i + 4 * g);
+#pragma unroll
+      for (int r = 0; r < 4; r++) d1 = mfma(w[r], in[r], d1);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) d1[r] *= gelu_d(z1[r], s1[r]);
+    *reinterpret_cast<f4 *>(lds + L_D1 + ho) = d1;
+    __syncthreads();
+    // gradients.  Rows past the batch have zero deltas.
 #pragma unroll
     for (int k = 0; k < TR; k += 4) {
-      const float *b1 = lds + L_D1 + (k + g) * S_H + 32 * wave + q, *b2 = b1 + (L_D2 - L_D1);
-      const float *ax = lds + L_X + (k + g) * S_X + q, *ah = lds + L_H1 + (k + g) * S_H + q;
-      const float *a2 = lds + L_H2 + (k + g) * S_H + 32 * wave + q;
-      const float dz3 = lds[L_D3 + (k + g) * S_O + q];
+      const float *a = lds + am + (k + g) * as + q, *b = lds + bm + (k + g) * bs + q;
 #pragma unroll
-      for (int n = 0; n < 2; n++) {
-#pragma unroll
-        for (int m = 0; m < 3; m++) g1[m][n] = mfma(ax[16 * m], b1[16 * n], g1[m][n]);
-#pragma unroll
-        for (int m = 0; m < 4; m++) g2[m][n] = mfma(ah[16 * m], b2[16 * n], g2[m][n]);
-        g3[n] = mfma(a2[16 * n], dz3, g3[n]);
-      }
+      for (int n = 0; n < 4; n++) gr[n] = mfma(a[n * an], b[n * bnn], gr[n]);
     }
+    if (tid < 2 * NH + NO) {
 #pragma unroll
-    for (int r = 0; r < TR; r++) {
-      gb += lds[(wave ? L_D2 : L_D1) + r * S_H + (tid & 63)];
-      if (tid < NO) gb3 += lds[L_D3 + r * S_O + tid];
+      for (int r = 0; r < TR; r++) gb += lds[gcol + r * gstr];
     }
   }
   float *out = partial + (long long)blockIdx.x * P_N;
+  const int om0 = wave < 3 ? P_W1 + 16 * wave * NH : wave < 7 ? P_W2 + 16 * (wave - 3) * NH : P_W3;
 #pragma unroll
-  for (int n = 0; n < 2; n++)
+  for (int n = 0; n < 4; n++)
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int col = 32 * wave + 16 * n + q, m0 = 4 * g + r;
-#pragma unroll
-      for (int m = 0; m < 3; m++) out[P_W1 + (16 * m + m0) * NH + col] = g1[m][n][r];
-#pragma unroll
-      for (int m = 0; m < 4; m++) out[P_W2 + (16 * m + m0) * NH + col] = g2[m][n][r];
-      out[P_W3 + (32 * wave + 16 * n + m0) * NO + q] = g3[n][r];
-    }
-  out[(wave ? P_B2 : P_B1) + (tid & 63)] = gb;
-  if (tid < NO) out[P_B3 + tid] = gb3;
+    for (int r = 0; r < 4; r++)
+      out[wave < 7 ? om0 + (4 * g + r) * NH + 16 * n + q : om0 + (16 * n + 4 * g + r) * NO + q] = gr[n][r];
+  if (tid < 2 * NH + NO) out[tid < NH ? P_B1 + tid : tid < 2 * NH ? P_B2 + tid - NH : P_B3 + tid - 2 * NH] = gb;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
-  if ((tid & 63) == 0) lred[wave] = loss;
+  if (u == 0 && (tid & 63) == 0) lred[grp] = loss;
   __syncthreads();
   if (tid == 0) lossp[blockIdx.x] = lred[0] + lred[1];
 }
@@ -362,7 +317,7 @@ int grad_enqueue(idfx_mlp *h, const float *X, const float *TAU, int B, const Ada
                  hipStream_t s) {
   const int nblk = train_blocks(B);
   const dim3 rgrid((P_N + 31) / 32);
-  hipLaunchKernelGGL(k_train, dim3(nblk), dim3(128), 0, s, X, TAU, B, h->P, h->partial, h->lossp);
+  hipLaunchKernelGGL(k_train, dim3(nblk), dim3(512), 0, s, X, TAU, B, h->P, h->partial, h->lossp);
   if (adam)
     hipLaunchKernelGGL(k_reduce<true>, rgrid, dim3(256), 0, s, h->partial, h->lossp, nblk, B, h->G,
                        h->loss, h->P, h->M, h->V, *adam);
