@@ -447,7 +447,7 @@ int idfx_ctx_create(const idfx_desc *desc, const double *dx1, const double *dx2,
   if (st == IDFX_OK) st = alloc_n(c, &c->Uc0, c->n3 * c->nvar);
   if (st == IDFX_OK && d.mhd) st = alloc_n(c, &c->Vs0, c->nvs);
   if (st == IDFX_OK && needs_unfused(c)) st = alloc_n(c, &c->Flux, c->n3 * c->nvar);
-  if (st == IDFX_OK) st = alloc_n(c, &c->dtmax, 1);
+  if (st == IDFX_OK) st = alloc_n(c, &c->dtmax, 2);  // maximum; blocks of publish_dt
   if (st == IDFX_OK && d.shock_flattening) st = alloc_n(c, &c->shock, c->n3);
   if (st == IDFX_OK) st = alloc_n(c, &c->divb, 1);
   if (st == IDFX_OK && d.recon == IDFX_RECON_MLP) {
@@ -494,7 +494,9 @@ int idfx_ctx_create(const idfx_desc *desc, const double *dx1, const double *dx2,
     bool user = false;
     for (int q = 0; q < d.dim; q++)
       user = user || d.lbound[q] == IDFX_BC_USERDEF || d.rbound[q] == IDFX_BC_USERDEF;
-    // without room for the second state the stages stay in place
+    // without room for the second state the stages stay in place, and so do those of a 1-D
+    // grid shorter than its ghost zones, whose sweep could not fill them
+    user = user || (d.dim == 1 && d.nx[0] < c->g.beg[0]);
     if (!user && alloc_n(c, &c->Vc2, c->n3 * c->nvar) == IDFX_OK) c->pp_ok = c->pp_hd_on = true;
     else (void)hipGetLastError();
   }
@@ -572,6 +574,21 @@ static bool all_periodic(const idfx_ctx *c) {
     if (c->d.lbound[d] != IDFX_BC_PERIODIC || c->d.rbound[d] != IDFX_BC_PERIODIC) return false;
   return true;
 }
+// Every ghost cell of a hydro box leads back to an interior one: no user-defined side, and no
+// direction shorter than its ghost zones (a reflection would end in the other side's).
+static bool hydro_box(const idfx_ctx *c) {
+  if (c->d.mhd) return false;
+  for (int d = 0; d < c->d.dim; d++)
+    if (c->d.lbound[d] == IDFX_BC_USERDEF || c->d.rbound[d] == IDFX_BC_USERDEF ||
+        c->g.end[d] - c->g.beg[d] < c->g.beg[d])
+      return false;
+  return true;
+}
+static BoxSides box_sides(const idfx_ctx *c) {
+  BoxSides b{};
+  for (int d = 0; d < c->d.dim; d++) b.lbc[d] = c->d.lbound[d], b.rbc[d] = c->d.rbound[d];
+  return b;
+}
 static int enforce_dir(idfx_ctx *c, int dir, double *Vc, double *Vs, DtTake tk, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   // built-in side types (user-defined sides are left alone by the kernel)
@@ -612,7 +629,9 @@ static int set_boundaries(idfx_ctx *c, double *Vc, double *Vs, DtTake tk, void *
 
 int idfx_set_boundaries(idfx_ctx *c, double *Vc, double *Vs, void *stream) {
   if (!c || !Vc || (c->d.mhd && !Vs)) return IDFX_E_ARGS;
-  // one kernel for the same values in a box periodic in every direction
+  // one kernel for the same values in a hydro box, or one periodic in every direction
+  if (hydro_box(c))
+    return check(c->ops->boundary_box(c->g, Vc, box_sides(c), DtTake{}, (hipStream_t)stream));
   if (all_periodic(c))
     return check(c->ops->boundary_periodic(c->g, Vc, Vs, true, DtTake{}, (hipStream_t)stream));
   return set_boundaries(c, Vc, Vs, DtTake{}, stream);
@@ -750,13 +769,14 @@ int idfx_check_divb(idfx_ctx *c, const double *Vs, double *divb, void *stream) {
   return IDFX_OK;
 }
 
-// Boundary step of a stage.  In a box periodic along every active direction one kernel
+// Boundary step of a stage.  A hydro box takes one kernel.  In a box periodic along every active direction one kernel
 // fills every ghost zone with the same values as the per-direction fill followed by
 // ReconstructVcField; the interior cell field is taken from the faces too unless it
 // already equals their average (every stage after the first of a cycle: the previous
 // stage's ConsToPrim wrote it).
 static int stage_boundaries(idfx_ctx *c, double *Vc, double *Vs, bool cell_field_consistent,
                             DtTake tk, hipStream_t s) {
+  if (hydro_box(c)) return check(c->ops->boundary_box(c->g, Vc, box_sides(c), tk, s));
   if (all_periodic(c))
     return check(c->ops->boundary_periodic(c->g, Vc, Vs, !cell_field_consistent, tk, s));
   return set_boundaries(c, Vc, Vs, tk, s);
@@ -764,11 +784,12 @@ static int stage_boundaries(idfx_ctx *c, double *Vc, double *Vs, bool cell_field
 
 // What a stage does for the next time step.  A cycle of several stages reduces InvDt in the
 // first (DT_REDUCE) and takes the maximum to the host, with ctx->ev_dt behind it, in the
-// second's boundary kernel (DT_TAKE); DT_ALL does everything in one stage.
-enum { DT_NONE, DT_REDUCE, DT_TAKE, DT_ALL };
+// second's boundary kernel (DT_TAKE), or both in the first's sweep (DT_SWEEP, 1-D hydro);
+// DT_ALL does everything in one stage.
+enum { DT_NONE, DT_REDUCE, DT_TAKE, DT_SWEEP, DT_ALL };
 // dtmax is cleared by its last reader, or here after any other use.
 static int dt_begin(idfx_ctx *c, int dt, hipStream_t s) {
-  if (dt != DT_REDUCE && dt != DT_ALL) return IDFX_OK;
+  if (dt != DT_REDUCE && dt != DT_SWEEP && dt != DT_ALL) return IDFX_OK;
   if (!c->dt_clean) {
     hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, c->dtmax);
     IDFX_TRY(check(hipGetLastError()));
@@ -801,12 +822,14 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
                          double *VcOut = nullptr) {
   static const double WC[2][2] = {{0.5, 0.0}, {0.25, 2.0 / 3.0}};
   static const double W0[2][2] = {{0.5, 0.0}, {0.75, 1.0 / 3.0}};
-  if (!skip_boundaries) {
+  // 1-D ping-pong: the sweep fills the ghost zones itself
+  const bool box = VcOut && c->d.dim == 1;
+  if (!skip_boundaries && !box) {
     Region r(c, IDFX_REGION_BOUNDARIES, s);
     IDFX_TRY(stage_boundaries(c, Vc, Vs, consistent, dt_take(c, dt_mode), s));
   }
   IDFX_TRY(dt_taken(c, dt_mode, s));
-  const bool want_dt = dt_mode == DT_REDUCE || dt_mode == DT_ALL;
+  const bool want_dt = dt_mode == DT_REDUCE || dt_mode == DT_SWEEP || dt_mode == DT_ALL;
   double wc = 0.0, w0 = 0.0;
   if (stage > 0) {
     wc = WC[nstages - 2][stage - 1];
@@ -847,6 +870,12 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
         flags |= SW_FINAL | (stage > 0 ? SW_RK : 0) | (write_uc ? SW_WRITE_UC : 0);
       SweepArgs a = sweep_args(c, dir, dt, Vc, Vs, Uc, InvDt, flags);
       a.VcOut = VcOut;
+      if (box) {
+        a.lbc = c->d.lbound[0];
+        a.rbc = c->d.rbound[0];
+        a.VcGhost = Vc;
+        a.dt_host = c->host;
+      }
       a.wc = wc;
       a.w0 = w0;
       IDFX_TRY(check(c->ops->sweep(dir, true, c->g, a, c->emf(), c->target_waves, s)));
@@ -869,6 +898,7 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
   } else if (c->d.mhd && stage > 0) {
     // 1-D MHD keeps Vs constant; AddAndStore still applies (a no-op on equal values)
   }
+  if (dt_mode == DT_SWEEP) IDFX_TRY(dt_taken(c, DT_TAKE, s));
   IDFX_TRY(dt_copy(c, dt_mode, s));
   const int lo[3] = {c->g.beg[0], c->g.beg[1], c->g.beg[2]};
   const int hi[3] = {c->g.end[0], c->g.end[1], c->g.end[2]};
@@ -1037,7 +1067,7 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
   // stage runs in place on the per-kernel schedule and the others alternate Vc -> Vc2 -> Vc;
   // 2-D turbulence 256^2: 154 us a cycle without it, 140 with it)
   const bool fused = c->fused2d_on && nstages >= 2 && Vs;
-  const bool pp3 = c->pp_ok && nstages >= 2 && (c->d.mhd ? c->fused3d_on && Vs : c->pp_hd_on);
+  bool pp3 = c->pp_ok && nstages >= 2 && (c->d.mhd ? c->fused3d_on && Vs : c->pp_hd_on);
   if ((pp3 || fused) && nstages == 3 && !c->Vc3 && !c->vc3_failed) {
     double *v = nullptr, *b = nullptr;
     if (alloc_n(c, &v, c->n3 * c->nvar) == IDFX_OK && (!fused || alloc_n(c, &b, c->nvs) == IDFX_OK)) {
@@ -1051,6 +1081,9 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
   double *pin[3] = {Vc, c->Vc2, Vc}, *pout[3] = {c->Vc2, Vc, nullptr};
   double *bin[3] = {Vs, c->Vs2, Vs}, *bout[3] = {c->Vs2, Vs, nullptr};
   int pp_first = 0;
+  // 1-D sweeps of the ping-pong schedule carry boundaries and time step: all stages or none
+  if (c->d.dim == 1 && nstages == 3 && !c->Vc3) pp3 = false;
+  const bool dt_sweep = pp3 && c->d.dim == 1;
   if (nstages == 3) {
     pp_first = c->Vc3 ? 0 : 1;
     pout[0] = c->Vc3, bout[0] = c->Vs3;
@@ -1064,7 +1097,9 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
   const double tstage[3] = {t0, t0 + *dt, 0.25 * (t0 + *dt + *dt) + 0.75 * t0};
   for (int stage = 0; stage < nstages; stage++) {
     c->t_bound = tstage[stage];
-    const int dt_mode = nstages == 1 ? DT_ALL : stage == 0 ? DT_REDUCE : stage == 1 ? DT_TAKE : DT_NONE;
+    const int dt_mode = nstages == 1 ? DT_ALL
+                        : dt_sweep   ? (stage == 0 ? DT_SWEEP : DT_NONE)
+                                     : (stage == 0 ? DT_REDUCE : stage == 1 ? DT_TAKE : DT_NONE);
     const bool last = stage == nstages - 1;
     if (stage < pp_first || !(pp3 || fused))
       IDFX_TRY(stage_enqueue(c, stage, nstages, *dt, Vc, Vs, Uc, InvDt, 0, last, dt_mode, s, stage > 0));

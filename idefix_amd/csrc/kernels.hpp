@@ -78,6 +78,10 @@ struct SweepArgs {
   const unsigned char *shock;  // shock flags per cell (shock flattening) or nullptr
   double *VcOut;      // SW_FINAL: output primitive state
   double wc, w0;      // SW_RK weights
+  // 1-D hydro FIN sweep: side types, and the host's copy of dtmax (dtmax[1] counts blocks)
+  int lbc, rbc;
+  double *VcGhost;    // = Vc, for its ghost cells
+  unsigned long long *dt_host;
 };
 
 // Element i of an array whose base is uniform across the wave, addressed as base + 32-bit
@@ -331,6 +335,42 @@ __device__ __forceinline__ void block_max_atomic(unsigned long long v, unsigned 
   }
 }
 
+// InvDt maximum to the host from the kernel that reduces it: the last block to arrive stores
+// it to pinned memory and clears it and the block count (dtmax[1]) for the next cycle.  Called
+// by one thread per block, after the block's own maximum.
+__device__ __forceinline__ void publish_dt(unsigned long long *dtmax, unsigned long long *host) {
+  const unsigned long long n =
+      __hip_atomic_fetch_add(dtmax + 1, 1ULL, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+  if (n != gridDim.x - 1) return;
+  const unsigned long long m = __hip_atomic_load(dtmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(host, m, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(dtmax, 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(dtmax + 1, 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+enum BcType { BC_PERIODIC = 0, BC_OUTFLOW = 1, BC_REFLECTIVE = 2, BC_USERDEF = 3 };
+
+// Ghost index q along d (hydro, nint >= ng): the interior index its value comes from, and its
+// side's type in bc and number in side; interior indices have bc = -1.
+__device__ __forceinline__ int ghost_source(const GridDesc &g, int d, int q, int lbc, int rbc,
+                                            int &bc, int &side) {
+  bc = -1;
+  side = q >= g.end[d];
+  if (!side && q >= g.beg[d]) return q;
+  bc = side ? rbc : lbc;
+  const int nint = g.end[d] - g.beg[d];
+  if (bc == BC_OUTFLOW) return side ? g.end[d] - 1 : g.beg[d];
+  if (bc == BC_REFLECTIVE) return 2 * (side ? g.end[d] : g.beg[d]) - q - 1;
+  return side ? q - nint : q + nint;
+}
+// ... and the value itself, from that of the source (normal: the velocity along d)
+__device__ __forceinline__ double ghost_value(double v, bool normal, int bc, int side) {
+  if (!normal) return v;
+  if (bc == BC_REFLECTIVE) return -v;
+  if (bc == BC_OUTFLOW && (side ? -v : v) >= 0.0) return 0.0;
+  return v;
+}
+
 // Passive tracers of one cell (tracer.hpp:58-111, tracer.cpp:13-47): the face value of
 // each tracer is upwinded by the sign of the Riemann mass flux with a van Leer slope, its
 // flux is F_rho * vface * A, and rho*tracer is updated like the fluid variables.  Both
@@ -516,9 +556,25 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
   constexpr int NW = window<C>();
   constexpr int H = NW / 2;
   constexpr int XF = x_first<C>();
+  // 1-D hydro on the ping-pong schedule is bound by its launches: every load of a ghost cell
+  // takes the interior cell the side's rule leads to, block 0 stores the ghost zones, which
+  // nothing in this kernel reads, and the last block hands over the time step.  (1000 cells:
+  // 25 us a cycle with two kernels, 31 with a boundary kernel before each.)
+  constexpr bool BOX = FIN && C::DIM == 1;
   const int lane = threadIdx.x & 63;
   const int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   unsigned long long red = 0;
+  if constexpr (BOX) {
+    const int ng = g.beg[0];
+    if (blockIdx.x == 0 && (int)threadIdx.x < 2 * ng) {
+      const int q = (int)threadIdx.x < ng ? (int)threadIdx.x : g.end[0] - ng + (int)threadIdx.x;
+      int bc, side;
+      const int r = ghost_source(g, 0, q, a.lbc, a.rbc, bc, side);
+#pragma unroll
+      for (int n = 0; n < NV; n++)
+        a.VcGhost[n * g.sv + q] = ghost_value(a.Vc[n * g.sv + r], n == C::MX1, bc, side);
+    }
+  }
   const int first = w * (63 - XF);  // the wave's first site
   if (first + XF < m.nsites) {
     // lanes past the last site repeat it; none of their faces or cells is theirs
@@ -535,8 +591,18 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
     // every load first: the limiters below branch, and loads between them would each wait
     // for memory on their own (512^3 PPM: 9.9 -> 8.1 ms a launch)
     T wv[NV][NW], bn = T(0);
+    if constexpr (BOX) {
 #pragma unroll
-    for (int n = 0; n < NV; n++) {
+      for (int s = 0; s < NW; s++) {
+        int bc, side;
+        const int q = ghost_source(g, 0, max(c + s - H, 0), a.lbc, a.rbc, bc, side);
+#pragma unroll
+        for (int n = 0; n < NV; n++)
+          wv[n][s] = (T)ghost_value(ld32(a.Vc + n * g.sv, row + (unsigned)q), n == C::MX1, bc, side);
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < (BOX ? 0 : NV); n++) {
       if (C::MHD && n == C::BX1) continue;  // the normal field comes from Vs
 #pragma unroll
       for (int s = 0; s < NW; s++) {
@@ -602,7 +668,10 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
     }
   }
   if constexpr (FUSED) {
-    if (a.flags & SW_DT_REDUCE) block_max_atomic(red, a.dtmax);
+    if (a.flags & SW_DT_REDUCE) {
+      block_max_atomic(red, a.dtmax);
+      if (BOX && threadIdx.x == 0) publish_dt(a.dtmax, a.dt_host);
+    }
   }
 }
 
@@ -1678,6 +1747,50 @@ __global__ __launch_bounds__(256) void k_boundary_periodic(GridDesc g, double *V
   }
 }
 
+// Ghost cells of a hydro box (built-in sides, at least nghost cells along each direction),
+// all directions at once: a ghost cell takes the interior cell that the direction-by-direction
+// fill of k_boundary leads back to, with the rules of the sides passed on the way in the order
+// of the directions.  Slabs as in k_boundary_periodic.  (181x133x120:
+// 14.8 us, in three launches 29.4.)
+struct BoxSides {
+  int lbc[3], rbc[3];
+};
+template <class C>
+__global__ __launch_bounds__(256) void k_boundary_box(GridDesc g, double *Vc, BoxSides b, DtTake tk) {
+  take_dt(tk);
+  unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+  for (int d = 0; d < C::DIM; d++) {
+    unsigned n[3], sz = 1;
+    for (int d2 = 0; d2 < 3; d2++) {
+      n[d2] = (d2 == d) ? 2u * g.beg[d] : (d2 < d) ? g.end[d2] - g.beg[d2] : g.nt[d2];
+      sz *= n[d2];
+    }
+    if (t >= sz) {
+      t -= sz;
+      continue;
+    }
+    int q[3], src[3], bc[3], side[3];
+    unsigned r = t;
+    for (int d2 = 0; d2 < 3; d2++) {
+      const unsigned rn = d2 < 2 ? r / n[d2] : 0;
+      const int v = (int)(r - rn * n[d2]);
+      r = rn;
+      q[d2] = d2 > d ? v : d2 < d ? g.beg[d2] + v : v < g.beg[d2] ? v : g.end[d2] + (v - g.beg[d2]);
+      src[d2] = q[d2];
+      if (d2 < C::DIM) src[d2] = ghost_source(g, d2, q[d2], b.lbc[d2], b.rbc[d2], bc[d2], side[d2]);
+    }
+    const unsigned ps = (unsigned)idx3(g, src[2], src[1], src[0]);
+    const unsigned pd = (unsigned)idx3(g, q[2], q[1], q[0]);
+    for (int v = 0; v < C::NVAR + g.ntr; v++) {
+      double val = ld32((const double *)Vc + v * g.sv, ps);
+#pragma unroll
+      for (int d2 = 0; d2 < C::DIM; d2++) val = ghost_value(val, v == C::MX1 + d2, bc[d2], side[d2]);
+      st32(Vc + v * g.sv, pd, val);
+    }
+    return;
+  }
+}
+
 // AddAndStore over whole arrays (stateContainer.cpp:91-98)
 static __global__ __launch_bounds__(256) void k_add_and_store(double *U, const double *U0, long long n,
                                                        double wl, double wr) {
@@ -1750,8 +1863,6 @@ __global__ __launch_bounds__(256) void k_divb_max(GridDesc g, const double *Vs,
 // ------------------------------------------------------------------------------------
 // Boundaries (boundary.hpp): one launch per direction fills both sides.
 // ------------------------------------------------------------------------------------
-enum BcType { BC_PERIODIC = 0, BC_OUTFLOW = 1, BC_REFLECTIVE = 2, BC_USERDEF = 3 };
-
 // Ghost cells of Vc along `dir`, and the tangential Vs components (all components for
 // periodic), for the sides whose type is not user-defined.
 template <class C>

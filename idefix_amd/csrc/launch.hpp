@@ -33,6 +33,9 @@ struct Ops {
   // (see k_boundary_periodic)
   hipError_t (*boundary_periodic)(const GridDesc &g, double *Vc, double *Vs, bool field,
                                   DtTake tk, hipStream_t s) = nullptr;
+  // hydro: every ghost zone of a box with built-in sides in one pass (see k_boundary_box)
+  hipError_t (*boundary_box)(const GridDesc &g, double *Vc, BoxSides b, DtTake tk,
+                             hipStream_t s) = nullptr;
   hipError_t (*boundary)(const GridDesc &g, double *Vc, double *Vs, int dir, int lbc, int rbc,
                          DtTake tk, hipStream_t s) = nullptr;
   hipError_t (*normal_field)(const GridDesc &g, double *Vs, int dir, int recL, int recR,
@@ -369,6 +372,17 @@ hipError_t launch_boundary_periodic(const GridDesc &g, double *Vc, double *Vs, b
 }
 
 template <class C>
+hipError_t launch_boundary_box(const GridDesc &g, double *Vc, BoxSides b, DtTake tk, hipStream_t s) {
+  long long total = 1, inner = 1;
+  for (int d = 0; d < 3; d++) {
+    total *= g.nt[d];
+    inner *= g.end[d] - g.beg[d];
+  }
+  hipLaunchKernelGGL((k_boundary_box<C>), dim3(blocks_for(total - inner)), dim3(256), 0, s, g, Vc, b, tk);
+  return hipGetLastError();
+}
+
+template <class C>
 hipError_t launch_normal_field(const GridDesc &g, double *Vs, int dir, int recL, int recR,
                                hipStream_t s) {
   if constexpr (C::MHD) {
@@ -566,6 +580,7 @@ Ops make_ops() {
   o.vc_field = &launch_vc_field<C>;
   o.boundary = &launch_boundary<C>;
   o.boundary_periodic = &launch_boundary_periodic<C>;
+  if constexpr (!C::MHD) o.boundary_box = &launch_boundary_box<C>;
   o.normal_field = &launch_normal_field<C>;
   o.correct_flux = &launch_correct_flux<C>;
   o.rhs = &launch_rhs<C>;

@@ -100,6 +100,45 @@ def test_hydro_ping_pong_equals_in_place(n, nstages, csiso):
     compare_state(o, g, what="hydro %s" % (n,))
 
 
+@pytest.mark.parametrize("n,recon,nstages,bc", [
+    (n, r, s, b) for n, r, s in [(2, "plm", 2), (3, "ppm", 2), (61, "plm", 3), (62, "ppm", 2),
+                                 (250, "plm", 2), (500, "ppm", 3)]
+    for b in ("periodic", "outflow", "reflective", [("reflective", "outflow")])] +
+    [(2, "ppm", 3, "periodic"), (2, "ppm", 3, "outflow")])
+def test_hd_1d_sides_in_the_sweep(n, recon, nstages, bc):
+    """1-D hydro sweeps that fill the ghost zones and hand over the time step themselves, at the
+    shortest grids (two PPM cells: one less than a ghost zone) and around a wave and a block,
+    against the schedule with a kernel for each: every bit of Vc, and dt, over three cycles; and
+    the oracle."""
+    import torch
+    kw = cfg_kwargs(1, (n,), mhd=False, solver="hllc", recon=recon, bc=bc, gamma=1.4, cfl=0.3,
+                    nstages=nstages)
+    o, g = make_pair(kw, problems.random_hd)
+    _, h = make_pair(kw, problems.random_hd)
+    h.set_fusion(0)
+    o.set_boundaries()
+    for _ in range(3):
+        assert o.cycle() == 0
+        g.cycle()
+        h.cycle()
+        assert g.dt == h.dt
+    assert torch.equal(g.interior(g.Vc), h.interior(h.Vc))
+    compare_state(o, g, what="%s %s %s" % (n, recon, bc))
+
+
+@pytest.mark.parametrize("bc", [["outflow", "reflective", "periodic"], ["reflective", "outflow", "outflow"],
+                                ["periodic", "outflow", "reflective"]])
+@pytest.mark.parametrize("n", [(4,), (3, 5), (64, 7), (2, 2), (4, 3, 5), (33, 6, 2)])
+def test_hd_box_ghost_zones(n, bc):
+    """The ghost zones of a hydro box in one kernel, corners included: every bit as the oracle
+    fills them direction by direction."""
+    kw = cfg_kwargs(len(n), n, mhd=False, solver="hllc", recon="plm", bc=bc[:len(n)], gamma=1.4)
+    o, g = make_pair(kw, problems.random_hd)
+    o.set_boundaries()
+    g.set_boundaries()
+    assert (g.download()[0] == o.Vc).all()
+
+
 @pytest.mark.parametrize("emf,recon", [("uct_hlld", "plm"), ("uct_hlld", "ppm"), ("uct_contact", "plm"),
                                        ("uct_contact", "ppm"), ("uct0", "plm"), ("arithmetic", "ppm")])
 @pytest.mark.parametrize("n", [(4, 3), (57, 4), (60, 5), (62, 3), (63, 9), (124, 4), (20, 70)])
