@@ -837,6 +837,8 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
   }
   const int dim = c->d.dim;
   IDFX_TRY(dt_begin(c, dt_mode, s));
+  int xflags = 0;
+  const bool xy = VcOut && c->ops->sweep_xy;
   for (int dir = 0; dir < dim; dir++) {
     int flags = 0;
     if (dir == 0) {
@@ -846,6 +848,10 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
     if (stage == 0) {
       flags |= (dir == 0) ? SW_INVDT_SET : SW_INVDT_ADD;
       if (dir == dim - 1 && want_dt) flags |= SW_DT_REDUCE;
+    }
+    if (xy && dir == 0) {  // with the y sweep
+      xflags = flags;
+      continue;
     }
     // the learned limiter's weights first, outside the sweep's region
     if (!needs_unfused(c)) IDFX_TRY(mlp_faces(c, dir, Vc, nullptr, s));
@@ -878,7 +884,10 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
       }
       a.wc = wc;
       a.w0 = w0;
-      IDFX_TRY(check(c->ops->sweep(dir, true, c->g, a, c->emf(), c->target_waves, s)));
+      if (xy && dir == 1)
+        IDFX_TRY(check(c->ops->sweep_xy(c->g, a, xflags, c->target_waves, s)));
+      else
+        IDFX_TRY(check(c->ops->sweep(dir, true, c->g, a, c->emf(), c->target_waves, s)));
     }
   }
   if (c->d.mhd && dim >= 2) {

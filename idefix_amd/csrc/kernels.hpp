@@ -420,7 +420,8 @@ __device__ __forceinline__ double cell_update(const GridDesc &g, const SweepArgs
                                               double A, int k, int j, int i, const T *Fm,
                                               const T *Fp, T cmaxm, T cmaxp,
                                               const double *u0pre = nullptr,
-                                              const double *upre = nullptr) {
+                                              const double *upre = nullptr,
+                                              const double *invpre = nullptr) {
   const double dtdV = a.uniform ? a.dtdV : a.dt / cell_dV<C::DIM>(g, k, j, i);
   double u[C::NVAR];
   if (a.flags & (SW_INIT_UC | SW_SAVE_UC0)) {
@@ -502,7 +503,7 @@ __device__ __forceinline__ double cell_update(const GridDesc &g, const SweepArgs
     if (a.flags & SW_INVDT_SET) {
       if (!(a.flags & SW_NO_INVDT_STORE)) st32(a.InvDt, p, inv);
     } else {
-      inv = ld32((const double *)a.InvDt, p) + inv;
+      inv = (invpre ? *invpre : ld32((const double *)a.InvDt, p)) + inv;
       st32(a.InvDt, p, inv);
     }
   }
@@ -875,6 +876,146 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
   if constexpr (FUSED) {
     if (a.flags & SW_DT_REDUCE) block_max_atomic(red, a.dtmax);
   }
+}
+
+// ------------------------------------------------------------------------------------
+// Hydro, x and y sweeps in one kernel: the y march of k_sweep_march (three-cell windows), whose
+// window in LDS also holds a row's x neighbours, so that the x fluxes of cell row f - 1 are solved
+// on the way to its y update.  The conserved state after the x sweep stays in registers: of
+// the passes over Vc (read), Uc (written, read) and InvDt, three of four go.  A wave has 64
+// sites of the x rows, dealt across row ends as in k_sweep_x; its outer lanes give states (0
+// and 63) and faces (1 and 62) only, so 60 of 64 own a cell.  (181x133x120 PLM: 111 us, the
+// two sweeps 176; 138 VGPRs.)
+// ------------------------------------------------------------------------------------
+struct XYGeom {
+  FastDiv ns;     // sites per row: cells beg - 2 .. end + 1
+  int nsites;     // sites of a plane's transverse rows
+  int ts, nseg;   // cells per segment along y, segments
+  int ncb, grp;   // as in MarchGeom
+  int xflags;     // the x sweep's flags (SW_SAVE_UC0, SW_INVDT_SET)
+};
+template <class C, typename T, bool FIN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+void k_sweep_xy(GridDesc g, SweepArgs a, XYGeom m) {
+  static_assert(!C::MHD && C::DIM >= 2 && window<C>() == 3, "hydro with three-cell windows");
+  constexpr int NV = C::NVAR;
+  const int lane = threadIdx.x & 63, tid = threadIdx.x;
+  const int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int cb = w / (m.grp * m.nseg) * m.grp + w % m.grp;
+  const int seg = w / m.grp % m.nseg;
+  unsigned long long red = 0;
+  __shared__ T ring[2 * NV][256], hand[NV][256];
+  if (cb < m.ncb) {
+    const int t = cb * 60 + lane;
+    const unsigned site = (unsigned)min(t, m.nsites - 1);
+    const unsigned tr = C::DIM >= 3 ? fast_div(site, m.ns) : 0;
+    const int i = g.beg[0] - 2 + (int)(site - tr * m.ns.d);
+    const int kk = g.beg[2] + (int)tr;
+    const int c0 = g.beg[1] + seg * m.ts;
+    const int c1 = min(c0 + m.ts, g.end[1]);
+    const unsigned sd = g.nt[0];
+    const unsigned col = (unsigned)idx3(g, kk, 0, i);
+    const double A = face_A<C::DIM, JDIR>(g, kk, 0, i);
+    const bool own = t < m.nsites && lane >= 2 && lane <= 61 && i >= g.beg[0] && i < g.end[0];
+    const int lt = lane > 0 ? tid - 1 : tid, rt = lane < 63 ? tid + 1 : tid;
+    auto row = [&](int r, int n, int l) -> T & { return ring[(r & 1) * NV + n][l]; };
+    // accesses of other lanes' LDS values stay on their side
+    auto wave_fence = [] {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    };
+    T Fprev[NV], cprev = 0, nxt[NV];
+#pragma unroll
+    for (int n = 0; n < NV; n++) {
+      Fprev[n] = 0;
+      T wv[3];
+#pragma unroll
+      for (int s = 0; s < 3; s++) {
+        wv[s] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 - 2 + s) * sd);
+        if (s >= 1) row(c0 - 2 + s, n, tid) = wv[s];
+      }
+      nxt[n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 + 1) * sd);
+      T dummy, right;
+      recon_cell<C>(wv, n, dummy, right, recon_dx<C, T>(g, JDIR, c0 - 1), false);
+      hand[n][tid] = right;
+    }
+    for (int f = c0; f <= c1; f++) {
+      const unsigned pc = col + (unsigned)(f - 1) * sd;  // cell f - 1, updated in this step
+      double u0pre[NV];
+      if constexpr (FIN) {
+        if ((a.flags & SW_RK) && f > c0 && own) {
+#pragma unroll
+          for (int n = 0; n < NV; n++) u0pre[n] = ld32((const double *)a.Uc0 + n * g.sv, pc);
+        }
+      }
+      // x sweep of row f - 1: u = U + rhs, inv = its InvDt
+      double u[NV], inv = 0.0;
+      if (f > c0) {
+        double v[NV];
+        if constexpr (!std::is_same<T, double>::value) {
+#pragma unroll
+          for (int n = 0; n < NV; n++) v[n] = ld32(a.Vc + n * g.sv, pc);
+        }
+        wave_fence();
+        T vL[NV], vR[NV], F[NV], cmax;
+#pragma unroll
+        for (int n = 0; n < NV; n++) {
+          const T wv[3] = {row(f - 1, n, lt), row(f - 1, n, tid), row(f - 1, n, rt)};
+          if constexpr (std::is_same<T, double>::value) v[n] = wv[1];
+          T right;
+          recon_cell<C>(wv, n, vR[n], right, recon_dx<C, T>(g, 0, i), false);
+          vL[n] = __shfl_up(right, 1);
+        }
+        wave_fence();
+        FaceEmf<T> E;
+        riemann<C, IDIR>(vL, vR, F, cmax, E, EMF_ARITHMETIC, eos_face<C, T>(g, pc - 1u, pc));
+        const T cmaxp = __shfl_down(cmax, 1);
+        prim2cons<C>(v, u, g.gamma);
+        if (own && (m.xflags & SW_SAVE_UC0)) {
+#pragma unroll
+          for (int n = 0; n < NV; n++) st32(a.Uc0 + n * g.sv, pc, u[n]);
+        }
+        const double dtdV = a.uniform ? a.dtdV : a.dt / cell_dV<C::DIM>(g, kk, f - 1, i);
+        const double Ax = a.uniform ? a.areax : face_A<C::DIM, IDIR>(g, kk, f - 1, i);
+#pragma unroll
+        for (int n = 0; n < NV; n++) {
+          const double fp = (double)__shfl_down(F[n], 1) * Ax;
+          const double fm = (double)F[n] * Ax;
+          u[n] = u[n] + -dtdV * (fp - fm);
+        }
+        if (m.xflags & SW_INVDT_SET) inv = 0.5 * ((double)cmaxp + (double)cmax) / (g.dx[0][i]);
+      }
+      // y sweep, as in k_sweep_march
+      T vL[NV], vR[NV];
+#pragma unroll
+      for (int n = 0; n < NV; n++) {
+        const T wv[3] = {row(f - 1, n, tid), row(f, n, tid), nxt[n]};
+        row(f + 1, n, tid) = nxt[n];
+        vL[n] = hand[n][tid];
+        T right;
+        recon_cell<C>(wv, n, vR[n], right, recon_dx<C, T>(g, JDIR, f), false);
+        hand[n][tid] = right;
+      }
+      if (f < c1) {
+#pragma unroll
+        for (int n = 0; n < NV; n++)
+          nxt[n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(f + 2) * sd);
+      }
+      T F[NV], cmax;
+      FaceEmf<T> E;
+      riemann<C, JDIR>(vL, vR, F, cmax, E, EMF_ARITHMETIC, eos_face<C, T>(g, pc, pc + sd));
+      if (f > c0 && own) {
+        const double r = cell_update<C, JDIR, false, FIN>(g, a, pc, A, kk, f - 1, i, Fprev, F, cprev,
+                                                          cmax, u0pre, u, &inv);
+        const unsigned long long b = __double_as_longlong(r);
+        red = b > red ? b : red;
+      }
+#pragma unroll
+      for (int n = 0; n < NV; n++) Fprev[n] = F[n];
+      cprev = cmax;
+    }
+  }
+  if (a.flags & SW_DT_REDUCE) block_max_atomic(red, a.dtmax);
 }
 
 // ------------------------------------------------------------------------------------

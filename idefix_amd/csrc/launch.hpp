@@ -33,6 +33,10 @@ struct Ops {
   // (see k_boundary_periodic)
   hipError_t (*boundary_periodic)(const GridDesc &g, double *Vc, double *Vs, bool field,
                                   DtTake tk, hipStream_t s) = nullptr;
+  // hydro with three-cell windows, 2-D and 3-D: x and y sweeps of the ping-pong schedule in one
+  // kernel (a: the y sweep's; xflags: the x sweep's flags)
+  hipError_t (*sweep_xy)(const GridDesc &g, const SweepArgs &a, int xflags, int target_waves,
+                         hipStream_t s) = nullptr;
   // hydro: every ghost zone of a box with built-in sides in one pass (see k_boundary_box)
   hipError_t (*boundary_box)(const GridDesc &g, double *Vc, BoxSides b, DtTake tk,
                              hipStream_t s) = nullptr;
@@ -160,6 +164,25 @@ hipError_t launch_sweep_xtra(const GridDesc &g, const SweepArgs &a, const EmfArr
     hipLaunchKernelGGL((k_sweep_march<C, T, DIR, FUSED, EMF, XTRA, FIN>), dim3(blocks_for(waves, 4)),
                        dim3(256), 0, s, g, a, e, m);
   }
+  return hipGetLastError();
+}
+
+template <class C, typename T>
+hipError_t launch_sweep_xy(const GridDesc &g, const SweepArgs &a, int xflags, int target_waves,
+                           hipStream_t s) {
+  constexpr bool FIN = C::DIM == 2;
+  const int n0 = g.end[0] - g.beg[0], nd = g.end[1] - g.beg[1];
+  XYGeom m;
+  m.ns = fast_div_of((unsigned)(n0 + 4));
+  m.nsites = (int)(m.ns.d * (unsigned)(g.end[2] - g.beg[2]));
+  m.ncb = (m.nsites - 4 + 59) / 60;
+  m.grp = std::min(m.ncb, (n0 + 63) / 60);
+  static const long long slots = resident_waves(k_sweep_xy<C, T, FIN>, target_waves);
+  m.ts = march_segment(m.ncb, nd, slots, march_fill<C, T>());
+  m.nseg = (nd + m.ts - 1) / m.ts;
+  m.xflags = xflags;
+  const long long waves = (long long)(m.ncb + m.grp - 1) / m.grp * m.grp * m.nseg;
+  hipLaunchKernelGGL((k_sweep_xy<C, T, FIN>), dim3(blocks_for(waves, 4)), dim3(256), 0, s, g, a, m);
   return hipGetLastError();
 }
 
@@ -581,6 +604,7 @@ Ops make_ops() {
   o.boundary = &launch_boundary<C>;
   o.boundary_periodic = &launch_boundary_periodic<C>;
   if constexpr (!C::MHD) o.boundary_box = &launch_boundary_box<C>;
+  if constexpr (!C::MHD && C::DIM >= 2 && window<C>() == 3) o.sweep_xy = &launch_sweep_xy<C, T>;
   o.normal_field = &launch_normal_field<C>;
   o.correct_flux = &launch_correct_flux<C>;
   o.rhs = &launch_rhs<C>;
