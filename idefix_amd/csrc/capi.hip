@@ -849,12 +849,12 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
       flags |= (dir == 0) ? SW_INVDT_SET : SW_INVDT_ADD;
       if (dir == dim - 1 && want_dt) flags |= SW_DT_REDUCE;
     }
+    // the learned limiter's weights first, outside the sweep's region
+    if (!needs_unfused(c)) IDFX_TRY(mlp_faces(c, dir, Vc, nullptr, s));
     if (xy && dir == 0) {  // with the y sweep
       xflags = flags;
       continue;
     }
-    // the learned limiter's weights first, outside the sweep's region
-    if (!needs_unfused(c)) IDFX_TRY(mlp_faces(c, dir, Vc, nullptr, s));
     Region r(c, IDFX_REGION_SWEEP_X + dir, s);
     if (needs_unfused(c)) {
       // reference sequence: PrimToCons, (begin copy), CalcFlux, CalcRightHandSide
@@ -885,7 +885,8 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
       a.wc = wc;
       a.w0 = w0;
       if (xy && dir == 1)
-        IDFX_TRY(check(c->ops->sweep_xy(c->g, a, xflags, c->target_waves, s)));
+        IDFX_TRY(check(c->ops->sweep_xy(c->g, a, xflags, c->mlp ? c->mlpW[0] : nullptr, c->emf(),
+                                         c->target_waves, s)));
       else
         IDFX_TRY(check(c->ops->sweep(dir, true, c->g, a, c->emf(), c->target_waves, s)));
     }

@@ -879,132 +879,205 @@ void k_sweep_march(GridDesc g, SweepArgs a, EmfArrays<T> e,
 }
 
 // ------------------------------------------------------------------------------------
-// Hydro, x and y sweeps in one kernel: the y march of k_sweep_march (three-cell windows), whose
+// x and y sweeps of the ping-pong schedule in one kernel: the y march of k_sweep_march, whose
 // window in LDS also holds a row's x neighbours, so that the x fluxes of cell row f - 1 are solved
 // on the way to its y update.  The conserved state after the x sweep stays in registers: of
 // the passes over Vc (read), Uc (written, read) and InvDt, three of four go.  A wave has 64
-// sites of the x rows, dealt across row ends as in k_sweep_x; its outer lanes give states (0
-// and 63) and faces (1 and 62) only, so 60 of 64 own a cell.  (181x133x120 PLM: 111 us, the
-// two sweeps 176; 138 VGPRs.)
+// sites of the x rows, dealt across row ends as in k_sweep_x; its outer lanes give states and
+// faces only, and 60 (three-cell windows) or 58 (PPM) own a cell.  MHD solves the x faces of one
+// more row on each side, at the ends of the first and last segment.  (Hydro PLM 181x133x120:
+// 111 us, the two sweeps 176, at 138 VGPRs; MHD PLM 128^3 181 against 220, at 205.)
 // ------------------------------------------------------------------------------------
 struct XYGeom {
-  FastDiv ns;     // sites per row: cells beg - 2 .. end + 1
-  int nsites;     // sites of a plane's transverse rows
+  FastDiv ns;     // sites per row: cells beg - 2 .. end + 1, PPM beg - 3 .. end + 2
+  int nsites;     // sites of all rows of x
   int ts, nseg;   // cells per segment along y, segments
   int ncb, grp;   // as in MarchGeom
   int xflags;     // the x sweep's flags (SW_SAVE_UC0, SW_INVDT_SET)
+  const float *mlpx;  // learned-limiter weights of the x faces (RECON_MLP; a.mlpw: y)
 };
-template <class C, typename T, bool FIN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-void k_sweep_xy(GridDesc g, SweepArgs a, XYGeom m) {
-  static_assert(!C::MHD && C::DIM >= 2 && window<C>() == 3, "hydro with three-cell windows");
+template <class C>
+constexpr int xy_first() {  // first lane that owns its cell
+  return C::ORDER == RECON_PPM ? 3 : 2;
+}
+template <class C>
+constexpr int xy_owned() {  // lanes that own their cell
+  return C::ORDER == RECON_PPM ? 58 : 60;
+}
+template <class C, typename T>
+constexpr int xy_waves_per_eu() {
+  return C::MHD && std::is_same<T, double>::value ? 2 : 3;
+}
+template <class C, typename T, int EMF, bool FIN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(xy_waves_per_eu<C, T>())))
+void k_sweep_xy(GridDesc g, SweepArgs a, EmfArrays<T> e, XYGeom m) {
+  static_assert(C::DIM >= 2 && window<C>() >= 3 && (!C::MHD || (C::DIM == 3 && EMF == EMF_UCT_CONTACT)),
+                "faces and extensions as below");
   constexpr int NV = C::NVAR;
+  constexpr int NW = window<C>();
+  constexpr int H = NW / 2;
+  constexpr bool PPM = C::ORDER == RECON_PPM;
+  constexpr int EXT = C::MHD ? 1 : 0;  // transverse extension of the faces (sweep_args)
+  constexpr int FO = xy_first<C>(), NO = xy_owned<C>();
+  constexpr int RW = NW - 1;  // rows of the ring, 2 or 4
   const int lane = threadIdx.x & 63, tid = threadIdx.x;
   const int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int cb = w / (m.grp * m.nseg) * m.grp + w % m.grp;
   const int seg = w / m.grp % m.nseg;
   unsigned long long red = 0;
-  __shared__ T ring[2 * NV][256], hand[NV][256];
+  __shared__ double ring[RW * NV][256];
+  __shared__ T hand[C::MHD ? NV - 1 : NV][256];
   if (cb < m.ncb) {
-    const int t = cb * 60 + lane;
-    const unsigned site = (unsigned)min(t, m.nsites - 1);
+    const int t = cb * NO + lane - EXT;
+    const unsigned site = (unsigned)min(max(t, 0), m.nsites - 1);
     const unsigned tr = C::DIM >= 3 ? fast_div(site, m.ns) : 0;
-    const int i = g.beg[0] - 2 + (int)(site - tr * m.ns.d);
-    const int kk = g.beg[2] + (int)tr;
+    const int i = g.beg[0] - (H + 1) + (int)(site - tr * m.ns.d);
+    const int kk = g.beg[2] - EXT + (int)tr;
     const int c0 = g.beg[1] + seg * m.ts;
     const int c1 = min(c0 + m.ts, g.end[1]);
     const unsigned sd = g.nt[0];
     const unsigned col = (unsigned)idx3(g, kk, 0, i);
     const double A = face_A<C::DIM, JDIR>(g, kk, 0, i);
-    const bool own = t < m.nsites && lane >= 2 && lane <= 61 && i >= g.beg[0] && i < g.end[0];
-    const int lt = lane > 0 ? tid - 1 : tid, rt = lane < 63 ? tid + 1 : tid;
-    auto row = [&](int r, int n, int l) -> T & { return ring[(r & 1) * NV + n][l]; };
+    const bool own = t < m.nsites && lane >= FO && lane < FO + NO;
+    const bool own_y = own && i >= g.beg[0] - EXT && i < g.end[0] + EXT;  // owns a y face
+    const bool own_x = own && i >= g.beg[0] && i <= g.end[0];             // ... an x face
+    const bool rhs_lane = own && i >= g.beg[0] && i < g.end[0] && kk >= g.beg[2] && kk < g.end[2];
+    const unsigned vcol = (unsigned)idxs(g, 0, kk, 0, i), vsd = g.vsn[0];
+    auto row = [&](int r, int n, int l) -> double & { return ring[(r & (RW - 1)) * NV + n][l]; };
+    auto at = [&](int dl) { return tid - lane + min(max(lane + dl, 0), 63); };  // lane + dl's slot
+    auto is_bx = [](int n) { return C::MHD && n == C::BX1; };
+    auto is_by = [](int n) { return C::MHD && n == C::BX1 + 1; };
+    auto slot = [](int n) { return C::MHD && n > C::BX1 + 1 ? n - 1 : n; };
     // accesses of other lanes' LDS values stay on their side
     auto wave_fence = [] {
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
     };
-    T Fprev[NV], cprev = 0, nxt[NV];
+    T Fprev[NV], fcar[NV], cprev = 0;
+    double nxt[NV];
 #pragma unroll
     for (int n = 0; n < NV; n++) {
       Fprev[n] = 0;
-      T wv[3];
+      T wv[NW];
 #pragma unroll
-      for (int s = 0; s < 3; s++) {
-        wv[s] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 - 2 + s) * sd);
-        if (s >= 1) row(c0 - 2 + s, n, tid) = wv[s];
+      for (int s = 0; s < NW; s++) {
+        const double v = ld32(a.Vc + n * g.sv, col + (unsigned)(c0 - 1 - H + s) * sd);
+        if (s >= 1) row(c0 - 1 - H + s, n, tid) = v;
+        wv[s] = (T)v;
       }
-      nxt[n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 + 1) * sd);
+      nxt[n] = ld32(a.Vc + n * g.sv, col + (unsigned)(c0 + H) * sd);
+      if (is_by(n)) continue;
       T dummy, right;
-      recon_cell<C>(wv, n, dummy, right, recon_dx<C, T>(g, JDIR, c0 - 1), false);
-      hand[n][tid] = right;
+      if constexpr (C::ORDER == RECON_MLP) {
+        recon_mlp<C, JDIR>(wv, n, a.mlpw, g.sv, col + (unsigned)(c0 - 1) * sd, sd, dummy, right);
+      } else if constexpr (PPM) {
+        fcar[n] = recon_face<C>(wv);
+        recon_ppm<C>(wv, n, ppm_face(wv[0], wv[1], wv[2], wv[3]), fcar[n], dummy, right);
+      } else {
+        recon_cell<C>(wv, n, dummy, right, recon_dx<C, T>(g, JDIR, c0 - 1), false);
+      }
+      hand[slot(n)][tid] = right;
     }
-    for (int f = c0; f <= c1; f++) {
+    const bool head = EXT && c0 == g.beg[1], tail = EXT && c1 == g.end[1];
+    for (int f = c0; f <= c1 + (tail ? 1 : 0); f++) {
       const unsigned pc = col + (unsigned)(f - 1) * sd;  // cell f - 1, updated in this step
+      const bool cell_row = f > c0 && f <= c1;
+      T bnx = T(0), bny = T(0);
+      if constexpr (C::MHD) {
+        bnx = (T)ld32(a.Vs, vcol + (unsigned)(f - 1) * vsd);
+        bny = (T)ld32(a.Vs + g.svs, vcol + (unsigned)f * vsd);
+      }
       double u0pre[NV];
       if constexpr (FIN) {
-        if ((a.flags & SW_RK) && f > c0 && own) {
+        if ((a.flags & SW_RK) && cell_row && rhs_lane) {
 #pragma unroll
           for (int n = 0; n < NV; n++) u0pre[n] = ld32((const double *)a.Uc0 + n * g.sv, pc);
         }
       }
       // x sweep of row f - 1: u = U + rhs, inv = its InvDt
       double u[NV], inv = 0.0;
-      if (f > c0) {
+      if (f > c0 || head) {
         double v[NV];
-        if constexpr (!std::is_same<T, double>::value) {
-#pragma unroll
-          for (int n = 0; n < NV; n++) v[n] = ld32(a.Vc + n * g.sv, pc);
-        }
         wave_fence();
         T vL[NV], vR[NV], F[NV], cmax;
 #pragma unroll
         for (int n = 0; n < NV; n++) {
-          const T wv[3] = {row(f - 1, n, lt), row(f - 1, n, tid), row(f - 1, n, rt)};
-          if constexpr (std::is_same<T, double>::value) v[n] = wv[1];
-          T right;
-          recon_cell<C>(wv, n, vR[n], right, recon_dx<C, T>(g, 0, i), false);
+          v[n] = row(f - 1, n, tid);
+          if (is_bx(n)) {
+            vL[n] = vR[n] = bnx;
+            continue;
+          }
+          T wv[NW], right;
+#pragma unroll
+          for (int s = 0; s < NW; s++) wv[s] = s == H ? (T)v[n] : (T)row(f - 1, n, at(s - H));
+          if constexpr (C::ORDER == RECON_MLP) {
+            recon_mlp<C, IDIR>(wv, n, m.mlpx, g.sv, pc, 1u, vR[n], right);
+          } else if constexpr (PPM) {
+            const T fr = recon_face<C>(wv);
+            recon_ppm<C>(wv, n, __shfl_up(fr, 1), fr, vR[n], right);
+          } else {
+            recon_cell<C>(wv, n, vR[n], right, recon_dx<C, T>(g, 0, i), false);
+          }
           vL[n] = __shfl_up(right, 1);
         }
         wave_fence();
         FaceEmf<T> E;
-        riemann<C, IDIR>(vL, vR, F, cmax, E, EMF_ARITHMETIC, eos_face<C, T>(g, pc - 1u, pc));
+        riemann<C, IDIR>(vL, vR, F, cmax, E, EMF, eos_face<C, T>(g, pc - 1u, pc));
+        if (own_x) store_face_emf<C, IDIR>(e, pc, EMF, E);
         const T cmaxp = __shfl_down(cmax, 1);
         prim2cons<C>(v, u, g.gamma);
-        if (own && (m.xflags & SW_SAVE_UC0)) {
+        if (cell_row && rhs_lane && (m.xflags & SW_SAVE_UC0)) {
 #pragma unroll
-          for (int n = 0; n < NV; n++) st32(a.Uc0 + n * g.sv, pc, u[n]);
+          for (int n = 0; n < NV; n++)
+            if (!C::is_ct_field(n)) st32(a.Uc0 + n * g.sv, pc, u[n]);
         }
         const double dtdV = a.uniform ? a.dtdV : a.dt / cell_dV<C::DIM>(g, kk, f - 1, i);
         const double Ax = a.uniform ? a.areax : face_A<C::DIM, IDIR>(g, kk, f - 1, i);
 #pragma unroll
         for (int n = 0; n < NV; n++) {
+          if (C::is_ct_field(n)) continue;
           const double fp = (double)__shfl_down(F[n], 1) * Ax;
           const double fm = (double)F[n] * Ax;
           u[n] = u[n] + -dtdV * (fp - fm);
         }
         if (m.xflags & SW_INVDT_SET) inv = 0.5 * ((double)cmaxp + (double)cmax) / (g.dx[0][i]);
       }
+      if (EXT && f > c1) break;
       // y sweep, as in k_sweep_march
       T vL[NV], vR[NV];
 #pragma unroll
       for (int n = 0; n < NV; n++) {
-        const T wv[3] = {row(f - 1, n, tid), row(f, n, tid), nxt[n]};
-        row(f + 1, n, tid) = nxt[n];
-        vL[n] = hand[n][tid];
+        T wv[NW];
+#pragma unroll
+        for (int s = 0; s < NW - 1; s++) wv[s] = (T)row(f - H + s, n, tid);
+        wv[NW - 1] = (T)nxt[n];
+        row(f + H, n, tid) = nxt[n];
+        if (is_by(n)) {
+          vL[n] = vR[n] = bny;
+          continue;
+        }
+        vL[n] = hand[slot(n)][tid];
         T right;
-        recon_cell<C>(wv, n, vR[n], right, recon_dx<C, T>(g, JDIR, f), false);
-        hand[n][tid] = right;
+        if constexpr (C::ORDER == RECON_MLP) {
+          recon_mlp<C, JDIR>(wv, n, a.mlpw, g.sv, col + (unsigned)f * sd, sd, vR[n], right);
+        } else if constexpr (PPM) {
+          const T fr = recon_face<C>(wv);
+          recon_ppm<C>(wv, n, fcar[n], fr, vR[n], right);
+          fcar[n] = fr;
+        } else {
+          recon_cell<C>(wv, n, vR[n], right, recon_dx<C, T>(g, JDIR, f), false);
+        }
+        hand[slot(n)][tid] = right;
       }
       if (f < c1) {
 #pragma unroll
-        for (int n = 0; n < NV; n++)
-          nxt[n] = (T)ld32(a.Vc + n * g.sv, col + (unsigned)(f + 2) * sd);
+        for (int n = 0; n < NV; n++) nxt[n] = ld32(a.Vc + n * g.sv, col + (unsigned)(f + 1 + H) * sd);
       }
       T F[NV], cmax;
       FaceEmf<T> E;
-      riemann<C, JDIR>(vL, vR, F, cmax, E, EMF_ARITHMETIC, eos_face<C, T>(g, pc, pc + sd));
-      if (f > c0 && own) {
+      riemann<C, JDIR>(vL, vR, F, cmax, E, EMF, eos_face<C, T>(g, pc, pc + sd));
+      if (own_y && (f < c1 || c1 == g.end[1])) store_face_emf<C, JDIR>(e, pc + sd, EMF, E);
+      if (cell_row && rhs_lane) {
         const double r = cell_update<C, JDIR, false, FIN>(g, a, pc, A, kk, f - 1, i, Fprev, F, cprev,
                                                           cmax, u0pre, u, &inv);
         const unsigned long long b = __double_as_longlong(r);

@@ -33,10 +33,11 @@ struct Ops {
   // (see k_boundary_periodic)
   hipError_t (*boundary_periodic)(const GridDesc &g, double *Vc, double *Vs, bool field,
                                   DtTake tk, hipStream_t s) = nullptr;
-  // hydro with three-cell windows, 2-D and 3-D: x and y sweeps of the ping-pong schedule in one
-  // kernel (a: the y sweep's; xflags: the x sweep's flags)
-  hipError_t (*sweep_xy)(const GridDesc &g, const SweepArgs &a, int xflags, int target_waves,
-                         hipStream_t s) = nullptr;
+  // 2-D and 3-D hydro, 3-D MHD with uct_contact: x and y sweeps of the ping-pong schedule in
+  // one kernel (a: the y sweep's arguments; xflags, mlpx: the x sweep's flags and
+  // learned-limiter weights)
+  hipError_t (*sweep_xy)(const GridDesc &g, const SweepArgs &a, int xflags, const float *mlpx,
+                         const void *emf, int target_waves, hipStream_t s) = nullptr;
   // hydro: every ghost zone of a box with built-in sides in one pass (see k_boundary_box)
   hipError_t (*boundary_box)(const GridDesc &g, double *Vc, BoxSides b, DtTake tk,
                              hipStream_t s) = nullptr;
@@ -168,22 +169,39 @@ hipError_t launch_sweep_xtra(const GridDesc &g, const SweepArgs &a, const EmfArr
 }
 
 template <class C, typename T>
-hipError_t launch_sweep_xy(const GridDesc &g, const SweepArgs &a, int xflags, int target_waves,
-                           hipStream_t s) {
+hipError_t launch_sweep_xy(const GridDesc &g, const SweepArgs &a, int xflags, const float *mlpx,
+                           const void *emf, int target_waves, hipStream_t s) {
   constexpr bool FIN = C::DIM == 2;
+  constexpr int EMF = C::MHD ? EMF_UCT_CONTACT : EMF_ARITHMETIC, EXT = C::MHD ? 1 : 0;
+  constexpr int FO = xy_first<C>(), NO = xy_owned<C>();
   const int n0 = g.end[0] - g.beg[0], nd = g.end[1] - g.beg[1];
+  for (int d = 0; d < C::DIM; d++)
+    if (d != 1 && a.ext[d] != EXT) return hipErrorInvalidValue;
   XYGeom m;
-  m.ns = fast_div_of((unsigned)(n0 + 4));
-  m.nsites = (int)(m.ns.d * (unsigned)(g.end[2] - g.beg[2]));
-  m.ncb = (m.nsites - 4 + 59) / 60;
-  m.grp = std::min(m.ncb, (n0 + 63) / 60);
-  static const long long slots = resident_waves(k_sweep_xy<C, T, FIN>, target_waves);
+  m.ns = fast_div_of((unsigned)(n0 + 2 * FO));
+  m.nsites = (int)(m.ns.d * (unsigned)(g.end[2] - g.beg[2] + 2 * EXT));
+  m.ncb = (m.nsites - 2 * (FO - EXT) + NO - 1) / NO;
+  m.grp = std::min(m.ncb, (n0 + 2 * FO + NO - 1) / NO);
+  static const long long slots = resident_waves(k_sweep_xy<C, T, EMF, FIN>, target_waves);
   m.ts = march_segment(m.ncb, nd, slots, march_fill<C, T>());
   m.nseg = (nd + m.ts - 1) / m.ts;
   m.xflags = xflags;
+  m.mlpx = mlpx;
   const long long waves = (long long)(m.ncb + m.grp - 1) / m.grp * m.grp * m.nseg;
-  hipLaunchKernelGGL((k_sweep_xy<C, T, FIN>), dim3(blocks_for(waves, 4)), dim3(256), 0, s, g, a, m);
+  EmfArrays<T> e{};
+  if constexpr (C::MHD) e = *static_cast<const EmfArrays<T> *>(emf);
+  hipLaunchKernelGGL((k_sweep_xy<C, T, EMF, FIN>), dim3(blocks_for(waves, 4)), dim3(256), 0, s, g, a, e, m);
   return hipGetLastError();
+}
+// Where k_sweep_xy is used.  Whole cycles with it, and with two sweeps: hydro 256^3 PLM 2687,
+// 3468 us, PPM 3473, 3874; 64^3 86, 96 and 130, 137.  MHD 256^3 PLM 6989, 7633 (FP32 stencils
+// 6116, 7017), 32^3 97, 104.  MHD with PPM is bound by instruction issue, which the lanes without
+// a cell add to: 203x150x97 2534, 2480 us (FP32 2132, 1971), 512^3 the same; it keeps its
+// sweeps.  Roe's MHD solver has no registers to spare.
+template <class C>
+constexpr bool has_sweep_xy() {
+  return C::DIM >= 2 && window<C>() >= 3 &&
+         (!C::MHD || (C::DIM == 3 && !C::ISO && window<C>() == 3 && C::SOLVER != SOLVER_ROE));
 }
 
 // The options that add per-cell work (shock flags, passive tracers) select the XTRA
@@ -604,7 +622,7 @@ Ops make_ops() {
   o.boundary = &launch_boundary<C>;
   o.boundary_periodic = &launch_boundary_periodic<C>;
   if constexpr (!C::MHD) o.boundary_box = &launch_boundary_box<C>;
-  if constexpr (!C::MHD && C::DIM >= 2 && window<C>() == 3) o.sweep_xy = &launch_sweep_xy<C, T>;
+  if constexpr (has_sweep_xy<C>()) o.sweep_xy = &launch_sweep_xy<C, T>;
   o.normal_field = &launch_normal_field<C>;
   o.correct_flux = &launch_correct_flux<C>;
   o.rhs = &launch_rhs<C>;

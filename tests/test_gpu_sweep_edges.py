@@ -5,7 +5,7 @@ are compared with the oracle cell by cell (FP64 bar of tests/pairs.py)."""
 import pytest
 
 from idefix_amd import problems
-from tests.pairs import cfg_kwargs, compare_state, make_pair
+from tests.pairs import cfg_kwargs, compare_state, interior_faces, make_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -137,6 +137,36 @@ def test_hd_box_ghost_zones(n, bc):
     o.set_boundaries()
     g.set_boundaries()
     assert (g.download()[0] == o.Vc).all()
+
+
+@pytest.mark.parametrize("mhd,recon,precision", [(True, "plm", "fp64"), (True, "plm", "fp32"),
+                                                 (True, "limo3", "fp64"), (False, "plm", "fp64"),
+                                                 (False, "ppm", "fp64")])
+@pytest.mark.parametrize("n", [(4, 3, 5), (3, 37, 4), (52, 4, 3), (54, 5, 3), (56, 4, 3), (58, 3, 3), (60, 5, 2),
+                               (62, 3, 3), (114, 4, 3), (118, 5, 3), (57, 130, 3)])
+def test_sweep_xy_equals_two_sweeps(n, mhd, recon, precision):
+    """x and y sweeps in one kernel (60 or 58 of a wave's 64 lanes own a cell, rows dealt across
+    their ends, several segments along y) against a kernel for each: every bit of Vc, Vs and
+    dt over two cycles; and the oracle."""
+    import torch
+    kw = cfg_kwargs(3, n, mhd=mhd, solver="hlld" if mhd else "hllc", emf="uct_contact", recon=recon,
+                    cfl=0.3, nstages=2)
+    ic = problems.random_mhd if mhd else problems.random_hd
+    o, g = make_pair(kw, ic, precision=precision)
+    _, h = make_pair(kw, ic, precision=precision)
+    h.set_fusion(0)
+    o.set_boundaries()
+    for _ in range(2):
+        assert o.cycle() == 0
+        g.cycle()
+        h.cycle()
+        assert g.dt == h.dt
+    assert torch.equal(g.interior(g.Vc), h.interior(h.Vc))
+    if mhd:
+        for a, b in zip(interior_faces(o, g.download()[1]), interior_faces(o, h.download()[1])):
+            assert (a == b).all()
+    if precision == "fp64":
+        compare_state(o, g, what="xy %s %s" % (recon, n))
 
 
 @pytest.mark.parametrize("emf,recon", [("uct_hlld", "plm"), ("uct_hlld", "ppm"), ("uct_contact", "plm"),
