@@ -81,7 +81,7 @@ struct SweepArgs {
   // 1-D hydro FIN sweep: side types, and the host's copy of dtmax (dtmax[1] counts blocks)
   int lbc, rbc;
   double *VcGhost;    // = Vc, for its ghost cells
-  unsigned long long *dt_host;
+  unsigned long long *dt_host, dt_seq;
 };
 
 // Element i of an array whose base is uniform across the wave, addressed as base + 32-bit
@@ -335,15 +335,22 @@ __device__ __forceinline__ void block_max_atomic(unsigned long long v, unsigned 
   }
 }
 
+// InvDt maximum to pinned memory: the value, then the cycle's number, which the host waits for.
+__device__ __forceinline__ void dt_to_host(unsigned long long *host, unsigned long long m,
+                                           unsigned long long seq) {
+  __hip_atomic_store(host, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(host + 1, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // InvDt maximum to the host from the kernel that reduces it: the last block to arrive stores
 // it to pinned memory and clears it and the block count (dtmax[1]) for the next cycle.  Called
 // by one thread per block, after the block's own maximum.
-__device__ __forceinline__ void publish_dt(unsigned long long *dtmax, unsigned long long *host) {
+__device__ __forceinline__ void publish_dt(unsigned long long *dtmax, unsigned long long *host,
+                                           unsigned long long seq) {
   const unsigned long long n =
       __hip_atomic_fetch_add(dtmax + 1, 1ULL, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
   if (n != gridDim.x - 1) return;
   const unsigned long long m = __hip_atomic_load(dtmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(host, m, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  dt_to_host(host, m, seq);
   __hip_atomic_store(dtmax, 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(dtmax + 1, 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -671,7 +678,7 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
   if constexpr (FUSED) {
     if (a.flags & SW_DT_REDUCE) {
       block_max_atomic(red, a.dtmax);
-      if (BOX && threadIdx.x == 0) publish_dt(a.dtmax, a.dt_host);
+      if (BOX && threadIdx.x == 0) publish_dt(a.dtmax, a.dt_host, a.dt_seq);
     }
   }
 }
@@ -1841,11 +1848,11 @@ __global__ __launch_bounds__(256) void k_vc_field(GridDesc g, const double *Vs, 
 // boundary kernel stores it to pinned memory and clears it for the next cycle, in place of a
 // clearing kernel and a copy.  dtmax == nullptr: nothing to take.
 struct DtTake {
-  unsigned long long *dtmax, *host;
+  unsigned long long *dtmax, *host, seq;
 };
 __device__ __forceinline__ void take_dt(const DtTake &tk) {
   if (tk.dtmax != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
-    __hip_atomic_store(tk.host, *tk.dtmax, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    dt_to_host(tk.host, *tk.dtmax, tk.seq);
     *tk.dtmax = 0ULL;
   }
 }
