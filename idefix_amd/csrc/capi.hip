@@ -127,6 +127,7 @@ struct idfx_ctx {
   // (SW_FINAL)
   bool pp_ok = false;
   bool pp_hd_on = false;  // hydro: off at fusion level 0 (MHD follows fused3d_on)
+  bool xy_all = false;    // fusion level 2: k_sweep_xy at every size
   double *Vc2 = nullptr, *Vs2 = nullptr;
   // ping-pong with three stages: the first stage's output (2-D MHD: and its faces)
   double *Vc3 = nullptr, *Vs3 = nullptr;
@@ -858,7 +859,9 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
   const int dim = c->d.dim;
   IDFX_TRY(dt_begin(c, dt_mode, s));
   int xflags = 0;
-  const bool xy = VcOut && c->ops->sweep_xy;
+  const bool xy = VcOut && c->ops->sweep_xy &&
+                  (c->xy_all || (long long)c->d.nx[0] * c->d.nx[1] * c->d.nx[2] >=
+                                    c->ops->sweep_xy_min_cells);
   for (int dir = 0; dir < dim; dir++) {
     int flags = 0;
     if (dir == 0) {
@@ -1065,6 +1068,7 @@ int idfx_ctx_set_fusion(idfx_ctx *c, int level) {
   c->fused2d_on = level >= 1 && c->fused2d_ok;
   c->fused3d_on = level >= 1 && c->fused3d_ok;
   c->pp_hd_on = level >= 1 && c->pp_ok;
+  c->xy_all = level == 2;
   c->ct3d_use = c->fused3d_on &&
                 (level == 2 || (long long)c->d.nx[0] * c->d.nx[1] * c->d.nx[2] >= CT3D_MIN_CELLS);
   return IDFX_OK;

@@ -932,7 +932,10 @@ void k_sweep_xy(GridDesc g, SweepArgs a, EmfArrays<T> e, XYGeom m) {
   const int cb = w / (m.grp * m.nseg) * m.grp + w % m.grp;
   const int seg = w / m.grp % m.nseg;
   unsigned long long red = 0;
-  __shared__ double ring[RW * NV][256];
+  // the window keeps the state in double for the conserved state of its centre, except with PPM,
+  // where FP32 rows leave room for a third wave per SIMD
+  using R = std::conditional_t<(C::MHD && NW == 5), T, double>;
+  __shared__ R ring[RW * NV][256];
   __shared__ T hand[C::MHD ? NV - 1 : NV][256];
   if (cb < m.ncb) {
     const int t = cb * NO + lane - EXT;
@@ -950,7 +953,7 @@ void k_sweep_xy(GridDesc g, SweepArgs a, EmfArrays<T> e, XYGeom m) {
     const bool own_x = own && i >= g.beg[0] && i <= g.end[0];             // ... an x face
     const bool rhs_lane = own && i >= g.beg[0] && i < g.end[0] && kk >= g.beg[2] && kk < g.end[2];
     const unsigned vcol = (unsigned)idxs(g, 0, kk, 0, i), vsd = g.vsn[0];
-    auto row = [&](int r, int n, int l) -> double & { return ring[(r & (RW - 1)) * NV + n][l]; };
+    auto row = [&](int r, int n, int l) -> R & { return ring[(r & (RW - 1)) * NV + n][l]; };
     auto at = [&](int dl) { return tid - lane + min(max(lane + dl, 0), 63); };  // lane + dl's slot
     auto is_bx = [](int n) { return C::MHD && n == C::BX1; };
     auto is_by = [](int n) { return C::MHD && n == C::BX1 + 1; };
@@ -961,7 +964,7 @@ void k_sweep_xy(GridDesc g, SweepArgs a, EmfArrays<T> e, XYGeom m) {
       __builtin_amdgcn_wave_barrier();
     };
     T Fprev[NV], fcar[NV], cprev = 0;
-    double nxt[NV];
+    R nxt[NV];
 #pragma unroll
     for (int n = 0; n < NV; n++) {
       Fprev[n] = 0;
@@ -969,10 +972,10 @@ void k_sweep_xy(GridDesc g, SweepArgs a, EmfArrays<T> e, XYGeom m) {
 #pragma unroll
       for (int s = 0; s < NW; s++) {
         const double v = ld32(a.Vc + n * g.sv, col + (unsigned)(c0 - 1 - H + s) * sd);
-        if (s >= 1) row(c0 - 1 - H + s, n, tid) = v;
+        if (s >= 1) row(c0 - 1 - H + s, n, tid) = (R)v;
         wv[s] = (T)v;
       }
-      nxt[n] = ld32(a.Vc + n * g.sv, col + (unsigned)(c0 + H) * sd);
+      nxt[n] = (R)ld32(a.Vc + n * g.sv, col + (unsigned)(c0 + H) * sd);
       if (is_by(n)) continue;
       T dummy, right;
       if constexpr (C::ORDER == RECON_MLP) {
@@ -1009,14 +1012,15 @@ void k_sweep_xy(GridDesc g, SweepArgs a, EmfArrays<T> e, XYGeom m) {
         T vL[NV], vR[NV], F[NV], cmax;
 #pragma unroll
         for (int n = 0; n < NV; n++) {
-          v[n] = row(f - 1, n, tid);
+          const R vc = row(f - 1, n, tid);
+          v[n] = std::is_same<R, double>::value ? (double)vc : ld32(a.Vc + n * g.sv, pc);
           if (is_bx(n)) {
             vL[n] = vR[n] = bnx;
             continue;
           }
           T wv[NW], right;
 #pragma unroll
-          for (int s = 0; s < NW; s++) wv[s] = s == H ? (T)v[n] : (T)row(f - 1, n, at(s - H));
+          for (int s = 0; s < NW; s++) wv[s] = s == H ? (T)vc : (T)row(f - 1, n, at(s - H));
           if constexpr (C::ORDER == RECON_MLP) {
             recon_mlp<C, IDIR>(wv, n, m.mlpx, g.sv, pc, 1u, vR[n], right);
           } else if constexpr (PPM) {
@@ -1078,7 +1082,7 @@ void k_sweep_xy(GridDesc g, SweepArgs a, EmfArrays<T> e, XYGeom m) {
       }
       if (f < c1) {
 #pragma unroll
-        for (int n = 0; n < NV; n++) nxt[n] = ld32(a.Vc + n * g.sv, col + (unsigned)(f + 1 + H) * sd);
+        for (int n = 0; n < NV; n++) nxt[n] = (R)ld32(a.Vc + n * g.sv, col + (unsigned)(f + 1 + H) * sd);
       }
       T F[NV], cmax;
       FaceEmf<T> E;

@@ -38,6 +38,7 @@ struct Ops {
   // learned-limiter weights)
   hipError_t (*sweep_xy)(const GridDesc &g, const SweepArgs &a, int xflags, const float *mlpx,
                          const void *emf, int target_waves, hipStream_t s) = nullptr;
+  long long sweep_xy_min_cells = 0;
   // hydro: every ghost zone of a box with built-in sides in one pass (see k_boundary_box)
   hipError_t (*boundary_box)(const GridDesc &g, double *Vc, BoxSides b, DtTake tk,
                              hipStream_t s) = nullptr;
@@ -195,13 +196,20 @@ hipError_t launch_sweep_xy(const GridDesc &g, const SweepArgs &a, int xflags, co
 }
 // Where k_sweep_xy is used.  Whole cycles with it, and with two sweeps: hydro 256^3 PLM 2687,
 // 3468 us, PPM 3473, 3874; 64^3 86, 96 and 130, 137.  MHD 256^3 PLM 6989, 7633 (FP32 stencils
-// 6116, 7017), 32^3 97, 104.  MHD with PPM is bound by instruction issue, which the lanes without
-// a cell add to: 203x150x97 2534, 2480 us (FP32 2132, 1971), 512^3 the same; it keeps its
-// sweeps.  Roe's MHD solver has no registers to spare.
-template <class C>
+// 6116, 7017), 32^3 97, 104.  Roe's MHD solver has no registers to spare.  MHD with PPM is
+// bound by instruction issue, which the lanes without a cell add to: in FP64 it keeps its sweeps
+// (203x150x97 2534, 2480 us; 512^3 the same), and with FP32 stencils it takes one kernel where the
+// passes it saves go to memory (512x512x256 27.2, 28.5 ms; 384^3 35.0, 36.1; but 203x150x97
+// 2026, 1963 us and 256^3 the same).
+template <class C, typename T>
 constexpr bool has_sweep_xy() {
   return C::DIM >= 2 && window<C>() >= 3 &&
-         (!C::MHD || (C::DIM == 3 && !C::ISO && window<C>() == 3 && C::SOLVER != SOLVER_ROE));
+         (!C::MHD || (C::DIM == 3 && !C::ISO && C::SOLVER != SOLVER_ROE &&
+                      (window<C>() == 3 || std::is_same<T, float>::value)));
+}
+template <class C>
+constexpr long long sweep_xy_min_cells() {
+  return C::MHD && window<C>() == 5 ? 1LL << 25 : 0;
 }
 
 // The options that add per-cell work (shock flags, passive tracers) select the XTRA
@@ -622,7 +630,10 @@ Ops make_ops() {
   o.boundary = &launch_boundary<C>;
   o.boundary_periodic = &launch_boundary_periodic<C>;
   if constexpr (!C::MHD) o.boundary_box = &launch_boundary_box<C>;
-  if constexpr (has_sweep_xy<C>()) o.sweep_xy = &launch_sweep_xy<C, T>;
+  if constexpr (has_sweep_xy<C, T>()) {
+    o.sweep_xy = &launch_sweep_xy<C, T>;
+    o.sweep_xy_min_cells = sweep_xy_min_cells<C>();
+  }
   o.normal_field = &launch_normal_field<C>;
   o.correct_flux = &launch_correct_flux<C>;
   o.rhs = &launch_rhs<C>;

@@ -140,7 +140,8 @@ def test_hd_box_ghost_zones(n, bc):
 
 
 @pytest.mark.parametrize("mhd,recon,precision", [(True, "plm", "fp64"), (True, "plm", "fp32"),
-                                                 (True, "limo3", "fp64"), (False, "plm", "fp64"),
+                                                 (True, "ppm", "fp32"), (True, "limo3", "fp64"),
+                                                 (False, "plm", "fp64"),
                                                  (False, "ppm", "fp64")])
 @pytest.mark.parametrize("n", [(4, 3, 5), (3, 37, 4), (52, 4, 3), (54, 5, 3), (56, 4, 3), (58, 3, 3), (60, 5, 2),
                                (62, 3, 3), (114, 4, 3), (118, 5, 3), (57, 130, 3)])
@@ -154,6 +155,8 @@ def test_sweep_xy_equals_two_sweeps(n, mhd, recon, precision):
     ic = problems.random_mhd if mhd else problems.random_hd
     o, g = make_pair(kw, ic, precision=precision)
     _, h = make_pair(kw, ic, precision=precision)
+    if recon == "ppm" and mhd:
+        g.set_fusion(2)  # large grids only by default
     h.set_fusion(0)
     o.set_boundaries()
     for _ in range(2):
