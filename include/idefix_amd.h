@@ -241,6 +241,9 @@ int idfx_cycle(idfx_ctx *ctx, int nstages, double cfl, double cfl_max_var, long 
  * the next state array, and a pointwise kernel adds pressure and cell field.  Hydro (same
  * conditions) starts with the last sweep doing both in full; level 0 makes ConvertConsToPrim
  * its own kernel there too.
+ * On these two schedules one kernel does the x and y sweeps of 2-D and 3-D hydro and of 3-D MHD
+ * with three-cell reconstructions (MHD with PPM: FP32 stencils from 2^25 cells on, and with
+ * level 2), and the sweep of 1-D hydro fills the ghost zones itself.
  * In 3-D, level 1 takes the fused CT kernel on blocks of at least 5 * 2^19 interior cells
  * and k_corner_emf + k_evolve_b below (the faster choice on MI355X); level 2 takes the
  * fused CT kernel at every size.  All levels give identical interior cells, faces and Uc.
