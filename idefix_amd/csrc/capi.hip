@@ -878,7 +878,7 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
       xflags = flags;
       continue;
     }
-    Region r(c, IDFX_REGION_SWEEP_X + dir, s);
+    Region r(c, IDFX_REGION_SWEEP_X + (xy && dir == 1 ? 0 : dir), s);
     if (needs_unfused(c)) {
       // reference sequence: PrimToCons, (begin copy), CalcFlux, CalcRightHandSide
       if (dir == 0) {

@@ -254,7 +254,8 @@ int idfx_ctx_set_fusion(idfx_ctx *ctx, int level);
 /* Regions of idfx_cycle / idfx_stage timed by the region profiler. */
 enum {
   IDFX_REGION_BOUNDARIES = 0,   /* SetBoundaries (ghost fill, normal field, cell B) */
-  IDFX_REGION_SWEEP_X = 1,      /* CalcFlux + CalcRightHandSide along x (y: 2, z: 3) */
+  IDFX_REGION_SWEEP_X = 1,      /* CalcFlux + CalcRightHandSide along x (y: 2, z: 3; one kernel for
+                                   x and y counts here) */
   IDFX_REGION_SWEEP_Y = 2,
   IDFX_REGION_SWEEP_Z = 3,
   IDFX_REGION_CORNER_EMF = 4,   /* CalcCornerEMF */
