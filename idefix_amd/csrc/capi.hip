@@ -70,6 +70,11 @@ __global__ void k_fill(double *p, long long n, double v) {
 
 using namespace idfx;
 
+// 1-D hydro cells up to which the first stage's sweep hands over the time step itself; beyond, the
+// second one does, because counting the blocks delays it more (us a cycle, first and second:
+// 1000 cells 16.0, 17.2; 8000 16.1, 17.4; 30,000 18.4, 17.9; 1,000,000 198, 75).
+constexpr int DT_SWEEP_MAX = 1 << 14;
+
 // Interior cells from which the fused CT kernel replaces k_corner_emf + k_evolve_b at
 // fusion level 1 (3-D uct_contact, per stage, fused against the two kernels: 128^3 126
 // against 122 us, FP32 110 against 107; 203x150x97 147 against 174 us; 512^3 5.2 against 8.3
@@ -903,8 +908,10 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
         a.lbc = c->d.lbound[0];
         a.rbc = c->d.rbound[0];
         a.VcGhost = Vc;
-        a.dt_host = c->host;
-        a.dt_seq = dt_mode == DT_SWEEP ? ++c->dt_seq : 0;
+        if (dt_mode == DT_SWEEP || dt_mode == DT_TAKE) {
+          a.dt_host = c->host;
+          a.dt_seq = ++c->dt_seq;
+        }
       }
       a.wc = wc;
       a.w0 = w0;
@@ -1118,7 +1125,7 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
   int pp_first = 0;
   // 1-D sweeps of the ping-pong schedule carry boundaries and time step: all stages or none
   if (c->d.dim == 1 && nstages == 3 && !c->Vc3) pp3 = false;
-  const bool dt_sweep = pp3 && c->d.dim == 1;
+  const bool dt_sweep = pp3 && c->d.dim == 1 && c->d.nx[0] <= DT_SWEEP_MAX;
   if (nstages == 3) {
     pp_first = c->Vc3 ? 0 : 1;
     pout[0] = c->Vc3, bout[0] = c->Vs3;

@@ -78,7 +78,7 @@ struct SweepArgs {
   const unsigned char *shock;  // shock flags per cell (shock flattening) or nullptr
   double *VcOut;      // SW_FINAL: output primitive state
   double wc, w0;      // SW_RK weights
-  // 1-D hydro FIN sweep: side types, and the host's copy of dtmax (dtmax[1] counts blocks)
+  // 1-D hydro FIN sweep: side types, and where dtmax goes (dtmax[1] counts blocks) or nullptr
   int lbc, rbc;
   double *VcGhost;    // = Vc, for its ghost cells
   unsigned long long *dt_host, dt_seq;
@@ -573,6 +573,11 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
   const int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   unsigned long long red = 0;
   if constexpr (BOX) {
+    // the previous stage's maximum, where that stage has too many blocks to count
+    if (a.dt_host && !(a.flags & SW_DT_REDUCE) && blockIdx.x == 0 && threadIdx.x == 0) {
+      dt_to_host(a.dt_host, *a.dtmax, a.dt_seq);
+      *a.dtmax = 0ULL;
+    }
     const int ng = g.beg[0];
     if (blockIdx.x == 0 && (int)threadIdx.x < 2 * ng) {
       const int q = (int)threadIdx.x < ng ? (int)threadIdx.x : g.end[0] - ng + (int)threadIdx.x;
@@ -678,7 +683,7 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
   if constexpr (FUSED) {
     if (a.flags & SW_DT_REDUCE) {
       block_max_atomic(red, a.dtmax);
-      if (BOX && threadIdx.x == 0) publish_dt(a.dtmax, a.dt_host, a.dt_seq);
+      if (BOX && a.dt_host && threadIdx.x == 0) publish_dt(a.dtmax, a.dt_host, a.dt_seq);
     }
   }
 }
