@@ -567,7 +567,8 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
   // 1-D hydro on the ping-pong schedule is bound by its launches: every load of a ghost cell
   // takes the interior cell the side's rule leads to, block 0 stores the ghost zones, which
   // nothing in this kernel reads, and the last block hands over the time step.  (1000 cells:
-  // 25 us a cycle with two kernels, 31 with a boundary kernel before each.)
+  // 25 us a cycle with two kernels, 31 with a boundary kernel before each; 18 since the host
+  // waits for the value and not for an event.)
   constexpr bool BOX = FIN && C::DIM == 1;
   const int lane = threadIdx.x & 63;
   const int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -696,9 +697,10 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
 // cycles: Orszag-Tang 128^3 1453 -> 1263 us, turbulence 512^3 133.4 -> 123.6 ms).
 //
 // With the window in LDS, the next row loaded a step ahead and every other load of a step
-// before its reconstruction, the 512^3 PPM sweeps take 7.2 (y) and 8.4 ms (z) a launch at
-// 228-238 VGPRs; with the window in registers and its leading row loaded when needed they
-// took 7.8 and 9.5 ms (256 VGPRs and 44 B of spills).
+// before its reconstruction, the 512^3 PPM sweeps took 7.2 (y) and 8.4 ms (z) a launch at
+// 228-238 VGPRs (6.8 and 8.1 at 212-222 since HLLD works out one side of a face only); with
+// the window in registers and its leading row loaded when needed they took 7.8 and 9.5 ms (256
+// VGPRs and 44 B of spills).
 // ------------------------------------------------------------------------------------
 struct MarchGeom {
   int ilo, ihi;   // x range (interior +- extension)
