@@ -218,9 +218,9 @@ template <class C, typename T, int DIR, bool FUSED, int EMF>
 hipError_t launch_sweep_dir(const GridDesc &g, const SweepArgs &a, const EmfArrays<T> &e,
                             int target_waves, hipStream_t s) {
   if (a.flags & SW_FINAL) {
-    // the last sweep of the ping-pong schedule (hydro; 3-D adiabatic MHD with uct_contact;
-    // no per-cell options)
-    if constexpr (DIR == C::DIM - 1 && FUSED &&
+    // the last sweep of the ping-pong schedule (hydro, in 2-D k_sweep_xy; 3-D adiabatic MHD
+    // with uct_contact; no per-cell options)
+    if constexpr (DIR == C::DIM - 1 && FUSED && !(C::DIM == 2 && has_sweep_xy<C, T>()) &&
                   (!C::MHD || (C::DIM == 3 && !C::ISO && EMF == EMF_UCT_CONTACT))) {
       if (a.shock != nullptr || g.ntr > 0) return hipErrorInvalidValue;
       return launch_sweep_xtra<C, T, DIR, FUSED, EMF, false, true>(g, a, e, target_waves, s);
