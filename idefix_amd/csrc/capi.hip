@@ -1116,6 +1116,10 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
       c->Vc3 = v;
       c->Vs3 = b;
     } else {
+      if (v && !c->allocs.empty() && c->allocs.back() == v) {  // no room for the faces
+        hipFree(v);
+        c->allocs.pop_back();
+      }
       c->vc3_failed = true;
       (void)hipGetLastError();  // the failed allocation must not surface as a launch error
     }
