@@ -164,8 +164,11 @@ int alloc_n(idfx_ctx *c, T **p, long long n) {
   if (hipMalloc(&q, sizeof(T) * (size_t)std::max<long long>(n, 1)) != hipSuccess) return IDFX_E_ALLOC;
   c->allocs.push_back(q);
   *p = static_cast<T *>(q);
-  // scratch starts at zero, as Kokkos views do
-  if (hipMemset(q, 0, sizeof(T) * (size_t)std::max<long long>(n, 1)) != hipSuccess) return IDFX_E_ALLOC;
+  // scratch starts at zero, as Kokkos views do.  The clear runs on the null stream and returns
+  // before it has ended; a caller's non-blocking stream would not wait for it.
+  if (hipMemset(q, 0, sizeof(T) * (size_t)std::max<long long>(n, 1)) != hipSuccess ||
+      hipStreamSynchronize(nullptr) != hipSuccess)
+    return IDFX_E_ALLOC;
   return IDFX_OK;
 }
 
