@@ -1060,7 +1060,9 @@ int idfx_ctx_set_mlp_params(idfx_ctx *c, const float *p) {
   for (int q = 0; q < 64; q++) b[q] = p[B1 + q];
   for (int q = 0; q < 64; q++) b[64 + q] = p[B2 + q];
   for (int q = 0; q < 16; q++) b[128 + q] = p[B3 + q];
-  if (hipMemcpy(c->mlp_wt, wt.data(), wt.size() * 2, hipMemcpyHostToDevice) != hipSuccess ||
+  // stages of the last cycle may still run, on a stream that the copies do not wait for
+  if (hipDeviceSynchronize() != hipSuccess ||
+      hipMemcpy(c->mlp_wt, wt.data(), wt.size() * 2, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(c->mlp_b, b.data(), b.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
     return IDFX_E_LAUNCH;
   c->net.valid = 1;

@@ -90,3 +90,29 @@ def test_two_contexts_in_flight():
         for (a, da), (b, db) in zip(w, r):
             assert da == db
             _equal(a, b)
+
+
+def test_new_weights_behind_a_running_cycle():
+    """The learned limiter's weights replaced right after a cycle returned on a side stream, its
+    last stages still running: they take the old weights."""
+    import numpy as np
+    import torch
+    from idefix_amd import learned
+    from idefix_amd.datablock import DataBlock
+    p = learned.init_params(8)
+    q = p + np.random.default_rng(9).normal(0, 0.05, p.shape).astype(np.float32)
+    out = []
+    for late in (False, True):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            g = DataBlock(2, (512, 384), comps=3, mhd=True, recon="mlp", precision="fp32", cfl=0.3,
+                          nstages=3, first_dt=1e-5)
+            g.upload(*problems.random_mhd(g))
+            g.set_mlp_params(q)
+            g.cycle()
+            if not late:
+                torch.cuda.current_stream().synchronize()
+            g.set_mlp_params(p)
+            torch.cuda.current_stream().synchronize()
+            out.append(g)
+    torch.cuda.synchronize()
+    _equal(*out)
