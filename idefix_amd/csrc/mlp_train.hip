@@ -307,7 +307,10 @@ int mlp_alloc(idfx_mlp *h, float **p, long long n) {
   void *q = nullptr;
   if (hipMalloc(&q, sizeof(float) * (size_t)std::max(n, 1LL)) != hipSuccess) return IDFX_E_ALLOC;
   h->allocs.push_back(q);
-  if (hipMemset(q, 0, sizeof(float) * (size_t)std::max(n, 1LL)) != hipSuccess) return IDFX_E_ALLOC;
+  // the clear has ended before the memory is handed out: a non-blocking stream does not wait for it
+  if (hipMemset(q, 0, sizeof(float) * (size_t)std::max(n, 1LL)) != hipSuccess ||
+      hipStreamSynchronize(nullptr) != hipSuccess)
+    return IDFX_E_ALLOC;
   *p = static_cast<float *>(q);
   return IDFX_OK;
 }
@@ -368,9 +371,12 @@ int idfx_mlp_destroy(idfx_mlp *h) {
 
 int idfx_mlp_set_params(idfx_mlp *h, const float *host) {
   if (!h || !host) return IDFX_E_ARGS;
-  if (hipMemcpy(h->P, host, sizeof(float) * P_N, hipMemcpyHostToDevice) != hipSuccess ||
+  // steps may be under way on a stream that does not wait for the null stream, nor it for them;
+  // the moments are clear before the call returns
+  if (hipDeviceSynchronize() != hipSuccess ||
+      hipMemcpy(h->P, host, sizeof(float) * P_N, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(h->M, 0, sizeof(float) * P_N) != hipSuccess ||
-      hipMemset(h->V, 0, sizeof(float) * P_N) != hipSuccess)
+      hipMemset(h->V, 0, sizeof(float) * P_N) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
     return IDFX_E_LAUNCH;
   h->step = 0;
   return IDFX_OK;
@@ -378,6 +384,8 @@ int idfx_mlp_set_params(idfx_mlp *h, const float *host) {
 
 int idfx_mlp_get_params(idfx_mlp *h, float *host) {
   if (!h || !host) return IDFX_E_ARGS;
+  // the steps enqueued so far, on whichever stream
+  if (hipDeviceSynchronize() != hipSuccess) return IDFX_E_LAUNCH;
   return hipMemcpy(host, h->P, sizeof(float) * P_N, hipMemcpyDeviceToHost) == hipSuccess
              ? IDFX_OK : IDFX_E_LAUNCH;
 }

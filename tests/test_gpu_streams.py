@@ -116,3 +116,36 @@ def test_new_weights_behind_a_running_cycle():
             out.append(g)
     torch.cuda.synchronize()
     _equal(*out)
+
+
+def test_training_on_a_side_stream():
+    """A trainer created, stepped, read and given new parameters on a side stream without waits
+    of the caller's: every parameter as on the default stream."""
+    import contextlib
+
+    import numpy as np
+    import torch
+    from idefix_amd import learned
+    rng = np.random.default_rng(2)
+    B = 20000
+    X = rng.uniform(-1, 1, (B, 72)).astype(np.float32)
+    tau = rng.uniform(-0.5, 0.5, (B, 8)).astype(np.float32)
+    p = learned.pack({k: v + 0.05 * rng.standard_normal(np.shape(v))
+                      for k, v in learned.unpack(learned.init_params(3)).items()})
+    got = []
+    for side in (False, True):
+        with torch.cuda.stream(torch.cuda.Stream()) if side else contextlib.nullcontext():
+            x, t = torch.from_numpy(X).cuda(), torch.from_numpy(tau).cuda()
+            torch.cuda.synchronize()
+            tr = learned.Trainer(B, p)
+            for _ in range(20):
+                tr.step(x, t, 1e-3)
+            first = tr.params()
+            for _ in range(20):
+                tr.step(x, t, 1e-3)
+            tr.set_params(p)
+            for _ in range(5):
+                tr.step(x, t, 1e-3)
+            got.append((first, tr.params()))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    assert not np.array_equal(got[0][0], p)
