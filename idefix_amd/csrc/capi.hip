@@ -1076,7 +1076,7 @@ int idfx_mlp_faces(idfx_ctx *c, int dir, const double *Vc, float *W, void *strea
 
 int idfx_ctx_set_fusion(idfx_ctx *c, int level) {
   if (!c || level < 0 || level > 2) return IDFX_E_ARGS;
-  if (level >= 1 && !c->fused2d_ok && !c->fused3d_ok) return IDFX_E_ARGS;
+  if (level >= 1 && !c->fused2d_ok && !c->fused3d_ok && !c->pp_ok) return IDFX_E_ARGS;
   c->fused2d_on = level >= 1 && c->fused2d_ok;
   c->fused3d_on = level >= 1 && c->fused3d_ok;
   c->pp_hd_on = level >= 1 && c->pp_ok;
