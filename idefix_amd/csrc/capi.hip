@@ -601,12 +601,24 @@ static BoxSides box_sides(const idfx_ctx *c) {
   for (int d = 0; d < c->d.dim; d++) b.lbc[d] = c->d.lbound[d], b.rbc[d] = c->d.rbound[d];
   return b;
 }
+// A reflecting side of a direction shorter than its ghost zone: the outer ghost cells mirror
+// ghost cells of the other side, as they are when the sides are filled left, then right.
+static bool mirrors_ghosts(const idfx_ctx *c, int dir) {
+  return c->g.end[dir] - c->g.beg[dir] < c->g.beg[dir] &&
+         (c->d.lbound[dir] == IDFX_BC_REFLECTIVE || c->d.rbound[dir] == IDFX_BC_REFLECTIVE);
+}
 static int enforce_dir(idfx_ctx *c, int dir, double *Vc, double *Vs, DtTake tk, void *stream) {
   hipStream_t s = (hipStream_t)stream;
-  // built-in side types (user-defined sides are left alone by the kernel)
-  IDFX_TRY(check(c->ops->boundary(c->g, Vc, Vs, dir, c->d.lbound[dir], c->d.rbound[dir], tk, s)));
+  const int lbc = c->d.lbound[dir], rbc = c->d.rbound[dir];
+  // built-in side types (user-defined sides are left alone by the kernel), both sides in one
+  // launch unless one reads what the other writes
+  const bool apart = mirrors_ghosts(c, dir);
+  if (!apart) IDFX_TRY(check(c->ops->boundary(c->g, Vc, Vs, dir, lbc, rbc, tk, s)));
   for (int side = 0; side < 2; side++) {
-    const int bc = side == 0 ? c->d.lbound[dir] : c->d.rbound[dir];
+    if (apart)
+      IDFX_TRY(check(c->ops->boundary(c->g, Vc, Vs, dir, side == 0 ? lbc : (int)IDFX_BC_USERDEF,
+                                      side == 1 ? rbc : (int)IDFX_BC_USERDEF, side == 0 ? tk : DtTake{}, s)));
+    const int bc = side == 0 ? lbc : rbc;
     if (bc != IDFX_BC_USERDEF) continue;
     // boundary.hpp:316-332: no enrolled function is a configuration error
     if (!c->user_fn) return IDFX_E_ARGS;

@@ -38,3 +38,28 @@ def test_levels_without_a_schedule_are_refused(kw):
     for level in (1, 2):
         with pytest.raises(Exception):
             g.set_fusion(level)
+
+
+SHORT = [(2, (2, 9), False, "reflective"), (2, (2, 9), True, "reflective"),
+         (2, (9, 2), True, ["outflow", ("reflective", "outflow")]), (2, (1, 8), False, [("outflow", "reflective"), "periodic"]),
+         (3, (66, 3, 2), False, ["outflow", "periodic", "reflective"]), (3, (5, 2, 7), True, "reflective"),
+         (3, (66, 3, 2), True, ["outflow", "periodic", "reflective"])]
+
+
+@pytest.mark.parametrize("dim,n,mhd,bc", SHORT)
+def test_reflection_in_a_direction_shorter_than_its_ghost_zone(dim, n, mhd, bc):
+    """The left side mirrors ghost cells of the right one as the last fill left them, the right
+    side those of the left one, just filled: every bit of cells and faces, over three fills,
+    as the oracle fills side by side in one array."""
+    import numpy as np
+    kw = cfg_kwargs(dim, n, mhd=mhd, solver="hlld" if mhd else "hllc", recon="ppm", bc=bc, gamma=1.4)
+    o, g = make_pair(kw, problems.random_mhd if mhd else problems.random_hd)
+    for _ in range(3):
+        o.set_boundaries()
+        g.set_boundaries()
+        Vc, Vs = g.download()
+        assert np.array_equal(Vc, o.Vc)
+        assert not mhd or np.array_equal(Vs, o.Vs)
+        # other values inside, exact in both
+        o.interior(o.Vc)[...] *= 0.75
+        g.interior(g.Vc).mul_(0.75)
