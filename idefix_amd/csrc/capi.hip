@@ -607,6 +607,11 @@ static bool mirrors_ghosts(const idfx_ctx *c, int dir) {
   return c->g.end[dir] - c->g.beg[dir] < c->g.beg[dir] &&
          (c->d.lbound[dir] == IDFX_BC_REFLECTIVE || c->d.rbound[dir] == IDFX_BC_REFLECTIVE);
 }
+static bool mirrors_ghosts(const idfx_ctx *c) {
+  bool m = false;
+  for (int d = 0; d < c->d.dim; d++) m = m || mirrors_ghosts(c, d);
+  return m;
+}
 static int enforce_dir(idfx_ctx *c, int dir, double *Vc, double *Vs, DtTake tk, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   const int lbc = c->d.lbound[dir], rbc = c->d.rbound[dir];
@@ -1125,8 +1130,10 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
   // Vc2 -> Vc (the third array allocated at the first such cycle; without it the first RK3
   // stage runs in place on the per-kernel schedule and the others alternate Vc -> Vc2 -> Vc;
   // 2-D turbulence 256^2: 154 us a cycle without it, 140 with it)
-  const bool fused = c->fused2d_on && nstages >= 2 && Vs;
-  bool pp3 = c->pp_ok && nstages >= 2 && (c->d.mhd ? c->fused3d_on && Vs : c->pp_hd_on);
+  // A ghost fill that reads older ghost cells needs them in one array from stage to stage.
+  const bool alternate = nstages >= 2 && !mirrors_ghosts(c);
+  const bool fused = alternate && c->fused2d_on && Vs;
+  bool pp3 = alternate && c->pp_ok && (c->d.mhd ? c->fused3d_on && Vs : c->pp_hd_on);
   if ((pp3 || fused) && nstages == 3 && !c->Vc3 && !c->vc3_failed) {
     double *v = nullptr, *b = nullptr;
     if (alloc_n(c, &v, c->n3 * c->nvar) == IDFX_OK && (!fused || alloc_n(c, &b, c->nvs) == IDFX_OK)) {

@@ -3,7 +3,7 @@ the caller's arrays."""
 import pytest
 
 from idefix_amd import problems
-from tests.pairs import cfg_kwargs, make_pair
+from tests.pairs import cfg_kwargs, interior_faces, make_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +63,24 @@ def test_reflection_in_a_direction_shorter_than_its_ghost_zone(dim, n, mhd, bc):
         # other values inside, exact in both
         o.interior(o.Vc)[...] *= 0.75
         g.interior(g.Vc).mul_(0.75)
+
+
+@pytest.mark.parametrize("nstages", [2, 3])
+@pytest.mark.parametrize("dim,n,mhd,bc", SHORT)
+def test_short_directions_at_every_level(dim, n, mhd, bc, nstages):
+    """Stages that need the last fill's ghost cells keep to one array: every bit, over three
+    cycles, as with a kernel per step."""
+    import torch
+    kw = cfg_kwargs(dim, n, mhd=mhd, solver="hlld" if mhd else "hllc", recon="ppm", bc=bc, gamma=1.4,
+                    cfl=0.3, nstages=nstages)
+    _, g = make_pair(kw, problems.random_mhd if mhd else problems.random_hd)
+    _, h = make_pair(kw, problems.random_mhd if mhd else problems.random_hd)
+    h.set_fusion(0)
+    for _ in range(3):
+        g.cycle()
+        h.cycle()
+        assert g.dt == h.dt
+    assert torch.equal(g.interior(g.Vc), h.interior(h.Vc))
+    if mhd:
+        for a, b in zip(interior_faces(g, g.download()[1]), interior_faces(h, h.download()[1])):
+            assert (a == b).all()
