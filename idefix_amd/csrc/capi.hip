@@ -826,8 +826,12 @@ static int dt_begin(idfx_ctx *c, int dt, hipStream_t s) {
   c->dt_clean = false;
   return IDFX_OK;
 }
+// The boundary step's first kernel takes the maximum and clears it; a user boundary called after
+// that kernel may use dtmax again (idfx_compute_timestep) and leave it so.
 static DtTake dt_take(idfx_ctx *c, int dt) {
-  return dt == DT_TAKE ? DtTake{c->dtmax, c->host, ++c->dt_seq} : DtTake{};
+  if (dt != DT_TAKE) return DtTake{};
+  c->dt_clean = true;
+  return DtTake{c->dtmax, c->host, ++c->dt_seq};
 }
 // The host reads the cycle's maximum as soon as the kernel has stored it.  (An event behind that
 // kernel costs a barrier on the stream and its signal's way to the host: 1000 hydro cells 25
@@ -874,7 +878,6 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
     Region r(c, IDFX_REGION_BOUNDARIES, s);
     IDFX_TRY(stage_boundaries(c, Vc, Vs, consistent, dt_take(c, dt_mode), s));
   }
-  if (dt_mode == DT_TAKE) c->dt_clean = true;
   const bool want_dt = dt_mode == DT_REDUCE || dt_mode == DT_SWEEP || dt_mode == DT_ALL;
   double wc = 0.0, w0 = 0.0;
   if (stage > 0) {
@@ -931,6 +934,7 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
         if (dt_mode == DT_SWEEP || dt_mode == DT_TAKE) {
           a.dt_host = c->host;
           a.dt_seq = ++c->dt_seq;
+          c->dt_clean = true;  // once the sweep has run
         }
       }
       a.wc = wc;
@@ -959,7 +963,6 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
   } else if (c->d.mhd && stage > 0) {
     // 1-D MHD keeps Vs constant; AddAndStore still applies (a no-op on equal values)
   }
-  if (dt_mode == DT_SWEEP) c->dt_clean = true;
   IDFX_TRY(dt_copy(c, dt_mode, s));
   const int lo[3] = {c->g.beg[0], c->g.beg[1], c->g.beg[2]};
   const int hi[3] = {c->g.end[0], c->g.end[1], c->g.end[2]};
@@ -986,7 +989,6 @@ static int stage_fused2d(idfx_ctx *c, int stage, int nstages, double dt, double 
     Region r(c, IDFX_REGION_BOUNDARIES, s);
     IDFX_TRY(stage_boundaries(c, Vc_in, Vs_in, consistent, dt_take(c, dt_mode), s));
   }
-  if (dt_mode == DT_TAKE) c->dt_clean = true;
   IDFX_TRY(dt_begin(c, dt_mode, s));
   const bool want_dt = dt_mode == DT_REDUCE || dt_mode == DT_ALL;
   int flags = SW_INIT_UC;
@@ -1165,23 +1167,28 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
   // stage times of the boundary calls (TimeIntegrator::Cycle advances t by dt after each
   // stage, then t = wc t + w0 t0): t0, t0 + dt, and t0 + dt/2 for the third RK3 stage
   const double tstage[3] = {t0, t0 + *dt, 0.25 * (t0 + *dt + *dt) + 0.75 * t0};
-  for (int stage = 0; stage < nstages; stage++) {
+  int st = IDFX_OK;
+  for (int stage = 0; stage < nstages && st == IDFX_OK; stage++) {
     c->t_bound = tstage[stage];
     const int dt_mode = nstages == 1 ? DT_ALL
                         : dt_sweep   ? (stage == 0 ? DT_SWEEP : DT_NONE)
                                      : (stage == 0 ? DT_REDUCE : stage == 1 ? DT_TAKE : DT_NONE);
     const bool last = stage == nstages - 1;
     if (stage < pp_first || !(pp3 || fused))
-      IDFX_TRY(stage_enqueue(c, stage, nstages, *dt, Vc, Vs, Uc, InvDt, 0, last, dt_mode, s, stage > 0));
+      st = stage_enqueue(c, stage, nstages, *dt, Vc, Vs, Uc, InvDt, 0, last, dt_mode, s, stage > 0);
     else if (pp3)
-      IDFX_TRY(stage_enqueue(c, stage, nstages, *dt, pin[stage], Vs, Uc, InvDt, 0, last, dt_mode, s,
-                             stage > 0, pout[stage]));
+      st = stage_enqueue(c, stage, nstages, *dt, pin[stage], Vs, Uc, InvDt, 0, last, dt_mode, s, stage > 0,
+                         pout[stage]);
     else
-      IDFX_TRY(stage_fused2d(c, stage, nstages, *dt, pin[stage], bin[stage], pout[stage], bout[stage],
-                             Uc, InvDt, last, dt_mode, s, stage > 0));
+      st = stage_fused2d(c, stage, nstages, *dt, pin[stage], bin[stage], pout[stage], bout[stage], Uc, InvDt,
+                         last, dt_mode, s, stage > 0);
   }
   // stage 0's InvDt maximum reaches the host while the later stages still run
-  IDFX_TRY(nstages == 1 ? check(hipEventSynchronize(c->ev_dt)) : dt_wait(c, s));
+  if (st == IDFX_OK) st = nstages == 1 ? check(hipEventSynchronize(c->ev_dt)) : dt_wait(c, s);
+  if (st != IDFX_OK) {
+    c->dt_clean = false;  // the kernel that takes the maximum may not have run
+    return st;
+  }
   const double newdt = cfl * (1.0 / bits_to_double(*c->host));
   *t = t0 + *dt;
   int status = IDFX_OK;
