@@ -96,7 +96,7 @@ struct idfx_ctx {
   double *Uc0 = nullptr, *Vs0 = nullptr;  // Runge-Kutta "begin" state
   unsigned long long *dtmax = nullptr, *divb = nullptr;  // device scalars
   unsigned char *shock = nullptr;  // shock flags (shock flattening on)
-  unsigned long long *host = nullptr;  // pinned readback: value, number of the cycle
+  unsigned long long *host = nullptr;  // pinned readback: a cycle's value, its number; read_u64's
   unsigned long long dt_seq = 0;       // cycles that handed their maximum over
   bool dt_clean = true;  // dtmax is zero (once the work enqueued so far has run)
   hipEvent_t ev_dt = nullptr;
@@ -290,9 +290,10 @@ int do_sweep_unfused(idfx_ctx *c, int dir, double dt, const double *Vc, const do
 }
 
 int read_u64(idfx_ctx *c, unsigned long long *dev, unsigned long long *out, hipStream_t s) {
-  IDFX_TRY(check(hipMemcpyAsync(c->host, dev, sizeof(unsigned long long), hipMemcpyDeviceToHost, s)));
+  // not where a cycle under way, whose user boundary may call this, keeps its maximum
+  IDFX_TRY(check(hipMemcpyAsync(c->host + 2, dev, sizeof(unsigned long long), hipMemcpyDeviceToHost, s)));
   IDFX_TRY(check(hipStreamSynchronize(s)));
-  *out = *c->host;
+  *out = c->host[2];
   return IDFX_OK;
 }
 
@@ -515,7 +516,7 @@ int idfx_ctx_create(const idfx_desc *desc, const double *dx1, const double *dx2,
     void *h = nullptr;
     if (hipHostMalloc(&h, 64, hipHostMallocDefault) != hipSuccess) st = IDFX_E_ALLOC;
     c->host = static_cast<unsigned long long *>(h);
-    if (c->host) c->host[0] = c->host[1] = 0;
+    if (c->host) c->host[0] = c->host[1] = c->host[2] = 0;
   }
   if (st == IDFX_OK && hipEventCreateWithFlags(&c->ev_dt, hipEventDisableTiming) != hipSuccess)
     st = IDFX_E_LAUNCH;

@@ -40,3 +40,14 @@ def test_time_step_of_a_boundary_that_computes_it(dim, n, mhd, nstages):
         for g in (a, b):
             g.Vc[1:prs + 1] *= 0.25  # velocities and pressure
     assert torch.equal(a.interior(a.Vc), b.interior(b.Vc))
+
+
+@pytest.mark.parametrize("nstages", [2, 3])
+def test_time_step_of_a_boundary_that_checks_divb(nstages):
+    """Nor does CheckDivB, whose result comes back through the same pinned block, change them."""
+    a = _block(2, (20, 12), True, nstages, [])
+    b = _block(2, (20, 12), True, nstages, ["check_divb", "compute_timestep", "check_divb"])
+    for _ in range(3):
+        a.cycle()
+        b.cycle()
+        assert a.dt == b.dt
