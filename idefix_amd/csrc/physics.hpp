@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
 
 namespace idfx {
 
@@ -184,6 +185,13 @@ __device__ __forceinline__ T ppm_div(T a, T b) {
   if constexpr (FAST) return a * __builtin_amdgcn_rcpf(b);
   else return div_(a, b);
 }
+// a / b for 0 <= a <= b, where b may be subnormal: FP64 scales both by 2^128, since quot() needs
+// a denominator whose reciprocal is in range (without, NaN, and the cell stays unlimited).
+template <typename T, bool FAST>
+__device__ __forceinline__ T ppm_ratio(T a, T b) {
+  if constexpr (std::is_same<T, double>::value) return div_(a * 0x1p128, b * 0x1p128);
+  else return ppm_div<T, FAST>(a, b);
+}
 template <typename T, bool FAST = false>
 __device__ __forceinline__ T ppm_face(T vm1, T v0, T vp1, T vp2) {
   const T sum = v0 + vp1;
@@ -217,7 +225,7 @@ __device__ __forceinline__ PpmStates<T> ppm_cell(T vm2, T vm1, T v0, T vp1, T vp
     const T qmax = fmx(fmx(fab(vm1), fab(v0)), fab(vp1));
     // q and qf carry the same sign: the quotient of their magnitudes
     T rho = 0;
-    if (fab(qf) > T(1e-12) * qmax) rho = ppm_div<T, FAST>(q, fab(qf));
+    if (fab(qf) > T(1e-12) * qmax) rho = ppm_ratio<T, FAST>(q, fab(qf));
     if (rho <= (T(1.0) - T(1e-12))) {
       l = v0 - rho * dl;
       r = v0 + rho * dr;
