@@ -69,10 +69,14 @@ __device__ __forceinline__ float sqrt_(float a) { return sqrtf(a); }
 // own expansion (two div_scale, a div_fmas that waits for VCC, two ldexp) and with the
 // reciprocal of a denominator refined once for all its quotients: v_rcp, two Newton steps,
 // then per quotient a product, its exact remainder and one correction (Markstein 1990).
-// div_fixup gives zero, infinite and NaN operands their IEEE results.  Equal to a / b bit
-// for bit while the denominator and the quotient are normal and the numerator is zero or
-// at least 2^-969 (its remainder is then exact; below, the last bit of a quotient may
-// differ), to sqrt(x) for x = 0 or x >= 2^-767.  An HLLD face has 20 quotients with 12
+// div_fixup gives zero, infinite and NaN operands their IEEE results.  In FP64 equal to a / b bit
+// for bit while the denominator is normal and below 2^1022, the quotient is normal and the
+// numerator is zero or at least 2^-969 (its remainder is then exact; below, the last bit of a
+// quotient may differ).  In FP32 the same with 2^126 and 2^-102.  A subnormal denominator or a
+// quotient that overflows gives NaN: densities and their roots are normal numbers, sums and
+// differences with a wave speed in them are zero or at least a unit in its last place, and
+// PPM's curvatures are scaled (ppm_ratio).  Square roots are IEEE's throughout: outside
+// [2^-767, inf) a branch takes the compiler's.  An HLLD face has 20 quotients with 12
 // denominators and 6 square roots; whole cycles: Orszag-Tang 512^2 147 -> 139 us, 128^3 1209
 // -> 1164 us, turbulence 203x150x97 3009 -> 2950 us.
 template <typename T>
@@ -112,7 +116,11 @@ __device__ __forceinline__ double sqrt_(double x) {
   g = __builtin_fma(g, e, g);
   g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
   g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-  return (x == 0.0 || x == __builtin_inf()) ? x : g;
+  // zero, infinite, negative, NaN, and below 2^-767, where a remainder may be subnormal (the
+  // branch costs no more than selecting zero and infinity: Orszag-Tang 512^2 and 128^3 the same)
+  const unsigned hi = (unsigned)((unsigned long long)__double_as_longlong(x) >> 32);
+  if (__builtin_expect(hi - 0x10000000u >= 0x6ff00000u, 0)) g = sqrt(x);
+  return g;
 }
 
 // ------------------------------------------------------------------------------------
