@@ -307,10 +307,7 @@ int mlp_alloc(idfx_mlp *h, float **p, long long n) {
   void *q = nullptr;
   if (hipMalloc(&q, sizeof(float) * (size_t)std::max(n, 1LL)) != hipSuccess) return IDFX_E_ALLOC;
   h->allocs.push_back(q);
-  // the clear has ended before the memory is handed out: a non-blocking stream does not wait for it
-  if (hipMemset(q, 0, sizeof(float) * (size_t)std::max(n, 1LL)) != hipSuccess ||
-      hipStreamSynchronize(nullptr) != hipSuccess)
-    return IDFX_E_ALLOC;
+  if (hipMemset(q, 0, sizeof(float) * (size_t)std::max(n, 1LL)) != hipSuccess) return IDFX_E_ALLOC;
   *p = static_cast<float *>(q);
   return IDFX_OK;
 }
@@ -353,6 +350,9 @@ int idfx_mlp_create(int max_batch, idfx_mlp **out) {
     h->loss = reinterpret_cast<double *>(l);
     h->lossp = h->loss ? h->loss + 1 : nullptr;
   }
+  // the clears have ended before the memory is handed out: a non-blocking stream does not wait
+  // for them
+  if (st == IDFX_OK && hipStreamSynchronize(nullptr) != hipSuccess) st = IDFX_E_ALLOC;
   if (st != IDFX_OK) {
     idfx_mlp_destroy(h);
     return st;
