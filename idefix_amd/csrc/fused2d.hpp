@@ -49,6 +49,7 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
   constexpr int NV = C::NVAR;
   constexpr int NW = window<C>();
   constexpr int H = NW / 2;
+  static_assert(NW >= 3, "the ring of window rows holds NW - 1 of them");
   constexpr int BX2 = C::BX2;
   const int lane = threadIdx.x & 63;
   const int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -91,10 +92,10 @@ void k_fused2d_y(GridDesc g, SweepArgs a, EmfArrays<T> e, Fused2dArgs s, MarchGe
     constexpr int S_S1 = S_E1 + 1;              //         svx of row f-1
     constexpr int NSLOT = HLLE ? S_AD + 4 : S_S1 + 1;
     // at least 56 KB in FP64, which keeps small solvers from a third wave per SIMD as well: its
-  // rows push the others' out of the caches on grids larger than those (TVDLF 2048^2 849 us
-  // a cycle with it, 767 without; 512^2 79, 74; FP32 is indifferent)
-  constexpr int NLDS = std::is_same<T, double>::value ? std::max(NSLOT, 28) : NSLOT;
-  __shared__ T lds[NLDS][256];
+    // rows push the others' out of the caches on grids larger than those (TVDLF 2048^2 849 us
+    // a cycle with it, 767 without; 512^2 79, 74; FP32 is indifferent)
+    constexpr int NLDS = std::is_same<T, double>::value ? std::max(NSLOT, 28) : NSLOT;
+    __shared__ T lds[NLDS][256];
     const int tid = threadIdx.x;
     auto sl = [](int n) { return n > BX2 ? n - 1 : n; };
     auto wslot = [&](int row, int n) -> T & { return lds[(row & (RW - 1)) * NS + sl(n)][tid]; };
