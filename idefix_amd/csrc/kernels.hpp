@@ -713,10 +713,11 @@ struct MarchGeom {
 };
 
 // 3 waves per SIMD fit the 2-D march of the 6-variable MHD state without spills; the 3-D
-// one and the 8-variable 2-D one would spill, so they stay at 2
+// one, the 8-variable 2-D one and Roe's would spill, so they stay at 2 (Roe 2048^2 with a kernel
+// per step, a cycle: 1162 us, at 3 waves 1375)
 template <class C>
 constexpr int march_waves_per_eu() {
-  return (window<C>() == 3 && C::DIM == 2 && C::NVAR < 8) ? 3 : 2;
+  return (window<C>() == 3 && C::DIM == 2 && C::NVAR < 8 && !(C::MHD && C::SOLVER == SOLVER_ROE)) ? 3 : 2;
 }
 template <class C, typename T, int DIR, bool FUSED, int EMF, bool XTRA, bool FIN = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(march_waves_per_eu<C>())))
