@@ -99,7 +99,6 @@ struct idfx_ctx {
   unsigned long long *host = nullptr;  // pinned readback: a cycle's value, its number; read_u64's
   unsigned long long dt_seq = 0;       // cycles that handed their maximum over
   bool dt_clean = true;  // dtmax is zero (once the work enqueued so far has run)
-  hipEvent_t ev_dt = nullptr;
   int target_waves = 8192;
   bool fp32 = false;
   bool uniform = false;  // every direction has one cell width
@@ -519,8 +518,6 @@ int idfx_ctx_create(const idfx_desc *desc, const double *dx1, const double *dx2,
     c->host = static_cast<unsigned long long *>(h);
     if (c->host) c->host[0] = c->host[1] = c->host[2] = 0;
   }
-  if (st == IDFX_OK && hipEventCreateWithFlags(&c->ev_dt, hipEventDisableTiming) != hipSuccess)
-    st = IDFX_E_LAUNCH;
   if (st == IDFX_OK) {
     int dev = 0, ncu = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
@@ -543,7 +540,6 @@ int idfx_ctx_destroy(idfx_ctx *c) {
   hipDeviceSynchronize();
   for (void *p : c->allocs) hipFree(p);
   if (c->host) hipHostFree(c->host);
-  if (c->ev_dt) hipEventDestroy(c->ev_dt);
   for (hipEvent_t e : c->ev_start) hipEventDestroy(e);
   for (hipEvent_t e : c->ev_stop) hipEventDestroy(e);
   delete c;
@@ -858,11 +854,13 @@ static int dt_wait(idfx_ctx *c, hipStream_t s) {
   }
   return IDFX_OK;
 }
-static int dt_copy(idfx_ctx *c, int dt, hipStream_t s) {
-  if (dt != DT_ALL) return IDFX_OK;
-  IDFX_TRY(check(hipMemcpyAsync(c->host, c->dtmax, sizeof(unsigned long long),
-                                hipMemcpyDeviceToHost, s)));
-  return check(hipEventRecord(c->ev_dt, s));
+// A single stage's maximum to the host, behind the sweeps (512x400 hydro, one stage a cycle:
+// RK1_FIG us with a copy, an event and a clearing kernel).
+static int dt_hand_over(idfx_ctx *c, hipStream_t s) {
+  hipLaunchKernelGGL(k_take_dt, dim3(1), dim3(64), 0, s, DtTake{c->dtmax, c->host, ++c->dt_seq});
+  IDFX_TRY(check(hipGetLastError()));
+  c->dt_clean = true;
+  return IDFX_OK;
 }
 
 // VcOut (ping-pong schedule, pp_ok): the last sweep writes the stage's new state into VcOut,
@@ -966,7 +964,7 @@ static int stage_enqueue(idfx_ctx *c, int stage, int nstages, double dt, double 
   } else if (c->d.mhd && stage > 0) {
     // 1-D MHD keeps Vs constant; AddAndStore still applies (a no-op on equal values)
   }
-  IDFX_TRY(dt_copy(c, dt_mode, s));
+  if (dt_mode == DT_ALL) IDFX_TRY(dt_hand_over(c, s));
   const int lo[3] = {c->g.beg[0], c->g.beg[1], c->g.beg[2]};
   const int hi[3] = {c->g.end[0], c->g.end[1], c->g.end[2]};
   const int flags = (stage > 0 ? 1 : 0) | (write_uc ? 2 : 0);
@@ -993,7 +991,7 @@ static int stage_fused2d(idfx_ctx *c, int stage, int nstages, double dt, double 
     IDFX_TRY(stage_boundaries(c, Vc_in, Vs_in, consistent, dt_take(c, dt_mode), s));
   }
   IDFX_TRY(dt_begin(c, dt_mode, s));
-  const bool want_dt = dt_mode == DT_REDUCE || dt_mode == DT_ALL;
+  const bool want_dt = dt_mode == DT_REDUCE;
   int flags = SW_INIT_UC;
   if (stage == 0 && nstages > 1) flags |= SW_SAVE_UC0;
   if (stage == 0) flags |= SW_INVDT_SET;
@@ -1024,7 +1022,6 @@ static int stage_fused2d(idfx_ctx *c, int stage, int nstages, double dt, double 
     Region r(c, IDFX_REGION_FUSED2D_Y, s);
     IDFX_TRY(check(c->ops->fused2d_y(c->g, ay, c->emf(), f, c->target_waves, s)));
   }
-  IDFX_TRY(dt_copy(c, dt_mode, s));
   return IDFX_OK;
 }
 
@@ -1119,7 +1116,7 @@ int idfx_stage(idfx_ctx *c, int stage, int nstages, double dt, double cfl, doubl
   IDFX_TRY(stage_enqueue(c, stage, nstages, dt, Vc, Vs, Uc, InvDt, skip_boundaries, write_uc,
                          want_dt ? DT_ALL : DT_NONE, s));
   if (want_dt) {
-    IDFX_TRY(check(hipEventSynchronize(c->ev_dt)));
+    IDFX_TRY(dt_wait(c, s));
     *newdt_host = cfl * (1.0 / bits_to_double(*c->host));
   }
   return IDFX_OK;
@@ -1188,7 +1185,7 @@ int idfx_cycle(idfx_ctx *c, int nstages, double cfl, double cfl_max_var, long nc
                          last, dt_mode, s, stage > 0);
   }
   // stage 0's InvDt maximum reaches the host while the later stages still run
-  if (st == IDFX_OK) st = nstages == 1 ? check(hipEventSynchronize(c->ev_dt)) : dt_wait(c, s);
+  if (st == IDFX_OK) st = dt_wait(c, s);
   if (st != IDFX_OK) {
     c->dt_clean = false;  // the kernel that takes the maximum may not have run
     return st;

@@ -1868,6 +1868,8 @@ __device__ __forceinline__ void take_dt(const DtTake &tk) {
     *tk.dtmax = 0ULL;
   }
 }
+// ... and by itself, where no such kernel follows
+static __global__ void k_take_dt(DtTake tk) { take_dt(tk); }
 
 // Ghost zones of a box periodic in every active direction, all directions at once: every
 // ghost cell of Vc and ghost face of each Vs component takes the value at the periodic
