@@ -49,7 +49,6 @@ enum : int {
   SW_INVDT_SET = 4,    // InvDt = term                (first direction after ResetStage)
   SW_INVDT_ADD = 8,    // InvDt += term
   SW_DT_REDUCE = 16,   // fold max(InvDt) of the updated cells into *dtmax
-  SW_NO_INVDT_STORE = 32,  // keep InvDt in registers only (requires SW_INVDT_SET)
   // last sweep of a stage on the ping-pong schedule (the FIN kernels; hydro, 3-D MHD): the
   // updated cell state goes through AddAndStore and ConsToPrim (with MHD its
   // field-independent part) into VcOut instead of back into Uc
@@ -508,7 +507,7 @@ __device__ __forceinline__ double cell_update(const GridDesc &g, const SweepArgs
     const double dl = g.dx[DIR][ig];
     inv = 0.5 * ((double)cmaxp + (double)cmaxm) / (dl);
     if (a.flags & SW_INVDT_SET) {
-      if (!(a.flags & SW_NO_INVDT_STORE)) st32(a.InvDt, p, inv);
+      st32(a.InvDt, p, inv);
     } else {
       inv = (invpre ? *invpre : ld32((const double *)a.InvDt, p)) + inv;
       st32(a.InvDt, p, inv);
@@ -690,7 +689,7 @@ void k_sweep_x(GridDesc g, SweepArgs a, EmfArrays<T> e, XGeom m) {
 }
 
 // ------------------------------------------------------------------------------------
-// y / z sweeps: marching along DIR with the stencil window in registers.  The columns of
+// y / z sweeps: marching along DIR with the stencil window in LDS.  The columns of
 // the transverse plane are numbered with x fastest and dealt to the lanes 64 at a time
 // across row ends: blocks of 64 along x would leave a row of 130 columns (128 cells and
 // their extension) with 48 % idle lanes in its three waves, one of 514 with 11 % (whole
@@ -1449,6 +1448,24 @@ __global__ __launch_bounds__(256) void k_evolve_b(GridDesc g, double *Vs, double
   }
 }
 
+// One face-field update of k_evolve_b's arithmetic (mode 0: Vs += rhs; 1: Vs0 = Vs, then
+// Vs += rhs; 2: Vs = wc (Vs + rhs) + w0 Vs0).
+__device__ __forceinline__ void evolve_face(double *Vs, double *Vs0, unsigned q, double rhs,
+                                            int mode, double wc, double w0) {
+  const double old = ld32(Vs, q);
+  const double upd = old + rhs;
+  if (mode == 1) st32(Vs0, q, old);
+  st32(Vs, q, (mode == 2) ? wc * upd + w0 * ld32(Vs0, q) : upd);
+}
+// The same with the face's old value (and, in mode 2, its RK begin value) loaded earlier.
+__device__ __forceinline__ void evolve_face_pre(double *Vs, double *Vs0, unsigned q, double old,
+                                                double old0, double rhs, int mode, double wc,
+                                                double w0) {
+  const double upd = old + rhs;
+  if (mode == 1) st32(Vs0, q, old);
+  st32(Vs, q, (mode == 2) ? wc * upd + w0 * old0 : upd);
+}
+
 // CalcCornerEMF (uct_contact) and EvolveMagField of a 3-D block in one kernel, for the
 // stage path (the reference-granularity entry points keep k_corner_emf + k_evolve_b).
 // A block of 12 waves covers 64 columns (i) x 12 rows (j), owns the 62 x 10 faces inside, and
@@ -1470,38 +1487,8 @@ __global__ __launch_bounds__(256) void k_evolve_b(GridDesc g, double *Vs, double
 // a time share their edge columns' cache lines and halo rows in its L2.  5.2 ms at 512^3 and
 // 147 us at 203x150x97; with every lane loading all four cells and the face data around its
 // edge, and tiles following each other along y, 7.6 ms and 208 us.
-// Cell EMFs of one cell from 32-bit offsets (the arithmetic of cell_emf).
-template <class C, typename T>
-__device__ __forceinline__ void cell_emf32(const double *Vc, long long sv, unsigned p, T &E1,
-                                           T &E2, T &E3) {
-  const T vx1 = (T)ld32(Vc + C::MX1 * sv, p), vx2 = (T)ld32(Vc + C::MX2 * sv, p);
-  const T vx3 = (T)ld32(Vc + C::MX3 * sv, p);
-  const T bx1 = (T)ld32(Vc + C::BX1 * sv, p), bx2 = (T)ld32(Vc + C::BX2 * sv, p);
-  const T bx3 = (T)ld32(Vc + C::BX3 * sv, p);
-  E1 = (vx3 * bx2 - vx2 * bx3);
-  E2 = (vx1 * bx3 - vx3 * bx1);
-  E3 = (vx2 * bx1 - vx1 * bx2);
-}
-
-// One face-field update of k_evolve_b's arithmetic (mode 0: Vs += rhs; 1: Vs0 = Vs, then
-// Vs += rhs; 2: Vs = wc (Vs + rhs) + w0 Vs0).
-__device__ __forceinline__ void evolve_face(double *Vs, double *Vs0, unsigned q, double rhs,
-                                            int mode, double wc, double w0) {
-  const double old = ld32(Vs, q);
-  const double upd = old + rhs;
-  if (mode == 1) st32(Vs0, q, old);
-  st32(Vs, q, (mode == 2) ? wc * upd + w0 * ld32(Vs0, q) : upd);
-}
-// The same with the face's old value (and, in mode 2, its RK begin value) loaded earlier.
-__device__ __forceinline__ void evolve_face_pre(double *Vs, double *Vs0, unsigned q, double old,
-                                                double old0, double rhs, int mode, double wc,
-                                                double w0) {
-  const double upd = old + rhs;
-  if (mode == 1) st32(Vs0, q, old);
-  st32(Vs, q, (mode == 2) ? wc * upd + w0 * old0 : upd);
-}
-
-// tile of k_ct3d: faces per block in i and j (512^3 FP64, 8 waves of 62 x 6: 5.5 ms, 12
+//
+// Tile of k_ct3d: faces per block in i and j (512^3 FP64, 8 waves of 62 x 6: 5.5 ms, 12
 // waves: 5.2 ms, 16 waves, which must fit 128 VGPRs: 5.9 ms)
 constexpr int CT_TI = 62, CT_TJ = 10;
 template <class C, typename T>

@@ -159,9 +159,6 @@ __device__ __forceinline__ T limo3_lim(T dvp, T dvm, T dx) {
   psi = (T(1) - (eta - T(1)) / eps) * q + (T(1) + (eta - T(1)) / eps) * psi;
   return T(0.5) * psi;
 }
-template <typename T>
-__device__ __forceinline__ int sgn(T v) { return (T(0) < v) - (v < T(0)); }
-
 // a - 2 b: the product is exact, so the fused form rounds the same difference.
 __device__ __forceinline__ double sub2(double a, double b) { return __builtin_fma(-2.0, b, a); }
 __device__ __forceinline__ float sub2(float a, float b) { return __builtin_fmaf(-2.0f, b, a); }
@@ -245,16 +242,6 @@ __device__ __forceinline__ PpmStates<T> ppm_cell(T vm2, T vm1, T v0, T vp1, T vp
     if (fab(dl) >= 2 * fab(d2)) l = v0 + 2 * d2;
   }
   return {l, r};
-}
-// Both states of a cell from its own window.
-template <typename T, bool FAST = false>
-__device__ __forceinline__ void ppm_states(T vm2, T vm1, T v0, T vp1, T vp2, T &vl_out,
-                                           T &vr_out) {
-  const PpmStates<T> s = ppm_cell<T, FAST>(vm2, vm1, v0, vp1, vp2,
-                                           ppm_face<T, FAST>(vm2, vm1, v0, vp1),
-                                           ppm_face<T, FAST>(vm1, v0, vp1, vp2));
-  vl_out = s.l;
-  vr_out = s.r;
 }
 
 // ------------------------------------------------------------------------------------
