@@ -75,11 +75,15 @@ using namespace idfx;
 // 1000 cells 16.0, 17.2; 8000 16.1, 17.4; 30,000 18.4, 17.9; 1,000,000 198, 75).
 constexpr int DT_SWEEP_MAX = 1 << 14;
 
-// Interior cells from which the fused CT kernel replaces k_corner_emf + k_evolve_b at
-// fusion level 1 (3-D uct_contact, per stage, fused against the two kernels: 128^3 126
-// against 122 us, FP32 110 against 107; 203x150x97 147 against 174 us; 512^3 5.2 against 8.3
-// ms).  Below, the chip's CUs are not filled by the fused kernel's blocks.
+// Interior cells and fill (ct3d_plan) from which the fused CT kernel replaces k_corner_emf +
+// k_evolve_b at fusion level 1 (3-D uct_contact).  Below the fill, rows that end early in their
+// tiles or rounds of blocks that end early leave its lanes idle.  Per stage, fused against the two
+// kernels, FP64 and FP32 (us): 8x600x600 (fill 0.13) 613, 215 and 524, 205; 64x1024x1024 (0.50) 4014,
+// 3350 and 3458, 2790; 128x128x160 (0.58) 154, 144 and 139, 119; 256x128x90 (0.63) 156, 165 and 137,
+// 140; 250^3 (0.66) 730, 817 and 637, 667; 203x150x97 (0.70) 148, 169 and 128, 144; 384^3 (0.81) 2299,
+// 3079 and 1990, 2450.  Fewer cells do not fill the chip: 128^3 (2^21) 126, 122 and 110, 107.
 constexpr long long CT3D_MIN_CELLS = 5LL << 19;
+constexpr double CT3D_MIN_FILL = 0.62;
 
 struct idfx_ctx {
   idfx_desc d;
@@ -124,7 +128,7 @@ struct idfx_ctx {
   bool fused3d_ok = false;   // 3-D MHD with uct_contact: fused CT kernel (k_ct3d)
   bool fused3d_on = false;
   // the fused CT kernel (k_ct3d) rather than k_corner_emf + k_evolve_b: fusion level 2, or
-  // level 1 on blocks of at least CT3D_MIN_CELLS interior cells, where it is the faster one
+  // level 1 where it is the faster one (ct3d_faster)
   bool ct3d_use = false;
   // 3-D adiabatic MHD and hydro, without per-cell options or user-defined sides:
   // idfx_cycle's stages ping-pong between Vc and Vc2, the last sweep writing the next state
@@ -259,6 +263,11 @@ SweepArgs sweep_args(idfx_ctx *c, int dir, double dt, const double *Vc, const do
     for (int d = 0; d < c->d.dim; d++) a.ext[d] = (d == dir) ? 0 : perp;
   }
   return a;
+}
+
+bool ct3d_faster(const idfx_ctx *c) {
+  return (long long)c->d.nx[0] * c->d.nx[1] * c->d.nx[2] >= CT3D_MIN_CELLS &&
+         ct3d_plan(c->g).fill >= CT3D_MIN_FILL;
 }
 
 // Learned limiter: interface weights of direction dir from Vc into the context's array
@@ -490,7 +499,7 @@ int idfx_ctx_create(const idfx_desc *desc, const double *dx1, const double *dx2,
   }
   if (st == IDFX_OK && d.mhd && d.dim == 3 && d.emf == IDFX_EMF_UCT_CONTACT && ops->ct3d) {
     c->fused3d_ok = c->fused3d_on = true;
-    c->ct3d_use = (long long)d.nx[0] * d.nx[1] * d.nx[2] >= CT3D_MIN_CELLS;
+    c->ct3d_use = ct3d_faster(c);
   }
   if (st == IDFX_OK && c->fused3d_ok && ops->prs_from_faces && !d.isothermal &&
       d.ntracer == 0 && !d.shock_flattening) {
@@ -1100,8 +1109,7 @@ int idfx_ctx_set_fusion(idfx_ctx *c, int level) {
   c->fused3d_on = level >= 1 && c->fused3d_ok;
   c->pp_hd_on = level >= 1 && c->pp_ok;
   c->xy_all = level == 2;
-  c->ct3d_use = c->fused3d_on &&
-                (level == 2 || (long long)c->d.nx[0] * c->d.nx[1] * c->d.nx[2] >= CT3D_MIN_CELLS);
+  c->ct3d_use = c->fused3d_on && (level == 2 || ct3d_faster(c));
   return IDFX_OK;
 }
 

@@ -308,33 +308,43 @@ hipError_t launch_evolve_b(const GridDesc &g, double *Vs, double *Vs0, const voi
   return hipSuccess;
 }
 
+// Tiles and k segments of k_ct3d: segments of kseg planes for the least rounds of the chip's 256
+// CUs (one block each) x (kseg + 2).  From 256 tiles on, 512 slots, which leads to fewer, longer
+// segments: the XCDs then work near one plane (512^3, 468 tiles: 5.2 against 5.6 ms;
+// 203x150x97, 64 tiles, with 512: 161 against 147 us).
+struct Ct3dPlan {
+  int nti, ntj, kseg, nseg;
+  double fill;  // faces the launch updates, over the faces its rounds of blocks have room for
+};
+inline Ct3dPlan ct3d_plan(const GridDesc &g) {
+  const int nfi = g.end[0] - g.beg[0] + 1, nfj = g.end[1] - g.beg[1] + 1, nfk = g.end[2] - g.beg[2] + 1;
+  Ct3dPlan p;
+  p.nti = (nfi + CT_TI - 1) / CT_TI;
+  p.ntj = (nfj + CT_TJ - 1) / CT_TJ;
+  const long long tiles = (long long)p.nti * p.ntj, slots = tiles >= 256 ? 512 : 256;
+  double best = 1e300;
+  for (int q = std::min(nfk, 4), n = 2; n > 1; q = n > 1 ? (nfk + n - 2) / (n - 1) : q) {
+    n = (nfk + q - 1) / q;  // next: the shortest segments that are fewer
+    const double cost = (double)((tiles * n + slots - 1) / slots) * (q + 2);
+    if (cost < best) {
+      best = cost;
+      p.kseg = q;
+      p.nseg = n;
+    }
+  }
+  p.fill = (double)nfi * nfj * nfk /
+           ((double)((tiles * p.nseg + 255) / 256) * (p.kseg + 2) * 256 * CT_TI * CT_TJ);
+  return p;
+}
 template <class C, typename T>
 hipError_t launch_ct3d(const GridDesc &g, const double *Vc, double *Vs, double *Vs0,
                        const void *emf, double dt, int mode, double wc, double w0,
                        hipStream_t s) {
   if constexpr (C::MHD && C::DIM == 3) {
-    // k segments of kseg planes: the least rounds of the chip's 256 CUs (one block each) x
-    // (kseg + 2).  From 256 tiles on, 512 slots, which leads to fewer, longer
-    // segments: the XCDs then work near one plane (512^3, 468 tiles: 5.2 against 5.6 ms;
-    // 203x150x97, 64 tiles, with 512: 161 against 147 us).
-    const int nfi = g.end[0] - g.beg[0] + 1, nfj = g.end[1] - g.beg[1] + 1;
-    const int nfk = g.end[2] - g.beg[2] + 1;
-    const int nti = (nfi + CT_TI - 1) / CT_TI, ntj = (nfj + CT_TJ - 1) / CT_TJ;
-    const long long tiles = (long long)nti * ntj;
-    const long long slots = tiles >= 256 ? 512 : 256;
-    int kseg = nfk;
-    double best = 1e300;
-    for (int q = std::min(nfk, 4); q <= nfk; q++) {
-      const double cost = (double)((tiles * ((nfk + q - 1) / q) + slots - 1) / slots) * (q + 2);
-      if (cost < best) {
-        best = cost;
-        kseg = q;
-      }
-    }
-    const int nseg = (nfk + kseg - 1) / kseg;
-    hipLaunchKernelGGL((k_ct3d<C, T>), dim3((unsigned)(tiles * nseg)), dim3((CT_TJ + 2) * 64), 0, s,
-                       g, Vc, Vs, Vs0, *static_cast<const EmfArrays<T> *>(emf), dt, mode, wc, w0,
-                       nti, ntj, kseg);
+    const Ct3dPlan p = ct3d_plan(g);
+    hipLaunchKernelGGL((k_ct3d<C, T>), dim3((unsigned)(p.nti * p.ntj * p.nseg)), dim3((CT_TJ + 2) * 64), 0,
+                       s, g, Vc, Vs, Vs0, *static_cast<const EmfArrays<T> *>(emf), dt, mode, wc, w0,
+                       p.nti, p.ntj, p.kseg);
     return hipGetLastError();
   }
   return hipErrorInvalidValue;

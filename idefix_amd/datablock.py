@@ -282,8 +282,9 @@ class DataBlock:
     def set_fusion(self, level):
         """Kernel schedule of cycle(): 0 = one kernel per reference step, 1 = the fused
         schedules (2-D MHD second half; 3-D ping-pong stage, with the fused CT kernel on
-        blocks of at least 5 * 2^19 interior cells), the default where supported, 2 = as 1 with
-        the fused 3-D CT and x-y sweep kernels at every size.  Results are identical."""
+        blocks of at least 5 * 2^19 interior cells whose extents fill its tiles), the default
+        where supported, 2 = as 1 with the fused 3-D CT and x-y sweep kernels at every size.
+        Results are identical."""
         capi.check(self._L.idfx_ctx_set_fusion(self.ctx, int(level)), "set_fusion")
 
     def set_profiling(self, on):

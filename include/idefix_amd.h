@@ -245,8 +245,8 @@ int idfx_cycle(idfx_ctx *ctx, int nstages, double cfl, double cfl_max_var, long 
  * with three-cell reconstructions (MHD with PPM: FP32 stencils from 2^25 cells on, and with
  * level 2), and the sweep of 1-D hydro fills the ghost zones itself.
  * In 3-D, level 1 takes the fused CT kernel on blocks of at least 5 * 2^19 interior cells
- * and k_corner_emf + k_evolve_b below (the faster choice on MI355X); level 2 takes the
- * fused CT kernel at every size.  All levels give identical interior cells, faces and Uc.
+ * whose extents fill its tiles, and k_corner_emf + k_evolve_b on others (the faster choice on
+ * MI355X); level 2 takes the fused CT kernel at every size.  All levels give identical interior cells, faces and Uc.
  * Returns IDFX_E_ARGS for levels 1 and 2 where the configuration supports none of these
  * schedules (2-D MHD, 3-D MHD, hydro), and for other levels. */
 int idfx_ctx_set_fusion(idfx_ctx *ctx, int level);

@@ -84,3 +84,30 @@ def test_short_directions_at_every_level(dim, n, mhd, bc, nstages):
     if mhd:
         for a, b in zip(interior_faces(g, g.download()[1]), interior_faces(h, h.download()[1])):
             assert (a == b).all()
+
+
+@pytest.mark.parametrize("n,fused", [((203, 150, 97), True), ((320, 200, 42), True), ((30, 300, 300), False),
+                                     ((16, 16, 10300), False), ((128, 128, 160), False), ((64, 60, 60), False)])
+def test_which_constrained_transport(n, fused):
+    """Level 1 takes the fused kernel where a block of enough cells fills its tiles; the other two
+    on narrow ones.  Every bit is that of the fused kernel, which level 2 takes."""
+    import torch
+    from idefix_amd.datablock import DataBlock
+    blocks = []
+    for level in (1, 2):
+        g = DataBlock(3, n, recon="plm", cfl=0.3, first_dt=1e-7)
+        gen = torch.Generator(device="cuda")
+        gen.manual_seed(3)
+        g.Vc.copy_(torch.rand(g.Vc.shape, generator=gen, device="cuda", dtype=torch.float64) * 0.3 + 0.5)
+        g.Vs.copy_(torch.rand(g.Vs.shape, generator=gen, device="cuda", dtype=torch.float64) * 0.2)
+        g.set_fusion(level)
+        g.set_profiling(True)
+        for _ in range(2):
+            g.cycle()
+        assert ("ct_fused" in g.region_times()) == (fused or level == 2)
+        blocks.append(g)
+    a, b = blocks
+    assert a.dt == b.dt
+    assert torch.equal(a.interior(a.Vc), b.interior(b.Vc))
+    for x, y in zip(interior_faces(a, a.Vs), interior_faces(b, b.Vs)):
+        assert torch.equal(x, y)
