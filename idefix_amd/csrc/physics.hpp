@@ -75,7 +75,7 @@ __device__ __forceinline__ float sqrt_(float a) { return sqrtf(a); }
 // quotient may differ).  In FP32 the same with 2^126 and 2^-102.  A subnormal denominator or a
 // quotient that overflows gives NaN: densities and their roots are normal numbers, sums and
 // differences with a wave speed in them are zero or at least a unit in its last place, and
-// PPM's curvatures are scaled (ppm_ratio).  Square roots are IEEE's throughout: outside
+// PPM's curvatures are scaled (ppm_cell).  Square roots are IEEE's throughout: outside
 // [2^-767, inf) a branch takes the compiler's.  An HLLD face has 20 quotients with 12
 // denominators and 6 square roots; whole cycles: Orszag-Tang 512^2 147 -> 139 us, 128^3 1209
 // -> 1164 us, turbulence 203x150x97 3009 -> 2950 us.
@@ -190,13 +190,6 @@ __device__ __forceinline__ T ppm_div(T a, T b) {
   if constexpr (FAST) return a * __builtin_amdgcn_rcpf(b);
   else return div_(a, b);
 }
-// a / b for 0 <= a <= b, where b may be subnormal: FP64 scales both by 2^128, since quot() needs
-// a denominator whose reciprocal is in range (without, NaN, and the cell stays unlimited).
-template <typename T, bool FAST>
-__device__ __forceinline__ T ppm_ratio(T a, T b) {
-  if constexpr (std::is_same<T, double>::value) return div_(a * 0x1p128, b * 0x1p128);
-  else return ppm_div<T, FAST>(a, b);
-}
 template <typename T, bool FAST = false>
 __device__ __forceinline__ T ppm_face(T vm1, T v0, T vp1, T vp2) {
   const T sum = v0 + vp1;
@@ -215,22 +208,26 @@ template <typename T>
 struct PpmStates {
   T l, r;
 };
+// FP64 holds the curvatures q and qf times 2^112, by the constants they are multiplied with anyway:
+// qf is the denominator of a quotient and, of values below 1e-307, subnormal (as it is, its
+// reciprocal overflows and the cell stays unlimited).
 template <typename T, bool FAST = false>
 __device__ __forceinline__ PpmStates<T> ppm_cell(T vm2, T vm1, T v0, T vp1, T vp2, T fl, T fr) {
+  constexpr T S = std::is_same<T, double>::value ? T(0x1p112) : T(1);
   const T dl = v0 - fl, dr = fr - v0;
   T l = fl, r = fr;
   if ((dr * dl <= T(0)) || (vm1 - v0) * (v0 - vp1) <= T(0)) {
-    const T qf = T(6.0) * sub2(fl + fr, v0);
+    const T qf = (S * T(6.0)) * sub2(fl + fr, v0);
     const T q0 = sub2(vm1 + vp1, v0);
     const T qp = sub2(v0 + vp2, vp1);
     const T qm = sub2(vm2 + v0, vm1);
     T q = fmn(flip(q0, qf), flip(qp, qf));
-    q = T(1.25) * fmn(flip(qm, qf), q);
+    q = (S * T(1.25)) * fmn(flip(qm, qf), q);
     q = fmx(fmn(fab(qf), q), T(0));
     const T qmax = fmx(fmx(fab(vm1), fab(v0)), fab(vp1));
     // q and qf carry the same sign: the quotient of their magnitudes
     T rho = 0;
-    if (fab(qf) > T(1e-12) * qmax) rho = ppm_ratio<T, FAST>(q, fab(qf));
+    if (fab(qf) > (S * T(1e-12)) * qmax) rho = ppm_div<T, FAST>(q, fab(qf));
     if (rho <= (T(1.0) - T(1e-12))) {
       l = v0 - rho * dl;
       r = v0 + rho * dr;
