@@ -1484,12 +1484,12 @@ __device__ __forceinline__ void evolve_face_pre(double *Vs, double *Vs0, unsigne
 //
 // The kernel is bound by HBM: 139 B a cell it cannot do without (3.9 ms at 512^3 at the
 // copy rate).  Tiles follow each other along x, then y, so that the tiles an XCD works on at
-// a time share their edge columns' cache lines and halo rows in its L2.  5.2 ms at 512^3 and
-// 147 us at 203x150x97; with every lane loading all four cells and the face data around its
-// edge, and tiles following each other along y, 7.6 ms and 208 us.
+// a time share their edge columns' cache lines and halo rows in its L2.  5.7 ms at 512^3 and
+// 148 us at 203x150x97 in whole cycles; with every lane loading all four cells and the face data
+// around its edge, and tiles following each other along y, 7.6 ms and 208 us.
 //
-// Tile of k_ct3d: faces per block in i and j (512^3 FP64, 8 waves of 62 x 6: 5.5 ms, 12
-// waves: 5.2 ms, 16 waves, which must fit 128 VGPRs: 5.9 ms)
+// Tile of k_ct3d: faces per block in i and j (512^3 FP64, its first stage, 8 waves of 62 x 6: 5.5 ms,
+// 12 waves: 5.2 ms, 16 waves, which must fit 128 VGPRs: 5.9 ms)
 constexpr int CT_TI = 62, CT_TJ = 10;
 template <class C, typename T>
 __global__ __launch_bounds__((CT_TJ + 2) * 64, 3) void k_ct3d(GridDesc g, const double *Vc, double *Vs,

@@ -198,7 +198,7 @@ hipError_t launch_sweep_xy(const GridDesc &g, const SweepArgs &a, int xflags, co
 // 3468 us, PPM 3473, 3874; 64^3 86, 96 and 130, 137.  MHD 256^3 PLM 6989, 7633 (FP32 stencils
 // 6116, 7017), 32^3 97, 104.  Roe's MHD solver has no registers to spare.  MHD with PPM is
 // bound by instruction issue, which the lanes without a cell add to: in FP64 it keeps its sweeps
-// (203x150x97 2534, 2480 us; 512^3 the same), and with FP32 stencils it takes one kernel where the
+// (203x150x97 2534, 2480 us; 512^3 92.4, 90.9 ms), and with FP32 stencils it takes one kernel where the
 // passes it saves go to memory (512x512x256 27.2, 28.5 ms; 384^3 35.0, 36.1; but 203x150x97
 // 2026, 1963 us and 256^3 the same).
 template <class C, typename T>
@@ -310,7 +310,7 @@ hipError_t launch_evolve_b(const GridDesc &g, double *Vs, double *Vs0, const voi
 
 // Tiles and k segments of k_ct3d: segments of kseg planes for the least rounds of the chip's 256
 // CUs (one block each) x (kseg + 2).  From 256 tiles on, 512 slots, which leads to fewer, longer
-// segments: the XCDs then work near one plane (512^3, 468 tiles: 5.2 against 5.6 ms;
+// segments: the XCDs then work near one plane (512^3, 468 tiles, first stage: 5.2 against 5.6 ms;
 // 203x150x97, 64 tiles, with 512: 161 against 147 us).
 struct Ct3dPlan {
   int nti, ntj, kseg, nseg;

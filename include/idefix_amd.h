@@ -224,7 +224,9 @@ int idfx_stage(idfx_ctx *ctx, int stage, int nstages, double dt, double cfl, dou
  * the ghost zones hold the boundary values of an earlier stage, which the next stage's
  * boundary fill rewrites before any use, and the corner (2-D also y-face) EMF scratch
  * arrays are not written.  The first RK3 cycle on these schedules allocates one more state array
- * (2-D MHD: and face array). */
+ * (2-D MHD: and face array).  A block with a reflecting side in a direction shorter than its ghost
+ * zone, whose fill mirrors ghost cells of the fill before it, is updated in place, as at level 0.
+ * Returns once *dt is known; the last stage may still run on the stream. */
 int idfx_cycle(idfx_ctx *ctx, int nstages, double cfl, double cfl_max_var, long ncycles,
                double *t, double *dt, double *Vc, double *Vs, double *Uc, double *InvDt,
                void *stream);
@@ -246,7 +248,8 @@ int idfx_cycle(idfx_ctx *ctx, int nstages, double cfl, double cfl_max_var, long 
  * level 2), and the sweep of 1-D hydro fills the ghost zones itself.
  * In 3-D, level 1 takes the fused CT kernel on blocks of at least 5 * 2^19 interior cells
  * whose extents fill its tiles, and k_corner_emf + k_evolve_b on others (the faster choice on
- * MI355X); level 2 takes the fused CT kernel at every size.  All levels give identical interior cells, faces and Uc.
+ * MI355X); level 2 takes the fused CT kernel at every size.  All levels give identical
+ * interior cells, faces and Uc.
  * Returns IDFX_E_ARGS for levels 1 and 2 where the configuration supports none of these
  * schedules (2-D MHD, 3-D MHD, hydro), and for other levels. */
 int idfx_ctx_set_fusion(idfx_ctx *ctx, int level);
@@ -299,11 +302,12 @@ int idfx_ctx_region_times(idfx_ctx *ctx, double *ms, long *count, int n);
  * high-resolution runs. */
 typedef struct idfx_mlp idfx_mlp;
 int idfx_mlp_param_count(void);
-/* Training state (FP32 parameters, Adam moments, activations for batches up to
+/* Training state (FP32 parameters, Adam moments, gradients per block of batches up to
  * max_batch rows).  Allocates device memory. */
 int idfx_mlp_create(int max_batch, idfx_mlp **out);
 int idfx_mlp_destroy(idfx_mlp *h);
-/* Host arrays of idfx_mlp_param_count() floats; set_params also resets Adam. */
+/* Host arrays of idfx_mlp_param_count() floats; set_params also resets Adam.  Both wait for the
+ * device: steps on any stream come before them. */
 int idfx_mlp_set_params(idfx_mlp *h, const float *params);
 int idfx_mlp_get_params(idfx_mlp *h, float *params);
 /* X: device [B][72] rows: the 48 features, the interface's 16 PPM weights and 8 loss
@@ -318,7 +322,8 @@ int idfx_mlp_train_step(idfx_mlp *h, const float *X, const float *tau, int B, fl
                         void *stream);
 int idfx_mlp_loss(idfx_mlp *h, double *loss, void *stream);
 /* Loads packed FP32 parameters (host) into an IDFX_RECON_MLP context as BF16 for MFMA
- * inference; params == NULL unloads them (every interface then takes the PPM weights). */
+ * inference; params == NULL unloads them (every interface then takes the PPM weights).  Waits for
+ * the device: stages under way keep the parameters they started with. */
 int idfx_ctx_set_mlp_params(idfx_ctx *ctx, const float *params);
 /* Interface weights of direction dir for the faces beg..end along dir (every transverse
  * index) from Vc, into W (device float [16][np_tot cells], or the context's own array
